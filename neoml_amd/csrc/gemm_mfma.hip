@@ -29,7 +29,7 @@
 // four consecutive k values  k0 + 4*half .. +3  with a single 128-bit LDS read and feeds them to four MFMAs.
 // MFMA j of a group therefore reduces over k = {k0 + j, k0 + 4 + j}; both operands use the same permutation of
 // k, which is all the dot product needs.
-#include "common.h"
+#include "gemm.h"
 #include <math.h>
 #include <map>
 #include <mutex>
@@ -38,100 +38,6 @@
 #include <vector>
 
 namespace nh {
-
-typedef float f32x16 __attribute__( ( ext_vector_type( 16 ) ) );
-
-// AM_Conv1x1 runs the same code as AM_Conv; the separate value gives 1x1 convolutions their own kernel symbols, so
-// that profiles tell them apart from the 3x3 ones
-// AM_ConvRows serves channel counts that are not a multiple of 4 (grey and RGB inputs): the reduction index runs
-// over Fh filter rows of RowPitch = ceil4( Fw * Cin ) values each. The Fw * Cin values that one filter row meets are
-// contiguous in a channels-last image (no dilation along the width), so they are fetched as 128-bit runs however
-// Cin divides; the 1-3 padding values per row are masked to zero on both operands.
-// AM_ConvClasses: the gradient by the input of a strided convolution, one stride-1 convolution per residue class of the
-// input pixels (blockIdx.y = class): AM_Conv whose geometry, filter and output rows come from args.Class[class].
-// AM_ConvTaps: AM_Conv for channel counts that are a multiple of the K step, without the strided gradient's exact-division
-// test: a step never straddles two taps, the reduction ends on a step, and everything that is only needed otherwise is
-// compiled out of the loop ( the 3x3 convolutions of the image networks ).
-enum TAMode { AM_RowsK = 0, AM_RowsM = 1, AM_Conv = 2, AM_Conv1x1 = 3, AM_ConvRows = 4, AM_ConvClasses = 5, AM_ConvTaps = 6 };
-// BM_ConvN: B is the im2col view of an N,H,W,C image read N-major: row k = output pixel, column n = ( kh, kw, ci ).
-// With A = the gradient by the convolution's output read M-major this is the gradient by the filter.
-enum TBMode { BM_RowsK = 0, BM_RowsN = 1, BM_ConvN = 2 };
-
-// One residue class ( ( hi + pad ) mod stride, same along the width ) of the input pixels of a strided convolution. Only
-// the filter taps kh with kh * dilation in the same class reach its pixels, Fh x Fw of them, and through them the
-// class is a stride-1 convolution over the output gradient. Its result rows are the pixels
-// ( OutH0 + j * strideH, OutW0 + i * strideW ), j < Ho, i < Wo, of every image.
-struct CConvClass {
-	int K, Fh, Fw, PadH, PadW, Ho, Wo, M, OutH0, OutW0;
-	long long BOffset; // of the class's filter [N][Fh][Fw][Cin] inside B, in floats
-};
-
-constexpr int MaxConvClasses = 4;
-
-struct CMatMulArgs {
-	const float* A;
-	const float* B;
-	float* C;
-	const float* Bias; // per column n, may be null
-	int M, N, K;
-	int Lda, Ldb, Ldc;
-	long long BatchStrideA, BatchStrideB, BatchStrideC;
-	int Accumulate; // C += instead of C =
-	int SplitK;     // number of K slices (grid z); > 1: partial products are added to C with atomics
-	int StepsPerSplit;
-	int TilesM, TilesN;
-	// convolution geometry (AM_Conv only): A is the image, M = batch * Ho * Wo
-	int H, W, Cin, Ho, Wo, Fh, Fw, PadH, PadW, StrideH, StrideW, DilH, DilW;
-	int RowK, RowPitch; // AM_ConvRows: Fw * Cin and its round-up to a multiple of 4; K = Fh * RowPitch
-	int AFloats, BFloats; // AM_ConvRows: sizes of the image and of the filter, the limit of a 128-bit load that reads past a run
-	// AM_Conv as the gradient by the input of a strided convolution: the tap's source coordinate is
-	// ( ho * StrideH - PadH + kh * DilH ) / UpH and only exists where that division is exact (values <= 1: no division)
-	int UpH, UpW;
-	int ManySlices; // the reduction is far longer than the output is large: as many K slices as fill the device
-	// Tail mode (FullTiles > 0, grid z = 1): the first FullTiles workgroups compute one whole tile each; the workgroups
-	// behind them share the TailTiles remaining tiles, TailSplit slices of TailSteps K steps per tile, and meet in C
-	// through atomic adds like the K slices above
-	int FullTiles, TailTiles, TailSplit, TailSteps;
-	// K slices that meet without atomics (Partials != null): every slice leaves its accumulators in Partials
-	// [ sliced tile ][ slice ][ 4096 ] and counts itself in Counters[ sliced tile ]; the slice that counts last adds
-	// them up in slice order, runs the ordinary epilogue and sets the counter back to zero for the next launch.
-	float* Partials;
-	unsigned* Counters;
-	// AM_ConvClasses: the dense result is [images][OutH][OutW][Ldc], DenseM pixels in all
-	int OutH, OutW, OutUpH, OutUpW, DenseM;
-	CConvClass Class[MaxConvClasses];
-	// epilogue of the fused blocks: C = act( A * B + bias ) + Residual; Residual has C's layout, may be C itself
-	CFusedActivation Act;
-	const float* Residual;
-	// floor( 2^32 / divisor ) for the divisions of the prologue ( pixel -> image, row, column; workgroup -> tile ): a
-	// multiplication and one correction instead of the twenty-odd instructions of a division by a run-time value
-	unsigned WoMagic, HoMagic, TilesNMagic;
-	// size of C in bytes when its rows can be addressed by 32-bit offsets from its start ( 0: they cannot ): the
-	// epilogue then stores through a buffer descriptor of that size, which drops the rows of a last tile that lie
-	// beyond the matrix by itself
-	unsigned CBytes;
-};
-
-// floor( 2^32 / d ), capped: with it q = mulhi( x, magic ) is floor( x / d ) or one less for every x < 2^32
-inline unsigned divisionMagic( int d )
-{
-	return d <= 1 ? 0xFFFFFFFFu : static_cast<unsigned>( 0x100000000ULL / static_cast<unsigned>( d ) );
-}
-
-__device__ __forceinline__ void fastDivMod( int x, int d, unsigned magic, int& quotient, int& remainder )
-{
-	unsigned q = __umulhi( static_cast<unsigned>( x ), magic );
-	unsigned r = static_cast<unsigned>( x ) - q * static_cast<unsigned>( d );
-	const bool low = r >= static_cast<unsigned>( d );
-	quotient = static_cast<int>( low ? q + 1 : q );
-	remainder = static_cast<int>( low ? r - static_cast<unsigned>( d ) : r );
-}
-
-constexpr int Threads = 256;
-
-#ifndef NH_KSTEP
-#define NH_KSTEP 16
-#endif
 
 // KGROUPS == 2: the workgroup has two groups of 4 wavefronts; each group runs the whole pipeline on its own LDS buffers
 // over one half of the K steps of the tile, then the second group hands its accumulators to the first through LDS.
@@ -2499,6 +2405,9 @@ static int matMulNTMeeting( hipStream_t stream, const float* a, int lda, const f
 	}
 	const bool vec = isAligned16( a ) && isAligned16( b ) && K % 4 == 0 && lda % 4 == 0 && ldb % 4 == 0
 		&& strideA % 4 == 0 && strideB % 4 == 0 && fitsBuffer( M, lda, K ) && fitsBuffer( N, ldb, K );
+	if( fixedMeeting == nullptr && trySplitProduct( stream, args, false, batch, vec, &rc ) ) {
+		return rc;
+	}
 	if( fixedMeeting == nullptr && tryLongProduct( stream, args, batch, vec, &rc ) ) {
 		return rc;
 	}
@@ -2826,6 +2735,10 @@ int convImplicitGemm( hipStream_t stream, const nhConvDesc& d, const float* sour
 		return launchMatMul<AM_ConvRows, BM_RowsK>( stream, args, 1, true, fixedMeeting );
 	}
 	if( vec && d.channels % NH_KSTEP == 0 ) {
+		int rc = NH_OK;
+		if( fixedMeeting == nullptr && trySplitProduct( stream, args, true, 1, vec, &rc ) ) {
+			return rc;
+		}
 		return launchMatMul<AM_ConvTaps, BM_RowsK>( stream, args, 1, true, fixedMeeting );
 	}
 	return launchMatMul<AM_Conv, BM_RowsK>( stream, args, 1, vec, fixedMeeting );
@@ -3328,6 +3241,9 @@ int convBackwardData( hipStream_t stream, const nhConvDesc& d, const float* outp
 		&& fitsBuffer( 1, 0, static_cast<long long>( d.batch ) * d.resultHeight * d.resultWidth * d.filterCount )
 		&& fitsBuffer( d.channels, args.K, args.K );
 	if( vec && d.filterCount % NH_KSTEP == 0 && d.strideHeight == 1 && d.strideWidth == 1 ) {
+		if( trySplitProduct( stream, args, true, 1, vec, &rc ) ) {
+			return rc;
+		}
 		return launchMatMul<AM_ConvTaps, BM_RowsK>( stream, args, 1, true );
 	}
 	return launchMatMul<AM_Conv, BM_RowsK>( stream, args, 1, vec );

@@ -1,0 +1,528 @@
+// fp32 matrix products and convolutions on the bf16 matrix instructions, each operand as the sum of three bf16 values.
+//
+// An fp32 value is exactly hi + mid + lo, where hi is the value rounded to bf16, mid what is left rounded to bf16, and lo
+// the rest: 8 significant bits each, signs of their own. Of the nine products of two such sums the six down to 2^-16 of the
+// largest are multiplied; the three that are left out ( mid lo, lo mid, lo lo ) are below 2^-26 of it, under the rounding of
+// an fp32 product. A matrix instruction sums 16 such products into the fp32 accumulator, where the fp32 one sums 2: six
+// roundings of the accumulator per 16 k instead of eight.
+#include "gemm.h"
+#include <type_traits>
+
+namespace nh {
+
+typedef __bf16 bf16x2 __attribute__( ( ext_vector_type( 2 ) ) );
+typedef __bf16 bf16x8 __attribute__( ( ext_vector_type( 8 ) ) );
+typedef float f32x2 __attribute__( ( ext_vector_type( 2 ) ) );
+
+// values ( x, y ) -> their three bf16 parts, packed
+__device__ __forceinline__ void splitPair( float x, float y, unsigned& hi, unsigned& mid, unsigned& lo )
+{
+	const f32x2 v = { x, y };
+	const bf16x2 h = __builtin_convertvector( v, bf16x2 );
+	hi = __builtin_bit_cast( unsigned, h );
+	const f32x2 r = { x - __uint_as_float( hi << 16 ), y - __uint_as_float( hi & 0xffff0000u ) };
+	const bf16x2 m = __builtin_convertvector( r, bf16x2 );
+	mid = __builtin_bit_cast( unsigned, m );
+	const f32x2 q = { r.x - __uint_as_float( mid << 16 ), r.y - __uint_as_float( mid & 0xffff0000u ) };
+	lo = __builtin_bit_cast( unsigned, __builtin_convertvector( q, bf16x2 ) );
+}
+
+constexpr int SplitStep = 16; // k per matrix instruction and per step
+
+// C[M x N] = act( A * B^T + bias ) (+ C, + residual), A rows of K values or the im2col view of an image whose channel count
+// is a multiple of the step ( a step stays inside a filter tap ), B rows of K values.
+// What bounds it: the card's power. Bare matrix instructions on random operands run at 1600 - 1700 TFLOP/s with the clock
+// held down to 1.5 GHz, a sixth of which is what can be had here; each value that is split ( 5.5 vector instructions ),
+// stored and read again costs on top, so the tiles are as large as the registers allow: a wavefront reads 2 x 2 blocks of
+// fragments for 24 matrix instructions. Measured against the fp32 instructions ( 64 x 64 and 128 x 128 tiles ), us:
+// 8192 x 2048 x 512 132 -> 102 ( 169 TFLOP/s ), 8192 x 512 x 2048 123 -> 107, 8192 x 512 x 512 35.5 -> 31.4, 8192 x 1024 x 256
+// 40 -> 29.5, 3x3 convolutions of 64 x 56 x 56 x 64 120 -> 107, 64 x 28 x 28 x 128 108 -> 91.
+// Error against 64 bits ( 2-norm ) on these: 2.4e-7 to 7.2e-7 where sequential fp32 sums have 2.9e-7 to 8.5e-7.
+// WGM x WGN wavefronts, each MI x NI blocks of 32 x 32; SETS: register sets of operands on their way from memory ( steps of
+// lead ); WPE: wavefronts per SIMD the registers must leave room for; RAGGED: K is not a multiple of the step.
+template<int AMODE, int WGM, int WGN, int MI, int NI, int SETS, int WPE, bool RAGGED>
+__global__ __launch_bounds__( 64 * WGM * WGN, WPE )
+void splitProductKernel( const CMatMulArgs args )
+{
+	constexpr bool IsTaps = ( AMODE == AM_ConvTaps );
+	static_assert( IsTaps || AMODE == AM_RowsK, "operands that are K-major" );
+	constexpr int KS = SplitStep;
+	constexpr int T = 64 * WGM * WGN;
+	constexpr int BM = 32 * WGM * MI, BN = 32 * WGN * NI;
+	// A tile's k step in LDS: three planes ( hi, mid, lo ) of [32-row block][k half][row][8 values], the order in which the
+	// lanes of a matrix instruction take their 16 bytes. The rows of the second half are rotated by eight, so that the 32
+	// lanes that store together, 8 rows of 4 quads, meet every bank once.
+	constexpr int AUnits = BM * 4, BUnits = BN * 4; // quads of k: a quarter of a tile row's step
+	constexpr int ASlots = ( AUnits + T - 1 ) / T, BSlots = ( BUnits + T - 1 ) / T;
+	constexpr int Plane = ( BM + BN ) * 32; // bytes
+	__shared__ __attribute__( ( aligned( 16 ) ) ) unsigned char lds[2][3 * Plane];
+
+	const int tid = threadIdx.x;
+	const int lane = tid & 63;
+	const int wave = __builtin_amdgcn_readfirstlane( tid >> 6 );
+	const int waveM = wave / WGN, waveN = wave % WGN;
+	const int l32 = lane & 31, half = lane >> 5;
+
+	const int batch = blockIdx.y;
+	const int M = args.M, N = args.N, K = args.K;
+	const float* baseA = args.A + batch * args.BatchStrideA;
+	const float* baseB = args.B + batch * args.BatchStrideB;
+	float* C = args.C + batch * args.BatchStrideC;
+	const int totalSteps = ( K + KS - 1 ) / KS;
+
+	const int tile = xcdSwizzle( blockIdx.x, gridDim.x );
+	int tileM, tileN;
+	fastDivMod( tile, args.TilesN, args.TilesNMagic, tileM, tileN );
+	const int m0 = tileM * BM, n0 = tileN * BN;
+
+	// position of output pixel m's window in the image, of a row of A otherwise
+	struct CRow {
+		unsigned Base; // in floats, of tap ( 0, 0 ): unsigned arithmetic, it may lie in front of the image
+		int H0, W0;
+	};
+	auto rowOf = [&]( int m ) -> CRow {
+		CRow row;
+		if constexpr( IsTaps ) {
+			int t, wo, n, ho;
+			fastDivMod( m, args.Wo, args.WoMagic, t, wo );
+			fastDivMod( t, args.Ho, args.HoMagic, n, ho );
+			row.H0 = m < M ? ho * args.StrideH - args.PadH : -0x40000000;
+			row.W0 = wo * args.StrideW - args.PadW;
+			row.Base = static_cast<unsigned>( n * args.H * args.W * args.Cin )
+				+ ( static_cast<unsigned>( row.H0 ) * static_cast<unsigned>( args.W ) + static_cast<unsigned>( row.W0 ) ) * static_cast<unsigned>( args.Cin );
+		} else {
+			row.H0 = m < M ? 0 : -1;
+			row.W0 = 0;
+			row.Base = static_cast<unsigned>( m ) * static_cast<unsigned>( args.Lda );
+		}
+		return row;
+	};
+	// byte offset of a row's values from k = 0 ( of the tap ) on
+	auto rowOffset = [&]( const CRow& row, int kh, int kw ) -> unsigned {
+		if constexpr( IsTaps ) {
+			const int dh = kh * args.DilH, dw = kw * args.DilW; // ( scalar )
+			const unsigned tapFloats = ( static_cast<unsigned>( dh ) * static_cast<unsigned>( args.W ) + static_cast<unsigned>( dw ) )
+				* static_cast<unsigned>( args.Cin );
+			const bool ok = kh < args.Fh && static_cast<unsigned>( row.H0 + dh ) < static_cast<unsigned>( args.H )
+				&& static_cast<unsigned>( row.W0 + dw ) < static_cast<unsigned>( args.W );
+			return ok ? ( row.Base + tapFloats ) * 4u : OutOfRange;
+		} else {
+			return row.H0 < 0 ? OutOfRange : row.Base * 4u;
+		}
+	};
+
+	// ---- this thread's quads: quad tid % 4 of tile rows tid / 4 + i T / 4, four lanes cover the 64 bytes of a row's step
+	CRow rowA[ASlots];
+	unsigned offA[ASlots], offB[BSlots];
+	int tapCi = 0, tapKh = 0, tapKw = 0;
+	const unsigned quad = tid & 3;
+	const int tileRow = tid >> 2;
+	constexpr int RowsPerSlot = T / 4;
+#pragma unroll
+	for( int i = 0; i < ASlots; ++i ) {
+		const int row = tileRow + i * RowsPerSlot;
+		rowA[i] = rowOf( m0 + row );
+		if( AUnits % T != 0 && row >= BM ) {
+			rowA[i].H0 = -0x40000000;
+		}
+		rowA[i].Base += quad * 4u;
+		offA[i] = rowOffset( rowA[i], tapKh, tapKw );
+	}
+#pragma unroll
+	for( int i = 0; i < BSlots; ++i ) {
+		const int row = tileRow + i * RowsPerSlot;
+		const int n = n0 + row;
+		offB[i] = ( BUnits % T == 0 || row < BN ) && n < N
+			? ( static_cast<unsigned>( n ) * static_cast<unsigned>( args.Ldb ) + quad * 4u ) * 4u : OutOfRange;
+	}
+
+	float4 regA[SETS][ASlots], regB[SETS][BSlots];
+	// Requests the quads of a step. A step behind the last is asked of a descriptor of size zero ( zeros, no memory
+	// access ): every step runs the same code.
+	auto load = [&]( int step, int set ) {
+		const unsigned range = step < totalSteps ? BufferBytes : 0u;
+		const __amdgpu_buffer_rsrc_t bufA = __builtin_amdgcn_make_buffer_rsrc( const_cast<float*>( baseA ), 0, range, 0x00020000 );
+		const __amdgpu_buffer_rsrc_t bufB = __builtin_amdgcn_make_buffer_rsrc( const_cast<float*>( baseB ), 0, range, 0x00020000 );
+		const unsigned uniB = static_cast<unsigned>( step ) * ( KS * 4u );
+		const unsigned uniA = IsTaps ? static_cast<unsigned>( tapCi ) * 4u : uniB;
+		// the last step of a K that is not a multiple of the step ( it is one of 4 )
+		const bool masked = RAGGED && step * KS + static_cast<int>( quad ) * 4 >= K;
+#pragma unroll
+		for( int i = 0; i < ASlots; ++i ) {
+			regA[set][i] = bufferLoad4( bufA, masked ? OutOfRange : offA[i], uniA );
+		}
+#pragma unroll
+		for( int i = 0; i < BSlots; ++i ) {
+			regB[set][i] = bufferLoad4( bufB, masked ? OutOfRange : offB[i], uniB );
+		}
+		if constexpr( IsTaps ) {
+			tapCi += KS;
+			if( tapCi >= args.Cin ) {
+				tapCi = 0;
+				if( ++tapKw == args.Fw ) {
+					tapKw = 0;
+					++tapKh;
+				}
+#pragma unroll
+				for( int i = 0; i < ASlots; ++i ) {
+					offA[i] = rowOffset( rowA[i], tapKh, tapKw );
+				}
+			}
+		}
+	};
+	const int quadAt = static_cast<int>( quad >> 1 ) * 512 + static_cast<int>( quad & 1 ) * 8;
+	auto unitAt = [&]( int row ) -> int {
+		return ( row >> 5 ) * 1024 + quadAt + ( ( row + static_cast<int>( quad >> 1 ) * 8 ) & 31 ) * 16;
+	};
+	auto storeUnit = [&]( int buf, int at, const float4& v ) {
+		uint2 hi, mid, lo;
+		splitPair( v.x, v.y, hi.x, mid.x, lo.x );
+		splitPair( v.z, v.w, hi.y, mid.y, lo.y );
+		*reinterpret_cast<uint2*>( &lds[buf][at] ) = hi;
+		*reinterpret_cast<uint2*>( &lds[buf][at + Plane] ) = mid;
+		*reinterpret_cast<uint2*>( &lds[buf][at + 2 * Plane] ) = lo;
+	};
+	auto store = [&]( int buf, int set ) {
+#pragma unroll
+		for( int i = 0; i < ASlots; ++i ) {
+			if( AUnits % T == 0 || tileRow + i * RowsPerSlot < BM ) {
+				storeUnit( buf, unitAt( tileRow + i * RowsPerSlot ), regA[set][i] );
+			}
+		}
+#pragma unroll
+		for( int i = 0; i < BSlots; ++i ) {
+			if( BUnits % T == 0 || tileRow + i * RowsPerSlot < BN ) {
+				storeUnit( buf, BM * 32 + unitAt( tileRow + i * RowsPerSlot ), regB[set][i] );
+			}
+		}
+	};
+
+	f32x16 acc[MI][NI];
+	auto clear = [&]() {
+#pragma unroll
+		for( int mi = 0; mi < MI; ++mi ) {
+#pragma unroll
+			for( int ni = 0; ni < NI; ++ni ) {
+#pragma unroll
+				for( int r = 0; r < 16; ++r ) {
+					acc[mi][ni][r] = 0.f;
+				}
+			}
+		}
+	};
+	clear();
+
+	const int fragLane = half * 512 + ( ( l32 + half * 8 ) & 31 ) * 16;
+	const int fragA = waveM * MI * 1024 + fragLane, fragB = BM * 32 + waveN * NI * 1024 + fragLane;
+	struct CFrag {
+		bf16x8 A[3][MI], B[3][NI];
+	};
+	CFrag frag[2];
+	auto readFrag = [&]( int buf, CFrag& f ) {
+#pragma unroll
+		for( int p = 2; p >= 0; --p ) {
+#pragma unroll
+			for( int mi = 0; mi < MI; ++mi ) {
+				f.A[p][mi] = *reinterpret_cast<const bf16x8*>( &lds[buf][p * Plane + fragA + mi * 1024] );
+			}
+#pragma unroll
+			for( int ni = 0; ni < NI; ++ni ) {
+				f.B[p][ni] = *reinterpret_cast<const bf16x8*>( &lds[buf][p * Plane + fragB + ni * 1024] );
+			}
+		}
+	};
+	auto product = [&]( const CFrag& f, int pa, int pb ) {
+#pragma unroll
+		for( int mi = 0; mi < MI; ++mi ) {
+#pragma unroll
+			for( int ni = 0; ni < NI; ++ni ) {
+				acc[mi][ni] = __builtin_amdgcn_mfma_f32_32x32x16_bf16( f.A[pa][mi], f.B[pb][ni], acc[mi][ni], 0, 0, 0 );
+			}
+		}
+	};
+
+	// Step s multiplies the fragments that step s - 1 read. Under its matrix instructions the fragments of step s + 1 are read
+	// from LDS buffer ( s + 1 ) % 2 and the values of step s + 2 are split and stored to buffer s % 2, whose last readers
+	// were in step s - 1; one barrier ends the step. Reads, stores and vector instructions are dealt evenly over the step.
+	load( 0, 0 );
+	store( 0, 0 );
+	load( 1, 0 );
+	store( 1, 0 );
+	load( 2, 0 );
+	if constexpr( SETS == 2 ) {
+		load( 3, 1 );
+	}
+	__syncthreads();
+	readFrag( 0, frag[0] );
+	__syncthreads();
+	constexpr int Products = 6 * MI * NI; // matrix instructions of a step
+	constexpr int SplitVector = ( ASlots + BSlots ) * 24; // vector instructions of a step's quads, about
+	auto step = [&]( int s, auto curOf ) {
+		constexpr int cur = decltype( curOf )::value, nxt = cur ^ 1;
+		constexpr int set = SETS == 2 ? cur : 0;
+		__builtin_amdgcn_sched_barrier( 0 );
+		readFrag( nxt, frag[nxt] );
+		store( cur, set );
+		product( frag[cur], 2, 0 );
+		product( frag[cur], 0, 2 );
+		product( frag[cur], 1, 1 );
+		product( frag[cur], 1, 0 );
+		product( frag[cur], 0, 1 );
+		product( frag[cur], 0, 0 );
+#pragma unroll
+		for( int i = 0; i < Products; ++i ) {
+			__builtin_amdgcn_sched_group_barrier( 0x008, 1, 0 ); // a matrix instruction
+			__builtin_amdgcn_sched_group_barrier( 0x100, ( 3 * ( MI + NI ) + Products - 1 ) / Products, 0 ); // LDS reads
+			__builtin_amdgcn_sched_group_barrier( 0x002, ( SplitVector + Products - 1 ) / Products, 0 ); // vector instructions under it
+			__builtin_amdgcn_sched_group_barrier( 0x200, ( 3 * ( ASlots + BSlots ) + Products - 1 ) / Products, 0 ); // LDS stores
+		}
+		__builtin_amdgcn_sched_barrier( 0 );
+		load( s + 2 + SETS, set );
+		__syncthreads();
+	};
+	int s = 0;
+	for( ; s + 1 < totalSteps; s += 2 ) {
+		step( s, std::integral_constant<int, 0>() );
+		step( s + 1, std::integral_constant<int, 1>() );
+	}
+	if( s < totalSteps ) {
+		step( s, std::integral_constant<int, 0>() );
+	}
+
+	// An operand that is infinite, NaN or rounds to infinity has no finite parts: infinity - infinity makes all it meets NaN.
+	// And parts of operands below 2^-108 fall under the smallest normal bf16 value. Either shows in the accumulators ( not
+	// finite; not zero but tiny ): such a wavefront multiplies its blocks again with the fp32 instructions, operands straight
+	// from memory.
+	float notFinite = 0.f, least = __builtin_inff();
+#pragma unroll
+	for( int mi = 0; mi < MI; ++mi ) {
+#pragma unroll
+		for( int ni = 0; ni < NI; ++ni ) {
+#pragma unroll
+			for( int r = 0; r < 16; ++r ) {
+				notFinite = __builtin_fmaf( acc[mi][ni][r], 0.f, notFinite );
+				least = fminf( least, fabsf( acc[mi][ni][r] ) );
+			}
+		}
+	}
+	constexpr float Tiny = 0x1p-80f;
+	bool again = notFinite != notFinite;
+	if( __builtin_amdgcn_ballot_w64( least < Tiny ) != 0 ) {
+#pragma unroll
+		for( int mi = 0; mi < MI; ++mi ) {
+#pragma unroll
+			for( int ni = 0; ni < NI; ++ni ) {
+#pragma unroll
+				for( int r = 0; r < 16; ++r ) {
+					again = again || ( acc[mi][ni][r] != 0.f && fabsf( acc[mi][ni][r] ) < Tiny );
+				}
+			}
+		}
+	}
+	if( __builtin_amdgcn_ballot_w64( again ) != 0 ) {
+		clear();
+		const __amdgpu_buffer_rsrc_t bufA = makeBuffer( baseA ), bufB = makeBuffer( baseB );
+		#pragma unroll 1
+		for( int k0 = 0; k0 < K; k0 += 8 ) {
+			int kh = 0, kw = 0, ci = k0;
+			if( IsTaps ) {
+				const int tap = k0 / args.Cin;
+				ci = k0 - tap * args.Cin;
+				kh = tap / args.Fw;
+				kw = tap - kh * args.Fw;
+			}
+			const bool inK = k0 + half * 4 < K;
+			float4 a[MI], b[NI];
+#pragma unroll
+			for( int mi = 0; mi < MI; ++mi ) {
+				const unsigned off = rowOffset( rowOf( m0 + ( waveM * MI + mi ) * 32 + l32 ), kh, kw );
+				a[mi] = bufferLoad4( bufA, inK && off != OutOfRange ? off + static_cast<unsigned>( ci + half * 4 ) * 4u : OutOfRange );
+			}
+#pragma unroll
+			for( int ni = 0; ni < NI; ++ni ) {
+				const int n = n0 + ( waveN * NI + ni ) * 32 + l32;
+				b[ni] = bufferLoad4( bufB, inK && n < N
+					? ( static_cast<unsigned>( n ) * static_cast<unsigned>( args.Ldb ) + static_cast<unsigned>( k0 + half * 4 ) ) * 4u : OutOfRange );
+			}
+#pragma unroll
+			for( int mi = 0; mi < MI; ++mi ) {
+#pragma unroll
+				for( int ni = 0; ni < NI; ++ni ) {
+					acc[mi][ni] = __builtin_amdgcn_mfma_f32_32x32x2f32( a[mi].x, b[ni].x, acc[mi][ni], 0, 0, 0 );
+					acc[mi][ni] = __builtin_amdgcn_mfma_f32_32x32x2f32( a[mi].y, b[ni].y, acc[mi][ni], 0, 0, 0 );
+					acc[mi][ni] = __builtin_amdgcn_mfma_f32_32x32x2f32( a[mi].z, b[ni].z, acc[mi][ni], 0, 0, 0 );
+					acc[mi][ni] = __builtin_amdgcn_mfma_f32_32x32x2f32( a[mi].w, b[ni].w, acc[mi][ni], 0, 0, 0 );
+				}
+			}
+		}
+	}
+
+	// C through a buffer descriptor that ends with the matrix: rows beyond it are dropped by the range check. A row adds a
+	// multiple of the row pitch to the lane's offset, in a scalar register where the tile lies inside the matrix.
+	const __amdgpu_buffer_rsrc_t bufC = __builtin_amdgcn_make_buffer_rsrc( C, 0, args.CBytes, 0x00020000 );
+	const float* residual = args.Residual != nullptr ? args.Residual + batch * args.BatchStrideC : nullptr;
+	const float actParam = withParam( args.Act ).Param; // ( the threshold may live in device memory )
+	const float reluTop = actParam > 0.f ? actParam : __builtin_inff();
+	const unsigned pitchBytes = static_cast<unsigned>( args.Ldc ) * 4u;
+	auto write = [&]( auto typeOf, auto extraOf, auto insideOf ) {
+		constexpr int Type = decltype( typeOf )::value;
+		constexpr bool Extra = decltype( extraOf )::value; // accumulate and / or residual
+		constexpr bool Inside = decltype( insideOf )::value;
+#pragma unroll
+		for( int ni = 0; ni < NI; ++ni ) {
+			const int n = n0 + ( waveN * NI + ni ) * 32 + l32;
+			const float bias = ( args.Bias != nullptr && n < N ) ? args.Bias[n] : 0.f;
+			const int rowBase = m0 + waveM * MI * 32 + half * 4;
+			const unsigned laneOffset = n < N ? static_cast<unsigned>( rowBase ) * pitchBytes + static_cast<unsigned>( n ) * 4u : OutOfRange;
+#pragma unroll
+			for( int mi = 0; mi < MI; ++mi ) {
+#pragma unroll
+				for( int r = 0; r < 16; ++r ) {
+					const int row = mi * 32 + ( r >> 2 ) * 8 + ( r & 3 );
+					// ( an offset that was out of range stays so: what is added is below 2^31 )
+					const unsigned groupOffset = laneOffset + static_cast<unsigned>( row & ~3 ) * pitchBytes;
+					const unsigned rowBytes = static_cast<unsigned>( row & 3 ) * pitchBytes;
+					float v = acc[mi][ni][r] + bias;
+					if constexpr( Extra ) {
+						const bool ok = n < N && rowBase + row < M;
+						const long long at = static_cast<long long>( rowBase + row ) * args.Ldc + n;
+						if( args.Accumulate && ok ) {
+							v += C[at];
+						}
+						v = applyActivationOf<Type>( v, reluTop );
+						if( residual != nullptr && ok ) {
+							v += residual[at];
+						}
+					} else {
+						v = applyActivationOf<Type>( v, reluTop );
+					}
+					if constexpr( Inside ) {
+						__builtin_amdgcn_raw_buffer_store_b32( __float_as_uint( v ), bufC, groupOffset, rowBytes, 0 );
+					} else {
+						__builtin_amdgcn_raw_buffer_store_b32( __float_as_uint( v ), bufC, groupOffset + rowBytes, 0, 0 );
+					}
+				}
+			}
+		}
+	};
+	auto writeAs = [&]( auto typeOf ) {
+		if( args.Accumulate || residual != nullptr ) {
+			write( typeOf, std::true_type(), std::false_type() );
+		} else if( m0 + BM <= M ) {
+			write( typeOf, std::false_type(), std::true_type() );
+		} else {
+			write( typeOf, std::false_type(), std::false_type() );
+		}
+	};
+	if( args.Act.Type == NH_ACT_RELU ) {
+		writeAs( std::integral_constant<int, NH_ACT_RELU>() );
+	} else if( args.Act.Type == NH_ACT_HSWISH ) {
+		writeAs( std::integral_constant<int, NH_ACT_HSWISH>() );
+	} else {
+		writeAs( std::integral_constant<int, NH_ACT_NONE>() );
+	}
+}
+
+// What a launch is expected to take, in microseconds, and its tiles.
+struct CSplitPlan {
+	double Cost;
+	int TilesM, TilesN;
+};
+
+// The shapes, as measured on products and 3x3 convolutions of 4 to 18 GFLOP with all compute units at work. The card holds
+// its power limit by lowering the clock, so these are times of a whole device: a step of 256 x 128 tiles on every compute
+// unit 1.25 us ( one workgroup of eight wavefronts each ), of 128 x 128 tiles 0.8 us with one workgroup to a unit and 1.3 us
+// with two, of 128 x 64 tiles 0.5 us with one and 0.49 us for each of up to four, of 256 x 64 tiles 0.94 us each.
+enum TSplitShape { SS_256x128, SS_128x128, SS_256x64, SS_128x64, SS_Count };
+
+static CSplitPlan splitPlan( int shape, const CMatMulArgs& a, int batch )
+{
+	const int bm = shape == SS_256x128 || shape == SS_256x64 ? 256 : 128;
+	const int bn = shape == SS_256x128 || shape == SS_128x128 ? 128 : 64;
+	const double steps = ceilDiv( a.K, SplitStep );
+	CSplitPlan plan = {};
+	plan.TilesM = ceilDiv( a.M, bm );
+	plan.TilesN = ceilDiv( a.N, bn );
+	const long long tiles = static_cast<long long>( plan.TilesM ) * plan.TilesN * batch;
+	const double deepest = static_cast<double>( ( tiles + 255 ) / 256 );
+	const double overhead = 6;
+	switch( shape ) {
+		case SS_256x128: plan.Cost = deepest * ( steps * 1.25 + overhead ); break;
+		case SS_128x128: plan.Cost = deepest <= 1 ? steps * 0.8 + overhead : deepest * ( steps * 0.65 + 3 ) + 3; break;
+		case SS_256x64: plan.Cost = deepest * ( steps * 0.94 + 3 ) + 3; break;
+		default: plan.Cost = deepest <= 1 ? steps * 0.5 + overhead : deepest * ( steps * 0.49 + 1.5 ) + 3; break;
+	}
+	return plan;
+}
+
+template<int AMODE, int WGM, int WGN, int MI, int NI, int SETS, int WPE>
+static void launchSplit( hipStream_t stream, const CMatMulArgs& args, const dim3& grid )
+{
+	const dim3 threads( 64 * WGM * WGN );
+	if constexpr( AMODE == AM_RowsK ) {
+		if( args.K % SplitStep != 0 ) {
+			hipLaunchKernelGGL( ( splitProductKernel<AMODE, WGM, WGN, MI, NI, SETS, WPE, true> ), grid, threads, 0, stream, args );
+			return;
+		}
+	}
+	hipLaunchKernelGGL( ( splitProductKernel<AMODE, WGM, WGN, MI, NI, SETS, WPE, false> ), grid, threads, 0, stream, args );
+}
+
+template<int AMODE>
+static void launchSplitShape( hipStream_t stream, int shape, const CMatMulArgs& args, const dim3& grid )
+{
+	switch( shape ) {
+		case SS_256x128: launchSplit<AMODE, 4, 2, 2, 2, 1, 2>( stream, args, grid ); break;
+		case SS_128x128: launchSplit<AMODE, 2, 2, 2, 2, 2, 2>( stream, args, grid ); break;
+		case SS_256x64: launchSplit<AMODE, 4, 1, 2, 2, 1, 2>( stream, args, grid ); break;
+		default: launchSplit<AMODE, 2, 2, 2, 1, 1, 4>( stream, args, grid ); break;
+	}
+}
+
+bool trySplitProduct( hipStream_t stream, const CMatMulArgs& given, bool convolution, int batch, bool vec, int* rc )
+{
+	CMatMulArgs args = given;
+	if( !vec || batch > 65535 || args.M < 128 || args.N < 48 || args.K < 128 || ( convolution && args.Cin % SplitStep != 0 ) ) {
+		return false;
+	}
+	const long long cBytes = ( static_cast<long long>( args.M - 1 ) * args.Ldc + args.N ) * 4;
+	if( args.Ldc < args.N || cBytes >= 0x7fffff00LL || args.Ldc > 0x1000000 ) {
+		return false;
+	}
+	int shape = 0;
+	CSplitPlan plan = {};
+	for( int s = 0; s < SS_Count; ++s ) {
+		const CSplitPlan p = splitPlan( s, args, batch );
+		if( s == 0 || p.Cost < plan.Cost ) {
+			plan = p;
+			shape = s;
+		}
+	}
+	// the fp32 instructions: 120 TFLOP/s at best on such sizes, and 4 us
+	const double flops = 2.0 * args.M * args.N * args.K * batch;
+	if( plan.Cost > 0.95 * ( flops / 120e6 + 4 ) ) {
+		return false;
+	}
+	args.TilesM = plan.TilesM;
+	args.TilesN = plan.TilesN;
+	args.TilesNMagic = divisionMagic( args.TilesN );
+	args.WoMagic = divisionMagic( args.Wo );
+	args.HoMagic = divisionMagic( args.Ho );
+	args.CBytes = static_cast<unsigned>( cBytes );
+	const dim3 grid( static_cast<unsigned>( plan.TilesM ) * plan.TilesN, batch );
+	if( convolution ) {
+		launchSplitShape<AM_ConvTaps>( stream, shape, args, grid );
+	} else {
+		launchSplitShape<AM_RowsK>( stream, shape, args, grid );
+	}
+	const hipError_t err = hipGetLastError();
+	if( err != hipSuccess ) {
+		setLastError( "split product: launch failed: %s", hipGetErrorString( err ) );
+		*rc = NH_ERR_HIP;
+	} else {
+		*rc = NH_OK;
+	}
+	return true;
+}
+
+} // namespace nh

@@ -1,0 +1,101 @@
+"""Products and convolutions that run on the bf16 matrix instructions with operands split in three, against 64 bits."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def hip():
+    import nhtest
+    return nhtest.Hip()
+
+
+def _check(got, a, b, k):
+    """a [M,K], b [N,K] in 64 bits. At most 6 roundings of the accumulator per 16 k, of partial sums below sum |a b|, and a
+    few for the dropped products and the epilogue."""
+    want = a @ b.T
+    bound = (6 * k / 16 + 8) * 2.0 ** -24 * (a.abs() @ b.abs().T)
+    excess = ((got.double() - want).abs() - bound).max().item()
+    assert excess <= 0, excess
+
+
+# the last tile row and column partly and all but empty, K that ends in each quad of a step, an odd pitch of C
+PRODUCTS = [(8192, 512, 512), (8129, 511, 516), (8065, 513, 264), (4097, 1025, 1004), (65537, 64, 200), (20000, 192, 392)]
+
+
+@pytest.mark.parametrize("m,n,k", PRODUCTS)
+def test_products(hip, m, n, k):
+    torch = hip.torch
+    g = torch.Generator(device=hip.dev).manual_seed(m + n + k)
+    a = torch.randn(m, k, generator=g, device=hip.dev)
+    b = torch.randn(n, k, generator=g, device=hip.dev)
+    c = torch.full((m, n), 7.0, device=hip.dev)
+    hip.call("nhMultiplyMatrixByTransposedMatrix", hip.p(a), m, k, k, hip.p(b), n, k, hip.p(c), n, c.numel())
+    _check(c, a.double(), b.double(), k)
+
+
+def _patches(torch, x, fh, fw, pad, stride):
+    x = torch.nn.functional.pad(x, (0, 0, pad, pad, pad, pad))
+    p = x.unfold(1, fh, stride).unfold(2, fw, stride)  # n, ho, wo, c, fh, fw
+    return p.permute(0, 1, 2, 4, 5, 3).reshape(-1, fh * fw * x.shape[3])
+
+
+# odd image sizes, windows over every edge, a filter other than 3x3, stride 2, a last tile row that is partly empty
+CONVOLUTIONS = [(64, 28, 28, 128, 128, 3, 1, 1), (33, 29, 31, 144, 130, 3, 1, 1), (64, 33, 30, 128, 256, 3, 1, 2), (16, 41, 37, 80, 96, 5, 2, 1),
+                (19, 53, 57, 64, 64, 3, 1, 1), (64, 14, 14, 256, 256, 3, 1, 1), (5, 3, 700, 256, 256, 3, 1, 1), (64, 7, 7, 512, 512, 3, 1, 1)]
+
+
+@pytest.mark.parametrize("n,h,w,cin,cout,f,pad,stride", CONVOLUTIONS)
+def test_convolutions(hip, n, h, w, cin, cout, f, pad, stride):
+    torch = hip.torch
+    g = torch.Generator(device=hip.dev).manual_seed(n * h * w)
+    x = torch.randn(n, h, w, cin, generator=g, device=hip.dev)
+    filt = torch.randn(cout, f, f, cin, generator=g, device=hip.dev)
+    bias = torch.randn(cout, generator=g, device=hip.dev)
+    d = hip.conv_desc(n, h, w, cin, cout, f, f, pad, pad, stride, stride)
+    y = torch.empty(n * d.resultHeight * d.resultWidth, cout, device=hip.dev)
+    import ctypes
+    hip.call("nhBlobConvolution", ctypes.byref(d), hip.p(x), hip.p(filt), hip.p(bias), hip.p(y))
+    a = _patches(torch, x.double(), f, f, pad, stride)
+    one = torch.ones(a.shape[0], 1, device=hip.dev, dtype=torch.float64)
+    _check(y, torch.cat([a, one], 1), torch.cat([filt.double().reshape(cout, -1), bias.double()[:, None]], 1), f * f * cin)
+
+
+def test_values_without_finite_parts(hip):
+    """Infinity, NaN, values that round to infinity in bf16, a product that overflows, values whose parts are too small:
+    what the fp32 instructions give, and the rows beside them untouched."""
+    torch = hip.torch
+    m, n, k = 8192, 512, 512
+    g = torch.Generator(device=hip.dev).manual_seed(5)
+    a = torch.randn(m, k, generator=g, device=hip.dev)
+    b = torch.randn(n, k, generator=g, device=hip.dev)
+    big = float(np.finfo(np.float32).max)
+    a[5, 7] = float("inf")
+    a[200, 0] = float("nan")
+    a[1000, :] = 0.0
+    a[1000, 3] = big
+    b[:, 3] = torch.where(b[:, 3].abs() < 1, b[:, 3], 0.5)
+    b[17, :] = 1.0
+    a[3000, :] = a[3000, :] * 1e-34
+    a[5000, :] = 1e38
+    a[8191, 511] = -float("inf")
+    b[100, 7] = 0.0
+    c = torch.empty(m, n, device=hip.dev)
+    hip.call("nhMultiplyMatrixByTransposedMatrix", hip.p(a), m, k, k, hip.p(b), n, k, hip.p(c), n, c.numel())
+    want = a.double() @ b.double().T
+    special = [5, 200, 5000, 8191]
+    plain = torch.ones(m, dtype=torch.bool, device=hip.dev)
+    plain[special] = False
+    plain[3000] = False
+    _check(c[plain], a[plain].double(), b.double(), k)
+    _check(c[3000:3001] * 2.0 ** 100, a[3000:3001].double() * 2.0 ** 100, b.double(), k)
+    for row in (5, 200, 8191):
+        assert torch.equal(c[row].isnan(), want[row].isnan()), row
+        assert torch.equal(c[row].isinf(), want[row].isinf()), row
+        assert torch.equal(c[row][c[row].isinf()].double(), want[row][want[row].isinf()]), row
+    # sums of 512 values up to 3e38: those far beyond the range are infinite, with their sign ( or NaN where partial sums of
+    # both signs left it ), none that stays well inside its running range may be anything but close
+    over = want[5000].abs() > 4 * big
+    assert not torch.isfinite(c[5000][over]).any()
+    assert c[5000, 17] == float("inf")
