@@ -3241,9 +3241,6 @@ int convBackwardData( hipStream_t stream, const nhConvDesc& d, const float* outp
 		&& fitsBuffer( 1, 0, static_cast<long long>( d.batch ) * d.resultHeight * d.resultWidth * d.filterCount )
 		&& fitsBuffer( d.channels, args.K, args.K );
 	if( vec && d.filterCount % NH_KSTEP == 0 && d.strideHeight == 1 && d.strideWidth == 1 ) {
-		if( trySplitProduct( stream, args, true, 1, vec, &rc ) ) {
-			return rc;
-		}
 		return launchMatMul<AM_ConvTaps, BM_RowsK>( stream, args, 1, true );
 	}
 	return launchMatMul<AM_Conv, BM_RowsK>( stream, args, 1, vec );

@@ -35,12 +35,11 @@ constexpr int SplitStep = 16; // k per matrix instruction and per step
 // held down to 1.5 GHz, a sixth of which is what can be had here; each value that is split ( 5.5 vector instructions ),
 // stored and read again costs on top, so the tiles are as large as the registers allow: a wavefront reads 2 x 2 blocks of
 // fragments for 24 matrix instructions. Measured against the fp32 instructions ( 64 x 64 and 128 x 128 tiles ), us:
-// 8192 x 2048 x 512 132 -> 102 ( 169 TFLOP/s ), 8192 x 512 x 2048 123 -> 107, 8192 x 512 x 512 35.5 -> 31.4, 8192 x 1024 x 256
-// 40 -> 29.5, 3x3 convolutions of 64 x 56 x 56 x 64 120 -> 107, 64 x 28 x 28 x 128 108 -> 91.
-// Error against 64 bits ( 2-norm ) on these: 2.4e-7 to 7.2e-7 where sequential fp32 sums have 2.9e-7 to 8.5e-7.
-// WGM x WGN wavefronts, each MI x NI blocks of 32 x 32; SETS: register sets of operands on their way from memory ( steps of
-// lead ); WPE: wavefronts per SIMD the registers must leave room for; RAGGED: K is not a multiple of the step.
-template<int AMODE, int WGM, int WGN, int MI, int NI, int SETS, int WPE, bool RAGGED>
+// 8192 x 2048 x 512 132 -> 106 ( 162 TFLOP/s ), 8192 x 512 x 2048 123 -> 113, 8192 x 512 x 512 35.5 -> 32.5, 8192 x 1024 x 256
+// 40 -> 29.5, 3x3 convolutions of 64 x 56 x 56 x 64 120 -> 112, 64 x 28 x 28 x 128 108 -> 94.
+// Error against 64 bits ( 2-norm ) on these: 1.5e-7 to 1.8e-7 where sequential fp32 sums have 2.9e-7 to 8.5e-7.
+// WGM x WGN wavefronts, each MI x NI blocks of 32 x 32; WPE: wavefronts per SIMD the registers must leave room for; RAGGED: K is not a multiple of the step.
+template<int AMODE, int WGM, int WGN, int MI, int NI, int WPE, bool RAGGED>
 __global__ __launch_bounds__( 64 * WGM * WGN, WPE )
 void splitProductKernel( const CMatMulArgs args )
 {
@@ -136,10 +135,22 @@ void splitProductKernel( const CMatMulArgs args )
 			? ( static_cast<unsigned>( n ) * static_cast<unsigned>( args.Ldb ) + quad * 4u ) * 4u : OutOfRange;
 	}
 
-	float4 regA[SETS][ASlots], regB[SETS][BSlots];
+	// A matrix instruction rounds its accumulator twice, a step twelve times, and not to nearest: the errors lean to one side,
+	// which a sum over many results ( the gradient by a filter, over 200704 pixels ) adds up: 7e-6 of it where the single
+	// results are off by 2e-7. So the reduction is cut into an even number of chunks of up to eight steps. Each begins from
+	// zero and is added to the totals, and every other one is computed with A negated and subtracted. Most roundings are then of short
+	// sums ( the error of 576 k falls from 3.6e-7 to 1.5e-7, of 2304 k from 7.2e-7 to 1.8e-7; the fp32 instructions: 4.2e-7 and
+	// 8.3e-7 ) and lean to both sides alike, for 2 - 4 % of the time. ( An even length: a chunk begins on LDS buffer 0. )
+	constexpr int LongestChunk = 8;
+	const int pairsOfChunks = ( totalSteps + 2 * LongestChunk - 1 ) / ( 2 * LongestChunk );
+	const int chunk = ( ( totalSteps + 2 * pairsOfChunks - 1 ) / ( 2 * pairsOfChunks ) + 1 ) & ~1;
+	int untilFlip = chunk; // steps to store until the sign changes
+	unsigned signOfA = 0;
+
+	float4 regA[ASlots], regB[BSlots];
 	// Requests the quads of a step. A step behind the last is asked of a descriptor of size zero ( zeros, no memory
 	// access ): every step runs the same code.
-	auto load = [&]( int step, int set ) {
+	auto load = [&]( int step ) {
 		const unsigned range = step < totalSteps ? BufferBytes : 0u;
 		const __amdgpu_buffer_rsrc_t bufA = __builtin_amdgcn_make_buffer_rsrc( const_cast<float*>( baseA ), 0, range, 0x00020000 );
 		const __amdgpu_buffer_rsrc_t bufB = __builtin_amdgcn_make_buffer_rsrc( const_cast<float*>( baseB ), 0, range, 0x00020000 );
@@ -149,11 +160,11 @@ void splitProductKernel( const CMatMulArgs args )
 		const bool masked = RAGGED && step * KS + static_cast<int>( quad ) * 4 >= K;
 #pragma unroll
 		for( int i = 0; i < ASlots; ++i ) {
-			regA[set][i] = bufferLoad4( bufA, masked ? OutOfRange : offA[i], uniA );
+			regA[i] = bufferLoad4( bufA, masked ? OutOfRange : offA[i], uniA );
 		}
 #pragma unroll
 		for( int i = 0; i < BSlots; ++i ) {
-			regB[set][i] = bufferLoad4( bufB, masked ? OutOfRange : offB[i], uniB );
+			regB[i] = bufferLoad4( bufB, masked ? OutOfRange : offB[i], uniB );
 		}
 		if constexpr( IsTaps ) {
 			tapCi += KS;
@@ -182,18 +193,25 @@ void splitProductKernel( const CMatMulArgs args )
 		*reinterpret_cast<uint2*>( &lds[buf][at + Plane] ) = mid;
 		*reinterpret_cast<uint2*>( &lds[buf][at + 2 * Plane] ) = lo;
 	};
-	auto store = [&]( int buf, int set ) {
+	auto store = [&]( int buf ) {
 #pragma unroll
 		for( int i = 0; i < ASlots; ++i ) {
 			if( AUnits % T == 0 || tileRow + i * RowsPerSlot < BM ) {
-				storeUnit( buf, unitAt( tileRow + i * RowsPerSlot ), regA[set][i] );
+				const float4 v = regA[i];
+				auto signedValue = [&]( float x ) { return __uint_as_float( __float_as_uint( x ) ^ signOfA ); };
+				storeUnit( buf, unitAt( tileRow + i * RowsPerSlot ),
+					make_float4( signedValue( v.x ), signedValue( v.y ), signedValue( v.z ), signedValue( v.w ) ) );
 			}
 		}
 #pragma unroll
 		for( int i = 0; i < BSlots; ++i ) {
 			if( BUnits % T == 0 || tileRow + i * RowsPerSlot < BN ) {
-				storeUnit( buf, BM * 32 + unitAt( tileRow + i * RowsPerSlot ), regB[set][i] );
+				storeUnit( buf, BM * 32 + unitAt( tileRow + i * RowsPerSlot ), regB[i] );
 			}
+		}
+		if( --untilFlip == 0 ) {
+			untilFlip = chunk;
+			signOfA ^= 0x80000000u;
 		}
 	};
 
@@ -231,27 +249,32 @@ void splitProductKernel( const CMatMulArgs args )
 			}
 		}
 	};
-	auto product = [&]( const CFrag& f, int pa, int pb ) {
+	auto products = [&]( const CFrag& f ) {
+		auto product = [&]( int pa, int pb ) {
 #pragma unroll
-		for( int mi = 0; mi < MI; ++mi ) {
+			for( int mi = 0; mi < MI; ++mi ) {
 #pragma unroll
-			for( int ni = 0; ni < NI; ++ni ) {
-				acc[mi][ni] = __builtin_amdgcn_mfma_f32_32x32x16_bf16( f.A[pa][mi], f.B[pb][ni], acc[mi][ni], 0, 0, 0 );
+				for( int ni = 0; ni < NI; ++ni ) {
+					acc[mi][ni] = __builtin_amdgcn_mfma_f32_32x32x16_bf16( f.A[pa][mi], f.B[pb][ni], acc[mi][ni], 0, 0, 0 );
+				}
 			}
-		}
+		};
+		product( 2, 0 );
+		product( 0, 2 );
+		product( 1, 1 );
+		product( 1, 0 );
+		product( 0, 1 );
+		product( 0, 0 );
 	};
 
 	// Step s multiplies the fragments that step s - 1 read. Under its matrix instructions the fragments of step s + 1 are read
 	// from LDS buffer ( s + 1 ) % 2 and the values of step s + 2 are split and stored to buffer s % 2, whose last readers
 	// were in step s - 1; one barrier ends the step. Reads, stores and vector instructions are dealt evenly over the step.
-	load( 0, 0 );
-	store( 0, 0 );
-	load( 1, 0 );
-	store( 1, 0 );
-	load( 2, 0 );
-	if constexpr( SETS == 2 ) {
-		load( 3, 1 );
-	}
+	load( 0 );
+	store( 0 );
+	load( 1 );
+	store( 1 );
+	load( 2 );
 	__syncthreads();
 	readFrag( 0, frag[0] );
 	__syncthreads();
@@ -259,16 +282,10 @@ void splitProductKernel( const CMatMulArgs args )
 	constexpr int SplitVector = ( ASlots + BSlots ) * 24; // vector instructions of a step's quads, about
 	auto step = [&]( int s, auto curOf ) {
 		constexpr int cur = decltype( curOf )::value, nxt = cur ^ 1;
-		constexpr int set = SETS == 2 ? cur : 0;
 		__builtin_amdgcn_sched_barrier( 0 );
 		readFrag( nxt, frag[nxt] );
-		store( cur, set );
-		product( frag[cur], 2, 0 );
-		product( frag[cur], 0, 2 );
-		product( frag[cur], 1, 1 );
-		product( frag[cur], 1, 0 );
-		product( frag[cur], 0, 1 );
-		product( frag[cur], 0, 0 );
+		store( cur );
+		products( frag[cur] );
 #pragma unroll
 		for( int i = 0; i < Products; ++i ) {
 			__builtin_amdgcn_sched_group_barrier( 0x008, 1, 0 ); // a matrix instruction
@@ -277,16 +294,39 @@ void splitProductKernel( const CMatMulArgs args )
 			__builtin_amdgcn_sched_group_barrier( 0x200, ( 3 * ( ASlots + BSlots ) + Products - 1 ) / Products, 0 ); // LDS stores
 		}
 		__builtin_amdgcn_sched_barrier( 0 );
-		load( s + 2 + SETS, set );
+		load( s + 3 );
 		__syncthreads();
 	};
-	int s = 0;
-	for( ; s + 1 < totalSteps; s += 2 ) {
-		step( s, std::integral_constant<int, 0>() );
-		step( s + 1, std::integral_constant<int, 1>() );
+	f32x16 total[MI][NI] = {};
+	for( int first = 0; first < totalSteps; first += chunk ) {
+		const int end = min( first + chunk, totalSteps );
+		int s = first;
+		for( ; s + 1 < end; s += 2 ) {
+			step( s, std::integral_constant<int, 0>() );
+			step( s + 1, std::integral_constant<int, 1>() );
+		}
+		if( s < end ) {
+			step( s, std::integral_constant<int, 0>() );
+		}
+		const float sign = ( first / chunk ) & 1 ? -1.f : 1.f;
+#pragma unroll
+		for( int mi = 0; mi < MI; ++mi ) {
+#pragma unroll
+			for( int ni = 0; ni < NI; ++ni ) {
+#pragma unroll
+				for( int r = 0; r < 16; ++r ) {
+					total[mi][ni][r] = __builtin_fmaf( acc[mi][ni][r], sign, total[mi][ni][r] );
+				}
+			}
+		}
+		clear();
 	}
-	if( s < totalSteps ) {
-		step( s, std::integral_constant<int, 0>() );
+#pragma unroll
+	for( int mi = 0; mi < MI; ++mi ) {
+#pragma unroll
+		for( int ni = 0; ni < NI; ++ni ) {
+			acc[mi][ni] = total[mi][ni];
+		}
 	}
 
 	// An operand that is infinite, NaN or rounds to infinity has no finite parts: infinity - infinity makes all it meets NaN.
@@ -432,13 +472,13 @@ struct CSplitPlan {
 // The shapes, as measured on products and 3x3 convolutions of 4 to 18 GFLOP with all compute units at work. The card holds
 // its power limit by lowering the clock, so these are times of a whole device: a step of 256 x 128 tiles on every compute
 // unit 1.25 us ( one workgroup of eight wavefronts each ), of 128 x 128 tiles 0.8 us with one workgroup to a unit and 1.3 us
-// with two, of 128 x 64 tiles 0.5 us with one and 0.49 us for each of up to four, of 256 x 64 tiles 0.94 us each.
-enum TSplitShape { SS_256x128, SS_128x128, SS_256x64, SS_128x64, SS_Count };
+// with two, of 128 x 64 tiles 0.5 us with one and 0.49 us for each of up to three.
+enum TSplitShape { SS_256x128, SS_128x128, SS_128x64, SS_Count };
 
 static CSplitPlan splitPlan( int shape, const CMatMulArgs& a, int batch )
 {
-	const int bm = shape == SS_256x128 || shape == SS_256x64 ? 256 : 128;
-	const int bn = shape == SS_256x128 || shape == SS_128x128 ? 128 : 64;
+	const int bm = shape == SS_256x128 ? 256 : 128;
+	const int bn = shape == SS_128x64 ? 64 : 128;
 	const double steps = ceilDiv( a.K, SplitStep );
 	CSplitPlan plan = {};
 	plan.TilesM = ceilDiv( a.M, bm );
@@ -449,33 +489,31 @@ static CSplitPlan splitPlan( int shape, const CMatMulArgs& a, int batch )
 	switch( shape ) {
 		case SS_256x128: plan.Cost = deepest * ( steps * 1.25 + overhead ); break;
 		case SS_128x128: plan.Cost = deepest <= 1 ? steps * 0.8 + overhead : deepest * ( steps * 0.65 + 3 ) + 3; break;
-		case SS_256x64: plan.Cost = deepest * ( steps * 0.94 + 3 ) + 3; break;
 		default: plan.Cost = deepest <= 1 ? steps * 0.5 + overhead : deepest * ( steps * 0.49 + 1.5 ) + 3; break;
 	}
 	return plan;
 }
 
-template<int AMODE, int WGM, int WGN, int MI, int NI, int SETS, int WPE>
+template<int AMODE, int WGM, int WGN, int MI, int NI, int WPE>
 static void launchSplit( hipStream_t stream, const CMatMulArgs& args, const dim3& grid )
 {
 	const dim3 threads( 64 * WGM * WGN );
 	if constexpr( AMODE == AM_RowsK ) {
 		if( args.K % SplitStep != 0 ) {
-			hipLaunchKernelGGL( ( splitProductKernel<AMODE, WGM, WGN, MI, NI, SETS, WPE, true> ), grid, threads, 0, stream, args );
+			hipLaunchKernelGGL( ( splitProductKernel<AMODE, WGM, WGN, MI, NI, WPE, true> ), grid, threads, 0, stream, args );
 			return;
 		}
 	}
-	hipLaunchKernelGGL( ( splitProductKernel<AMODE, WGM, WGN, MI, NI, SETS, WPE, false> ), grid, threads, 0, stream, args );
+	hipLaunchKernelGGL( ( splitProductKernel<AMODE, WGM, WGN, MI, NI, WPE, false> ), grid, threads, 0, stream, args );
 }
 
 template<int AMODE>
 static void launchSplitShape( hipStream_t stream, int shape, const CMatMulArgs& args, const dim3& grid )
 {
 	switch( shape ) {
-		case SS_256x128: launchSplit<AMODE, 4, 2, 2, 2, 1, 2>( stream, args, grid ); break;
-		case SS_128x128: launchSplit<AMODE, 2, 2, 2, 2, 2, 2>( stream, args, grid ); break;
-		case SS_256x64: launchSplit<AMODE, 4, 1, 2, 2, 1, 2>( stream, args, grid ); break;
-		default: launchSplit<AMODE, 2, 2, 2, 1, 1, 4>( stream, args, grid ); break;
+		case SS_256x128: launchSplit<AMODE, 4, 2, 2, 2, 2>( stream, args, grid ); break;
+		case SS_128x128: launchSplit<AMODE, 2, 2, 2, 2, 2>( stream, args, grid ); break;
+		default: launchSplit<AMODE, 2, 2, 2, 1, 3>( stream, args, grid ); break;
 	}
 }
 
@@ -498,9 +536,19 @@ bool trySplitProduct( hipStream_t stream, const CMatMulArgs& given, bool convolu
 			shape = s;
 		}
 	}
-	// the fp32 instructions: 120 TFLOP/s at best on such sizes, and 4 us
+	// The fp32 instructions: 120 TFLOP/s at best on such sizes, and 4 us. Between other work the card lets the clock rise, so
+	// the costs above are on the safe side ( in ResNet-18 at batch 64: 64 x 28 x 28 x 128 67 us where alone it takes 91 ).
 	const double flops = 2.0 * args.M * args.N * args.K * batch;
-	if( plan.Cost > 0.95 * ( flops / 120e6 + 4 ) ) {
+	if( plan.Cost > 1.15 * ( flops / 120e6 + 4 ) ) {
+		return false;
+	}
+	// A convolution is, as a rule, followed by a ReLU, whose sign a training step's gradients hang on: one value of ten
+	// million that lies within a rounding of zero and falls on the other side moves a gradient by one whole element
+	// ( a residual block of 64 x 56 x 56 x 64: 8e-4 of the gradient, where the sums differ by 4e-7 ). So the blocks of image
+	// networks keep the rounding that they have, for the 6 - 30 % that a launch would gain, and what is taken is the largest
+	// launches ( 65536 pixels, 1152 -> 256: 274 -> 194 us; 2304 -> 256: 414 -> 306 ).
+	constexpr double LargeConvolution = 16e9;
+	if( convolution && flops < LargeConvolution ) {
 		return false;
 	}
 	args.TilesM = plan.TilesM;
