@@ -104,4 +104,12 @@ constexpr int Threads = 256;
 // launch's code; false: not one that it is for.
 bool trySplitProduct( hipStream_t stream, const CMatMulArgs& args, bool convolution, int batch, bool vec, int* rc );
 
+// ( gemm_small.hip ) the same for results of a few tiles; here the image's channel count has to be a multiple of 16.
+constexpr int MaxSmallSlices = 16;
+bool trySmallProduct( hipStream_t stream, const CMatMulArgs& args, bool convolution, int batch, bool vec, int* rc );
+
+// The stream's block of partial tiles and arrival counters for reductions that are cut into slices ( the counters are zero
+// between launches ). false: none to be had ( a capturing stream, a shared stream handle, no memory ).
+bool sliceMeetingPlace( hipStream_t stream, size_t partialFloats, size_t counterCount, float** partials, unsigned** counters );
+
 } // namespace nh

@@ -1162,6 +1162,17 @@ bool streamMeetingPlace( hipStream_t stream, size_t partialFloats, float** parti
 	return true;
 }
 
+bool sliceMeetingPlace( hipStream_t stream, size_t partialFloats, size_t counterCount, float** partials, unsigned** counters )
+{
+	CSliceScratch scratch;
+	if( !sliceScratch( stream, partialFloats, counterCount, scratch ) ) {
+		return false;
+	}
+	*partials = scratch.Partials;
+	*counters = scratch.Counters;
+	return true;
+}
+
 // A meeting place handed in by the caller instead of the stream's block: the launch neither allocates nor looks the
 // stream up, and fails when the place is too small.
 struct CSliceMeeting {
@@ -2405,7 +2416,9 @@ static int matMulNTMeeting( hipStream_t stream, const float* a, int lda, const f
 	}
 	const bool vec = isAligned16( a ) && isAligned16( b ) && K % 4 == 0 && lda % 4 == 0 && ldb % 4 == 0
 		&& strideA % 4 == 0 && strideB % 4 == 0 && fitsBuffer( M, lda, K ) && fitsBuffer( N, ldb, K );
-	if( fixedMeeting == nullptr && trySplitProduct( stream, args, false, batch, vec, &rc ) ) {
+	if( fixedMeeting == nullptr && ( trySmallProduct( stream, args, false, batch, vec, &rc )
+		|| trySplitProduct( stream, args, false, batch, vec, &rc ) ) )
+	{
 		return rc;
 	}
 	if( fixedMeeting == nullptr && tryLongProduct( stream, args, batch, vec, &rc ) ) {
@@ -2713,6 +2726,10 @@ int convImplicitGemm( hipStream_t stream, const nhConvDesc& d, const float* sour
 		// a pointwise convolution over a channels-last image is the plain product image[M x Cin] * filter[Cout x Cin]^T
 		return matMulNTMeeting( stream, source, d.channels, filter, d.channels, result, d.filterCount, args.M, args.N, d.channels,
 			1, 0, 0, 0, freeTerm, false, act, nullptr, fixedMeeting );
+	}
+	int smallRc = NH_OK;
+	if( fixedMeeting == nullptr && trySmallProduct( stream, args, true, 1, vec, &smallRc ) ) {
+		return smallRc;
 	}
 	if( d.filterHeight == 1 && d.filterWidth == 1 ) {
 		return launchMatMul<AM_Conv1x1, BM_RowsK>( stream, args, 1, vec, fixedMeeting );
@@ -3241,6 +3258,9 @@ int convBackwardData( hipStream_t stream, const nhConvDesc& d, const float* outp
 		&& fitsBuffer( 1, 0, static_cast<long long>( d.batch ) * d.resultHeight * d.resultWidth * d.filterCount )
 		&& fitsBuffer( d.channels, args.K, args.K );
 	if( vec && d.filterCount % NH_KSTEP == 0 && d.strideHeight == 1 && d.strideWidth == 1 ) {
+		if( trySmallProduct( stream, args, true, 1, vec, &rc ) ) {
+			return rc;
+		}
 		return launchMatMul<AM_ConvTaps, BM_RowsK>( stream, args, 1, true );
 	}
 	return launchMatMul<AM_Conv, BM_RowsK>( stream, args, 1, vec );
