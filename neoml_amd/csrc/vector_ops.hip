@@ -500,7 +500,7 @@ struct CTanhDiffOutOp : CNoScalar { __device__ float operator()( float y, float 
 //
 // The same queue serves the passes of a layer over a whole blob: a call over more than TinyWideMaxCount elements begins
 // a chain that only calls of its own count join ( an activation's or a solver's passes over one blob, the passes of a
-// normalisation over its matrix, whose vectors per row or column are "spread" operands ). Such a chain never has barriers;
+// normalisation over its matrix, whose vectors per row or column are "spread" operands, of whatever count ). Such a chain never has barriers;
 // it runs four elements per thread with 128-bit accesses where the operands allow it ( quadChainKernel ), through a kernel
 // of its own if it is one of a few known sequences ( launchKnownChain ), and a call that nothing joined goes out as the
 // launch it always was. In every chain without barriers whose calls have one count, a result that a later call
@@ -522,8 +522,8 @@ struct CTinyOp {
 	alignas( 8 ) unsigned char Functor[TinyFunctorBytes];
 	// The second operand of a call over a matrix of rows of Width elements may be a vector spread over it: one value per row
 	// ( TS_PerRow: In[1][i / Width], AddVectorToMatrixColumns, MultiplyDiagMatrixByMatrix ) or per column ( TS_PerColumn:
-	// In[1][i % Width], AddVectorToMatrixRows, MultiplyMatrixByDiagMatrix ). Only calls over more than TinyWideMaxCount
-	// elements come with one, so a chain with barriers never holds any.
+	// In[1][i % Width], AddVectorToMatrixRows, MultiplyMatrixByDiagMatrix ). A chain that holds such a call holds calls of
+	// its count only and has no barriers.
 	short Spread;
 	// The result is not stored: a later call of the chain writes the same elements, and every call in between that reads
 	// them has them in registers ( chains without barriers whose calls all have one count; set when the chain is launched ).
@@ -1099,6 +1099,14 @@ static bool launchKnownChain( hipStream_t stream, const CTinyChain& chain )
 		}
 		return false;
 	}
+	// CEltwiseSumLayer and CReLULayer in place over it ( larger sums wait for their ReLU by themselves, CPendingSum )
+	if( chain.Length == 2 && isKind<CAddOp<float>>( op[0] ) && isKind<CReLUOp>( op[1] ) && op[0].Spread == TS_None
+		&& op[1].In[0] == op[0].Out && op[1].Out == op[0].Out ) {
+		CAddReLUOp sum; sum.Ptr = op[1].Scalar; sum.Threshold = 0;
+		( void )launchEltwisePlain<2, float, float>( stream, op[0].In[0], op[0].In[1], static_cast<const float*>( nullptr ), op[0].Out,
+			op[0].Count, sum );
+		return true;
+	}
 	if( chain.Length == 2 && isKind<CAddOp<float>>( op[0] ) && isKind<CMulOp<float>>( op[1] ) && op[0].Spread == TS_PerRow
 		&& op[1].Spread == TS_None ) {
 		float* y = op[0].Out;
@@ -1132,7 +1140,7 @@ static bool launchTinyChain( hipStream_t stream, CTinyQueue& queue )
 		}
 		return true;
 	}
-	bool barrier = false, quads = true, oneCount = true;
+	bool barrier = false, quads = true, oneCount = true, spreads = false;
 	int longest = 0;
 	for( int k = 0; k < chain.Length; ++k ) {
 		CTinyOp& op = chain.Ops[k];
@@ -1140,6 +1148,7 @@ static bool launchTinyChain( hipStream_t stream, CTinyQueue& queue )
 		barrier = barrier || op.Barrier != 0;
 		oneCount = oneCount && op.Count == chain.Ops[0].Count;
 		longest = op.Count > longest ? op.Count : longest;
+		spreads = spreads || op.Spread != TS_None;
 		quads = quads && op.Count == chain.Ops[0].Count && op.Count % 4 == 0 && isAligned16( op.Out )
 			&& isAligned16( op.In[0] ) && isAligned16( op.In[1] ) && isAligned16( op.In[2] )
 			&& ( op.Spread == TS_None || op.Width % 4 == 0 );
@@ -1166,7 +1175,8 @@ static bool launchTinyChain( hipStream_t stream, CTinyQueue& queue )
 			}
 		}
 	}
-	if( !barrier && quads && longest > TinyOpMaxCount ) {
+	// ( calls with a spread operand: known sequences, at any count )
+	if( !barrier && quads && ( longest > TinyOpMaxCount || spreads ) ) {
 		if( !launchKnownChain( stream, chain ) ) {
 			chain.Straight = 4;
 			chain.Blocks = ceilDiv( longest / 4, QuadThreads * QuadsPerThread );
@@ -1484,6 +1494,24 @@ bool deferColumnSum( nhStream s, float* result, const float* matrix, int height,
 				sum.Result = result; sum.Matrix = matrix; sum.Height = height; sum.Width = width;
 				sum.AddFirst = added.First; sum.AddSecond = added.Second;
 				sum.SquareOf = nullptr; sum.SquareShift = nullptr;
+				return true;
+			}
+		}
+		if( waiting != tinyQueues().end() && !waiting->second.LaunchWaits() && waiting->second.Chain.Length == 1 ) {
+			// the same for a sum that waits as a chain of one call ( those that are not large, deferEltwise )
+			CTinyChain& chain = waiting->second.Chain;
+			const CTinyOp& added = chain.Ops[0];
+			const long long count = static_cast<long long>( height ) * width;
+			const float* resultEnd = result + height;
+			auto apart = [&]( const float* p ) { return resultEnd <= p || p + count <= result; };
+			if( added.Kind == CKindOf<CAddOp<float>, CTinyKinds>::Value && added.Spread == TS_None && added.Out == matrix
+				&& added.Count == count && apart( added.Out ) && apart( added.In[0] ) && apart( added.In[1] ) ) {
+				CPendingColumnSum& sum = waiting->second.ColumnSum;
+				sum.Pending = true;
+				sum.Result = result; sum.Matrix = matrix; sum.Height = height; sum.Width = width;
+				sum.AddFirst = added.In[0]; sum.AddSecond = added.In[1];
+				sum.SquareOf = nullptr; sum.SquareShift = nullptr;
+				chain.Length = 0; // ( one thing waits where one waited )
 				return true;
 			}
 		}
@@ -1863,8 +1891,17 @@ static bool deferEltwise( nhStream s, const TIn* a, const TIn* b, const TIn* c, 
 		}
 		CTinyQueue& queue = found->second;
 		CTinyChain& chain = queue.Chain;
-		if( chain.Length > 0 && ( n > TinyWideMaxCount || chain.Ops[0].Count > TinyWideMaxCount ) && chain.Ops[0].Count != n ) {
-			launchTinyChain( stream, queue ); // ( a chain with a call that large holds calls of one count only )
+		bool oneCount = n > TinyWideMaxCount || spread != TS_None;
+		for( int k = 0; k < chain.Length; ++k ) {
+			oneCount = oneCount || chain.Ops[k].Count > TinyWideMaxCount || chain.Ops[k].Spread != TS_None;
+		}
+		if( oneCount ) {
+			for( int k = 0; k < chain.Length; ++k ) {
+				if( chain.Ops[k].Count != n || chain.Ops[k].Barrier != 0 ) {
+					launchTinyChain( stream, queue ); // ( a chain with a call that large or spread holds calls of one count only )
+					break;
+				}
+			}
 		}
 		if( chain.Length == TinyChainMax ) {
 			launchTinyChain( stream, queue );
@@ -1905,9 +1942,9 @@ static bool deferEltwise( nhStream s, const TIn* a, const TIn* b, const TIn* c, 
 		}
 		writes.Lo = out;
 		writes.Hi = out + n;
-		bool barrier = false, wide = n > TinyOpMaxCount;
+		bool barrier = false, wide = n > TinyOpMaxCount || spread != TS_None;
 		for( int k = 0; k < chain.Length; ++k ) {
-			wide = wide || chain.Ops[k].Count > TinyOpMaxCount;
+			wide = wide || chain.Ops[k].Count > TinyOpMaxCount || chain.Ops[k].Spread != TS_None;
 		}
 		for( int k = 0; k < chain.Length && !barrier; ++k ) {
 			const CTinyOp& front = chain.Ops[k];
@@ -1960,7 +1997,7 @@ bool deferSpreadOp( nhStream s, bool multiply, int spread, const float* matrix, 
 	CSpreadAlone alone )
 {
 	const long long count = static_cast<long long>( height ) * width;
-	if( __atomic_load_n( &tinyDeferringStreams, __ATOMIC_RELAXED ) == 0 || count <= TinyWideMaxCount || count > 0x7fffffffLL
+	if( __atomic_load_n( &tinyDeferringStreams, __ATOMIC_RELAXED ) == 0 || height <= 0 || width <= 0 || count > 0x7fffffffLL
 		|| matrix == nullptr || vector == nullptr || result == nullptr || alone == nullptr
 		|| ( spread != TS_PerRow && spread != TS_PerColumn ) ) {
 		return false;

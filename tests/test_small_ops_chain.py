@@ -865,3 +865,88 @@ def test_row_sums_wait_for_the_calls_over_them(streams):
     got = streams.run(streams.deferring, [("nhSumMatrixColumns", [at(sums), at(x), rows, width])] + tails["mean"], start)
     mean = start[:rows * width].astype(np.float64).reshape(rows, width).mean(1)
     assert np.allclose(got[sums:sums + rows], -mean, rtol=1e-5, atol=1e-6)
+
+
+@pytest.mark.parametrize("rows,width,o", [(37, 512, 0), (1, 64, 0), (3, 7, 0), (40, 263, 3), (130, 128, 0), (257, 4, 1), (512, 512, 0)])
+def test_passes_over_a_small_matrix_with_vectors_spread_over_it(streams, rows, width, o):
+    """Calls with a vector spread over the matrix join a chain at any size. A residual sum, its normalisation, a sum with
+    its ReLU, and random runs of such calls with others of the same and of other counts between them, over operands that
+    overlap in every way the calls allow: the bits of the separate launches."""
+    import torch
+    lib, na = streams.lib, streams.na
+    n = rows * width
+    P = lambda t, at=0: ctypes.c_void_p(t.data_ptr() + 4 * int(at))
+
+    def run(stream, program):
+        g = torch.Generator(device=streams.dev).manual_seed(n + o)
+        new = lambda count: torch.randn(count, generator=g, device=streams.dev)
+        m = [new(n + 8) for _ in range(4)]
+        r, c, f = [new(rows + 4) for _ in range(3)], [new(width + 4) for _ in range(3)], [new(1).abs() for _ in range(2)]
+        torch.cuda.synchronize()
+        program(stream, m, r, c, f)
+        na.check(lib.nhStreamSynchronize(stream))
+        return [t.cpu().numpy() for t in m + r + c]
+
+    def layer(s, m, r, c, f):
+        x, y, sq, out = m
+        mean, dev = r[0], r[1]
+        na.check(lib.nhVectorAdd(s, P(x, o), P(y, o), P(y, o), n))
+        na.check(lib.nhSumMatrixColumns(s, P(mean), P(y, o), rows, width))
+        na.check(lib.nhVectorNegMultiply(s, P(mean), P(mean), rows, P(f[0])))
+        na.check(lib.nhAddVectorToMatrixColumns(s, P(y, o), P(sq, o), rows, width, P(mean)))
+        na.check(lib.nhVectorEltwiseMultiply(s, P(sq, o), P(sq, o), P(sq, o), n))
+        na.check(lib.nhSumMatrixColumns(s, P(dev), P(sq, o), rows, width))
+        na.check(lib.nhVectorMultiply(s, P(dev), P(dev), rows, P(f[0])))
+        na.check(lib.nhVectorAddValue(s, P(dev), P(dev), rows, P(f[1])))
+        na.check(lib.nhVectorSqrt(s, P(dev), P(dev), rows))
+        na.check(lib.nhVectorInv(s, P(dev), P(dev), rows))
+        na.check(lib.nhAddVectorToMatrixColumns(s, P(y, o), P(out, o), rows, width, P(mean)))
+        na.check(lib.nhMultiplyDiagMatrixByMatrix(s, P(dev), rows, P(out, o), width, P(out, o), n))
+        na.check(lib.nhBatchMultiplyMatrixByDiagMatrix(s, 1, P(out, o), rows, width, 0, P(c[0]), 0, P(out, o), n))
+        na.check(lib.nhAddVectorToMatrixRows(s, 1, P(out, o), P(out, o), rows, width, P(c[1])))
+        na.check(lib.nhVectorAdd(s, P(out, o), P(x, o), P(x, o), n))
+        na.check(lib.nhVectorReLU(s, P(x, o), P(x, o), n, P(f[0])))
+        # sums that land in an operand of the sum in front of them, and sums over fewer rows than that has
+        na.check(lib.nhVectorAdd(s, P(out, o), P(y, o), P(out, o), n))
+        na.check(lib.nhSumMatrixColumns(s, P(y, o), P(out, o), rows, width))
+        na.check(lib.nhVectorAdd(s, P(x, o), P(sq, o), P(sq, o), n))
+        na.check(lib.nhSumMatrixColumns(s, P(r[2]), P(sq, o), max(1, rows - 1), width))
+
+    def random_calls(seed):
+        def program(s, m, r, c, f):
+            g = rng(seed)
+            for _ in range(60):
+                b = P(m[g.integers(4)], o + (0 if g.random() < 0.8 else 1))
+                kind = g.integers(11)
+                if kind == 0:
+                    i, j = g.permutation(4)[:2]  # ( the vector may be the beginning of another matrix )
+                    row = P(r[g.integers(3)], g.integers(2)) if g.random() < 0.7 else P(m[i])
+                    na.check(lib.nhAddVectorToMatrixColumns(s, P(m[j], o), P(m[j], o), rows, width, row))
+                elif kind == 1:
+                    na.check(lib.nhAddVectorToMatrixRows(s, 1, b, b, rows, width, P(c[g.integers(3)])))
+                elif kind == 2:
+                    na.check(lib.nhMultiplyDiagMatrixByMatrix(s, P(r[g.integers(3)]), rows, b, width, b, n))
+                elif kind == 3:
+                    na.check(lib.nhBatchMultiplyMatrixByDiagMatrix(s, 1, b, rows, width, 0, P(c[g.integers(3)]), 0, b, n))
+                elif kind == 4:
+                    na.check(lib.nhVectorEltwiseMultiply(s, b, b, b, n))
+                elif kind == 5:
+                    na.check(lib.nhVectorTanh(s, b, b, n))
+                elif kind == 6:
+                    na.check(lib.nhVectorTanh(s, P(r[0]), P(r[0]), rows))
+                elif kind == 7:
+                    na.check(lib.nhVectorSigmoid(s, P(c[1]), P(c[1]), width))
+                elif kind == 8:
+                    na.check(lib.nhSumMatrixColumns(s, P(r[1]), b, rows, width))
+                elif kind == 9:
+                    i, j = g.permutation(4)[:2]
+                    na.check(lib.nhVectorAdd(s, P(m[i], o), P(m[j], o), P(m[j], o), n))
+                else:
+                    i = g.integers(4)
+                    na.check(lib.nhVectorTanh(s, P(m[i], o), P(m[i], o), n))
+        return program
+
+    for program in [layer] + [random_calls(seed) for seed in range(6)]:
+        got, want = run(streams.deferring, program), run(streams.plain, program)
+        for x, y in zip(got, want):
+            assert same_bits(x, y)
