@@ -35,7 +35,7 @@ constexpr int SplitStep = 16; // k per matrix instruction and per step
 // held down to 1.5 GHz, a sixth of which is what can be had here; each value that is split ( 5.5 vector instructions ),
 // stored and read again costs on top, so the tiles are as large as the registers allow: a wavefront reads 2 x 2 blocks of
 // fragments for 24 matrix instructions. Measured against the fp32 instructions ( 64 x 64 and 128 x 128 tiles ), us:
-// 8192 x 2048 x 512 132 -> 106 ( 162 TFLOP/s ), 8192 x 512 x 2048 123 -> 113, 8192 x 512 x 512 35.5 -> 32.5, 8192 x 1024 x 256
+// 8192 x 2048 x 512 132 -> 106 ( 162 TFLOP/s ), 8192 x 512 x 2048 123 -> 113, 8192 x 512 x 512 35.5 -> 29.5, 8192 x 1024 x 256
 // 40 -> 29.5, 3x3 convolutions of 64 x 56 x 56 x 64 120 -> 112, 64 x 28 x 28 x 128 108 -> 94.
 // Error against 64 bits ( 2-norm ) on these: 1.5e-7 to 1.8e-7 where sequential fp32 sums have 2.9e-7 to 8.5e-7.
 // WGM x WGN wavefronts, each MI x NI blocks of 32 x 32; WPE: wavefronts per SIMD the registers must leave room for; RAGGED: K is not a multiple of the step.
@@ -471,8 +471,9 @@ struct CSplitPlan {
 
 // The shapes, as measured on products and 3x3 convolutions of 4 to 18 GFLOP with all compute units at work. The card holds
 // its power limit by lowering the clock, so these are times of a whole device: a step of 256 x 128 tiles on every compute
-// unit 1.25 us ( one workgroup of eight wavefronts each ), of 128 x 128 tiles 0.8 us with one workgroup to a unit and 1.3 us
-// with two, of 128 x 64 tiles 0.5 us with one and 0.49 us for each of up to three.
+// unit 1.25 us, of 128 x 128 tiles 0.8 us ( one workgroup of eight wavefronts each, the second shape with 64 x 32 of the tile to a
+// wavefront: four wavefronts of 64 x 64 take 33.2 us instead of 29.5 for 8192 x 512 x 512, 116 instead of 113 for
+// 8192 x 512 x 2048 ), of 128 x 64 tiles 0.5 us with one workgroup of four to a unit and 0.49 us for each of up to three.
 enum TSplitShape { SS_256x128, SS_128x128, SS_128x64, SS_Count };
 
 static CSplitPlan splitPlan( int shape, const CMatMulArgs& a, int batch )
@@ -488,7 +489,7 @@ static CSplitPlan splitPlan( int shape, const CMatMulArgs& a, int batch )
 	const double overhead = 6;
 	switch( shape ) {
 		case SS_256x128: plan.Cost = deepest * ( steps * 1.25 + overhead ); break;
-		case SS_128x128: plan.Cost = deepest <= 1 ? steps * 0.8 + overhead : deepest * ( steps * 0.65 + 3 ) + 3; break;
+		case SS_128x128: plan.Cost = deepest * ( steps * 0.8 + 4 ) + 2; break;
 		default: plan.Cost = deepest <= 1 ? steps * 0.5 + overhead : deepest * ( steps * 0.49 + 1.5 ) + 3; break;
 	}
 	return plan;
@@ -512,7 +513,7 @@ static void launchSplitShape( hipStream_t stream, int shape, const CMatMulArgs& 
 {
 	switch( shape ) {
 		case SS_256x128: launchSplit<AMODE, 4, 2, 2, 2, 2>( stream, args, grid ); break;
-		case SS_128x128: launchSplit<AMODE, 2, 2, 2, 2, 2>( stream, args, grid ); break;
+		case SS_128x128: launchSplit<AMODE, 2, 4, 2, 1, 2>( stream, args, grid ); break;
 		default: launchSplit<AMODE, 2, 2, 2, 1, 3>( stream, args, grid ); break;
 	}
 }
