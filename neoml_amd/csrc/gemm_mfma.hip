@@ -2046,6 +2046,8 @@ static bool tryShortReduction( hipStream_t stream, const float* a, int lda, cons
 }
 
 // ---- plain products with long reductions and large results -------------------------------------------------------
+// ( What reaches it: results whose rows lie beyond 32-bit offsets. The others go to gemm_split.hip, whose figures stand
+// there; those below are of this kernel when it took them. )
 // C[M x N] (+)= act( A[M x K] * B[N x K]^T + bias ) (+ residual), both operands K-major: the products of fully connected
 // layers over thousands of rows ( transformer feed-forward 8192 x 2048 x 512 and 8192 x 512 x 2048, the input product of
 // an LSTM layer 8192 x 1024 x 256 ).
