@@ -99,12 +99,12 @@ constexpr int Threads = 256;
 #define NH_KSTEP 16
 #endif
 
-// ( gemm_split.hip ) C = act( A * B^T + bias ) (+ C, + residual) for operands that are K-major, A also as the im2col view of
-// an image whose channel count is a multiple of the K step ( args as the fp32 kernels take them ). true: launched, *rc is the
-// launch's code; false: not one that it is for.
-bool trySplitProduct( hipStream_t stream, const CMatMulArgs& args, bool convolution, int batch, bool vec, int* rc );
+// ( gemm_split.hip ) C = act( A * B^T + bias ) (+ C, + residual) for operands that are K-major ( args as the fp32 kernels take
+// them ). true: launched, *rc is the launch's code; false: not one that it is for.
+bool trySplitProduct( hipStream_t stream, const CMatMulArgs& args, int batch, bool vec, int* rc );
 
-// ( gemm_small.hip ) the same for results of a few tiles; here the image's channel count has to be a multiple of 16.
+// ( gemm_small.hip ) the same for results of a few tiles; A also as the im2col view of an image whose channel count is a multiple
+// of 16.
 constexpr int MaxSmallSlices = 16;
 bool trySmallProduct( hipStream_t stream, const CMatMulArgs& args, bool convolution, int batch, bool vec, int* rc );
 

@@ -2419,7 +2419,7 @@ static int matMulNTMeeting( hipStream_t stream, const float* a, int lda, const f
 	const bool vec = isAligned16( a ) && isAligned16( b ) && K % 4 == 0 && lda % 4 == 0 && ldb % 4 == 0
 		&& strideA % 4 == 0 && strideB % 4 == 0 && fitsBuffer( M, lda, K ) && fitsBuffer( N, ldb, K );
 	if( fixedMeeting == nullptr && ( trySmallProduct( stream, args, false, batch, vec, &rc )
-		|| trySplitProduct( stream, args, false, batch, vec, &rc ) ) )
+		|| trySplitProduct( stream, args, batch, vec, &rc ) ) )
 	{
 		return rc;
 	}
@@ -2754,10 +2754,6 @@ int convImplicitGemm( hipStream_t stream, const nhConvDesc& d, const float* sour
 		return launchMatMul<AM_ConvRows, BM_RowsK>( stream, args, 1, true, fixedMeeting );
 	}
 	if( vec && d.channels % NH_KSTEP == 0 ) {
-		int rc = NH_OK;
-		if( fixedMeeting == nullptr && trySplitProduct( stream, args, true, 1, vec, &rc ) ) {
-			return rc;
-		}
 		return launchMatMul<AM_ConvTaps, BM_RowsK>( stream, args, 1, true, fixedMeeting );
 	}
 	return launchMatMul<AM_Conv, BM_RowsK>( stream, args, 1, vec, fixedMeeting );

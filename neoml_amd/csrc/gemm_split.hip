@@ -1,4 +1,4 @@
-// fp32 matrix products and convolutions on the bf16 matrix instructions, each operand as the sum of three bf16 values.
+// fp32 matrix products on the bf16 matrix instructions, each operand as the sum of three bf16 values.
 //
 // An fp32 value is exactly hi + mid + lo, where hi is the value rounded to bf16, mid what is left rounded to bf16, and lo
 // the rest: 8 significant bits each, signs of their own. Of the nine products of two such sums the six down to 2^-16 of the
@@ -29,22 +29,19 @@ __device__ __forceinline__ void splitPair( float x, float y, unsigned& hi, unsig
 
 constexpr int SplitStep = 16; // k per matrix instruction and per step
 
-// C[M x N] = act( A * B^T + bias ) (+ C, + residual), A rows of K values or the im2col view of an image whose channel count
-// is a multiple of the step ( a step stays inside a filter tap ), B rows of K values.
+// C[M x N] = act( A * B^T + bias ) (+ C, + residual), A and B rows of K values.
 // What bounds it: the card's power. Bare matrix instructions on random operands run at 1600 - 1700 TFLOP/s with the clock
 // held down to 1.5 GHz, a sixth of which is what can be had here; each value that is split ( 5.5 vector instructions ),
 // stored and read again costs on top, so the tiles are as large as the registers allow: a wavefront reads 2 x 2 blocks of
 // fragments for 24 matrix instructions. Measured against the fp32 instructions ( 64 x 64 and 128 x 128 tiles ), us:
 // 8192 x 2048 x 512 132 -> 106 ( 162 TFLOP/s ), 8192 x 512 x 2048 123 -> 113, 8192 x 512 x 512 35.5 -> 29.5, 8192 x 1024 x 256
-// 40 -> 29.5, 3x3 convolutions of 64 x 56 x 56 x 64 120 -> 112, 64 x 28 x 28 x 128 108 -> 94.
+// 40 -> 29.5.
 // Error against 64 bits ( 2-norm ) on these: 1.5e-7 to 1.8e-7 where sequential fp32 sums have 2.9e-7 to 8.5e-7.
 // WGM x WGN wavefronts, each MI x NI blocks of 32 x 32; WPE: wavefronts per SIMD the registers must leave room for; RAGGED: K is not a multiple of the step.
-template<int AMODE, int WGM, int WGN, int MI, int NI, int WPE, bool RAGGED>
+template<int WGM, int WGN, int MI, int NI, int WPE, bool RAGGED>
 __global__ __launch_bounds__( 64 * WGM * WGN, WPE )
 void splitProductKernel( const CMatMulArgs args )
 {
-	constexpr bool IsTaps = ( AMODE == AM_ConvTaps );
-	static_assert( IsTaps || AMODE == AM_RowsK, "operands that are K-major" );
 	constexpr int KS = SplitStep;
 	constexpr int T = 64 * WGM * WGN;
 	constexpr int BM = 32 * WGM * MI, BN = 32 * WGN * NI;
@@ -74,58 +71,17 @@ void splitProductKernel( const CMatMulArgs args )
 	fastDivMod( tile, args.TilesN, args.TilesNMagic, tileM, tileN );
 	const int m0 = tileM * BM, n0 = tileN * BN;
 
-	// position of output pixel m's window in the image, of a row of A otherwise
-	struct CRow {
-		unsigned Base; // in floats, of tap ( 0, 0 ): unsigned arithmetic, it may lie in front of the image
-		int H0, W0;
-	};
-	auto rowOf = [&]( int m ) -> CRow {
-		CRow row;
-		if constexpr( IsTaps ) {
-			int t, wo, n, ho;
-			fastDivMod( m, args.Wo, args.WoMagic, t, wo );
-			fastDivMod( t, args.Ho, args.HoMagic, n, ho );
-			row.H0 = m < M ? ho * args.StrideH - args.PadH : -0x40000000;
-			row.W0 = wo * args.StrideW - args.PadW;
-			row.Base = static_cast<unsigned>( n * args.H * args.W * args.Cin )
-				+ ( static_cast<unsigned>( row.H0 ) * static_cast<unsigned>( args.W ) + static_cast<unsigned>( row.W0 ) ) * static_cast<unsigned>( args.Cin );
-		} else {
-			row.H0 = m < M ? 0 : -1;
-			row.W0 = 0;
-			row.Base = static_cast<unsigned>( m ) * static_cast<unsigned>( args.Lda );
-		}
-		return row;
-	};
-	// byte offset of a row's values from k = 0 ( of the tap ) on
-	auto rowOffset = [&]( const CRow& row, int kh, int kw ) -> unsigned {
-		if constexpr( IsTaps ) {
-			const int dh = kh * args.DilH, dw = kw * args.DilW; // ( scalar )
-			const unsigned tapFloats = ( static_cast<unsigned>( dh ) * static_cast<unsigned>( args.W ) + static_cast<unsigned>( dw ) )
-				* static_cast<unsigned>( args.Cin );
-			const bool ok = kh < args.Fh && static_cast<unsigned>( row.H0 + dh ) < static_cast<unsigned>( args.H )
-				&& static_cast<unsigned>( row.W0 + dw ) < static_cast<unsigned>( args.W );
-			return ok ? ( row.Base + tapFloats ) * 4u : OutOfRange;
-		} else {
-			return row.H0 < 0 ? OutOfRange : row.Base * 4u;
-		}
-	};
-
 	// ---- this thread's quads: quad tid % 4 of tile rows tid / 4 + i T / 4, four lanes cover the 64 bytes of a row's step
-	CRow rowA[ASlots];
 	unsigned offA[ASlots], offB[BSlots];
-	int tapCi = 0, tapKh = 0, tapKw = 0;
 	const unsigned quad = tid & 3;
 	const int tileRow = tid >> 2;
 	constexpr int RowsPerSlot = T / 4;
 #pragma unroll
 	for( int i = 0; i < ASlots; ++i ) {
 		const int row = tileRow + i * RowsPerSlot;
-		rowA[i] = rowOf( m0 + row );
-		if( AUnits % T != 0 && row >= BM ) {
-			rowA[i].H0 = -0x40000000;
-		}
-		rowA[i].Base += quad * 4u;
-		offA[i] = rowOffset( rowA[i], tapKh, tapKw );
+		const int m = m0 + row;
+		offA[i] = ( AUnits % T == 0 || row < BM ) && m < M
+			? ( static_cast<unsigned>( m ) * static_cast<unsigned>( args.Lda ) + quad * 4u ) * 4u : OutOfRange;
 	}
 #pragma unroll
 	for( int i = 0; i < BSlots; ++i ) {
@@ -154,31 +110,16 @@ void splitProductKernel( const CMatMulArgs args )
 		const unsigned range = step < totalSteps ? BufferBytes : 0u;
 		const __amdgpu_buffer_rsrc_t bufA = __builtin_amdgcn_make_buffer_rsrc( const_cast<float*>( baseA ), 0, range, 0x00020000 );
 		const __amdgpu_buffer_rsrc_t bufB = __builtin_amdgcn_make_buffer_rsrc( const_cast<float*>( baseB ), 0, range, 0x00020000 );
-		const unsigned uniB = static_cast<unsigned>( step ) * ( KS * 4u );
-		const unsigned uniA = IsTaps ? static_cast<unsigned>( tapCi ) * 4u : uniB;
+		const unsigned uni = static_cast<unsigned>( step ) * ( KS * 4u );
 		// the last step of a K that is not a multiple of the step ( it is one of 4 )
 		const bool masked = RAGGED && step * KS + static_cast<int>( quad ) * 4 >= K;
 #pragma unroll
 		for( int i = 0; i < ASlots; ++i ) {
-			regA[i] = bufferLoad4( bufA, masked ? OutOfRange : offA[i], uniA );
+			regA[i] = bufferLoad4( bufA, masked ? OutOfRange : offA[i], uni );
 		}
 #pragma unroll
 		for( int i = 0; i < BSlots; ++i ) {
-			regB[i] = bufferLoad4( bufB, masked ? OutOfRange : offB[i], uniB );
-		}
-		if constexpr( IsTaps ) {
-			tapCi += KS;
-			if( tapCi >= args.Cin ) {
-				tapCi = 0;
-				if( ++tapKw == args.Fw ) {
-					tapKw = 0;
-					++tapKh;
-				}
-#pragma unroll
-				for( int i = 0; i < ASlots; ++i ) {
-					offA[i] = rowOffset( rowA[i], tapKh, tapKw );
-				}
-			}
+			regB[i] = bufferLoad4( bufB, masked ? OutOfRange : offB[i], uni );
 		}
 	};
 	const int quadAt = static_cast<int>( quad >> 1 ) * 512 + static_cast<int>( quad & 1 ) * 8;
@@ -364,19 +305,13 @@ void splitProductKernel( const CMatMulArgs args )
 		const __amdgpu_buffer_rsrc_t bufA = makeBuffer( baseA ), bufB = makeBuffer( baseB );
 		#pragma unroll 1
 		for( int k0 = 0; k0 < K; k0 += 8 ) {
-			int kh = 0, kw = 0, ci = k0;
-			if( IsTaps ) {
-				const int tap = k0 / args.Cin;
-				ci = k0 - tap * args.Cin;
-				kh = tap / args.Fw;
-				kw = tap - kh * args.Fw;
-			}
 			const bool inK = k0 + half * 4 < K;
 			float4 a[MI], b[NI];
 #pragma unroll
 			for( int mi = 0; mi < MI; ++mi ) {
-				const unsigned off = rowOffset( rowOf( m0 + ( waveM * MI + mi ) * 32 + l32 ), kh, kw );
-				a[mi] = bufferLoad4( bufA, inK && off != OutOfRange ? off + static_cast<unsigned>( ci + half * 4 ) * 4u : OutOfRange );
+				const int m = m0 + ( waveM * MI + mi ) * 32 + l32;
+				a[mi] = bufferLoad4( bufA, inK && m < M
+					? ( static_cast<unsigned>( m ) * static_cast<unsigned>( args.Lda ) + static_cast<unsigned>( k0 + half * 4 ) ) * 4u : OutOfRange );
 			}
 #pragma unroll
 			for( int ni = 0; ni < NI; ++ni ) {
@@ -469,7 +404,7 @@ struct CSplitPlan {
 	int TilesM, TilesN;
 };
 
-// The shapes, as measured on products and 3x3 convolutions of 4 to 18 GFLOP with all compute units at work. The card holds
+// The shapes, as measured on products of 4 to 18 GFLOP with all compute units at work. The card holds
 // its power limit by lowering the clock, so these are times of a whole device: a step of 256 x 128 tiles on every compute
 // unit 1.25 us, of 128 x 128 tiles 0.8 us ( one workgroup of eight wavefronts each, the second shape with 64 x 32 of the tile to a
 // wavefront: four wavefronts of 64 x 64 take 33.2 us instead of 29.5 for 8192 x 512 x 512, 116 instead of 113 for
@@ -495,33 +430,27 @@ static CSplitPlan splitPlan( int shape, const CMatMulArgs& a, int batch )
 	return plan;
 }
 
-template<int AMODE, int WGM, int WGN, int MI, int NI, int WPE>
+template<int WGM, int WGN, int MI, int NI, int WPE>
 static void launchSplit( hipStream_t stream, const CMatMulArgs& args, const dim3& grid )
 {
 	const dim3 threads( 64 * WGM * WGN );
-	if constexpr( AMODE == AM_RowsK ) {
-		if( args.K % SplitStep != 0 ) {
-			hipLaunchKernelGGL( ( splitProductKernel<AMODE, WGM, WGN, MI, NI, WPE, true> ), grid, threads, 0, stream, args );
-			return;
-		}
-	}
-	hipLaunchKernelGGL( ( splitProductKernel<AMODE, WGM, WGN, MI, NI, WPE, false> ), grid, threads, 0, stream, args );
-}
-
-template<int AMODE>
-static void launchSplitShape( hipStream_t stream, int shape, const CMatMulArgs& args, const dim3& grid )
-{
-	switch( shape ) {
-		case SS_256x128: launchSplit<AMODE, 4, 2, 2, 2, 2>( stream, args, grid ); break;
-		case SS_128x128: launchSplit<AMODE, 2, 4, 2, 1, 2>( stream, args, grid ); break;
-		default: launchSplit<AMODE, 2, 2, 2, 1, 3>( stream, args, grid ); break;
+	if( args.K % SplitStep != 0 ) {
+		hipLaunchKernelGGL( ( splitProductKernel<WGM, WGN, MI, NI, WPE, true> ), grid, threads, 0, stream, args );
+	} else {
+		hipLaunchKernelGGL( ( splitProductKernel<WGM, WGN, MI, NI, WPE, false> ), grid, threads, 0, stream, args );
 	}
 }
 
-bool trySplitProduct( hipStream_t stream, const CMatMulArgs& given, bool convolution, int batch, bool vec, int* rc )
+// Products, a pointwise convolution's among them. 3x3 convolutions would be done in 0.66 to 0.9 of the time ( us: 65536 pixels,
+// 1152 -> 256, 282 -> 190; 64 x 28 x 28 x 128, 116 -> 83; 64 x 56 x 56 x 64, 119 -> 104 ), but the ReLU behind one decides by a
+// value's sign what a training step's gradients are made of. Another rounding, also a smaller one, moves a value next to zero to the
+// other side, and with each such value of the 1.3e7 of 64 x 56 x 56 x 64 a residual block's gradients move by 3e-4, where the sums
+// differ by 4e-7. A convolution cannot know what it is computed for, and its size says nothing about it: at every size they keep the
+// rounding that they have had.
+bool trySplitProduct( hipStream_t stream, const CMatMulArgs& given, int batch, bool vec, int* rc )
 {
 	CMatMulArgs args = given;
-	if( !vec || batch > 65535 || args.M < 128 || args.N < 48 || args.K < 128 || ( convolution && args.Cin % SplitStep != 0 ) ) {
+	if( !vec || batch > 65535 || args.M < 128 || args.N < 48 || args.K < 128 ) {
 		return false;
 	}
 	const long long cBytes = ( static_cast<long long>( args.M - 1 ) * args.Ldc + args.N ) * 4;
@@ -537,32 +466,20 @@ bool trySplitProduct( hipStream_t stream, const CMatMulArgs& given, bool convolu
 			shape = s;
 		}
 	}
-	// The fp32 instructions: 120 TFLOP/s at best on such sizes, and 4 us. Between other work the card lets the clock rise, so
-	// the costs above are on the safe side ( in ResNet-18 at batch 64: 64 x 28 x 28 x 128 67 us where alone it takes 91 ).
+	// The fp32 instructions: 120 TFLOP/s at best on such sizes, and 4 us.
 	const double flops = 2.0 * args.M * args.N * args.K * batch;
 	if( plan.Cost > 1.15 * ( flops / 120e6 + 4 ) ) {
-		return false;
-	}
-	// A convolution is, as a rule, followed by a ReLU, whose sign a training step's gradients hang on: one value of ten
-	// million that lies within a rounding of zero and falls on the other side moves a gradient by one whole element
-	// ( a residual block of 64 x 56 x 56 x 64: 8e-4 of the gradient, where the sums differ by 4e-7 ). So the blocks of image
-	// networks keep the rounding that they have, for the 6 - 30 % that a launch would gain, and what is taken is the largest
-	// launches ( 65536 pixels, 1152 -> 256: 274 -> 194 us; 2304 -> 256: 414 -> 306 ).
-	constexpr double LargeConvolution = 16e9;
-	if( convolution && flops < LargeConvolution ) {
 		return false;
 	}
 	args.TilesM = plan.TilesM;
 	args.TilesN = plan.TilesN;
 	args.TilesNMagic = divisionMagic( args.TilesN );
-	args.WoMagic = divisionMagic( args.Wo );
-	args.HoMagic = divisionMagic( args.Ho );
 	args.CBytes = static_cast<unsigned>( cBytes );
 	const dim3 grid( static_cast<unsigned>( plan.TilesM ) * plan.TilesN, batch );
-	if( convolution ) {
-		launchSplitShape<AM_ConvTaps>( stream, shape, args, grid );
-	} else {
-		launchSplitShape<AM_RowsK>( stream, shape, args, grid );
+	switch( shape ) {
+		case SS_256x128: launchSplit<4, 2, 2, 2, 2>( stream, args, grid ); break;
+		case SS_128x128: launchSplit<2, 4, 2, 1, 2>( stream, args, grid ); break;
+		default: launchSplit<2, 2, 2, 1, 3>( stream, args, grid ); break;
 	}
 	const hipError_t err = hipGetLastError();
 	if( err != hipSuccess ) {

@@ -1,4 +1,5 @@
-"""Products and convolutions that run on the bf16 matrix instructions with operands split in three, against 64 bits."""
+"""Products that run on the bf16 matrix instructions with operands split in three, and convolutions of such sizes, which do not,
+against 64 bits."""
 import numpy as np
 import pytest
 
@@ -78,6 +79,24 @@ def test_convolutions(hip, n, h, w, cin, cout, f, pad, stride):
     a = _patches(torch, x.double(), f, f, pad, stride)
     one = torch.ones(a.shape[0], 1, device=hip.dev, dtype=torch.float64)
     _check(y, torch.cat([a, one], 1), torch.cat([filt.double().reshape(cout, -1), bias.double()[:, None]], 1), f * f * cin)
+
+
+def test_a_convolution_rounds_alike_at_every_batch(hip):
+    """The ReLU behind a convolution decides by a value's sign: what is computed of an image does not change with the images beside
+    it. ( The last tiles of a launch may be cut into slices of the reduction: the images in front of them, to the bit. )"""
+    torch = hip.torch
+    import ctypes
+    g = torch.Generator(device=hip.dev).manual_seed(6)
+    x = torch.rand(70, 56, 56, 64, generator=g, device=hip.dev)
+    filt = torch.randn(64, 3, 3, 64, generator=g, device=hip.dev) * 0.06
+    bias = torch.randn(64, generator=g, device=hip.dev) * 0.01
+    results = []
+    for batch in (64, 70):  # 14.8 and 16.2 GFLOP
+        d = hip.conv_desc(batch, 56, 56, 64, 64, 3, 3, 1, 1, 1, 1)
+        y = torch.empty(batch, 56, 56, 64, device=hip.dev)
+        hip.call("nhBlobConvolution", ctypes.byref(d), hip.p(x), hip.p(filt), hip.p(bias), hip.p(y))
+        results.append(y)
+    assert torch.equal(results[0][:52], results[1][:52])
 
 
 def test_values_without_finite_parts(hip):
