@@ -29,6 +29,11 @@ __device__ __forceinline__ void splitPair( float x, float y, unsigned& hi, unsig
 
 constexpr int SplitStep = 16; // k per matrix instruction and per step
 
+// The lowest bit of a value is 2^-23 of its power of two: below 2^-103 some of its parts lie under the smallest normal number, 2^-126,
+// and are lost, whatever the value is multiplied by. So operands are split times 2^24, which every normal value's parts bear and
+// which the sums are relieved of again as they are added up. ( Denormal values count as zero, here as in the fp32 instructions. )
+constexpr float OperandScale = 0x1p24f, SumScale = 0x1p-48f;
+
 // C[M x N] = act( A * B^T + bias ) (+ C, + residual), A and B rows of K values.
 // What bounds it: the card's power. Bare matrix instructions on random operands run at 1600 - 1700 TFLOP/s with the clock
 // held down to 1.5 GHz, a sixth of which is what can be had here; each value that is split ( 5.5 vector instructions ),
@@ -101,7 +106,7 @@ void splitProductKernel( const CMatMulArgs args )
 	const int pairsOfChunks = ( totalSteps + 2 * LongestChunk - 1 ) / ( 2 * LongestChunk );
 	const int chunk = ( ( totalSteps + 2 * pairsOfChunks - 1 ) / ( 2 * pairsOfChunks ) + 1 ) & ~1;
 	int untilFlip = chunk; // steps to store until the sign changes
-	unsigned signOfA = 0;
+	float scaleOfA = OperandScale;
 
 	float4 regA[ASlots], regB[BSlots];
 	// Requests the quads of a step. A step behind the last is asked of a descriptor of size zero ( zeros, no memory
@@ -139,20 +144,21 @@ void splitProductKernel( const CMatMulArgs args )
 		for( int i = 0; i < ASlots; ++i ) {
 			if( AUnits % T == 0 || tileRow + i * RowsPerSlot < BM ) {
 				const float4 v = regA[i];
-				auto signedValue = [&]( float x ) { return __uint_as_float( __float_as_uint( x ) ^ signOfA ); };
 				storeUnit( buf, unitAt( tileRow + i * RowsPerSlot ),
-					make_float4( signedValue( v.x ), signedValue( v.y ), signedValue( v.z ), signedValue( v.w ) ) );
+					make_float4( v.x * scaleOfA, v.y * scaleOfA, v.z * scaleOfA, v.w * scaleOfA ) );
 			}
 		}
 #pragma unroll
 		for( int i = 0; i < BSlots; ++i ) {
 			if( BUnits % T == 0 || tileRow + i * RowsPerSlot < BN ) {
-				storeUnit( buf, BM * 32 + unitAt( tileRow + i * RowsPerSlot ), regB[i] );
+				const float4 v = regB[i];
+				storeUnit( buf, BM * 32 + unitAt( tileRow + i * RowsPerSlot ),
+					make_float4( v.x * OperandScale, v.y * OperandScale, v.z * OperandScale, v.w * OperandScale ) );
 			}
 		}
 		if( --untilFlip == 0 ) {
 			untilFlip = chunk;
-			signOfA ^= 0x80000000u;
+			scaleOfA = -scaleOfA;
 		}
 	};
 
@@ -220,7 +226,7 @@ void splitProductKernel( const CMatMulArgs args )
 	readFrag( 0, frag[0] );
 	__syncthreads();
 	constexpr int Products = 6 * MI * NI; // matrix instructions of a step
-	constexpr int SplitVector = ( ASlots + BSlots ) * 24; // vector instructions of a step's quads, about
+	constexpr int SplitVector = ( ASlots + BSlots ) * 26; // vector instructions of a step's quads, about
 	auto step = [&]( int s, auto curOf ) {
 		constexpr int cur = decltype( curOf )::value, nxt = cur ^ 1;
 		__builtin_amdgcn_sched_barrier( 0 );
@@ -249,7 +255,7 @@ void splitProductKernel( const CMatMulArgs args )
 		if( s < end ) {
 			step( s, std::integral_constant<int, 0>() );
 		}
-		const float sign = ( first / chunk ) & 1 ? -1.f : 1.f;
+		const float sign = ( first / chunk ) & 1 ? -SumScale : SumScale;
 #pragma unroll
 		for( int mi = 0; mi < MI; ++mi ) {
 #pragma unroll
@@ -270,11 +276,10 @@ void splitProductKernel( const CMatMulArgs args )
 		}
 	}
 
-	// An operand that is infinite, NaN or rounds to infinity has no finite parts: infinity - infinity makes all it meets NaN.
-	// And parts of operands below 2^-108 fall under the smallest normal bf16 value. Either shows in the accumulators ( not
-	// finite; not zero but tiny ): such a wavefront multiplies its blocks again with the fp32 instructions, operands straight
-	// from memory.
-	float notFinite = 0.f, least = __builtin_inff();
+	// An operand that is infinite or NaN, or that times its factor rounds to infinity, has no finite parts: infinity - infinity makes
+	// all it meets NaN. And a sum beyond 2^80 overflows times the factors. Either shows in the totals: such a wavefront multiplies its
+	// blocks again with the fp32 instructions, operands straight from memory.
+	float notFinite = 0.f;
 #pragma unroll
 	for( int mi = 0; mi < MI; ++mi ) {
 #pragma unroll
@@ -282,24 +287,10 @@ void splitProductKernel( const CMatMulArgs args )
 #pragma unroll
 			for( int r = 0; r < 16; ++r ) {
 				notFinite = __builtin_fmaf( acc[mi][ni][r], 0.f, notFinite );
-				least = fminf( least, fabsf( acc[mi][ni][r] ) );
 			}
 		}
 	}
-	constexpr float Tiny = 0x1p-80f;
-	bool again = notFinite != notFinite;
-	if( __builtin_amdgcn_ballot_w64( least < Tiny ) != 0 ) {
-#pragma unroll
-		for( int mi = 0; mi < MI; ++mi ) {
-#pragma unroll
-			for( int ni = 0; ni < NI; ++ni ) {
-#pragma unroll
-				for( int r = 0; r < 16; ++r ) {
-					again = again || ( acc[mi][ni][r] != 0.f && fabsf( acc[mi][ni][r] ) < Tiny );
-				}
-			}
-		}
-	}
+	const bool again = notFinite != notFinite;
 	if( __builtin_amdgcn_ballot_w64( again ) != 0 ) {
 		clear();
 		const __amdgpu_buffer_rsrc_t bufA = makeBuffer( baseA ), bufB = makeBuffer( baseB );

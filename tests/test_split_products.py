@@ -136,3 +136,49 @@ def test_values_without_finite_parts(hip):
     over = want[5000].abs() > 4 * big
     assert not torch.isfinite(c[5000][over]).any()
     assert c[5000, 17] == float("inf")
+
+
+# ( a product for each of the three tile shapes )
+@pytest.mark.parametrize("m,n,k", [(8192, 2048, 512), (8192, 512, 1024), (2048, 1024, 516)])
+@pytest.mark.parametrize("of_a,of_b", [(-104, 60), (-116, 60), (60, -116), (-125, 100), (-110, 10)])
+def test_small_values_with_large_partners(hip, m, n, k, of_a, of_b):
+    """Normal values whose lower parts would lie under the smallest normal number, against partners that bring the products back
+    into the middle of the range. In the 2-norm k products that are added one by one, the partial sums growing as a random walk, are
+    off by 2^-24 sqrt( k / 6 ) ( each rounding 2^-24 / sqrt( 3 ) of a partial sum )."""
+    torch = hip.torch
+    g = torch.Generator(device=hip.dev).manual_seed(m + k)
+
+    def values(rows, power):
+        v = torch.rand(rows, k, generator=g, device=hip.dev, dtype=torch.float64) + 1
+        sign = torch.randint(0, 2, (rows, k), generator=g, device=hip.dev, dtype=torch.float64) * 2 - 1
+        return (v * sign * 2.0 ** power).float()
+
+    a, b = values(m, of_a), values(n, of_b)
+    c = torch.empty(m, n, device=hip.dev)
+    hip.call("nhMultiplyMatrixByTransposedMatrix", hip.p(a), m, k, k, hip.p(b), n, k, hip.p(c), n, c.numel())
+    want = a.double() @ b.double().T
+    assert ((c.double() - want).norm() / want.norm()).item() < 2.0 ** -24 * (k / 6) ** 0.5
+
+
+@pytest.mark.parametrize("m,n,k", [(8192, 2048, 512), (8192, 512, 1024), (2048, 1024, 516)])
+def test_one_small_value(hip, m, n, k):
+    """One such value in a row of A, one in a row of B, by itself in its row: the results are its products, rounded once."""
+    torch = hip.torch
+    g = torch.Generator(device=hip.dev).manual_seed(k)
+    a = torch.randn(m, k, generator=g, device=hip.dev)
+    b = torch.randn(n, k, generator=g, device=hip.dev)
+    for one, other, row, at in ((a, b, m - 3, k - 1), (b, a, n // 2, 5)):
+        one[row] = 0.0
+        one[row, at] = 1.2345678 * 2.0 ** -118
+        other[:, at] = torch.rand(other.shape[0], generator=g, device=hip.dev) * 2.0 ** 80
+        other[m - 3 if other is a else n // 2, at] = 0.0
+    c = torch.empty(m, n, device=hip.dev)
+    hip.call("nhMultiplyMatrixByTransposedMatrix", hip.p(a), m, k, k, hip.p(b), n, k, hip.p(c), n, c.numel())
+    want = a.double() @ b.double().T
+    for got, right in ((c[m - 3], want[m - 3]), (c[:, n // 2], want[:, n // 2])):
+        assert ((got.double() - right).abs() <= 2.0 ** -23 * right.abs()).all()
+    rest = torch.ones(m, n, dtype=torch.bool, device=hip.dev)
+    rest[m - 3] = False
+    rest[:, n // 2] = False
+    bound = (6 * k / 16 + 8) * 2.0 ** -24 * (a.double().abs() @ b.double().abs().T)
+    assert ((c.double() - want).abs() <= bound)[rest].all()
