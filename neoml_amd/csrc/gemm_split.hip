@@ -6,6 +6,7 @@
 // an fp32 product. A matrix instruction sums 16 such products into the fp32 accumulator, where the fp32 one sums 2: six
 // roundings of the accumulator per 16 k instead of eight.
 #include "gemm.h"
+#include <algorithm>
 #include <type_traits>
 
 namespace nh {
@@ -401,11 +402,15 @@ struct CSplitPlan {
 	int TilesM, TilesN;
 };
 
-// The shapes, as measured on products of 4 to 18 GFLOP with all compute units at work. The card holds
-// its power limit by lowering the clock, so these are times of a whole device: a step of 256 x 128 tiles on every compute
-// unit 1.25 us, of 128 x 128 tiles 0.8 us ( one workgroup of eight wavefronts each, the second shape with 64 x 32 of the tile to a
-// wavefront: four wavefronts of 64 x 64 take 33.2 us instead of 29.5 for 8192 x 512 x 512, 116 instead of 113 for
-// 8192 x 512 x 2048 ), of 128 x 64 tiles 0.5 us with one workgroup of four to a unit and 0.49 us for each of up to three.
+// A launch takes what the compute unit with the most tiles takes, or, where the matrix instructions of all units together draw more
+// power than there is, what the card's rate leaves: the longer of the two. Fitted to 443 products of 0.3 to 40 GFLOP, K from 128 to
+// 4092, one or up to 64 of them, repeated until the clock had settled ( fitted over measured, 5th and 95th percentile: 0.90 and 1.10
+// for the largest tiles, 0.86 and 1.12, 0.82 and 1.15 ). A step of a tile takes
+//   256 x 128 tiles: 0.84 us, one workgroup to a unit; the card 213 TFLOP/s;
+//   128 x 128 tiles by eight wavefronts of 64 x 32: 0.525 us, 188 TFLOP/s ( by four of 64 x 64: 33.2 us instead of 29.5 for
+//   8192 x 512 x 512, 116 instead of 113 for 8192 x 512 x 2048 );
+//   128 x 64 tiles: 0.46 us, 0.39 us for each of several side by side ( three to a unit ), 166 TFLOP/s;
+// and a tile costs what its prologue and epilogue take on top.
 enum TSplitShape { SS_256x128, SS_128x128, SS_128x64, SS_Count };
 
 static CSplitPlan splitPlan( int shape, const CMatMulArgs& a, int batch )
@@ -418,11 +423,11 @@ static CSplitPlan splitPlan( int shape, const CMatMulArgs& a, int batch )
 	plan.TilesN = ceilDiv( a.N, bn );
 	const long long tiles = static_cast<long long>( plan.TilesM ) * plan.TilesN * batch;
 	const double deepest = static_cast<double>( ( tiles + 255 ) / 256 );
-	const double overhead = 6;
+	const double megaflops = static_cast<double>( tiles ) * steps * ( 2e-6 * SplitStep * bm * bn );
 	switch( shape ) {
-		case SS_256x128: plan.Cost = deepest * ( steps * 1.25 + overhead ); break;
-		case SS_128x128: plan.Cost = deepest * ( steps * 0.8 + 4 ) + 2; break;
-		default: plan.Cost = deepest <= 1 ? steps * 0.5 + overhead : deepest * ( steps * 0.49 + 1.5 ) + 3; break;
+		case SS_256x128: plan.Cost = std::max( deepest * steps * 0.84, megaflops / 213 ) + deepest * 8; break;
+		case SS_128x128: plan.Cost = std::max( deepest * steps * 0.525, megaflops / 188 ) + deepest * 3.5 + 1.9; break;
+		default: plan.Cost = std::max( steps * std::max( 0.46, 0.39 * deepest ), megaflops / 166 ) + deepest * 0.5 + 3.5; break;
 	}
 	return plan;
 }
@@ -463,9 +468,13 @@ bool trySplitProduct( hipStream_t stream, const CMatMulArgs& given, int batch, b
 			shape = s;
 		}
 	}
-	// The fp32 instructions: 120 TFLOP/s at best on such sizes, and 4 us.
+	// The fp32 instructions at their best on such sizes: 130 TFLOP/s, three steps' time for the ends of a tile, 3 us. What is taken is
+	// what is expected to be faster. Of the 443 products one was slower so, 15265 x 128 x 1048 with 43.9 us instead of 42.7; all together
+	// take 0.881 of the time of the fp32 instructions, the faster kernel every time would take 0.864. ( 1792 x 1024 x 512 20.2 -> 17.3,
+	// 4096 x 512 x 256 12.2 -> 10.9, 4096 x 768 x 128 12.0 -> 9.8; not 1024 x 512 x 512, 10.5 and 16.3, or 6272 x 160 x 960, 23 and 32. )
+	const double steps = ceilDiv( args.K, SplitStep );
 	const double flops = 2.0 * args.M * args.N * args.K * batch;
-	if( plan.Cost > 1.15 * ( flops / 120e6 + 4 ) ) {
+	if( plan.Cost > flops / 130e6 * ( steps + 3 ) / steps + 3 ) {
 		return false;
 	}
 	args.TilesM = plan.TilesM;

@@ -606,6 +606,20 @@ def assert_close(actual, expected, what="", rtol=RTOL, atol=ATOL):
 # ---------------------------------------------------------------------------------------------------------
 # device side: the same front-end, through the C ABI of libneoml_hip.so on torch-owned device memory
 
+def kernel_names(calls):
+    """The names of the kernels that each of the calls launches ( kernel_names.py says how a call is written ), without template
+    arguments' types and parameters: "splitProductKernel<4, 2, 2, 2, 2, true>"."""
+    import json
+    import subprocess
+    import sys
+    here = os.path.dirname(os.path.abspath(__file__))
+    paths = [os.path.dirname(here)] + [p for p in os.environ.get("PYTHONPATH", "").split(os.pathsep) if p]
+    out = subprocess.run([sys.executable, os.path.join(here, "kernel_names.py")], input=json.dumps(calls), stdout=subprocess.PIPE, text=True,
+                         check=True, timeout=100, env=dict(os.environ, PYTHONPATH=os.pathsep.join(paths)))
+    names = json.loads(out.stdout.strip().splitlines()[-1])
+    return [[n.split("nh::", 1)[1].split("(")[0] for n in launched] for launched in names]
+
+
 class Hip:
     """Calls the HIP library through its C ABI. Inputs are numpy arrays; they are uploaded into torch CUDA
     tensors (plumbing only), the kernel runs on torch's current stream, and the result comes back as numpy."""
