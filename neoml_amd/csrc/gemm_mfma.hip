@@ -865,7 +865,7 @@ void matMulKernel( const CMatMulArgs launchArgs )
 		if( args.CBytes != 0 && splitK == 1 && !args.Accumulate && args.Residual == nullptr ) {
 			const __amdgpu_buffer_rsrc_t bufC = __builtin_amdgcn_make_buffer_rsrc( C, 0, args.CBytes, 0x00020000 );
 			const float actParam = withParam( args.Act ).Param; // ( the threshold may live in device memory )
-			const float reluTop = actParam > 0.f ? actParam : __builtin_inff();
+	const float reluTop = actParam > 0.f ? actParam : __builtin_inff();
 			const unsigned pitchBytes = static_cast<unsigned>( args.Ldc ) * 4u;
 			const bool inside = m0 + BM <= M;
 			auto store = [&]( auto typeOf, auto insideOf ) {
@@ -928,7 +928,7 @@ void matMulKernel( const CMatMulArgs launchArgs )
 		}
 		const float bias = ( args.Bias != nullptr ) ? args.Bias[n] : 0.f;
 		const float actParam = withParam( args.Act ).Param; // ( the threshold may live in device memory )
-			const float reluTop = actParam > 0.f ? actParam : __builtin_inff();
+	const float reluTop = actParam > 0.f ? actParam : __builtin_inff();
 		// Mode: 0 adds onto C with atomics ( K slices that meet in C: it was set to the free term, or left as it was when
 		// accumulating, before the launch ), 1 stores act( acc + bias ), 2 also accumulates and / or adds the residual.
 		// What is the same for the whole tile is decided once per tile, not per element: with up to eight wavefronts per SIMD
@@ -2046,26 +2046,16 @@ static bool tryShortReduction( hipStream_t stream, const float* a, int lda, cons
 }
 
 // ---- plain products with long reductions and large results -------------------------------------------------------
-// ( What reaches it: results whose rows lie beyond 32-bit offsets. The others go to gemm_split.hip, whose figures stand
-// there; those below are of this kernel when it took them. )
-// C[M x N] (+)= act( A[M x K] * B[N x K]^T + bias ) (+ residual), both operands K-major: the products of fully connected
-// layers over thousands of rows ( transformer feed-forward 8192 x 2048 x 512 and 8192 x 512 x 2048, the input product of
-// an LSTM layer 8192 x 1024 x 256 ).
-// Workgroup tile 128 x 128, K step 16, two LDS buffers of [row][16 + 4], in two shapes:
-//   eight wavefronts ( 2 x 4 ), each 64 rows x 32 columns = two 32 x 32 MFMA blocks that share their B operand; three
-//   workgroups fit a compute unit;
-//   four wavefronts ( 2 x 2 ), each 64 x 64 = four blocks; four workgroups fit a compute unit.
+// C[M x N] (+)= act( A[M x K] * B[N x K]^T + bias ) (+ residual), both operands K-major, for results whose rows lie beyond 32-bit
+// offsets: the kernel of gemm_split.hip, which takes the others where they gain by it, stores by such offsets.
+// Workgroup tile 128 x 128 of eight wavefronts ( 2 x 4 ), each 64 rows x 32 columns = two 32 x 32 MFMA blocks that share their B
+// operand; K step 16, two LDS buffers of [row][16 + 4]; three workgroups fit a compute unit.
 // Against the 64 x 64 tile of matMulKernel every value that reaches LDS feeds twice as many MFMAs and every fragment
-// read 1.5 to 2 times as many, which on this part shows as a higher sustained clock as much as in fewer stalls, and
-// eight waves per workgroup keep two to six waves on every SIMD even when the tiles only just cover the compute units.
-// Measured against the 64 x 64 tile ( us ): 8192 x 512 x 2048 129 -> 123, 8192 x 512 x 512 39 -> 35, 8192 x 1024 x 256
-// 40 -> 36.5, 8192 x 2048 x 2048 550 -> 469 ( 146.5 TFLOP/s ) with eight wavefronts. With 1024 tiles and a reduction of 32
-// steps ( 8192 x 2048 x 512 ) the eight-wave shape runs 768 workgroups at once and the remaining 256 afterwards on a
-// device that is three quarters idle: 130 to 150 us, depending on how far the first ones had drifted apart; four
-// workgroups of four waves per compute unit hold all 1024 at once: 130 us.
-// Each thread fetches 128-bit pieces of A and B ( raw buffer loads: rows beyond the matrix read as zeros ) into SETS
-// register sets; with one set the values wait a whole step before they go to LDS, which is enough while several
-// workgroups share a compute unit; two sets pay where a compute unit holds one workgroup.
+// read 1.5 times as many, which on this part shows as a higher sustained clock as much as in fewer stalls. Measured against
+// it ( us ): 32800 x 16400 x 128 1425 -> 1253, x 256 2518 -> 2189, x 512 4693 -> 4069 ( 135 TFLOP/s ), 600000 x 1000 x 512
+// 5096 -> 4576; at 64 columns, half the tile, the two are equal.
+// Each thread fetches 128-bit pieces of A and B ( raw buffer loads: rows beyond the matrix read as zeros ); the values wait
+// a whole step before they go to LDS, which is enough while several workgroups share a compute unit.
 struct CLongProductArgs {
 	const float* A;
 	const float* B;
@@ -2082,12 +2072,12 @@ struct CLongProductArgs {
 
 constexpr int LongTile = 128;
 
-// WGM x WGN wavefronts, each MI x NI blocks of 32 x 32; WPE: wavefronts per SIMD the registers must leave room for
 // RAGGED: K is not a multiple of the step
-template<int WGM, int WGN, int MI, int NI, int SETS, int WPE, bool RAGGED>
-__global__ __launch_bounds__( 64 * WGM * WGN, WPE )
+template<bool RAGGED>
+__global__ __launch_bounds__( 512, 6 )
 void longProductKernel( const CLongProductArgs args )
 {
+	constexpr int WGM = 2, WGN = 4, MI = 2, NI = 1; // wavefronts, each MI x NI blocks of 32 x 32
 	constexpr int KS = NH_KSTEP, LdsK = KS + 4, KQ = KS / 4;
 	constexpr int T = 64 * WGM * WGN;
 	constexpr int BM = 32 * WGM * MI, BN = 32 * WGN * NI;
@@ -2130,14 +2120,14 @@ void longProductKernel( const CLongProductArgs args )
 	const int kSteps = ( K + KS - 1 ) / KS;
 	const bool inLastStep = ( kSteps - 1 ) * KS + kq < K; // RAGGED: the last step has columns beyond K, they must read as zeros
 
-	float4 rA[SETS][ASlots], rB[SETS][BSlots];
+	float4 rA[ASlots], rB[BSlots];
 	// Every step of the reduction, the last ones included, runs the same code with the same number of loads in flight
 	// ( the waits in front of the LDS stores count them ): a step behind the last one is requested through a descriptor of
 	// size zero, which answers with zeros without touching memory and costs two scalar instructions. No vector
 	// instruction: a wave's vector instructions wait for its MFMAs in flight, and two selects per step on the lanes'
 	// offsets cost 3 % ( 8192 x 2048 x 2048: 469 -> 484 us ). Only a K that ends inside a step ( RAGGED, a kernel of its
 	// own ) pays them, for the per-lane mask of its last step.
-	auto load = [&]( int step, int set ) {
+	auto load = [&]( int step ) {
 		const unsigned uni = static_cast<unsigned>( step ) * ( KS * 4u );
 		const unsigned range = step < kSteps ? BufferBytes : 0u;
 		const __amdgpu_buffer_rsrc_t bufA = __builtin_amdgcn_make_buffer_rsrc( const_cast<float*>( baseA ), 0, range, 0x00020000 );
@@ -2145,21 +2135,21 @@ void longProductKernel( const CLongProductArgs args )
 		const bool masked = RAGGED && step == kSteps - 1 && !inLastStep;
 #pragma unroll
 		for( int i = 0; i < ASlots; ++i ) {
-			rA[set][i] = bufferLoad4( bufA, masked ? OutOfRange : offA[i], uni );
+			rA[i] = bufferLoad4( bufA, masked ? OutOfRange : offA[i], uni );
 		}
 #pragma unroll
 		for( int i = 0; i < BSlots; ++i ) {
-			rB[set][i] = bufferLoad4( bufB, masked ? OutOfRange : offB[i], uni );
+			rB[i] = bufferLoad4( bufB, masked ? OutOfRange : offB[i], uni );
 		}
 	};
-	auto store = [&]( int buf, int set ) {
+	auto store = [&]( int buf ) {
 #pragma unroll
 		for( int i = 0; i < ASlots; ++i ) {
-			*reinterpret_cast<float4*>( &lds[buf][rowOfSlot( i ) * LdsK + kq] ) = rA[set][i];
+			*reinterpret_cast<float4*>( &lds[buf][rowOfSlot( i ) * LdsK + kq] ) = rA[i];
 		}
 #pragma unroll
 		for( int i = 0; i < BSlots; ++i ) {
-			*reinterpret_cast<float4*>( &lds[buf][( BM + rowOfSlot( i ) ) * LdsK + kq] ) = rB[set][i];
+			*reinterpret_cast<float4*>( &lds[buf][( BM + rowOfSlot( i ) ) * LdsK + kq] ) = rB[i];
 		}
 	};
 
@@ -2209,16 +2199,14 @@ void longProductKernel( const CLongProductArgs args )
 	};
 
 	// Step ks multiplies out of LDS buffer ks % 2 while the operands of step ks + 1 go from registers to the other buffer
-	// and those of step ks + 1 + SETS are requested. The one barrier of a step sits between its two groups of 8 k: the
+	// and those of step ks + 2 are requested. The one barrier of a step sits between its two groups of 8 k: the
 	// second group's fragments were fetched ahead of it, so behind it nobody reads the buffer any more ( it is the one
 	// the next step stores to ), and the first fragments of the next step are fetched right behind it.
-	constexpr int Ahead = SETS + 1;
 	auto step = [&]( int ks, auto parity ) {
 		constexpr int nxt = decltype( parity )::value; // == ( ks + 1 ) % 2
 		constexpr int cur = nxt ^ 1;
-		constexpr int set = SETS == 2 ? nxt : 0;
-		store( nxt, set ); // ( behind the last step: zeros that nobody multiplies )
-		load( ks + Ahead, set );
+		store( nxt ); // ( behind the last step: zeros that nobody multiplies )
+		load( ks + 2 );
 		__builtin_amdgcn_sched_barrier( 0 );
 		readFrag( cur, 1, frag[1] );
 		__builtin_amdgcn_sched_barrier( 0 );
@@ -2231,14 +2219,9 @@ void longProductKernel( const CLongProductArgs args )
 		__builtin_amdgcn_sched_barrier( 0 );
 	};
 
-	load( 0, 0 );
-	store( 0, 0 );
-	if( SETS == 2 ) {
-		load( 1, 1 );
-		load( 2, 0 );
-	} else {
-		load( 1, 0 );
-	}
+	load( 0 );
+	store( 0 );
+	load( 1 );
 	__syncthreads();
 	readFrag( 0, 0, frag[0] );
 	int ks = 0;
@@ -2254,7 +2237,7 @@ void longProductKernel( const CLongProductArgs args )
 	float* C = args.C + batch * args.BatchStrideC;
 	const float* residual = args.Residual != nullptr ? args.Residual + batch * args.BatchStrideC : nullptr;
 	const float actParam = withParam( args.Act ).Param; // ( the threshold may live in device memory )
-			const float reluTop = actParam > 0.f ? actParam : __builtin_inff();
+	const float reluTop = actParam > 0.f ? actParam : __builtin_inff();
 	const bool accumulate = args.Accumulate != 0;
 	const int rowBase = m0 + waveM * 32 * MI + half * 4;
 	// what is the same for the whole tile is decided once, here, and not per element: 32 or 64 elements per lane and up
@@ -2313,12 +2296,15 @@ void longProductKernel( const CLongProductArgs args )
 	}
 }
 
-// true ( and launched ) when the product is one this kernel is for: vector loads possible, a reduction of at least eight
-// steps, and enough 128 x 128 tiles to give every compute unit the same number of workgroups to within a quarter ( results
-// with fewer tiles, or tiles that would be mostly padding, stay with the 64 x 64 tiles and their K slices )
+// true ( and launched ) when the product is one this kernel is for: a result beyond 32-bit offsets, vector loads possible, a
+// reduction of at least eight steps, and enough 128 x 128 tiles to give every compute unit the same number of workgroups to within
+// a quarter ( results with fewer tiles, or tiles that would be mostly padding, stay with the 64 x 64 tiles and their K slices ).
+// Smaller results that the split does not take have few tiles or short reductions, where the 64 x 64 tiles are faster ( us:
+// 2753 x 2188 x 140 25 here, 22 there, 829 x 3564 x 160 16 and 12.5 ).
 static bool tryLongProduct( hipStream_t stream, const CMatMulArgs& a, int batch, bool vec, int* rc )
 {
-	if( !vec || a.K < 8 * NH_KSTEP || a.M < LongTile || a.N < LongTile / 2 || batch > 65535 ) {
+	const long long cBytes = ( static_cast<long long>( a.M - 1 ) * a.Ldc + a.N ) * 4;
+	if( !vec || cBytes < 0x7fffff00LL || a.K < 8 * NH_KSTEP || a.M < LongTile || a.N < LongTile / 2 || batch > 65535 ) {
 		return false;
 	}
 	const long long tilesM = ceilDiv( a.M, LongTile ), tilesN = ceilDiv( a.N, LongTile );
@@ -2342,24 +2328,10 @@ static bool tryLongProduct( hipStream_t stream, const CMatMulArgs& a, int batch,
 	args.Accumulate = a.Accumulate;
 	args.Act = a.Act;
 	const dim3 grid( static_cast<unsigned>( tilesM * tilesN ), batch );
-	const int kSteps = ceilDiv( a.K, NH_KSTEP );
-	auto launch = [&]( auto ragged ) {
-		constexpr bool Ragged = decltype( ragged )::value;
-		if( tiles <= unitsAtOnce ) {
-			// one workgroup per compute unit: two waves per SIMD, the operands get two steps to arrive
-			hipLaunchKernelGGL( ( longProductKernel<2, 4, 2, 1, 2, 4, Ragged> ), grid, dim3( 512 ), 0, stream, args );
-		} else if( tiles > 3 * unitsAtOnce && tiles <= 4 * unitsAtOnce && kSteps <= 64 ) {
-			// more than the three workgroups of eight waves that fit a compute unit, and a reduction too short for them
-			// to drift apart: four workgroups of four waves hold all the tiles at once
-			hipLaunchKernelGGL( ( longProductKernel<2, 2, 2, 2, 1, 4, Ragged> ), grid, dim3( 256 ), 0, stream, args );
-		} else {
-			hipLaunchKernelGGL( ( longProductKernel<2, 4, 2, 1, 1, 6, Ragged> ), grid, dim3( 512 ), 0, stream, args );
-		}
-	};
 	if( a.K % NH_KSTEP != 0 ) {
-		launch( std::true_type() );
+		hipLaunchKernelGGL( ( longProductKernel<true> ), grid, dim3( 512 ), 0, stream, args );
 	} else {
-		launch( std::false_type() );
+		hipLaunchKernelGGL( ( longProductKernel<false> ), grid, dim3( 512 ), 0, stream, args );
 	}
 	const hipError_t err = hipGetLastError();
 	if( err != hipSuccess ) {
