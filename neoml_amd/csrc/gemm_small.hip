@@ -237,6 +237,25 @@ void smallProductKernel( const CMatMulArgs args )
 	}
 }
 
+// What this kernel is expected to take, in microseconds, with shares of so many groups. Fitted to some 1700 launches over
+// 478 products and convolutions of up to 256 tiles, K from 128 to 8196, as all figures here are.
+static double smallCost( int waves, int share, int slices, long long tiles )
+{
+	// ( the groups that all compute units have to do, to each: loads and matrix instructions share what there is )
+	const double fill = static_cast<double>( tiles ) * slices * share / 256;
+	const double meeting = slices > 1 ? 1.2 + 0.05 * slices : 0.0;
+	return waves == 8 ? 4.6 + 0.25 * share + 0.83 * ( ( share + 1 ) / 2 ) + 0.45 * fill + meeting : 4.4 + 0.27 * share + 0.2 * fill + meeting;
+}
+
+// What the 64 x 64 tiles take: chains of steps below 32 steps, slices of them from there on.
+static double tilesCost( int steps, long long tiles64, bool convolution )
+{
+	if( steps < 32 ) {
+		return 3.3 + 0.256 * steps + ( convolution ? 0.6 : 0.0 );
+	}
+	return 6.7 + steps * ( 0.033 + 0.0008 * static_cast<double>( tiles64 ) ) + ( convolution ? 0.3 : 0.0 );
+}
+
 bool trySmallProduct( hipStream_t stream, const CMatMulArgs& given, bool convolution, int batch, bool vec, int* rc )
 {
 	if( !vec || batch > 65535 || given.K < 128 || ( convolution && given.Cin % 16 != 0 ) ) {
@@ -244,24 +263,35 @@ bool trySmallProduct( hipStream_t stream, const CMatMulArgs& given, bool convolu
 	}
 	const long long tilesM = ceilDiv( given.M, 32 ), tilesN = ceilDiv( given.N, 32 );
 	const long long tiles = tilesM * tilesN * batch;
+	if( tiles > 256 ) { // ( a second workgroup on a compute unit waits for the first )
+		return false;
+	}
 	const int groups = ceilDiv( given.K, 16 );
 	const int waves = groups >= 16 ? 8 : 4;
-	// slices until the compute units have a workgroup each, as long as a wavefront's share is more than three groups
-	int slices = 1;
-	while( batch == 1 && slices < MaxSmallSlices && tiles * slices * 2 <= 256 && groups > slices * waves * 3 ) {
-		slices *= 2;
+	// as many slices as are expected to pay, up to a workgroup for every compute unit
+	int slices = 0;
+	double cost = 0;
+	for( int s = 1; s <= ( batch == 1 ? MaxSmallSlices : 1 ) && tiles * s <= 256; ++s ) {
+		const int share = ceilDiv( groups, static_cast<long long>( s ) * waves );
+		if( ceilDiv( groups, static_cast<long long>( share ) * waves ) != s ) {
+			continue; // ( fewer slices have the same share )
+		}
+		const double c = smallCost( waves, share, s, tiles );
+		if( slices == 0 || c < cost ) {
+			slices = s;
+			cost = c;
+		}
 	}
-	// A group costs a compute unit's eight wavefronts 0.47 us ( the fp32 matrix instructions' rate ) on top of some 6 us, slices
-	// 2 us more. Measured against the 64 x 64 tiles and their slices, us: 49 x 320 x 960 9.4 -> 8.0, 196 x 64 x 384 9.3 -> 7.7,
-	// 37 x 512 x 2048 11.7 -> 9.1, 1 x 1000 x 1280 10.8 -> 8.5, 1024 x 256 x 256 7.4 -> 6.6, 3x3 convolutions of 14 x 14 x 256 13.4 -> 11.9,
-	// of 7 x 7 x 512 17.3 -> 12.2. Where the shares stay long ( 9 x 6 x 7 x 512: 27 -> 36 ) or two slices only save a group or
-	// two ( 37 x 512 x 512: 7.5 -> 7.9 ) those stay.
-	if( tiles * slices > 256 || groups > slices * waves * 5 || ( groups > 24 && groups < 40 ) ) {
+	// Of the 478 one was slower so ( 196 x 384 x 512 8.0 -> 8.2 us ); all together take 0.856 of the tiles' time, the faster kernel with
+	// the best count of slices 0.850. us: 1 x 1000 x 1280 10.8 -> 7.7, 37 x 512 x 400 9.7 -> 6.9, 196 x 96 x 576 8.2 -> 7.8, 37 x 512 x 768
+	// 8.4 -> 8.1, x 2048 11.7 -> 8.9, 49 x 160 x 960 9.4 -> 7.7, 100 x 512 x 960 9.8 -> 8.4, 1024 x 256 x 256 7.3 -> 6.7; convolutions of
+	// 7 x 7 x 512 17.2 -> 12.3, 14 x 14 x 256 13.3 -> 11.7, 30 x 30 x 48 10.4 -> 6.8. Not 512 x 512 x 768 ( 10.3 and 10.5 ) or
+	// 9 x 6 x 7 x 512 ( 26 and 35 ).
+	if( cost > tilesCost( groups, static_cast<long long>( ceilDiv( given.M, 64 ) ) * ceilDiv( given.N, 64 ) * batch, convolution ) ) {
 		return false;
 	}
 	CMatMulArgs args = given;
 	args.StepsPerSplit = ceilDiv( groups, static_cast<long long>( slices ) * waves );
-	slices = ceilDiv( groups, static_cast<long long>( args.StepsPerSplit ) * waves );
 	if( slices > 1 && !sliceMeetingPlace( stream, static_cast<size_t>( tiles ) * slices * 1024, static_cast<size_t>( tiles ), &args.Partials, &args.Counters ) ) {
 		return false;
 	}
