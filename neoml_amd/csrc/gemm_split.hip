@@ -1,10 +1,10 @@
 // fp32 matrix products on the bf16 matrix instructions, each operand as the sum of three bf16 values.
 //
 // An fp32 value is exactly hi + mid + lo, where hi is the value rounded to bf16, mid what is left rounded to bf16, and lo
-// the rest: 8 significant bits each, signs of their own. Of the nine products of two such sums the six down to 2^-16 of the
-// largest are multiplied; the three that are left out ( mid lo, lo mid, lo lo ) are below 2^-26 of it, under the rounding of
-// an fp32 product. A matrix instruction sums 16 such products into the fp32 accumulator, where the fp32 one sums 2: six
-// roundings of the accumulator per 16 k instead of eight.
+// the rest: 8 significant bits each, signs of their own. Of the nine products of two such sums six are multiplied, down to
+// 2^-16 of the largest. The three that are left out ( mid lo, lo mid, lo lo ) come to 2^-24 of the product at most ( 1 + 2^-8 - 2^-17
+// squared: 0.99 of that ) and to 2^-27 as a rule. What that and the instruction's own roundings leave is measured at the
+// kernel: less than the fp32 instructions do.
 #include "gemm.h"
 #include <algorithm>
 #include <type_traits>
@@ -36,13 +36,12 @@ constexpr int SplitStep = 16; // k per matrix instruction and per step
 constexpr float OperandScale = 0x1p24f, SumScale = 0x1p-48f;
 
 // C[M x N] = act( A * B^T + bias ) (+ C, + residual), A and B rows of K values.
-// What bounds it: the card's power. Bare matrix instructions on random operands run at 1600 - 1700 TFLOP/s with the clock
-// held down to 1.5 GHz, a sixth of which is what can be had here; each value that is split ( 5.5 vector instructions ),
-// stored and read again costs on top, so the tiles are as large as the registers allow: a wavefront reads 2 x 2 blocks of
-// fragments for 24 matrix instructions. Measured against the fp32 instructions ( 64 x 64 and 128 x 128 tiles ), us:
-// 8192 x 2048 x 512 132 -> 106 ( 162 TFLOP/s ), 8192 x 512 x 2048 123 -> 113, 8192 x 512 x 512 35.5 -> 29.5, 8192 x 1024 x 256
-// 40 -> 29.5.
-// Error against 64 bits ( 2-norm ) on these: 1.5e-7 to 1.8e-7 where sequential fp32 sums have 2.9e-7 to 8.5e-7.
+// What bounds it: the instructions of a SIMD's one or two wavefronts, which a barrier a step keeps together ( 8192 x 2048 x 512: the
+// matrix pipe busy 52 % of the cycles, the vector instructions that split the operands another 36 % ), and the card's power ( back
+// to back the clock is 1.9 GHz; on zeros 2.4, 69 us instead of 90 ). So the tiles are as large as the registers allow: a wavefront
+// reads 2 x 2 blocks of fragments for 24 matrix instructions. Measured against the fp32 instructions, us: 8192 x 2048 x 512
+// 130 -> 93 ( 185 TFLOP/s ), 8192 x 512 x 2048 125 -> 94, 8192 x 512 x 512 37.4 -> 27.2, 8192 x 1024 x 256 37.2 -> 28.0.
+// Error against 64 bits ( 2-norm ), K from 132 to 2064: 1.2e-7 to 1.8e-7 where the fp32 instructions have 2.9e-7 to 8.5e-7.
 // WGM x WGN wavefronts, each MI x NI blocks of 32 x 32; WPE: wavefronts per SIMD the registers must leave room for; RAGGED: K is not a multiple of the step.
 template<int WGM, int WGN, int MI, int NI, int WPE, bool RAGGED>
 __global__ __launch_bounds__( 64 * WGM * WGN, WPE )
@@ -104,15 +103,13 @@ void splitProductKernel( const CMatMulArgs args )
 	// sums ( the error of 576 k falls from 3.6e-7 to 1.5e-7, of 2304 k from 7.2e-7 to 1.8e-7; the fp32 instructions: 4.2e-7 and
 	// 8.3e-7 ) and lean to both sides alike, for 2 - 4 % of the time. A chunk is a number of pairs of steps, so that it begins on
 	// LDS buffer 0; the numbers differ by one at most, and the longer chunks are the last ones, where a step may be missing.
-	// ( Mean error in 264, 288, 640, 1152 k: 3e-10, 1e-9 ( two of eighteen steps more with one sign ), 1e-10, 1e-10; with an odd number of chunks 4e-9, 5e-9, 4e-9, 3e-9. )
+	// ( Mean error in 264, 288, 640, 1152 k: 3e-10, 1e-9 ( two of eighteen steps more with one sign ), 1e-10, 1e-10; with an odd number
+	// of chunks 4e-9, 5e-9, 4e-9, 3e-9. )
 	constexpr int LongestChunk = 8;
 	const int chunks = ( totalSteps + 2 * LongestChunk - 1 ) / ( 2 * LongestChunk ) * 2;
 	const int pairsOfSteps = ( totalSteps + 1 ) >> 1;
 	const int chunkPairs = pairsOfSteps / chunks, firstLonger = chunks - ( pairsOfSteps - chunkPairs * chunks );
 	auto chunkSteps = [&]( int index ) -> int { return ( chunkPairs + ( index < firstLonger ? 0 : 1 ) ) * 2; };
-	int storedChunk = 0; // of the next step to store
-	int untilFlip = chunkSteps( 0 ); // steps to store until the sign changes
-	float scaleOfA = OperandScale;
 
 	float4 regA[ASlots], regB[BSlots];
 	// Requests the quads of a step. A step behind the last is asked of a descriptor of size zero ( zeros, no memory
@@ -145,7 +142,7 @@ void splitProductKernel( const CMatMulArgs args )
 		*reinterpret_cast<uint2*>( &lds[buf][at + Plane] ) = mid;
 		*reinterpret_cast<uint2*>( &lds[buf][at + 2 * Plane] ) = lo;
 	};
-	auto store = [&]( int buf ) {
+	auto store = [&]( int buf, float scaleOfA ) {
 #pragma unroll
 		for( int i = 0; i < ASlots; ++i ) {
 			if( AUnits % T == 0 || tileRow + i * RowsPerSlot < BM ) {
@@ -161,10 +158,6 @@ void splitProductKernel( const CMatMulArgs args )
 				storeUnit( buf, BM * 32 + unitAt( tileRow + i * RowsPerSlot ),
 					make_float4( v.x * OperandScale, v.y * OperandScale, v.z * OperandScale, v.w * OperandScale ) );
 			}
-		}
-		if( --untilFlip == 0 ) {
-			untilFlip = chunkSteps( ++storedChunk );
-			scaleOfA = -scaleOfA;
 		}
 	};
 
@@ -224,20 +217,20 @@ void splitProductKernel( const CMatMulArgs args )
 	// from LDS buffer ( s + 1 ) % 2 and the values of step s + 2 are split and stored to buffer s % 2, whose last readers
 	// were in step s - 1; one barrier ends the step. Reads, stores and vector instructions are dealt evenly over the step.
 	load( 0 );
-	store( 0 );
+	store( 0, OperandScale );
 	load( 1 );
-	store( 1 );
+	store( 1, OperandScale );
 	load( 2 );
 	__syncthreads();
 	readFrag( 0, frag[0] );
 	__syncthreads();
 	constexpr int Products = 6 * MI * NI; // matrix instructions of a step
 	constexpr int SplitVector = ( ASlots + BSlots ) * 26; // vector instructions of a step's quads, about
-	auto step = [&]( int s, auto curOf ) {
+	auto step = [&]( int s, float scaleOfStored, auto curOf ) {
 		constexpr int cur = decltype( curOf )::value, nxt = cur ^ 1;
 		__builtin_amdgcn_sched_barrier( 0 );
 		readFrag( nxt, frag[nxt] );
-		store( cur );
+		store( cur, scaleOfStored );
 		products( frag[cur] );
 #pragma unroll
 		for( int i = 0; i < Products; ++i ) {
@@ -254,12 +247,14 @@ void splitProductKernel( const CMatMulArgs args )
 	int s = 0, end = 0;
 	for( int chunk = 0; chunk < chunks; ++chunk ) {
 		end = min( end + chunkSteps( chunk ), totalSteps );
+		const float scale = chunk & 1 ? -OperandScale : OperandScale;
 		for( ; s + 1 < end; s += 2 ) {
-			step( s, std::integral_constant<int, 0>() );
-			step( s + 1, std::integral_constant<int, 1>() );
+			const float scaleOfStored = s + 2 < end ? scale : -scale; // ( the last pair stores the next chunk's first )
+			step( s, scaleOfStored, std::integral_constant<int, 0>() );
+			step( s + 1, scaleOfStored, std::integral_constant<int, 1>() );
 		}
 		if( s < end ) {
-			step( s, std::integral_constant<int, 0>() );
+			step( s, scale, std::integral_constant<int, 0>() );
 			++s;
 		}
 		const float sign = chunk & 1 ? -SumScale : SumScale;
@@ -447,8 +442,8 @@ static void launchSplit( hipStream_t stream, const CMatMulArgs& args, const dim3
 // 1152 -> 256, 282 -> 190; 64 x 28 x 28 x 128, 116 -> 83; 64 x 56 x 56 x 64, 119 -> 104 ), but the ReLU behind one decides by a
 // value's sign what a training step's gradients are made of. Another rounding, also a smaller one, moves a value next to zero to the
 // other side, and with each such value of the 1.3e7 of 64 x 56 x 56 x 64 a residual block's gradients move by 3e-4, where the sums
-// differ by 4e-7. A convolution cannot know what it is computed for, and its size says nothing about it: at every size they keep the
-// rounding that they have had.
+// differ by 4e-7. A convolution cannot know what it is computed for, and its size says nothing about it: they stay on the fp32
+// instructions at every size.
 bool trySplitProduct( hipStream_t stream, const CMatMulArgs& given, int batch, bool vec, int* rc )
 {
 	CMatMulArgs args = given;
