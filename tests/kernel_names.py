@@ -1,7 +1,7 @@
 """Which kernels the engine's calls launch: a program of its own, so that the profiler it asks stays out of the tests' process.
 
-Standard input: a JSON list of calls, ["nt", batch, m, n, k, pitch of C], ["conv", n, h, w, cin, cout, filter size, padding, stride] or
-["conv_backward", ...the same]. Standard output: a JSON list of lists of the kernels' names."""
+Standard input: a JSON list of calls, ["nt", batch, m, n, k, pitch of C], ["conv", n, h, w, cin, cout, filter size, padding, stride],
+["conv_backward", ...the same] or ["lstm", steps, batch, width, hidden]. Standard output: a JSON list of lists of the kernels' names."""
 import ctypes
 import json
 import sys
@@ -25,6 +25,15 @@ def main():
             if batch > 1:
                 return (a, b, c), lambda: hip.call("nhBatchMultiplyMatrixByTransposedMatrix", batch, hip.p(a), m, k, hip.p(b), n, hip.p(c), c.numel())
             return (a, b, c), lambda: hip.call("nhMultiplyMatrixByTransposedMatrix", hip.p(a), m, k, k, hip.p(b), n, k, hip.p(c), pitch, c.numel())
+        if kind == "lstm":
+            steps, batch, width, hidden = sizes
+            size = ctypes.c_size_t(0)
+            hip.na.check(hip.lib.nhLstmWorkspaceSize(hidden, width, steps, batch, ctypes.byref(size)))
+            x, y, work = blob(steps, batch, width), blob(steps, batch, hidden), blob(size.value // 4 + 1)
+            w_in, w_rec, free = blob(4 * hidden, width), blob(4 * hidden, hidden), blob(4 * hidden)
+            return (x, y, work, w_in, w_rec, free), lambda: hip.call(
+                "nhLstm", hidden, width, hip.p(w_in), hip.p(free), hip.p(w_rec), hip.p(free), 0, steps, batch, None, None, hip.p(x), None,
+                hip.p(y), hip.p(work), size)
         batch, h, w, cin, cout, f, pad, stride = sizes
         d = hip.conv_desc(batch, h, w, cin, cout, f, f, pad, pad, stride, stride)
         x, filt, y = blob(batch, h, w, cin), blob(cout, f, f, cin), blob(batch, d.resultHeight, d.resultWidth, cout)

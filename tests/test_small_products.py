@@ -26,6 +26,7 @@ SHAPES = [(1, 1, 128), (1, 1000, 1280), (31, 33, 132), (32, 32, 384), (33, 65, 2
 BATCHES = [(8, 33, 65, 132), (4, 60, 100, 256), (3, 1, 50, 388), (200, 7, 31, 128)]
 CONVOLUTIONS = [(1, 7, 7, 512, 512, 3, 1, False), (1, 14, 14, 256, 256, 3, 1, True), (1, 28, 28, 256, 512, 1, 2, False),
                 (2, 5, 3, 80, 36, 5, 2, True), (1, 2, 50, 256, 250, 3, 1, True), (3, 9, 11, 16, 48, 3, 1, False), (1, 30, 30, 48, 48, 3, 1, True)]
+STEPS = [(132, 5), (260, 33)]  # ( hidden, batch )
 # ( batch, height, width, channels, filters, filter size, padding )
 GRADIENTS = [(1, 7, 7, 256, 256, 3, 1), (2, 9, 11, 80, 48, 5, 2), (1, 5, 6, 33, 512, 3, 0), (1, 30, 29, 48, 32, 3, 1)]
 
@@ -35,7 +36,7 @@ def launched():
     import nhtest
     calls = [("nt", 1, m, n, k, n + 3) for m, n, k in SHAPES] + [("nt", b, m, n, k, n) for b, m, n, k in BATCHES]
     calls += [("conv", n, h, w, cin, cout, f, f // 2, stride) for n, h, w, cin, cout, f, stride, _ in CONVOLUTIONS]
-    calls += [("conv_backward",) + c + (1,) for c in GRADIENTS]
+    calls += [("conv_backward",) + c + (1,) for c in GRADIENTS] + [("lstm", 2, batch, 24, hidden) for hidden, batch in STEPS]
     return dict(zip(calls, nhtest.kernel_names(calls)))
 
 
@@ -70,9 +71,10 @@ def test_batches(hip, launched, batch, m, n, k):
         _check(c[i], a[i].double(), b[i].double(), k)
 
 
-@pytest.mark.parametrize("hidden,batch", [(132, 5), (260, 33)])
-def test_products_added_to_the_result(hip, hidden, batch):
+@pytest.mark.parametrize("hidden,batch", STEPS)
+def test_products_added_to_the_result(hip, launched, hidden, batch):
     """The steps of an LSTM whose width no other path takes: gates += h * W^T."""
+    assert "smallProductKernel<0, %d>" % (8 if hidden > 240 else 4) in launched["lstm", 2, batch, 24, hidden]
     import numpy as np
     from nhtest import Cpu, assert_close
     g = np.random.default_rng(hidden)

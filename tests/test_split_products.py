@@ -190,12 +190,12 @@ def test_values_without_finite_parts(hip):
     assert c[5000, 17] == float("inf")
 
 
-# ( a product for each of the three tile shapes )
+# ( a product for each of the three tile shapes; no sums next to the smallest normal number, where 2^-126 is lost to any kernel )
 @pytest.mark.parametrize("m,n,k", [(8192, 2048, 512), (8192, 512, 1024), (2048, 1024, 516)])
-@pytest.mark.parametrize("of_a,of_b", [(-104, 60), (-116, 60), (60, -116), (-125, 100), (-110, 10)])
+@pytest.mark.parametrize("of_a,of_b", [(-104, 60), (-116, 60), (60, -116), (-125, 100), (-110, 10), (-50, -50), (110, -60), (-90, 103), (45, 45)])
 def test_small_values_with_large_partners(hip, m, n, k, of_a, of_b):
     """Normal values whose lower parts would lie under the smallest normal number, against partners that bring the products back
-    into the middle of the range. In the 2-norm k products that are added one by one, the partial sums growing as a random walk, are
+    into the middle of the range; small products of both; values and sums that overflow times the factors of the split. In the 2-norm k products that are added one by one, the partial sums growing as a random walk, are
     off by 2^-24 sqrt( k / 6 ) ( each rounding 2^-24 / sqrt( 3 ) of a partial sum )."""
     torch = hip.torch
     g = torch.Generator(device=hip.dev).manual_seed(m + k)
