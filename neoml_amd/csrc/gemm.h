@@ -66,6 +66,7 @@ struct CMatMulArgs {
 	// AM_ConvClasses: the dense result is [images][OutH][OutW][Ldc], DenseM pixels in all
 	int OutH, OutW, OutUpH, OutUpW, DenseM;
 	CConvClass Class[MaxConvClasses];
+	int SmallTile; // smallProductKernel: 0: 16 x 16, 1: 16 x 32, 2: 32 x 32
 	// epilogue of the fused blocks: C = act( A * B + bias ) + Residual; Residual has C's layout, may be C itself
 	CFusedActivation Act;
 	const float* Residual;
@@ -103,10 +104,20 @@ constexpr int Threads = 256;
 // them ). true: launched, *rc is the launch's code; false: not one that it is for.
 bool trySplitProduct( hipStream_t stream, const CMatMulArgs& args, int batch, bool vec, int* rc );
 
+// A meeting place handed in by the caller instead of the stream's block: the launch neither allocates nor looks the
+// stream up, and fails when the place is too small.
+struct CSliceMeeting {
+	float* Partials;
+	size_t PartialFloats;
+	unsigned* Counters;
+	size_t CounterCount;
+};
+
 // ( gemm_small.hip ) the same for results of a few tiles; A also as the im2col view of an image whose channel count is a multiple
-// of 16.
+// of 16. fixedMeeting: where its slices meet ( none if they would not fit ) instead of the stream's block.
 constexpr int MaxSmallSlices = 16;
-bool trySmallProduct( hipStream_t stream, const CMatMulArgs& args, bool convolution, int batch, bool vec, int* rc );
+bool trySmallProduct( hipStream_t stream, const CMatMulArgs& args, bool convolution, int batch, bool vec, int* rc,
+	const CSliceMeeting* fixedMeeting = nullptr );
 
 // The stream's block of partial tiles and arrival counters for reductions that are cut into slices ( the counters are zero
 // between launches ). false: none to be had ( a capturing stream, a shared stream handle, no memory ).

@@ -1173,15 +1173,6 @@ bool sliceMeetingPlace( hipStream_t stream, size_t partialFloats, size_t counter
 	return true;
 }
 
-// A meeting place handed in by the caller instead of the stream's block: the launch neither allocates nor looks the
-// stream up, and fails when the place is too small.
-struct CSliceMeeting {
-	float* Partials;
-	size_t PartialFloats;
-	unsigned* Counters;
-	size_t CounterCount;
-};
-
 // The meeting place of nhBlobConvolutionNoAlloc: a fixed array in the library's own device image, one copy per GPU,
 // held from the moment the library is loaded on that GPU until the process ends. Partial tiles first, the arrival
 // counters behind them. Every call on a GPU shares that GPU's copy, so calls that overlap there race.
@@ -2390,8 +2381,8 @@ static int matMulNTMeeting( hipStream_t stream, const float* a, int lda, const f
 	}
 	const bool vec = isAligned16( a ) && isAligned16( b ) && K % 4 == 0 && lda % 4 == 0 && ldb % 4 == 0
 		&& strideA % 4 == 0 && strideB % 4 == 0 && fitsBuffer( M, lda, K ) && fitsBuffer( N, ldb, K );
-	if( fixedMeeting == nullptr && ( trySmallProduct( stream, args, false, batch, vec, &rc )
-		|| trySplitProduct( stream, args, batch, vec, &rc ) ) )
+	if( trySmallProduct( stream, args, false, batch, vec, &rc, fixedMeeting )
+		|| ( fixedMeeting == nullptr && trySplitProduct( stream, args, batch, vec, &rc ) ) )
 	{
 		return rc;
 	}
@@ -2702,7 +2693,7 @@ int convImplicitGemm( hipStream_t stream, const nhConvDesc& d, const float* sour
 			1, 0, 0, 0, freeTerm, false, act, nullptr, fixedMeeting );
 	}
 	int smallRc = NH_OK;
-	if( fixedMeeting == nullptr && trySmallProduct( stream, args, true, 1, vec, &smallRc ) ) {
+	if( trySmallProduct( stream, args, true, 1, vec, &smallRc, fixedMeeting ) ) {
 		return smallRc;
 	}
 	if( d.filterHeight == 1 && d.filterWidth == 1 ) {

@@ -8,33 +8,37 @@ typedef float f32x4 __attribute__( ( ext_vector_type( 4 ) ) );
 
 // C[M x N] = act( A * B^T + bias ) (+ C, + residual), A rows of K values or the im2col view of an image whose channel count is
 // a multiple of 16, B rows of K values.
-// What bounds such a product is latency: a chain of K steps, each with a barrier, on a few workgroups.
-// So a workgroup is one 32 x 32 tile whose reduction is dealt to its WAVES wavefronts and, where the tiles leave compute
-// units idle, to several workgroups. A wavefront fetches its share straight into operand registers, 16 k at a time: lane
-// ( row, quad ) holds k = 16 g + 4 quad .. + 3 of its rows, so that four lanes cover 64 bytes of a row, for 2 x 2 blocks of
-// v_mfma_f32_16x16x4_f32; eight such groups are in flight. It meets no barrier until its share is done. The shares are
-// summed through LDS in the order of k, the slices through scratch memory by the one that arrives last, which fetches the
-// others' tiles all at once.
-template<int AMODE, int WAVES>
-__global__ __launch_bounds__( 64 * WAVES, 2 )
-void smallProductKernel( const CMatMulArgs args )
+// What bounds such a product is latency: a chain of K steps, each with a barrier, on a few workgroups, and the instructions in
+// front of its first load and behind its last sum ( a launch by itself takes 1.6 us, a few hundred instructions of a wavefront 1 us ).
+// So a workgroup is one tile of 16 MB x 16 NB whose reduction is dealt to its WAVES wavefronts and, where the tiles leave compute
+// units idle, to several workgroups. A wavefront fetches its share into registers, 16 k at a time with DEPTH such groups in flight,
+// turns them round in its own part of LDS ( pass, below ) and multiplies MB x NB blocks by v_mfma_f32_16x16x4_f32, one group behind
+// what it turns. It meets no barrier until its share is done. The shares are summed through LDS in the order of k, the
+// slices through scratch memory by the one that arrives last, which fetches the others' tiles all at once.
+// us, for operands loaded straight into the matrix instructions' layout and 32 x 32 tiles only, and now: 37 x 512 x 512 7.5 -> 3.9,
+// x 2048 x 512 8.1 -> 5.2, x 512 x 2048 9.2 -> 7.1, 49 x 160 x 960 7.6 -> 5.0, 196 x 64 x 384 7.6 -> 3.1, 1 x 1000 x 1280 7.7 -> 4.9;
+// 3 x 3 convolutions of 56 x 56 x 64 9.8 -> 6.7, 28 x 28 x 128 12.0 -> 7.1, 14 x 14 x 256 12.0 -> 7.9, 7 x 7 x 512 12.6 -> 10.2.
+template<int AMODE, int WAVES, int MB, int NB, int DEPTH>
+__device__ __forceinline__ void smallProductTile( const CMatMulArgs& args, float* lds, unsigned* arrived )
 {
 	constexpr bool IsTaps = ( AMODE == AM_ConvTaps );
 	static_assert( IsTaps || AMODE == AM_RowsK, "operands that are K-major" );
+	static_assert( MB * NB <= MB + NB && MB + NB <= 4, "the sums take the place of the operands in LDS" );
 	constexpr int T = 64 * WAVES;
-	constexpr int Batch = 2, Sets = 4; // groups of 16 k to a register set, sets
-	constexpr int PerThread = 1024 / T; // elements of the tile that a thread sums and writes
-	__shared__ float lds[WAVES][16][64];
-	__shared__ unsigned arrived;
+	constexpr int Regs = 4 * MB * NB; // accumulators of a lane
+	constexpr int Elements = 64 * Regs;
+	constexpr int Stage = ( MB + NB ) * 256; // floats of LDS that a wavefront stages its operands in
+	constexpr int PerThread = ( Elements + T - 1 ) / T; // elements of the tile that a thread sums and writes
 
 	const int tid = threadIdx.x;
 	const int lane = tid & 63;
 	const int wave = __builtin_amdgcn_readfirstlane( tid >> 6 );
-	const int l16 = lane & 15, quad = lane >> 4;
+	const int l16 = lane & 15, quad = lane >> 4; // of the matrix instructions' operands
+	const int loadRow = lane >> 2, loadQuad = lane & 3; // of the loads
 	const int tile = xcdSwizzle( blockIdx.x, gridDim.x );
 	int tileM, tileN;
 	fastDivMod( tile, args.TilesN, args.TilesNMagic, tileM, tileN );
-	const int m0 = tileM * 32, n0 = tileN * 32;
+	const int m0 = tileM * 16 * MB, n0 = tileN * 16 * NB;
 	const int batch = blockIdx.y, slice = blockIdx.z;
 	const int M = args.M, N = args.N, K = args.K;
 	const float* baseA = args.A + batch * args.BatchStrideA;
@@ -45,26 +49,30 @@ void smallProductKernel( const CMatMulArgs args )
 	const int firstGroup = ( slice * WAVES + wave ) * args.StepsPerSplit;
 	const int lastGroup = min( firstGroup + args.StepsPerSplit, groups );
 
-	// the lane's two rows of A and of B
-	unsigned offA[2], offB[2];
-	unsigned baseOfA[2] = {}; // in floats, of tap ( 0, 0 ): unsigned arithmetic, it may lie in front of the image
-	int imageH0[2] = {}, imageW0[2] = {};
+	// the lane's rows of A and of B
+	unsigned offA[MB], offB[NB];
+	unsigned baseOfA[MB] = {}; // in floats, of tap ( 0, 0 ): unsigned arithmetic, it may lie in front of the image
+	int imageH0[MB] = {}, imageW0[MB] = {};
 	int tapCi = 0, tapKh = 0, tapKw = 0;
 	auto tapOffsets = [&]() {
 		const int dh = tapKh * args.DilH, dw = tapKw * args.DilW; // ( scalar )
 		const unsigned tapFloats = ( static_cast<unsigned>( dh ) * static_cast<unsigned>( args.W ) + static_cast<unsigned>( dw ) )
 			* static_cast<unsigned>( args.Cin );
 #pragma unroll
-		for( int i = 0; i < 2; ++i ) {
+		for( int i = 0; i < MB; ++i ) {
 			const bool ok = tapKh < args.Fh && static_cast<unsigned>( imageH0[i] + dh ) < static_cast<unsigned>( args.H )
 				&& static_cast<unsigned>( imageW0[i] + dw ) < static_cast<unsigned>( args.W );
 			offA[i] = ok ? ( baseOfA[i] + tapFloats ) * 4u : OutOfRange;
 		}
 	};
 #pragma unroll
-	for( int i = 0; i < 2; ++i ) {
-		const int n = n0 + i * 16 + l16, m = m0 + i * 16 + l16;
-		offB[i] = n < N ? ( static_cast<unsigned>( n ) * static_cast<unsigned>( args.Ldb ) + quad * 4u ) * 4u : OutOfRange;
+	for( int i = 0; i < NB; ++i ) {
+		const int n = n0 + i * 16 + loadRow;
+		offB[i] = n < N ? ( static_cast<unsigned>( n ) * static_cast<unsigned>( args.Ldb ) + loadQuad * 4u ) * 4u : OutOfRange;
+	}
+#pragma unroll
+	for( int i = 0; i < MB; ++i ) {
+		const int m = m0 + i * 16 + loadRow;
 		if constexpr( IsTaps ) {
 			int t, wo, image, ho;
 			fastDivMod( m, args.Wo, args.WoMagic, t, wo );
@@ -72,9 +80,9 @@ void smallProductKernel( const CMatMulArgs args )
 			imageH0[i] = m < M ? ho * args.StrideH - args.PadH : -0x40000000;
 			imageW0[i] = wo * args.StrideW - args.PadW;
 			baseOfA[i] = static_cast<unsigned>( image * args.H * args.W * args.Cin ) + ( static_cast<unsigned>( imageH0[i] )
-				* static_cast<unsigned>( args.W ) + static_cast<unsigned>( imageW0[i] ) ) * static_cast<unsigned>( args.Cin ) + quad * 4u;
+				* static_cast<unsigned>( args.W ) + static_cast<unsigned>( imageW0[i] ) ) * static_cast<unsigned>( args.Cin ) + loadQuad * 4u;
 		} else {
-			offA[i] = m < M ? ( static_cast<unsigned>( m ) * static_cast<unsigned>( args.Lda ) + quad * 4u ) * 4u : OutOfRange;
+			offA[i] = m < M ? ( static_cast<unsigned>( m ) * static_cast<unsigned>( args.Lda ) + loadQuad * 4u ) * 4u : OutOfRange;
 		}
 	}
 	if constexpr( IsTaps ) {
@@ -85,114 +93,212 @@ void smallProductKernel( const CMatMulArgs args )
 		tapOffsets();
 	}
 
-	float4 a[Sets][Batch][2], b[Sets][Batch][2];
-	// ( a group behind the share's last is asked of a descriptor of size zero: zeros, no memory access )
-	auto load = [&]( int group, int set ) {
+	// what the thread adds behind the sums, asked for in front of them: columns of its elements e = tid + i T ( see below )
+	float free[PerThread] = {};
+	const CFusedActivation act = withParam( args.Act );
+	if( args.Bias != nullptr ) {
+		const __amdgpu_buffer_rsrc_t bias = __builtin_amdgcn_make_buffer_rsrc( const_cast<float*>( args.Bias ), 0, N * 4u, 0x00020000 );
 #pragma unroll
-		for( int g = 0; g < Batch; ++g ) {
-			const unsigned range = group + g < lastGroup ? BufferBytes : 0u;
-			const __amdgpu_buffer_rsrc_t bufA = __builtin_amdgcn_make_buffer_rsrc( const_cast<float*>( baseA ), 0, range, 0x00020000 );
-			const __amdgpu_buffer_rsrc_t bufB = __builtin_amdgcn_make_buffer_rsrc( const_cast<float*>( baseB ), 0, range, 0x00020000 );
-			const unsigned uniB = static_cast<unsigned>( group + g ) * 64u;
-			const bool inK = IsTaps || ( group + g ) * 16 + quad * 4 < K; // ( K is a multiple of 4 )
-#pragma unroll
-			for( int i = 0; i < 2; ++i ) {
-				a[set][g][i] = bufferLoad4( bufA, inK ? offA[i] : OutOfRange, IsTaps ? static_cast<unsigned>( tapCi ) * 4u : uniB );
-				b[set][g][i] = bufferLoad4( bufB, inK ? offB[i] : OutOfRange, uniB );
-			}
-			if constexpr( IsTaps ) {
-				tapCi += 16;
-				if( tapCi >= args.Cin ) {
-					tapCi = 0;
-					if( ++tapKw == args.Fw ) {
-						tapKw = 0;
-						++tapKh;
-					}
-					tapOffsets();
-				}
-			}
+		for( int i = 0; i < PerThread; ++i ) {
+			free[i] = bufferLoad1( bias, ( n0 + ( ( wave + i * WAVES ) / 4 % NB ) * 16 + l16 ) * 4u );
 		}
-	};
-	f32x4 acc[2][2];
-#pragma unroll
-	for( int r = 0; r < 16; ++r ) {
-		acc[r >> 3][( r >> 2 ) & 1][r & 3] = 0.f;
 	}
-	auto multiply = [&]( int set ) {
+
+	const __amdgpu_buffer_rsrc_t bufA = makeBuffer( baseA ), bufB = makeBuffer( baseB );
+	float4 a[DEPTH][MB], b[DEPTH][NB];
+	unsigned uniform = static_cast<unsigned>( firstGroup ) * 64u; // of the next group, in bytes
+	const unsigned ragged = !IsTaps && ( K & 15 ) != 0 ? static_cast<unsigned>( groups - 1 ) * 64u : OutOfRange;
+	auto load = [&]( int set ) {
+		if( !IsTaps && uniform == ragged ) { // the last group of all: some quads lie behind K ( a multiple of 4 )
+			const bool inK = static_cast<int>( uniform >> 2 ) + loadQuad * 4 < K;
 #pragma unroll
-		for( int g = 0; g < Batch; ++g ) {
-			auto product = [&]( auto partOf ) {
+			for( int i = 0; i < MB; ++i ) {
+				offA[i] = inK ? offA[i] : OutOfRange;
+			}
 #pragma unroll
-				for( int mi = 0; mi < 2; ++mi ) {
+			for( int i = 0; i < NB; ++i ) {
+				offB[i] = inK ? offB[i] : OutOfRange;
+			}
+		}
 #pragma unroll
-					for( int ni = 0; ni < 2; ++ni ) {
-						acc[mi][ni] = __builtin_amdgcn_mfma_f32_16x16x4f32( partOf( a[set][g][mi] ), partOf( b[set][g][ni] ), acc[mi][ni], 0, 0, 0 );
-					}
+		for( int i = 0; i < MB; ++i ) {
+			a[set][i] = bufferLoad4( bufA, offA[i], IsTaps ? static_cast<unsigned>( tapCi ) * 4u : uniform );
+		}
+#pragma unroll
+		for( int i = 0; i < NB; ++i ) {
+			b[set][i] = bufferLoad4( bufB, offB[i], uniform );
+		}
+		uniform += 64u;
+		if constexpr( IsTaps ) {
+			tapCi += 16;
+			if( tapCi >= args.Cin ) {
+				tapCi = 0;
+				if( ++tapKw == args.Fw ) {
+					tapKw = 0;
+					++tapKh;
 				}
-			};
-			product( []( const float4& v ) { return v.x; } );
-			product( []( const float4& v ) { return v.y; } );
-			product( []( const float4& v ) { return v.z; } );
-			product( []( const float4& v ) { return v.w; } );
+				tapOffsets();
+			}
 		}
 	};
-	auto step = [&]( int group, auto setOf ) {
-		constexpr int set = decltype( setOf )::value;
-		multiply( set );
-		__builtin_amdgcn_sched_barrier( 0 );
-		load( group + Sets * Batch, set );
-		__builtin_amdgcn_sched_barrier( 0 );
+	// ( a block of its own has two accumulators, of the even and the odd quarters: a matrix instruction waits for the one whose sum
+	// it continues )
+	constexpr int Chains = MB * NB == 1 ? 2 : 1;
+	f32x4 acc[Chains][MB][NB];
+#pragma unroll
+	for( int c = 0; c < Chains; ++c ) {
+#pragma unroll
+		for( int mi = 0; mi < MB; ++mi ) {
+#pragma unroll
+			for( int ni = 0; ni < NB; ++ni ) {
+				acc[c][mi][ni] = f32x4{ 0.f, 0.f, 0.f, 0.f };
+			}
+		}
+	}
+	// A wavefront's operands pass through its own part of LDS ( instructions of one wavefront are executed there in their order: no
+	// barrier, one buffer ): asked for with four lanes to a row and read back with rows across lanes, as the matrix instructions
+	// want them. Where consecutive lanes ask for 16 bytes of different rows the memory unit delivers 16 bytes a clock, where four
+	// lanes ask for 64 neighbouring bytes 64 ( 288 KB by one workgroup in 9.2 and 4.1 us ). The quads of a row are dealt so that
+	// 16 lanes of a read meet all banks.
+	float4* stage = reinterpret_cast<float4*>( lds + wave * Stage ); // blocks of 16 rows x 64 bytes
+	float4* stageWrite = stage + loadRow * 4 + ( loadQuad ^ ( ( loadRow >> 2 ) & 3 ) );
+	const float4* stageRead = stage + l16 * 4 + ( quad ^ ( ( l16 >> 2 ) & 3 ) );
+	struct COperands { float4 X[MB], Y[NB]; } even, odd; // of this step and the next
+	auto pass = [&]( int set, COperands& to ) {
+#pragma unroll
+		for( int i = 0; i < MB; ++i ) {
+			stageWrite[i * 64] = a[set][i];
+		}
+#pragma unroll
+		for( int i = 0; i < NB; ++i ) {
+			stageWrite[( MB + i ) * 64] = b[set][i];
+		}
+		__builtin_amdgcn_wave_barrier();
+		asm volatile( "" ::: "memory" );
+#pragma unroll
+		for( int i = 0; i < MB; ++i ) {
+			to.X[i] = stageRead[i * 64];
+		}
+#pragma unroll
+		for( int i = 0; i < NB; ++i ) {
+			to.Y[i] = stageRead[( MB + i ) * 64];
+		}
+		__builtin_amdgcn_wave_barrier();
+		asm volatile( "" ::: "memory" );
 	};
-	if( firstGroup < lastGroup ) {
-		load( firstGroup, 0 );
-		load( firstGroup + Batch, 1 );
-		load( firstGroup + 2 * Batch, 2 );
-		load( firstGroup + 3 * Batch, 3 );
-		for( int group = firstGroup; group < lastGroup; group += Sets * Batch ) {
-			step( group, std::integral_constant<int, 0>() );
-			if( group + Batch < lastGroup ) {
-				step( group + Batch, std::integral_constant<int, 1>() );
+	auto multiply = [&]( const COperands& of ) {
+		auto product = [&]( int chain, auto partOf ) {
+#pragma unroll
+			for( int mi = 0; mi < MB; ++mi ) {
+#pragma unroll
+				for( int ni = 0; ni < NB; ++ni ) {
+					acc[chain][mi][ni] = __builtin_amdgcn_mfma_f32_16x16x4f32( partOf( of.X[mi] ), partOf( of.Y[ni] ), acc[chain][mi][ni], 0, 0, 0 );
+				}
 			}
-			if( group + 2 * Batch < lastGroup ) {
-				step( group + 2 * Batch, std::integral_constant<int, 2>() );
+		};
+		product( 0, []( const float4& v ) { return v.x; } );
+		product( Chains - 1, []( const float4& v ) { return v.y; } );
+		product( 0, []( const float4& v ) { return v.z; } );
+		product( Chains - 1, []( const float4& v ) { return v.w; } );
+	};
+	static_assert( DEPTH % 2 == 0, "steps alternate" );
+	const int sets = lastGroup - firstGroup;
+	if( sets > 0 ) {
+#pragma unroll
+		for( int u = 0; u < DEPTH; ++u ) {
+			if( u < sets ) {
+				load( u );
 			}
-			if( group + 3 * Batch < lastGroup ) {
-				step( group + 3 * Batch, std::integral_constant<int, 3>() );
+		}
+		pass( 0, even );
+		// ( no condition inside: a wait counts the loads behind the awaited one, which all paths to it must have asked for )
+		int left = sets;
+		for( ; left >= 2 * DEPTH; left -= DEPTH ) {
+#pragma unroll
+			for( int u = 0; u < DEPTH; u += 2 ) {
+				__builtin_amdgcn_sched_barrier( 0 );
+				load( u );
+				pass( u + 1, odd );
+				__builtin_amdgcn_sched_barrier( 0 );
+				multiply( even );
+				__builtin_amdgcn_sched_barrier( 0 );
+				load( u + 1 );
+				pass( ( u + 2 ) % DEPTH, even );
+				__builtin_amdgcn_sched_barrier( 0 );
+				multiply( odd );
+			}
+		}
+		if( left >= DEPTH ) {
+			left -= DEPTH;
+#pragma unroll
+			for( int u = 0; u < DEPTH; u += 2 ) {
+				if( u < left ) {
+					load( u );
+				}
+				pass( u + 1, odd );
+				multiply( even );
+				if( u + 1 < left ) {
+					load( u + 1 );
+				}
+				pass( ( u + 2 ) % DEPTH, even ); // ( of the last step, where nothing is left: values that are not used )
+				multiply( odd );
+			}
+		}
+#pragma unroll
+		for( int u = 0; u + 1 < DEPTH; u += 2 ) {
+			if( u < left ) {
+				pass( u + 1, odd );
+				multiply( even );
+			}
+			if( u + 1 < left ) {
+				if( u + 2 < DEPTH ) {
+					pass( u + 2, even );
+				}
+				multiply( odd );
 			}
 		}
 	}
 
 #pragma unroll
-	for( int r = 0; r < 16; ++r ) {
-		lds[wave][r][lane] = acc[r >> 3][( r >> 2 ) & 1][r & 3];
+	for( int r = 0; r < Regs; ++r ) {
+		float v = acc[0][r / ( 4 * NB )][( r / 4 ) % NB][r & 3];
+		if constexpr( Chains == 2 ) {
+			v += acc[1][0][0][r & 3];
+		}
+		lds[wave * Stage + r * 64 + lane] = v;
 	}
 	__syncthreads();
-	// from here on a thread owns elements ( r = wave + i WAVES, lane ) of the tile
+	// from here on a thread owns elements e = tid + i T of the tile: of register e / 64 of lane e % 64
 	float sum[PerThread];
+	const bool owns = Elements % T == 0 || tid < Elements;
 #pragma unroll
 	for( int i = 0; i < PerThread; ++i ) {
 		sum[i] = 0.f;
+		if( owns ) {
 #pragma unroll
-		for( int w = 0; w < WAVES; ++w ) {
-			sum[i] += lds[w][wave + i * WAVES][lane];
+			for( int w = 0; w < WAVES; ++w ) {
+				sum[i] += lds[w * Stage + tid + i * T];
+			}
 		}
 	}
 	const int slices = args.SplitK;
 	if( slices > 1 ) {
 		// Values cross between the L2 caches of the XCDs through agent-scope atomic accesses, which go past them; a wave's
 		// stores are complete before the barrier in front of the count, and the reads come behind the barrier that follows it.
-		unsigned* first = reinterpret_cast<unsigned*>( args.Partials ) + static_cast<long long>( tile ) * slices * 1024 + tid;
+		unsigned* first = reinterpret_cast<unsigned*>( args.Partials ) + static_cast<long long>( tile ) * slices * Elements + tid;
+		if( owns ) {
 #pragma unroll
-		for( int i = 0; i < PerThread; ++i ) {
-			__hip_atomic_store( first + slice * 1024 + i * T, __float_as_uint( sum[i] ), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT );
+			for( int i = 0; i < PerThread; ++i ) {
+				__hip_atomic_store( first + slice * Elements + i * T, __float_as_uint( sum[i] ), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT );
+			}
 		}
 		__builtin_amdgcn_s_waitcnt( 0x0F70 ); // vmcnt( 0 ): this wave's stores have been acknowledged
 		__syncthreads();
 		if( tid == 0 ) {
-			arrived = __hip_atomic_fetch_add( args.Counters + tile, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT );
+			*arrived = __hip_atomic_fetch_add( args.Counters + tile, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT );
 		}
 		__syncthreads();
-		if( arrived != static_cast<unsigned>( slices - 1 ) ) {
+		if( *arrived != static_cast<unsigned>( slices - 1 ) ) {
 			return;
 		}
 		unsigned v[MaxSmallSlices][PerThread];
@@ -200,7 +306,7 @@ void smallProductKernel( const CMatMulArgs args )
 		for( int s = 0; s < MaxSmallSlices; ++s ) {
 #pragma unroll
 			for( int i = 0; i < PerThread; ++i ) {
-				v[s][i] = s < slices ? __hip_atomic_load( first + s * 1024 + i * T, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT ) : 0u;
+				v[s][i] = s < slices && owns ? __hip_atomic_load( first + s * Elements + i * T, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT ) : 0u;
 			}
 		}
 #pragma unroll
@@ -215,16 +321,18 @@ void smallProductKernel( const CMatMulArgs args )
 			__hip_atomic_store( args.Counters + tile, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT );
 		}
 	}
-	// element ( r, lane ): block ( r / 8, r / 4 % 2 ), of it column lane % 16 of row 4 ( lane / 16 ) + r % 4
+	if( !owns ) {
+		return;
+	}
+	// element ( r, lane ): block ( r / ( 4 NB ), r / 4 % NB ), of it column lane % 16 of row 4 ( lane / 16 ) + r % 4
 	float* C = args.C + batch * args.BatchStrideC;
-	const CFusedActivation act = withParam( args.Act );
 #pragma unroll
 	for( int i = 0; i < PerThread; ++i ) {
 		const int r = wave + i * WAVES;
-		const int row = m0 + ( r >> 3 ) * 16 + quad * 4 + ( r & 3 ), n = n0 + ( ( r >> 2 ) & 1 ) * 16 + l16;
+		const int row = m0 + ( r / ( 4 * NB ) ) * 16 + quad * 4 + ( r & 3 ), n = n0 + ( ( r / 4 ) % NB ) * 16 + l16;
 		if( row < M && n < N ) {
 			const long long at = static_cast<long long>( row ) * args.Ldc + n;
-			float v = sum[i] + ( args.Bias != nullptr ? args.Bias[n] : 0.f );
+			float v = sum[i] + free[i];
 			if( args.Accumulate ) {
 				v += C[at];
 			}
@@ -237,65 +345,112 @@ void smallProductKernel( const CMatMulArgs args )
 	}
 }
 
-// What this kernel is expected to take, in microseconds, with shares of so many groups. Fitted to some 1700 launches over
-// 478 products and convolutions of up to 256 tiles, K from 128 to 8196, as all figures here are.
-static double smallCost( int waves, int share, int slices, long long tiles )
+// The tile is chosen per launch ( CMatMulArgs::SmallTile ).
+template<int AMODE, int WAVES>
+__global__ __launch_bounds__( 64 * WAVES, 2 )
+void smallProductKernel( const CMatMulArgs args )
 {
-	// ( the groups that all compute units have to do, to each: loads and matrix instructions share what there is )
-	const double fill = static_cast<double>( tiles ) * slices * share / 256;
-	const double meeting = slices > 1 ? 1.2 + 0.05 * slices : 0.0;
-	return waves == 8 ? 4.6 + 0.25 * share + 0.83 * ( ( share + 1 ) / 2 ) + 0.45 * fill + meeting : 4.4 + 0.27 * share + 0.2 * fill + meeting;
+	__shared__ float lds[WAVES * 1024];
+	__shared__ unsigned arrived;
+	if( args.SmallTile == 0 ) {
+		smallProductTile<AMODE, WAVES, 1, 1, 6>( args, lds, &arrived );
+	} else if( args.SmallTile == 1 ) {
+		smallProductTile<AMODE, WAVES, 1, 2, 4>( args, lds, &arrived );
+	} else {
+		smallProductTile<AMODE, WAVES, 2, 2, 4>( args, lds, &arrived );
+	}
 }
 
-// What the 64 x 64 tiles take: chains of steps below 32 steps, slices of them from there on.
-static double tilesCost( int steps, long long tiles64, bool convolution )
+constexpr int SmallTiles = 3;
+constexpr int SmallTileM[SmallTiles] = { 16, 16, 32 }, SmallTileN[SmallTiles] = { 16, 32, 32 };
+constexpr int MaxSmallWorkgroups = 384;
+
+// What this kernel is expected to take, in microseconds. Fitted to 2177 launches over 302 products and convolutions ( 1 to 17000
+// rows, 16 to 2500 columns, K from 28 to 4608 ), standard deviation 9 %.
+static double smallCost( int tile, int waves, int share, int slices, long long tiles, bool convolution )
 {
-	if( steps < 32 ) {
-		return 3.3 + 0.256 * steps + ( convolution ? 0.6 : 0.0 );
-	}
-	return 6.7 + steps * ( 0.033 + 0.0008 * static_cast<double>( tiles64 ) ) + ( convolution ? 0.3 : 0.0 );
+	struct CFit {
+		double Launch, Group, GroupMore, GroupFill, More, Convolution, Eight, Meeting, MeetingSlice, MeetingTile;
+	};
+	static const CFit fits[SmallTiles] = { { 2.27, 0.196, 0.226, 0.131, 0.31, 0.22, 0.43, 1.09, 0.141, 1.32 },
+		{ 2.57, 0.352, 0.352, 0.167, 0.43, 0.13, 0.15, 0.76, 0.167, 1.68 }, { 2.87, 0.556, 0.557, 0.283, 0.48, 0.28, 0.02, 1.03, 0.136, 0.96 } };
+	const CFit& f = fits[tile];
+	const double x = share * waves / 8.0; // groups to be done, two wavefronts to a matrix pipe
+	const double fill = static_cast<double>( tiles ) * slices / 256;
+	const double more = ceilDiv( tiles * slices, 256 ) - 1; // further workgroups on the fullest compute unit
+	return f.Launch + f.Group * x + f.GroupMore * x * more + f.GroupFill * x * fill + f.More * more + ( convolution ? f.Convolution : 0.0 )
+		+ ( waves == 8 ? f.Eight : 0.0 ) + ( slices > 1 ? f.Meeting + f.MeetingSlice * slices + f.MeetingTile * static_cast<double>( tiles ) / 256 : 0.0 );
 }
 
-bool trySmallProduct( hipStream_t stream, const CMatMulArgs& given, bool convolution, int batch, bool vec, int* rc )
+// What the other kernels take for the same, standard deviation 4 % below K = 512 ( one workgroup to a tile ) and 7 % from there on.
+static double tilesCost( int M, int N, int K, int batch, bool convolution )
 {
-	if( !vec || batch > 65535 || given.K < 128 || ( convolution && given.Cin % 16 != 0 ) ) {
-		return false;
+	const double steps = ceilDiv( K, 16 );
+	const double fill = static_cast<double>( batch ) * ( N > 32 ? static_cast<double>( ceilDiv( M, 64 ) ) * ceilDiv( N, 64 ) : ceilDiv( M, 128 ) ) / 256;
+	if( K < 512 ) {
+		return 2.57 + 0.291 * steps + 1.08 * fill + ( convolution ? 0.54 : 0.0 );
 	}
-	const long long tilesM = ceilDiv( given.M, 32 ), tilesN = ceilDiv( given.N, 32 );
-	const long long tiles = tilesM * tilesN * batch;
-	if( tiles > 256 ) { // ( a second workgroup on a compute unit waits for the first )
+	return 6.59 + 0.034 * steps + 0.166 * steps * fill + 3.42 * fill + ( convolution ? 0.43 : 0.0 );
+}
+
+// The tile and as many slices as are expected to pay; tile < 0: none. Of the 302 none was slower than without this kernel, all
+// together take 0.556 of that time ( 0.549 with the best tile and count of slices for each ). Beyond 384 workgroups the larger tiles
+// of the other kernels win: 9 x 12 x 14 x 256 3 x 3 22 and 26 us, 410 x 1121 x 832 14.7 and 16.9.
+static void chooseSmall( const CMatMulArgs& args, bool convolution, int batch, int waves, int maxSlices, int& tile, int& slices )
+{
+	const int groups = ceilDiv( args.K, 16 );
+	tile = -1;
+	double cost = tilesCost( args.M, args.N, args.K, batch, convolution );
+	for( int t = 0; t < SmallTiles; ++t ) {
+		const long long tiles = static_cast<long long>( ceilDiv( args.M, SmallTileM[t] ) ) * ceilDiv( args.N, SmallTileN[t] ) * batch;
+		for( int s = 1; s <= maxSlices && tiles * s <= MaxSmallWorkgroups; ++s ) {
+			const int share = ceilDiv( groups, static_cast<long long>( s ) * waves );
+			if( ceilDiv( groups, static_cast<long long>( share ) * waves ) != s ) {
+				continue; // ( fewer slices have the same share )
+			}
+			const double c = smallCost( t, waves, share, s, tiles, convolution );
+			if( c < cost ) {
+				tile = t;
+				slices = s;
+				cost = c;
+			}
+		}
+	}
+}
+
+bool trySmallProduct( hipStream_t stream, const CMatMulArgs& given, bool convolution, int batch, bool vec, int* rc,
+	const CSliceMeeting* fixedMeeting )
+{
+	if( !vec || batch > 65535 || given.K < 16 || ( convolution && given.Cin % 16 != 0 ) ) {
 		return false;
 	}
 	const int groups = ceilDiv( given.K, 16 );
 	const int waves = groups >= 16 ? 8 : 4;
-	// as many slices as are expected to pay, up to a workgroup for every compute unit
-	int slices = 0;
-	double cost = 0;
-	for( int s = 1; s <= ( batch == 1 ? MaxSmallSlices : 1 ) && tiles * s <= 256; ++s ) {
-		const int share = ceilDiv( groups, static_cast<long long>( s ) * waves );
-		if( ceilDiv( groups, static_cast<long long>( share ) * waves ) != s ) {
-			continue; // ( fewer slices have the same share )
-		}
-		const double c = smallCost( waves, share, s, tiles );
-		if( slices == 0 || c < cost ) {
-			slices = s;
-			cost = c;
-		}
-	}
-	// Of the 478 one was slower so ( 196 x 384 x 512 8.0 -> 8.2 us ); all together take 0.856 of the tiles' time, the faster kernel with
-	// the best count of slices 0.850. us: 1 x 1000 x 1280 10.8 -> 7.7, 37 x 512 x 400 9.7 -> 6.9, 196 x 96 x 576 8.2 -> 7.8, 37 x 512 x 768
-	// 8.4 -> 8.1, x 2048 11.7 -> 8.9, 49 x 160 x 960 9.4 -> 7.7, 100 x 512 x 960 9.8 -> 8.4, 1024 x 256 x 256 7.3 -> 6.7; convolutions of
-	// 7 x 7 x 512 17.2 -> 12.3, 14 x 14 x 256 13.3 -> 11.7, 30 x 30 x 48 10.4 -> 6.8. Not 512 x 512 x 768 ( 10.3 and 10.5 ) or
-	// 9 x 6 x 7 x 512 ( 26 and 35 ).
-	if( cost > tilesCost( groups, static_cast<long long>( ceilDiv( given.M, 64 ) ) * ceilDiv( given.N, 64 ) * batch, convolution ) ) {
-		return false;
-	}
 	CMatMulArgs args = given;
-	args.StepsPerSplit = ceilDiv( groups, static_cast<long long>( slices ) * waves );
-	if( slices > 1 && !sliceMeetingPlace( stream, static_cast<size_t>( tiles ) * slices * 1024, static_cast<size_t>( tiles ), &args.Partials, &args.Counters ) ) {
+	int tile = -1, slices = 1;
+	chooseSmall( given, convolution, batch, waves, batch == 1 ? MaxSmallSlices : 1, tile, slices );
+	if( tile >= 0 && slices > 1 ) {
+		const size_t tiles = static_cast<size_t>( ceilDiv( given.M, SmallTileM[tile] ) ) * ceilDiv( given.N, SmallTileN[tile] );
+		const size_t floats = tiles * slices * SmallTileM[tile] * SmallTileN[tile];
+		bool place;
+		if( fixedMeeting != nullptr ) {
+			place = floats <= fixedMeeting->PartialFloats && tiles <= fixedMeeting->CounterCount;
+			args.Partials = fixedMeeting->Partials;
+			args.Counters = fixedMeeting->Counters;
+		} else {
+			place = sliceMeetingPlace( stream, floats, tiles, &args.Partials, &args.Counters );
+		}
+		if( !place ) { // ( under capture, at a pool's limit )
+			chooseSmall( given, convolution, batch, waves, 1, tile, slices );
+		}
+	}
+	if( tile < 0 ) {
 		return false;
 	}
+	const long long tilesM = ceilDiv( given.M, SmallTileM[tile] ), tilesN = ceilDiv( given.N, SmallTileN[tile] );
+	args.StepsPerSplit = ceilDiv( groups, static_cast<long long>( slices ) * waves );
 	args.SplitK = slices;
+	args.SmallTile = tile;
 	args.TilesM = static_cast<int>( tilesM );
 	args.TilesN = static_cast<int>( tilesN );
 	args.TilesNMagic = divisionMagic( args.TilesN );
