@@ -630,6 +630,12 @@ static int sumMatrixRowsImpl( nhStream s, int batchSize, float* result, const fl
 			return rc;
 		}
 	}
+	if( slices == 1 && matrixHeight < 256 && batchSize <= 65535 ) {
+		if( !accumulate && deferRowSums( s, batchSize, result, matrix, matrixHeight, matrixWidth ) ) {
+			return NH_OK;
+		}
+		return sumShortRows( toStream( s ), batchSize, result, matrix, matrixHeight, matrixWidth, accumulate );
+	}
 	const int rowsPerSlice = ceilDiv( matrixHeight, slices );
 	slices = matrixHeight == 0 ? 1 : ceilDiv( matrixHeight, rowsPerSlice );
 	if( batchSize > 65535 || slices > 65535 ) {

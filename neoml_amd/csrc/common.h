@@ -44,6 +44,9 @@ bool deferSpreadOp( nhStream s, bool multiply, int spread, const float* matrix, 
 	CSpreadAlone alone );
 // The sums of a matrix's rows ( nhSumMatrixColumns ) wait for the element-wise calls in place over them: one launch
 bool deferColumnSum( nhStream s, float* result, const float* matrix, int height, int width );
+// ... and so do the sums of each of `batch` matrices' columns ( nhSumMatrixRows ) where sumShortRows is their launch
+bool deferRowSums( nhStream s, int batch, float* result, const float* matrix, int height, int width );
+int sumShortRows( hipStream_t stream, int batch, float* result, const float* matrix, int height, int width, bool accumulate );
 // An image blob padded with a constant ( nhBlobResizeImage ) that waits for the call behind it: a 3 x 3 max pooling over the
 // padded blob ( CImageResizeLayer + CMaxPoolingLayer, the way a pooling layer without padding of its own gets its border )
 // writes the padded blob and the pooled one in one pass over the image.

@@ -1,0 +1,37 @@
+"""nhSumMatrixRows over up to a few hundred rows, by itself and waiting for the calls in place over its sums."""
+import ctypes
+
+import numpy as np
+import pytest
+
+from test_small_ops_chain import ARENA, at, same_bits, streams  # noqa: F401 ( a fixture )
+
+pytestmark = pytest.mark.gpu
+
+RESULT, MATRIX, SCALAR, OTHER = 0, 1 << 16, (1 << 16) - 8, ARENA - 4096
+
+
+# one row, a lane's first row and one beside it, the last height; columns beside a workgroup's runs of 32 and 8, off the 16-byte boundaries
+@pytest.mark.parametrize("batch,height,width,shift", [
+    (1, 1, 1, 0), (1, 49, 1280, 0), (3, 49, 512, 0), (2, 31, 33, 0), (2, 32, 36, 0), (5, 33, 7, 0), (1, 255, 132, 0), (2, 255, 9, 1), (1, 49, 512, 1), (4, 0, 12, 0)])
+def test_sums(streams, batch, height, width, shift):  # noqa: F811
+    g = np.random.default_rng(height * width + shift)
+    start = g.uniform(-1, 1, ARENA).astype(np.float32)
+    m = MATRIX + shift
+    values = start[m:m + batch * height * width].reshape(batch, height, width).astype(np.float64)
+    want = values.sum(axis=1)
+    bound = (height + 2) * 2.0 ** -24 * np.abs(values).sum(axis=1) + 1e-30
+    count = batch * width
+    for name, first in (("nhSumMatrixRows", 0.0), ("nhSumMatrixRowsAdd", start[:count].reshape(batch, width).astype(np.float64))):
+        out = streams.run(streams.plain, [(name, [batch, at(RESULT), at(m), height, width])], start)
+        got = out[:count].reshape(batch, width).astype(np.float64)
+        assert (np.abs(got - want - first) <= bound + 2.0 ** -23 * np.abs(first)).all()
+        assert same_bits(out[count:], start[count:])
+    # the calls that follow: its tail, or a call that is none ( part of the sums, the scalar among them, into another vector, an operand more )
+    scale = ("nhVectorMultiply", [at(RESULT), at(RESULT), count, at(SCALAR)])
+    tails = [[], [scale], [scale, ("nhVectorAddValue", [at(RESULT), at(RESULT), count, at(SCALAR)]), ("nhVectorSqrt", [at(RESULT), at(RESULT), count])],
+             [("nhVectorMultiply", [at(RESULT), at(RESULT), max(1, count - 1), at(SCALAR)])], [("nhVectorMultiply", [at(RESULT), at(RESULT), count, at(RESULT)])],
+             [("nhVectorMultiply", [at(RESULT), at(OTHER), min(count, 4000), at(SCALAR)])], [("nhVectorAdd", [at(RESULT), at(MATRIX), at(RESULT), count])], [scale] * 11]
+    for tail in tails:
+        program = [("nhSumMatrixRows", [batch, at(RESULT), at(m), height, width])] + tail
+        assert same_bits(streams.run(streams.plain, program, start), streams.run(streams.deferring, program, start))
