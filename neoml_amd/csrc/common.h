@@ -73,6 +73,8 @@ bool deferConvolution( nhStream s, bool channelwise, const nhConvDesc& d, const 
 	const float* freeTerm, float* result );
 bool fusePendingConvolution( nhStream s, const float* first, float* result, long long count, int activation,
 	const float* upperThreshold, int* rc );
+// VectorAdd asks whether a convolution that waits takes it along: the sum in place over its result ( true: that waits on )
+bool joinPendingConvolution( nhStream s, const float* first, const float* second, float* result, long long count );
 
 inline hipStream_t toStream( nhStream s )
 {
@@ -201,6 +203,9 @@ struct CFusedActivation {
 	// where the threshold lives in device memory instead ( the engine's VectorReLU takes it there ): a kernel that is
 	// handed one reads it once, through withParam, before it looks at Param
 	const float* ParamPtr;
+	// A launch that is also handed a residual adds it behind the activation ( the fused blocks ) or, with this set, in front of it ( the
+	// junction of a residual block ).
+	int BehindResidual;
 };
 
 __device__ __forceinline__ CFusedActivation withParam( CFusedActivation a )

@@ -15,9 +15,10 @@ namespace nh {
 // matrix products defined in gemm_mfma.hip
 struct CSliceMeeting;
 int convImplicitGemm( hipStream_t stream, const nhConvDesc& d, const float* source, const float* filter,
-	const float* freeTerm, float* result, const CFusedActivation& act, const CSliceMeeting* fixedMeeting );
+	const float* freeTerm, float* result, const CFusedActivation& act, const CSliceMeeting* fixedMeeting,
+	const float* residual );
 int launchDeferredConvolution( hipStream_t stream, bool channelwise, const nhConvDesc& d, const float* source, const float* filter,
-	const float* freeTerm, float* result, const CFusedActivation& act );
+	const float* freeTerm, float* result, const CFusedActivation& act, const float* residual );
 int matMulNT( hipStream_t stream, const float* a, int lda, const float* b, int ldb, float* c, int ldc,
 	int M, int N, int K, int batch, long long strideA, long long strideB, long long strideC,
 	const float* bias, bool accumulate );
@@ -3199,12 +3200,12 @@ static int channelwiseConvolution( nhStream s, const nhConvDesc* d, const float*
 
 // a convolution that waited for its successor ( vector_ops.hip ), with the activation the successor turned out to be
 int nh::launchDeferredConvolution( hipStream_t stream, bool channelwise, const nhConvDesc& d, const float* source, const float* filter,
-	const float* freeTerm, float* result, const CFusedActivation& act )
+	const float* freeTerm, float* result, const CFusedActivation& act, const float* residual )
 {
 	if( channelwise ) {
 		return channelwiseConvolution( reinterpret_cast<nhStream>( stream ), &d, source, filter, freeTerm, result, act );
 	}
-	return convImplicitGemm( stream, d, source, filter, freeTerm, result, act, nullptr );
+	return convImplicitGemm( stream, d, source, filter, freeTerm, result, act, nullptr, residual );
 }
 
 extern "C" {

@@ -861,16 +861,22 @@ void matMulKernel( const CMatMulArgs launchArgs )
 	// ( in a scalar register for tiles that lie inside the matrix: no vector instruction per element beyond the bias and
 	// the activation; as a vector addition for the last tile row, whose rows beyond M the range check drops ). Per tile
 	// and wavefront this takes some 150 vector instructions out of an epilogue that cost as much as ten K steps.
+	// A residual is fetched for all of a block's elements before the first of them is stored: it may be C itself as far as the
+	// compiler knows, and a load behind each store would wait for its memory sixteen times.
 	if constexpr( !IsClasses && BMODE != BM_ConvN ) {
-		if( args.CBytes != 0 && splitK == 1 && !args.Accumulate && args.Residual == nullptr ) {
+		if( args.CBytes != 0 && splitK == 1 && !args.Accumulate ) {
 			const __amdgpu_buffer_rsrc_t bufC = __builtin_amdgcn_make_buffer_rsrc( C, 0, args.CBytes, 0x00020000 );
+			const __amdgpu_buffer_rsrc_t bufR = __builtin_amdgcn_make_buffer_rsrc(
+				const_cast<float*>( args.Residual != nullptr ? args.Residual + batch * args.BatchStrideC : C ), 0, args.CBytes, 0x00020000 );
 			const float actParam = withParam( args.Act ).Param; // ( the threshold may live in device memory )
-	const float reluTop = actParam > 0.f ? actParam : __builtin_inff();
+			const float reluTop = actParam > 0.f ? actParam : __builtin_inff();
 			const unsigned pitchBytes = static_cast<unsigned>( args.Ldc ) * 4u;
 			const bool inside = m0 + BM <= M;
-			auto store = [&]( auto typeOf, auto insideOf ) {
+			// residualOf: 0 none, 1 added behind the activation, 2 in front of it
+			auto store = [&]( auto typeOf, auto insideOf, auto residualOf ) {
 				constexpr int Type = decltype( typeOf )::value;
 				constexpr bool Inside = decltype( insideOf )::value;
+				constexpr int Residual = decltype( residualOf )::value;
 #pragma unroll
 				for( int ni = 0; ni < NI; ++ni ) {
 					const int n = n0 + waveN * WN + ni * 32 + l32;
@@ -879,10 +885,28 @@ void matMulKernel( const CMatMulArgs launchArgs )
 						? static_cast<unsigned>( ( m0 + waveM * WM + half * 4 ) * args.Ldc + n ) * 4u : OutOfRange;
 #pragma unroll
 					for( int mi = 0; mi < MI; ++mi ) {
+						auto rowBytesOf = [&]( int r ) {
+							return static_cast<unsigned>( mi * 32 + ( r >> 2 ) * 8 + ( r & 3 ) ) * pitchBytes;
+						};
+						float other[16];
+						if constexpr( Residual != 0 ) {
+#pragma unroll
+							for( int r = 0; r < 16; ++r ) {
+								other[r] = __uint_as_float( Inside ? __builtin_amdgcn_raw_buffer_load_b32( bufR, laneOffset, rowBytesOf( r ), 0 )
+									: __builtin_amdgcn_raw_buffer_load_b32( bufR, laneOffset + rowBytesOf( r ), 0, 0 ) );
+							}
+						}
 #pragma unroll
 						for( int r = 0; r < 16; ++r ) {
-							const unsigned rowBytes = static_cast<unsigned>( mi * 32 + ( r >> 2 ) * 8 + ( r & 3 ) ) * pitchBytes;
-							const float v = applyActivationOf<Type>( acc[mi][ni][r] + bias, reluTop );
+							const unsigned rowBytes = rowBytesOf( r );
+							float v = acc[mi][ni][r] + bias;
+							if constexpr( Residual == 2 ) {
+								v += other[r];
+							}
+							v = applyActivationOf<Type>( v, reluTop );
+							if constexpr( Residual == 1 ) {
+								v += other[r];
+							}
 							if constexpr( Inside ) {
 								__builtin_amdgcn_raw_buffer_store_b32( __float_as_uint( v ), bufC, laneOffset, rowBytes, 0 );
 							} else {
@@ -893,11 +917,20 @@ void matMulKernel( const CMatMulArgs launchArgs )
 					}
 				}
 			};
-			auto storeAs = [&]( auto typeOf ) {
+			auto storeBy = [&]( auto typeOf, auto residualOf ) {
 				if( inside ) {
-					store( typeOf, std::true_type() );
+					store( typeOf, std::true_type(), residualOf );
 				} else {
-					store( typeOf, std::false_type() );
+					store( typeOf, std::false_type(), residualOf );
+				}
+			};
+			auto storeAs = [&]( auto typeOf ) {
+				if( args.Residual == nullptr ) {
+					storeBy( typeOf, std::integral_constant<int, 0>() );
+				} else if( args.Act.BehindResidual == 0 || decltype( typeOf )::value == NH_ACT_NONE ) {
+					storeBy( typeOf, std::integral_constant<int, 1>() );
+				} else {
+					storeBy( typeOf, std::integral_constant<int, 2>() );
 				}
 			};
 			if( args.Act.Type == NH_ACT_RELU ) {
@@ -960,11 +993,11 @@ void matMulKernel( const CMatMulArgs launchArgs )
 									v += *p;
 								}
 							}
-							v = applyActivationOf<Type>( v, reluTop );
 							if constexpr( Mode == 2 ) {
-								if( args.Residual != nullptr ) {
-									v += args.Residual[batch * args.BatchStrideC + row * args.Ldc + n];
-								}
+								const float r = args.Residual != nullptr ? args.Residual[batch * args.BatchStrideC + row * args.Ldc + n] : 0.f;
+								v = args.Act.BehindResidual != 0 ? applyActivationOf<Type>( v + r, reluTop ) : applyActivationOf<Type>( v, reluTop ) + r;
+							} else {
+								v = applyActivationOf<Type>( v, reluTop );
 							}
 							*p = v;
 						}
@@ -1357,7 +1390,7 @@ static int launchTile( hipStream_t stream, CMatMulArgs& args, int batch, bool ve
 	const int slots = 256 * 5; // planned as above: the five that saturate a compute unit, not the eight that fit
 	long long gridX = tiles;
 	int tailRow = 0;
-	if( splits == 1 && !twoGroups && batch == 1 && AMODE != AM_ConvClasses && args.Residual == nullptr && tiles >= slots && totalSteps >= 16 ) {
+	if( splits == 1 && !twoGroups && batch == 1 && AMODE != AM_ConvClasses && tiles >= slots && totalSteps >= 16 ) {
 		long long full = tiles / slots * slots;
 		full -= full % args.TilesN; // whole rows of tiles: the preset below covers the rows behind them
 		const long long rest = tiles - full;
@@ -1420,11 +1453,13 @@ static int launchTile( hipStream_t stream, CMatMulArgs& args, int batch, bool ve
 		}
 	}
 	const bool meetInScratch = args.Partials != nullptr;
-	if( args.Residual != nullptr && args.SplitK > 1 && !meetInScratch ) {
+	if( args.Residual != nullptr && ( args.SplitK > 1 || args.FullTiles > 0 ) && !meetInScratch ) {
 		// The residual is added by the one workgroup that writes a tile, which is the last slice to arrive at the meeting;
 		// slices that add onto C with atomics have no such workgroup. No scratch ( a capturing stream ): one slice.
 		args.StepsPerSplit = totalSteps;
 		args.SplitK = 1;
+		args.FullTiles = 0;
+		gridX = tiles;
 	}
 	// the rows of the tail tiles as a matrix product of their own: what the preset and the activation pass cover
 	CMatMulArgs tail = args;
@@ -1888,6 +1923,15 @@ void shortReductionKernel( const float* A, const float* W, const float* bias, fl
 				for( int q = 0; q < 4; ++q ) {
 					v[q] = *reinterpret_cast<const float4*>( patch + ( q * 8 + ( lane >> 3 ) ) * PatchPitch + col4 );
 				}
+				if( RES && act.BehindResidual != 0 ) {
+#pragma unroll
+					for( int q = 0; q < 4; ++q ) {
+						v[q].x += res[q].x;
+						v[q].y += res[q].y;
+						v[q].z += res[q].z;
+						v[q].w += res[q].w;
+					}
+				}
 				if( act.Type == NH_ACT_RELU ) {
 #pragma unroll
 					for( int q = 0; q < 4; ++q ) {
@@ -1909,7 +1953,7 @@ void shortReductionKernel( const float* A, const float* W, const float* bias, fl
 				const unsigned o = outOffset( block, nb + t );
 #pragma unroll
 				for( int q = 0; q < 4; ++q ) {
-					if( RES ) {
+					if( RES && act.BehindResidual == 0 ) {
 						v[q].x += res[q].x;
 						v[q].y += res[q].y;
 						v[q].z += res[q].z;
@@ -2257,11 +2301,11 @@ void longProductKernel( const CLongProductArgs args )
 								v += C[at];
 							}
 						}
-						v = applyActivationOf<Type>( v, reluTop );
 						if constexpr( Extra ) {
-							if( residual != nullptr ) {
-								v += residual[at];
-							}
+							const float r = residual != nullptr ? residual[at] : 0.f;
+							v = args.Act.BehindResidual != 0 ? applyActivationOf<Type>( v + r, reluTop ) : applyActivationOf<Type>( v, reluTop ) + r;
+						} else {
+							v = applyActivationOf<Type>( v, reluTop );
 						}
 						C[at] = v;
 					}
@@ -2664,10 +2708,12 @@ static bool tryWindowReduction( hipStream_t stream, const nhConvDesc& d, const f
 }
 
 int convImplicitGemm( hipStream_t stream, const nhConvDesc& d, const float* source, const float* filter,
-	const float* freeTerm, float* result, const CFusedActivation& act, const CSliceMeeting* fixedMeeting = nullptr )
+	const float* freeTerm, float* result, const CFusedActivation& act, const CSliceMeeting* fixedMeeting = nullptr,
+	const float* residual = nullptr )
 {
 	CMatMulArgs args = {};
 	args.Act = act;
+	args.Residual = residual;
 	args.A = source; args.B = filter; args.C = result; args.Bias = freeTerm;
 	const long long m = static_cast<long long>( d.batch ) * d.resultHeight * d.resultWidth;
 	args.M = static_cast<int>( m );
@@ -2690,7 +2736,7 @@ int convImplicitGemm( hipStream_t stream, const nhConvDesc& d, const float* sour
 	{
 		// a pointwise convolution over a channels-last image is the plain product image[M x Cin] * filter[Cout x Cin]^T
 		return matMulNTMeeting( stream, source, d.channels, filter, d.channels, result, d.filterCount, args.M, args.N, d.channels,
-			1, 0, 0, 0, freeTerm, false, act, nullptr, fixedMeeting );
+			1, 0, 0, 0, freeTerm, false, act, residual, fixedMeeting );
 	}
 	int smallRc = NH_OK;
 	if( trySmallProduct( stream, args, true, 1, vec, &smallRc, fixedMeeting ) ) {
@@ -2701,7 +2747,7 @@ int convImplicitGemm( hipStream_t stream, const nhConvDesc& d, const float* sour
 	}
 	if( d.channels % 4 != 0 ) {
 		int rc = NH_OK;
-		if( tryWindowReduction( stream, d, source, filter, freeTerm, result, act, &rc ) ) {
+		if( residual == nullptr && tryWindowReduction( stream, d, source, filter, freeTerm, result, act, &rc ) ) {
 			return rc;
 		}
 	}

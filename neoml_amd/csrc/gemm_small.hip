@@ -326,6 +326,7 @@ __device__ __forceinline__ void smallProductTile( const CMatMulArgs& args, float
 	}
 	// element ( r, lane ): block ( r / ( 4 NB ), r / 4 % NB ), of it column lane % 16 of row 4 ( lane / 16 ) + r % 4
 	float* C = args.C + batch * args.BatchStrideC;
+	const float* residual = args.Residual != nullptr ? args.Residual + batch * args.BatchStrideC : nullptr;
 #pragma unroll
 	for( int i = 0; i < PerThread; ++i ) {
 		const int r = wave + i * WAVES;
@@ -336,9 +337,11 @@ __device__ __forceinline__ void smallProductTile( const CMatMulArgs& args, float
 			if( args.Accumulate ) {
 				v += C[at];
 			}
-			v = applyActivation( v, act );
-			if( args.Residual != nullptr ) {
-				v += args.Residual[batch * args.BatchStrideC + at];
+			if( residual != nullptr ) {
+				const float r = residual[at];
+				v = act.BehindResidual != 0 ? applyActivation( v + r, act ) : applyActivation( v, act ) + r;
+			} else {
+				v = applyActivation( v, act );
 			}
 			C[at] = v;
 		}

@@ -331,6 +331,7 @@ void splitProductKernel( const CMatMulArgs args )
 	const float* residual = args.Residual != nullptr ? args.Residual + batch * args.BatchStrideC : nullptr;
 	const float actParam = withParam( args.Act ).Param; // ( the threshold may live in device memory )
 	const float reluTop = actParam > 0.f ? actParam : __builtin_inff();
+	const bool behind = args.Act.BehindResidual != 0;
 	const unsigned pitchBytes = static_cast<unsigned>( args.Ldc ) * 4u;
 	auto write = [&]( auto typeOf, auto extraOf, auto insideOf ) {
 		constexpr int Type = decltype( typeOf )::value;
@@ -357,10 +358,8 @@ void splitProductKernel( const CMatMulArgs args )
 						if( args.Accumulate && ok ) {
 							v += C[at];
 						}
-						v = applyActivationOf<Type>( v, reluTop );
-						if( residual != nullptr && ok ) {
-							v += residual[at];
-						}
+						const float r = residual != nullptr && ok ? residual[at] : 0.f;
+						v = behind ? applyActivationOf<Type>( v + r, reluTop ) : applyActivationOf<Type>( v, reluTop ) + r;
 					} else {
 						v = applyActivationOf<Type>( v, reluTop );
 					}

@@ -808,6 +808,14 @@ struct CPendingConvolution {
 	const float* Filter = nullptr;
 	const float* FreeTerm = nullptr;
 	float* Result = nullptr;
+	// what a VectorAdd in place over the result adds to it ( the junction of a residual block, CEltwiseSumLayer ); the ReLU may
+	// still follow
+	const float* Residual = nullptr;
+
+	long long ResultCount() const
+	{
+		return static_cast<long long>( Desc.batch ) * Desc.resultHeight * Desc.resultWidth * Desc.filterCount;
+	}
 };
 
 // The sum of two large vectors ( the junction of a residual block, CEltwiseSumLayer ) followed by CReLULayer in place:
@@ -866,6 +874,10 @@ struct CTinyQueue {
 	CSpreadAlone FirstSpreadAlone = nullptr; // ( the same for a call with a spread operand: its own kernel lives with its entry point )
 	CPendingProduct Product;
 	CPendingConvolution Convolution;
+	// A second convolution with a result of the same size, behind the first: a block's last convolution may be followed by that of
+	// its shortcut, and only then by the sum of the two over the first one's result. The sum launches the second one and waits on
+	// with the first ( pending only while that is ).
+	CPendingConvolution Shortcut;
 	CPendingSum Sum;
 	CPendingBatched Batched;
 	CPendingPadding Padding;
@@ -880,7 +892,7 @@ struct CTinyQueue {
 static int launchPlainSum( hipStream_t stream, const CPendingSum& sum );
 
 int launchDeferredConvolution( hipStream_t stream, bool channelwise, const nhConvDesc& d, const float* source, const float* filter,
-	const float* freeTerm, float* result, const CFusedActivation& act );
+	const float* freeTerm, float* result, const CFusedActivation& act, const float* residual );
 
 int matMulNT( hipStream_t stream, const float* a, int lda, const float* b, int ldb, float* c, int ldc,
 	int M, int N, int K, int batch, long long strideA, long long strideB, long long strideC, const float* bias, bool accumulate );
@@ -888,6 +900,11 @@ int matMulNT( hipStream_t stream, const float* a, int lda, const float* b, int l
 int matMulNN( hipStream_t stream, const float* a, int lda, const float* b, int ldb, float* c, int ldc,
 	int M, int N, int K, int batch, long long strideA, long long strideB, long long strideC, bool accumulate,
 	const float* scale, bool* scaled );
+
+static int launchPendingConvolution( hipStream_t stream, const CPendingConvolution& c, const CFusedActivation& act )
+{
+	return launchDeferredConvolution( stream, c.Channelwise, c.Desc, c.Source, c.Filter, c.FreeTerm, c.Result, act, c.Residual );
+}
 
 static int launchBatched( hipStream_t stream, const CPendingBatched& p, const float* scale, bool* scaled )
 {
@@ -1382,11 +1399,15 @@ static bool launchPending( hipStream_t stream, CTinyQueue& queue )
 		return true;
 	}
 	if( queue.Convolution.Pending ) {
-		const CPendingConvolution c = queue.Convolution;
+		const CPendingConvolution c = queue.Convolution, shortcut = queue.Shortcut;
 		queue.Convolution.Pending = false;
+		queue.Shortcut.Pending = false;
 		__atomic_fetch_sub( &tinyChainsPending, 1, __ATOMIC_RELAXED );
 		const CFusedActivation none = { NH_ACT_NONE, 0.f };
-		( void )launchDeferredConvolution( stream, c.Channelwise, c.Desc, c.Source, c.Filter, c.FreeTerm, c.Result, none );
+		( void )launchPendingConvolution( stream, c, none );
+		if( shortcut.Pending ) {
+			( void )launchPendingConvolution( stream, shortcut, none );
+		}
 		return true;
 	}
 	if( queue.Batched.Pending ) {
@@ -1866,16 +1887,54 @@ static bool fusePendingSum( nhStream s, const float* first, float* result, int c
 	return true;
 }
 
+static bool rangesMeet( const float* a, long long countA, const float* b, long long countB )
+{
+	return a != nullptr && b != nullptr && a < b + countB && b < a + countA;
+}
+
+// whether the convolution reads or writes any of these values
+static bool touches( const CPendingConvolution& c, const float* p, long long count )
+{
+	const nhConvDesc& d = c.Desc;
+	return rangesMeet( c.Source, static_cast<long long>( d.batch ) * d.height * d.width * d.channels, p, count )
+		|| rangesMeet( c.Filter, static_cast<long long>( d.filterCount ) * d.filterHeight * d.filterWidth * d.channels, p, count )
+		|| rangesMeet( c.FreeTerm, d.filterCount, p, count ) || rangesMeet( c.Result, c.ResultCount(), p, count );
+}
+
+static CTinyQueue* deferringQueue( hipStream_t stream )
+{
+	int device = 0;
+	if( hipGetDevice( &device ) != hipSuccess ) {
+		( void )hipGetLastError();
+		return nullptr;
+	}
+	auto found = tinyQueues().find( std::make_pair( device, stream ) );
+	return found != tinyQueues().end() && found->second.Enabled ? &found->second : nullptr;
+}
+
 bool deferConvolution( nhStream s, bool channelwise, const nhConvDesc& d, const float* source, const float* filter,
 	const float* freeTerm, float* result )
 {
 	if( __atomic_load_n( &tinyDeferringStreams, __ATOMIC_RELAXED ) == 0 || d.batch <= 0 ) {
 		return false;
 	}
+	CPendingConvolution c;
+	c.Pending = true;
+	c.Channelwise = channelwise;
+	c.Desc = d;
+	c.Source = source; c.Filter = filter; c.FreeTerm = freeTerm; c.Result = result;
+	if( !channelwise && __atomic_load_n( &tinyChainsPending, __ATOMIC_RELAXED ) != 0 ) {
+		std::lock_guard<std::recursive_mutex> guard( tinyLock );
+		CTinyQueue* queue = deferringQueue( reinterpret_cast<hipStream_t>( s ) );
+		if( queue != nullptr && queue->Convolution.Pending && !queue->Convolution.Channelwise && queue->Convolution.Residual == nullptr
+			&& !queue->Shortcut.Pending && queue->Convolution.ResultCount() == c.ResultCount() ) {
+			queue->Shortcut = c;
+			return true;
+		}
+	}
 	const hipStream_t stream = toStream( s ); // ( what the stream holds goes out first )
-	int device = 0;
 	hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-	if( hipGetDevice( &device ) != hipSuccess || hipStreamIsCapturing( stream, &capture ) != hipSuccess ) {
+	if( hipStreamIsCapturing( stream, &capture ) != hipSuccess ) {
 		( void )hipGetLastError();
 		return false;
 	}
@@ -1883,17 +1942,68 @@ bool deferConvolution( nhStream s, bool channelwise, const nhConvDesc& d, const 
 		return false;
 	}
 	std::lock_guard<std::recursive_mutex> guard( tinyLock );
-	auto found = tinyQueues().find( std::make_pair( device, stream ) );
-	if( found == tinyQueues().end() || !found->second.Enabled || found->second.Chain.Length != 0 || found->second.LaunchWaits() )
-	{
+	CTinyQueue* queue = deferringQueue( stream );
+	if( queue == nullptr || queue->Chain.Length != 0 || queue->LaunchWaits() ) {
 		return false;
 	}
-	CPendingConvolution& c = found->second.Convolution;
-	c.Pending = true;
-	c.Channelwise = channelwise;
-	c.Desc = d;
-	c.Source = source; c.Filter = filter; c.FreeTerm = freeTerm; c.Result = result;
+	queue->Convolution = c;
+	queue->Shortcut.Pending = false;
 	__atomic_fetch_add( &tinyChainsPending, 1, __ATOMIC_RELAXED );
+	return true;
+}
+
+bool joinPendingConvolution( nhStream s, const float* first, const float* second, float* result, long long count )
+{
+	if( first == nullptr || second == nullptr || result == nullptr || first == second ) {
+		return false;
+	}
+	const hipStream_t stream = reinterpret_cast<hipStream_t>( s );
+	CPendingConvolution shortcut, c;
+	{
+		std::lock_guard<std::recursive_mutex> guard( tinyLock );
+		CTinyQueue* queue = deferringQueue( stream );
+		if( queue == nullptr || !queue->Convolution.Pending || queue->Convolution.Channelwise || queue->Convolution.Residual != nullptr ) {
+			return false;
+		}
+		c = queue->Convolution;
+		shortcut = queue->Shortcut;
+		if( c.Desc.channels % 4 != 0 ) {
+			return false; // ( the loader of first layers' windows has no residual )
+		}
+		const float* other = first == c.Result ? second : first;
+		if( ( first != c.Result && second != c.Result ) || result != c.Result || count != c.ResultCount()
+			|| rangesMeet( other, count, c.Result, count ) ) {
+			return false; // ( the caller's own launch sends the convolutions out first, as they were asked for )
+		}
+		if( !shortcut.Pending ) {
+			queue->Convolution.Residual = other;
+			return true;
+		}
+		// the other summand has to be the second convolution's result, and that convolution has to be free to go first
+		if( other != shortcut.Result || touches( c, shortcut.Result, count ) || touches( shortcut, c.Result, count ) ) {
+			return false;
+		}
+		// ( both leave the queue: the launch may ask a pool for memory, which sends out what the queues hold )
+		queue->Convolution.Pending = false;
+		queue->Shortcut.Pending = false;
+		__atomic_fetch_sub( &tinyChainsPending, 1, __ATOMIC_RELAXED );
+	}
+	const CFusedActivation none = { NH_ACT_NONE, 0.f };
+	( void )launchPendingConvolution( stream, shortcut, none );
+	if( __atomic_load_n( &lstmPartnersAwaited, __ATOMIC_RELAXED ) != 0 ) {
+		noteStreamUse( stream );
+	}
+	c.Residual = shortcut.Result;
+	{
+		std::lock_guard<std::recursive_mutex> guard( tinyLock );
+		CTinyQueue* queue = deferringQueue( stream );
+		if( queue != nullptr && queue->Chain.Length == 0 && !queue->LaunchWaits() ) {
+			queue->Convolution = c;
+			__atomic_fetch_add( &tinyChainsPending, 1, __ATOMIC_RELAXED );
+			return true;
+		}
+	}
+	( void )launchPendingConvolution( stream, c, none );
 	return true;
 }
 
@@ -1901,28 +2011,31 @@ bool fusePendingConvolution( nhStream s, const float* first, float* result, long
 	const float* upperThreshold, int* rc )
 {
 	const hipStream_t stream = reinterpret_cast<hipStream_t>( s );
-	int device = 0;
-	if( hipGetDevice( &device ) != hipSuccess ) {
-		( void )hipGetLastError();
-		return false;
-	}
-	CPendingConvolution c;
+	CPendingConvolution c, front;
 	{
 		std::lock_guard<std::recursive_mutex> guard( tinyLock );
-		auto found = tinyQueues().find( std::make_pair( device, stream ) );
-		if( found == tinyQueues().end() || !found->second.Convolution.Pending ) {
+		CTinyQueue* queue = deferringQueue( stream );
+		if( queue == nullptr || !queue->Convolution.Pending ) {
 			return false;
 		}
-		c = found->second.Convolution;
-		const long long resultCount = static_cast<long long>( c.Desc.batch ) * c.Desc.resultHeight * c.Desc.resultWidth * c.Desc.filterCount;
-		if( first != c.Result || result != c.Result || count != resultCount || ( activation == NH_ACT_RELU && upperThreshold == nullptr ) ) {
+		c = queue->Convolution;
+		if( queue->Shortcut.Pending ) { // ( the call behind the second one: the first goes out as it was asked for )
+			front = queue->Convolution;
+			c = queue->Shortcut;
+		}
+		if( first != c.Result || result != c.Result || count != c.ResultCount() || ( activation == NH_ACT_RELU && ( upperThreshold == nullptr || rangesMeet( upperThreshold, 1, c.Result, count ) ) ) ) {
 			return false; // ( the caller's own launch sends the convolution out first, as it was asked for )
 		}
-		found->second.Convolution.Pending = false;
+		queue->Convolution.Pending = false;
+		queue->Shortcut.Pending = false;
 		__atomic_fetch_sub( &tinyChainsPending, 1, __ATOMIC_RELAXED );
 	}
-	const CFusedActivation act = { activation, 0.f, activation == NH_ACT_RELU ? upperThreshold : nullptr };
-	*rc = launchDeferredConvolution( stream, c.Channelwise, c.Desc, c.Source, c.Filter, c.FreeTerm, c.Result, act );
+	if( front.Pending ) {
+		const CFusedActivation none = { NH_ACT_NONE, 0.f };
+		( void )launchPendingConvolution( stream, front, none );
+	}
+	const CFusedActivation act = { activation, 0.f, activation == NH_ACT_RELU ? upperThreshold : nullptr, c.Residual != nullptr ? 1 : 0 };
+	*rc = launchPendingConvolution( stream, c, act );
 	if( __atomic_load_n( &lstmPartnersAwaited, __ATOMIC_RELAXED ) != 0 ) {
 		noteStreamUse( stream );
 	}
@@ -2473,7 +2586,12 @@ NH_BINARY( nhVectorEltwiseMax, float, CMaxOp )
 NH_BINARY( nhVectorEltwiseMin, float, CMinOp )
 extern "C" int nhVectorAdd( nhStream s, const float* first, const float* second, float* result, int vectorSize )
 {
-	// ( on a stream that puts calls aside a large sum waits for the call behind it: a ReLU over it in place is the same pass )
+	// ( on a stream that puts calls aside a sum over the result of a convolution that waits goes into that convolution's launch )
+	if( vectorSize > 0 && __atomic_load_n( &tinyChainsPending, __ATOMIC_RELAXED ) != 0
+		&& joinPendingConvolution( s, first, second, result, vectorSize ) ) {
+		return NH_OK;
+	}
+	// ( a large sum waits for the call behind it: a ReLU over it in place is the same pass )
 	if( vectorSize > TinyWideMaxCount && deferSum( s, first, second, result, vectorSize ) ) {
 		return NH_OK;
 	}
