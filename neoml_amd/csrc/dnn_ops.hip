@@ -1,7 +1,7 @@
 // Bandwidth-bound blob kernels of IDnnEngine on channels-last images: depthwise (channelwise) convolution,
 // 2-D max / mean pooling, image padding / cropping, split / merge along a blob dimension, and the LSTM
 // recurrence (matrix products on the MFMA kernels + one fused gate kernel per step).
-#include "common.h"
+#include "gemm.h"
 #include <float.h>
 #include <math.h>
 #include <stdlib.h>
@@ -226,6 +226,68 @@ void channelwiseConv3x3Kernel( const nhConvDesc d, const float* source, const fl
 			}
 			outRowOffset += outRowBytes;
 		}
+	}
+}
+
+// The same convolution for layers that are a few wavefronts per compute unit: one thread owns 4 channels of WPT pixels of one output
+// row, with everything it reads asked for at once. What bounds such a layer is how many instructions a wavefront has in front of it: a
+// strip of four rows, four pixels wide, is some 900 of them, 2 us at one wavefront to a SIMD. The sums in the same order, the same bits.
+template<int STRIDE, int WPT, int ACT>
+__global__ __launch_bounds__( 256 )
+void channelwiseConv3x3SmallKernel( const nhConvDesc d, const float* source, const float* filter, const float* freeTerm, float* result,
+	int wGroups, unsigned wGroupsMagic, int cg, unsigned cgMagic, unsigned heightMagic, int totalItems, const CFusedActivation actAsGiven,
+	int flipTaps, unsigned resultBytes )
+{
+	constexpr int NC = ( WPT - 1 ) * STRIDE + 3;
+	const int item = xcdSwizzle( blockIdx.x, gridDim.x ) * 256 + threadIdx.x;
+	if( item >= totalItems ) {
+		return;
+	}
+	int t, c4, wGroup, n, ho;
+	fastDivMod( item, cg, cgMagic, t, c4 );
+	fastDivMod( t, wGroups, wGroupsMagic, t, wGroup );
+	fastDivMod( t, d.resultHeight, heightMagic, n, ho );
+	const unsigned c = static_cast<unsigned>( c4 ) * 16u; // ( in bytes )
+	const __amdgpu_buffer_rsrc_t image = makeBuffer( source ), taps = makeBuffer( filter );
+	const unsigned pixelBytes = static_cast<unsigned>( d.channels ) * 4u;
+	const unsigned rowBytes = static_cast<unsigned>( d.width ) * pixelBytes;
+	const int hi0 = ho * STRIDE - d.paddingHeight, wi0 = wGroup * WPT * STRIDE - d.paddingWidth;
+	const unsigned corner = static_cast<unsigned>( n * d.height + hi0 ) * rowBytes + static_cast<unsigned>( wi0 ) * pixelBytes + c;
+	float4 in[3][NC], f[9];
+#pragma unroll
+	for( int kh = 0; kh < 3; ++kh ) {
+		const bool rowInside = static_cast<unsigned>( hi0 + kh ) < static_cast<unsigned>( d.height );
+#pragma unroll
+		for( int j = 0; j < NC; ++j ) {
+			const bool inside = rowInside && static_cast<unsigned>( wi0 + j ) < static_cast<unsigned>( d.width );
+			in[kh][j] = bufferLoad4( image, inside ? corner + static_cast<unsigned>( kh ) * rowBytes + static_cast<unsigned>( j ) * pixelBytes : OutOfRange );
+		}
+	}
+#pragma unroll
+	for( int k = 0; k < 9; ++k ) {
+		f[k] = bufferLoad4( taps, c, static_cast<unsigned>( flipTaps != 0 ? 8 - k : k ) * pixelBytes );
+	}
+	const float4 bias = freeTerm != nullptr ? bufferLoad4( makeBuffer( freeTerm ), c ) : make_float4( 0.f, 0.f, 0.f, 0.f );
+	const CFusedActivation act = withParam( actAsGiven );
+	const float reluTop = act.Param > 0.f ? act.Param : __builtin_inff();
+	const __amdgpu_buffer_rsrc_t out = __builtin_amdgcn_make_buffer_rsrc( result, 0, resultBytes, 0x00020000 );
+	const unsigned outOffset = ( static_cast<unsigned>( n * d.resultHeight + ho ) * static_cast<unsigned>( d.resultWidth )
+		+ static_cast<unsigned>( wGroup * WPT ) ) * pixelBytes + c;
+#pragma unroll
+	for( int j = 0; j < WPT; ++j ) {
+		float4 acc = bias;
+#pragma unroll
+		for( int kh = 0; kh < 3; ++kh ) {
+#pragma unroll
+			for( int kw = 0; kw < 3; ++kw ) {
+				acc = CChanVec<4>::fma( in[kh][j * STRIDE + kw], f[kh * 3 + kw], acc );
+			}
+		}
+		acc.x = applyActivationOf<ACT>( acc.x, reluTop );
+		acc.y = applyActivationOf<ACT>( acc.y, reluTop );
+		acc.z = applyActivationOf<ACT>( acc.z, reluTop );
+		acc.w = applyActivationOf<ACT>( acc.w, reluTop );
+		bufferStore4( out, wGroup * WPT + j < d.resultWidth ? outOffset + static_cast<unsigned>( j ) * pixelBytes : OutOfRange, acc );
 	}
 }
 
@@ -2717,10 +2779,49 @@ static int channelwise3x3Launch( nhStream s, const nhConvDesc* d, const float* s
 }
 
 template<int STRIDE, int WPT>
+static int channelwise3x3SmallLaunch( nhStream s, const nhConvDesc* d, const float* source, const float* filter, const float* freeTerm,
+	float* result, const CFusedActivation& act, bool flipTaps )
+{
+	const int wGroups = ceilDiv( d->resultWidth, WPT ), cg = d->channels / 4;
+	const int items = d->batch * d->resultHeight * wGroups * cg;
+	const unsigned resultBytes = static_cast<unsigned>( static_cast<long long>( d->batch ) * d->resultHeight * d->resultWidth * d->channels * 4 );
+	auto launch = [&]( auto actOf ) {
+		constexpr int Act = decltype( actOf )::value;
+		hipLaunchKernelGGL( ( channelwiseConv3x3SmallKernel<STRIDE, WPT, Act> ), dim3( ceilDiv( items, 256 ) ), dim3( 256 ), 0, toStream( s ), *d,
+			source, filter, freeTerm, result, wGroups, divisionMagic( wGroups ), cg, divisionMagic( cg ), divisionMagic( d->resultHeight ), items, act,
+			flipTaps ? 1 : 0, resultBytes );
+	};
+	if( act.Type == NH_ACT_RELU ) {
+		launch( std::integral_constant<int, NH_ACT_RELU>() );
+	} else if( act.Type == NH_ACT_HSWISH ) {
+		launch( std::integral_constant<int, NH_ACT_HSWISH>() );
+	} else {
+		launch( std::integral_constant<int, NH_ACT_NONE>() );
+	}
+	NH_LAUNCH_CHECK();
+	return NH_OK;
+}
+
+template<int STRIDE, int WPT>
 static int channelwise3x3Impl( nhStream s, const nhConvDesc* d, const float* source, const float* filter,
 	const float* freeTerm, float* result, const CFusedActivation& act, bool flipTaps = false )
 {
 	const long long sourceBytes = static_cast<long long>( d->batch ) * d->height * d->width * d->channels * 4;
+	const long long quads = static_cast<long long>( d->batch ) * d->resultHeight * d->resultWidth * ( d->channels / 4 );
+	// ( us, strips and pixels: 14 x 14 x 384 3.85 -> 2.54, 56 x 56 x 144 4.03 -> 2.94, two of 112 x 112 x 32 4.21 -> 3.39, 14 x 14 x 576 stride 2
+	// 3.83 -> 2.51; one pixel to a thread up to 2^16 quads ( 2^16.2: 3.18, two pixels 2.85 ), two up to 2^17 ( 2^17.2: 3.59, four 3.27 ), at
+	// stride 1 four up to 2^18, where they meet the strips' time: 2^17.8 3.47 and 4.27, 2^18.2 4.44 and 4.61, 2^18.8 5.24 and 4.91 )
+	if( quads <= 65536 ) {
+		return channelwise3x3SmallLaunch<STRIDE, 1>( s, d, source, filter, freeTerm, result, act, flipTaps );
+	}
+	if( quads <= 131072 ) {
+		return channelwise3x3SmallLaunch<STRIDE, 2>( s, d, source, filter, freeTerm, result, act, flipTaps );
+	}
+	if constexpr( STRIDE == 1 ) {
+		if( quads <= 262144 ) {
+			return channelwise3x3SmallLaunch<STRIDE, 4>( s, d, source, filter, freeTerm, result, act, flipTaps );
+		}
+	}
 	if( sourceBytes < ( 64LL << 20 ) ) {
 		// served by the caches: what counts is how many waves work at once, not what is read twice
 		const long long perRow = static_cast<long long>( d->batch ) * ceilDiv( d->resultWidth, WPT ) * ( d->channels / 4 );
