@@ -3177,7 +3177,212 @@ void expandDepthwiseKernel( const nhSeparableBlockDesc d, int outH, int outW, co
 	}
 }
 
+// The same two stages for blocks of a few images, where each of the launches is mostly the launch: a workgroup computes 16 channels of
+// the expanded tensor for `rows` output rows of the whole width and the rows around them, in LDS, and convolves them there. Its
+// wavefronts take 16 pixels at a time, weights as the matrix instructions' first operand, so that a lane ends up with four channels
+// of a pixel. The pixels come row by row ( four lanes to 64 bytes of a pixel ) and are turned round in the wavefront's own kilobyte of
+// LDS, those of its next 16 pixels on their way meanwhile. What bounds it is latency; the rows that neighbouring workgroups both
+// expand are the price of one launch less.
+template<int STRIDE, int KG>
+__global__ __launch_bounds__( 256 )
+void expandDepthwiseSmallKernel( const nhSeparableBlockDesc d, int outH, int outW, int rows, int rowGroups, int chunks, unsigned widthMagic,
+	unsigned outWMagic, const float* input, const float* expandFilter, const float* expandBias, const float* dwFilter, const float* dwBias,
+	float* reduced, const CFusedActivation expandActAsGiven, const CFusedActivation dwActAsGiven )
+{
+	extern __shared__ float4 expandLds[];
+	const int tid = threadIdx.x, lane = tid & 63;
+	const int wave = __builtin_amdgcn_readfirstlane( tid >> 6 );
+	const int l16 = lane & 15, quad = lane >> 4;
+	const int loadRow = lane >> 2, loadQuad = lane & 3;
+	const int cin = d.inputChannels, E = d.expandedChannels, W = d.width, pitch = W + 2;
+	int t = xcdSwizzle( blockIdx.x, gridDim.x );
+	const int e0 = ( t % chunks ) * 16; t /= chunks;
+	const int ho0 = ( t % rowGroups ) * rows, n = t / rowGroups;
+	const int rowsHere = min( rows, outH - ho0 );
+	const int rowsIn = ( rowsHere - 1 ) * STRIDE + 3;
+	const int hi0 = ho0 * STRIDE - 1;
+	const int hiBegin = max( hi0, 0 ), hiEnd = min( hi0 + rowsIn, d.height );
+	float4* stage = expandLds + wave * 64;
+	float4* region = expandLds + 256; // [rowsIn][W + 2][16 channels], zeros around the image
+
+	const CFusedActivation expandAct = withParam( expandActAsGiven ), dwAct = withParam( dwActAsGiven );
+	const int c = e0 + ( tid & 3 ) * 4; // the thread's channels in the second stage
+	float4 f[9];
+#pragma unroll
+	for( int k = 0; k < 9; ++k ) {
+		f[k] = *reinterpret_cast<const float4*>( dwFilter + k * E + c );
+	}
+	const float4 zero = make_float4( 0.f, 0.f, 0.f, 0.f );
+	const float4 dwFree = dwBias != nullptr ? *reinterpret_cast<const float4*>( dwBias + c ) : zero;
+	const float4 expandFree = expandBias != nullptr ? *reinterpret_cast<const float4*>( expandBias + e0 + quad * 4 ) : zero;
+
+	const int pixels = ( hiEnd - hiBegin ) * W;
+	const __amdgpu_buffer_rsrc_t bufIn = __builtin_amdgcn_make_buffer_rsrc(
+		const_cast<float*>( input + ( static_cast<long long>( n ) * d.height + hiBegin ) * W * cin ), 0, static_cast<unsigned>( pixels * cin ) * 4u, 0x00020000 );
+	const __amdgpu_buffer_rsrc_t bufW = __builtin_amdgcn_make_buffer_rsrc(
+		const_cast<float*>( expandFilter + static_cast<long long>( e0 ) * cin ), 0, static_cast<unsigned>( 16 * cin ) * 4u, 0x00020000 );
+	// ( quads behind the last channel and rows behind the last pixel are out of the descriptors' range: zeros )
+	auto load = [&]( __amdgpu_buffer_rsrc_t from, int row, float4 ( &to )[KG] ) {
+#pragma unroll
+		for( int g = 0; g < KG; ++g ) {
+			const int k = g * 16 + loadQuad * 4;
+			to[g] = bufferLoad4( from, k < cin ? static_cast<unsigned>( ( row + loadRow ) * cin + k ) * 4u : OutOfRange );
+		}
+	};
+	// ( one wavefront's instructions are executed in order by the LDS unit: no barrier )
+	auto turn = [&]( const float4& v ) {
+		stage[loadRow * 4 + ( loadQuad ^ ( ( loadRow >> 2 ) & 3 ) )] = v;
+		__builtin_amdgcn_wave_barrier();
+		asm volatile( "" ::: "memory" );
+		const float4 r = stage[l16 * 4 + ( quad ^ ( ( l16 >> 2 ) & 3 ) )];
+		__builtin_amdgcn_wave_barrier();
+		asm volatile( "" ::: "memory" );
+		return r;
+	};
+	float4 weights[KG], next[KG];
+	load( bufW, 0, weights );
+	load( bufIn, wave * 16, next );
+	// the border: a column on either side, and the rows that lie outside the image
+	for( int i = tid; i < rowsIn * 8; i += 256 ) {
+		region[( ( i >> 3 ) * pitch + ( ( i & 4 ) != 0 ? W + 1 : 0 ) ) * 4 + ( i & 3 )] = zero;
+	}
+	if( hi0 < 0 ) {
+		for( int i = tid; i < W * 4; i += 256 ) {
+			region[4 + i] = zero;
+		}
+	}
+	if( hi0 + rowsIn > d.height ) {
+		for( int i = tid; i < W * 4; i += 256 ) {
+			region[( rowsIn - 1 ) * pitch * 4 + 4 + i] = zero;
+		}
+	}
+#pragma unroll
+	for( int g = 0; g < KG; ++g ) {
+		weights[g] = turn( weights[g] );
+	}
+	typedef float f32x4 __attribute__( ( ext_vector_type( 4 ) ) );
+	for( int p0 = wave * 16; p0 < pixels; p0 += 64 ) {
+		float4 x[KG];
+#pragma unroll
+		for( int g = 0; g < KG; ++g ) {
+			x[g] = next[g];
+		}
+		load( bufIn, p0 + 64, next );
+		f32x4 acc[2] = { { 0.f, 0.f, 0.f, 0.f }, { 0.f, 0.f, 0.f, 0.f } };
+#pragma unroll
+		for( int g = 0; g < KG; ++g ) {
+			const float4 v = turn( x[g] );
+			acc[0] = __builtin_amdgcn_mfma_f32_16x16x4f32( weights[g].x, v.x, acc[0], 0, 0, 0 );
+			acc[1] = __builtin_amdgcn_mfma_f32_16x16x4f32( weights[g].y, v.y, acc[1], 0, 0, 0 );
+			acc[0] = __builtin_amdgcn_mfma_f32_16x16x4f32( weights[g].z, v.z, acc[0], 0, 0, 0 );
+			acc[1] = __builtin_amdgcn_mfma_f32_16x16x4f32( weights[g].w, v.w, acc[1], 0, 0, 0 );
+		}
+		// lane ( l16, quad ): channels e0 + 4 quad .. + 3 of pixel p0 + l16
+		const int p = p0 + l16;
+		int row, column;
+		fastDivMod( p, W, widthMagic, row, column );
+		float4 v;
+		v.x = applyActivation( acc[0][0] + acc[1][0] + expandFree.x, expandAct );
+		v.y = applyActivation( acc[0][1] + acc[1][1] + expandFree.y, expandAct );
+		v.z = applyActivation( acc[0][2] + acc[1][2] + expandFree.z, expandAct );
+		v.w = applyActivation( acc[0][3] + acc[1][3] + expandFree.w, expandAct );
+		if( p < pixels ) {
+			region[( ( row + hiBegin - hi0 ) * pitch + column + 1 ) * 4 + quad] = v;
+		}
+	}
+	__syncthreads();
+	float* out = reduced + ( static_cast<long long>( n ) * outH + ho0 ) * outW * E + c;
+	for( int o = tid >> 2; o < rowsHere * outW; o += 64 ) {
+		int row, column;
+		fastDivMod( o, outW, outWMagic, row, column );
+		const float4* corner = region + ( row * STRIDE * pitch + column * STRIDE ) * 4 + ( tid & 3 );
+		float4 acc = dwFree;
+#pragma unroll
+		for( int kh = 0; kh < 3; ++kh ) {
+#pragma unroll
+			for( int kw = 0; kw < 3; ++kw ) {
+				acc = CChanVec<4>::fma( corner[( kh * pitch + kw ) * 4], f[kh * 3 + kw], acc );
+			}
+		}
+		*reinterpret_cast<float4*>( out + static_cast<long long>( o ) * E ) = CChanVec<4>::activate( acc, dwAct );
+	}
+}
+
+// Values of the expanded tensor, times the groups of 16 input channels behind each: where the rows expanded twice and the workgroups'
+// rounds cost what the launch costs. us of a whole block with the two launches and with this one, up to the line: 112 x 112 x 16 -> 96 stride 2,
+// one image 10.9 and 9.8, four 25.5 and 16.8; 56 x 56 x 24 -> 144, one 10.5 and 9.2, four 18.0 and 17.4; 28 x 28 x 32 -> 192, one 9.2 and
+// 7.2, 16 19.8 and 19.1; 14 x 14 x 64 -> 384, one 9.5 and 7.2, 16 16.9 and 14.8; 7 x 7 x 160 -> 960, one 10.8 and 9.7, eight 14.9 and 12.0; and
+// beyond it: 14 x 14 x 96 -> 576, eight 16.2 and 17.2; 7 x 7 x 160 -> 960, 16 17.0 and 18.1; 56 x 56 x 24 -> 144, 16 36.2 and 47.6.
+constexpr long long MaxExpandSmall = 5 << 20;
+constexpr int ExpandSmallLdsQuads = 3840; // 60 KB: a region of a workgroup, next to the 4 KB that its wavefronts turn operands in
+
 } // namespace nh
+
+// true ( and launched ) for blocks of a few images
+static bool tryExpandDepthwiseSmall( nhStream s, const nhSeparableBlockDesc* d, const nhConvDesc& dw, const float* input,
+	const float* expandFilter, const float* expandBias, const float* dwFilter, const float* dwBias, float* reduced )
+{
+	const int cin = d->inputChannels, E = d->expandedChannels;
+	const long long pixelsIn = static_cast<long long>( d->batch ) * d->height * d->width;
+	const auto aligned = []( const float* p ) { return isAligned16( p ); };
+	if( cin % 4 != 0 || cin > 160 || E % 16 != 0 || !aligned( input ) || !aligned( expandFilter ) || !aligned( expandBias ) || !aligned( dwFilter )
+		|| !aligned( dwBias ) || !aligned( reduced ) || pixelsIn * cin * 4 > 0x7fffffffLL || pixelsIn * E * ceilDiv( cin, 16 ) > MaxExpandSmall ) {
+		return false;
+	}
+	const int groups = ceilDiv( cin, 16 ), chunks = E / 16, outH = dw.resultHeight, outW = dw.resultWidth, stride = d->stride;
+	// the rows of a workgroup: as long as its slowest wavefront's pixels and a thread's outputs, in rounds of workgroups
+	int rows = 0;
+	double best = 0;
+	for( int r = 1; r <= outH; ++r ) {
+		const int rowsIn = ( r - 1 ) * stride + 3;
+		if( rowsIn * ( d->width + 2 ) * 4 > ExpandSmallLdsQuads ) {
+			break;
+		}
+		const double workgroups = static_cast<double>( ceilDiv( outH, r ) ) * d->batch * chunks;
+		const double length = 2000 + ceilDiv( rowsIn * d->width, 64 ) * ( groups * 170.0 + 250 ) + ceilDiv( r * outW, 64 ) * 350.0;
+		const double cost = length * ( workgroups <= 256 ? 1.0 : 0.4 + 0.6 * workgroups / 256 );
+		if( rows == 0 || cost < best ) {
+			rows = r;
+			best = cost;
+		}
+	}
+	if( rows == 0 ) {
+		return false;
+	}
+	const int rowGroups = ceilDiv( outH, rows );
+	const long long workgroups = static_cast<long long>( rowGroups ) * d->batch * chunks;
+	if( workgroups > 0x7ffffff0LL ) {
+		return false;
+	}
+	const size_t lds = ( 256 + static_cast<size_t>( ( rows - 1 ) * stride + 3 ) * ( d->width + 2 ) * 4 ) * sizeof( float4 );
+	const CFusedActivation expandAct = { d->expandActivation, d->expandParam };
+	const CFusedActivation dwAct = { d->channelwiseActivation, d->channelwiseParam };
+	auto launch = [&]( auto strideOf, auto groupsOf ) {
+		constexpr int Stride = decltype( strideOf )::value, Groups = decltype( groupsOf )::value;
+		hipLaunchKernelGGL( ( expandDepthwiseSmallKernel<Stride, Groups> ), dim3( static_cast<unsigned>( workgroups ) ), dim3( 256 ), lds, toStream( s ), *d,
+			outH, outW, rows, rowGroups, chunks, divisionMagic( d->width ), divisionMagic( outW ), input, expandFilter, expandBias, dwFilter, dwBias,
+			reduced, expandAct, dwAct );
+	};
+	auto launchGroups = [&]( auto strideOf ) {
+		if( groups <= 1 ) {
+			launch( strideOf, std::integral_constant<int, 1>() );
+		} else if( groups <= 2 ) {
+			launch( strideOf, std::integral_constant<int, 2>() );
+		} else if( groups <= 4 ) {
+			launch( strideOf, std::integral_constant<int, 4>() );
+		} else if( groups <= 6 ) {
+			launch( strideOf, std::integral_constant<int, 6>() );
+		} else {
+			launch( strideOf, std::integral_constant<int, 10>() );
+		}
+	};
+	if( stride == 1 ) {
+		launchGroups( std::integral_constant<int, 1>() );
+	} else {
+		launchGroups( std::integral_constant<int, 2>() );
+	}
+	return true;
+}
 
 // true ( and launched ) where the fused kernel is built for the block and the expanded tensor is too large for the caches
 static bool tryExpandDepthwise( nhStream s, const nhSeparableBlockDesc* d, const nhConvDesc& dw, const float* input,
@@ -3884,7 +4089,8 @@ int nhMobileNetV2Block( nhStream s, const nhSeparableBlockDesc* d, const float* 
 	const CFusedActivation expandAct = { d->expandActivation, d->expandParam };
 	const CFusedActivation channelwiseAct = { d->channelwiseActivation, d->channelwiseParam };
 	const CFusedActivation none = { NH_ACT_NONE, 0.f };
-	if( tryExpandDepthwise( s, d, dw, input, expandFilter, expandFreeTerm, channelwiseFilter, channelwiseFreeTerm, reduced ) ) {
+	if( tryExpandDepthwiseSmall( s, d, dw, input, expandFilter, expandFreeTerm, channelwiseFilter, channelwiseFreeTerm, reduced )
+		|| tryExpandDepthwise( s, d, dw, input, expandFilter, expandFreeTerm, channelwiseFilter, channelwiseFreeTerm, reduced ) ) {
 		NH_LAUNCH_CHECK();
 	} else {
 		rc = matMulNTFused( toStream( s ), input, d->inputChannels, expandFilter, d->inputChannels, expanded, d->expandedChannels,
