@@ -864,8 +864,18 @@ struct CPendingColumnSum {
 	int Count() const { return ColumnsOf > 0 ? ColumnsOf * Width : Height; }
 };
 
+// Sums of rows with their tails that wait on while the calls behind them are queued: those of a normalisation, whose mean and
+// inverse deviation the passes over the matrix read ( CObjectNormalizationLayer, see launchNormalization ). They go out in front of
+// whatever else the queue holds.
+struct CParkedSum {
+	CPendingColumnSum Sum;
+	CTinyChain Tail;
+};
+
 struct CTinyQueue {
 	bool Enabled = false;
+	CParkedSum Parked[2] = {};
+	int ParkedCount = 0;
 	CTinyChain Chain = {};
 	// A call over more than TinyWideMaxCount elements begins a chain that only calls of the same count join ( the passes
 	// of an activation or of a solver over one blob, quadChainKernel ); if none does, the call goes out as the launch it
@@ -1142,11 +1152,25 @@ static bool launchKnownChain( hipStream_t stream, const CTinyChain& chain )
 	return false;
 }
 
+static void launchColumnSum( hipStream_t stream, const CPendingColumnSum& sum, const CTinyChain& tail );
+
+static bool launchParked( hipStream_t stream, CTinyQueue& queue )
+{
+	const int count = queue.ParkedCount;
+	queue.ParkedCount = 0;
+	for( int i = 0; i < count; ++i ) {
+		launchColumnSum( stream, queue.Parked[i].Sum, queue.Parked[i].Tail );
+		__atomic_fetch_sub( &tinyChainsPending, 1, __ATOMIC_RELAXED );
+	}
+	return count > 0;
+}
+
 static bool launchTinyChain( hipStream_t stream, CTinyQueue& queue )
 {
 	CTinyChain& chain = queue.Chain;
+	const bool parked = launchParked( stream, queue );
 	if( chain.Length == 0 ) {
-		return false;
+		return parked;
 	}
 	// ( a call that nothing has joined goes out as the launch it would have been on any other stream: the large ones for
 	// their kernels' rates, the small ones because a chain's launch takes 5 us where theirs takes 4 )
@@ -1361,29 +1385,242 @@ int sumShortRows( hipStream_t stream, int batch, float* result, const float* mat
 	return NH_OK;
 }
 
+static bool rangesMeet( const float* a, long long countA, const float* b, long long countB )
+{
+	return a != nullptr && b != nullptr && a < b + countB && b < a + countA;
+}
+
+// The thirteen calls of CObjectNormalizationLayer::runOnceImpl ( NeoML/src/Dnn/Layers/ObjectNormalizationLayer.cpp:181-242 ), and the sum of
+// two in front of them, as one pass: a wavefront holds its row in registers and walks over it three times. With the expressions of
+// the separate launches and their order of additions ( sumColumnsTailKernel, normalizeChainKernel ): the same bits.
+// Bound by memory for many rows and by launches for few; us, three launches and one: 8192 x 512 ( five blobs of 16 MB ) 24.0 and 13.7
+// = 6.1 TB/s, 2048 x 384 11.2 and 4.1, 37 x 512 9.4 and 2.8, 300 x 2048 12.6 and 5.5.
+template<int QUADS, bool ADD>
+__global__ __launch_bounds__( 256 )
+void normalizeRowsKernel( const float* first, const float* second, float* matrix, float* square, float* centred, float* out, float* mean,
+	float* deviation, const float* scale, const float* bias, const float* negInvWidth, const float* invWidth, const float* epsilon, int height,
+	int width )
+{
+#pragma clang fp contract( off )
+	const int row = blockIdx.x * 4 + ( threadIdx.x >> 6 );
+	if( row >= height ) {
+		return;
+	}
+	const int lane = threadIdx.x & 63;
+	const int w4 = width >> 2;
+	const long long offset = static_cast<long long>( row ) * width;
+	// ( the functors of these calls, written out: theirs may be contracted into a fused multiply-add once they are inlined here )
+	const float negFactor = *negInvWidth, varianceFactor = *invWidth, addition = *epsilon;
+	float4 v[QUADS], factor[QUADS], shift[QUADS];
+#pragma unroll
+	for( int q = 0; q < QUADS; ++q ) {
+		const int i = lane + q * 64;
+		v[q] = make_float4( 0.f, 0.f, 0.f, 0.f );
+		if( i < w4 ) {
+			v[q] = reinterpret_cast<const float4*>( first + offset )[i];
+			if( ADD ) {
+				const float4 y = reinterpret_cast<const float4*>( second + offset )[i];
+				v[q] = make_float4( v[q].x + y.x, v[q].y + y.y, v[q].z + y.z, v[q].w + y.w );
+			}
+			factor[q] = reinterpret_cast<const float4*>( scale )[i];
+			shift[q] = reinterpret_cast<const float4*>( bias )[i];
+		}
+	}
+	float s = 0.f;
+#pragma unroll
+	for( int q = 0; q < QUADS; ++q ) {
+		if( lane + q * 64 < w4 ) {
+			if( ADD ) {
+				reinterpret_cast<float4*>( matrix + offset )[lane + q * 64] = v[q];
+			}
+			s += ( v[q].x + v[q].y ) + ( v[q].z + v[q].w );
+		}
+	}
+	const float toRow = -waveReduceSum( s ) * negFactor;
+	s = 0.f;
+#pragma unroll
+	for( int q = 0; q < QUADS; ++q ) {
+		if( lane + q * 64 < w4 ) {
+			v[q] = make_float4( v[q].x + toRow, v[q].y + toRow, v[q].z + toRow, v[q].w + toRow );
+			const float4 squared = make_float4( v[q].x * v[q].x, v[q].y * v[q].y, v[q].z * v[q].z, v[q].w * v[q].w );
+			reinterpret_cast<float4*>( square + offset )[lane + q * 64] = squared;
+			s += ( squared.x + squared.y ) + ( squared.z + squared.w );
+		}
+	}
+	const float variance = waveReduceSum( s ) * varianceFactor;
+	const float byRow = CInvOp()( CSqrtOp()( variance + addition, 0.f, 0.f ), 0.f, 0.f );
+	if( lane == 0 ) {
+		mean[row] = toRow;
+		deviation[row] = byRow;
+	}
+#pragma unroll
+	for( int q = 0; q < QUADS; ++q ) {
+		if( lane + q * 64 < w4 ) {
+			const float4 c = make_float4( v[q].x * byRow, v[q].y * byRow, v[q].z * byRow, v[q].w * byRow );
+			const float4 f = factor[q], b = shift[q];
+			if( out != centred ) {
+				reinterpret_cast<float4*>( centred + offset )[lane + q * 64] = c;
+			}
+			const float4 scaled = make_float4( c.x * f.x, c.y * f.y, c.z * f.z, c.w * f.w );
+			reinterpret_cast<float4*>( out + offset )[lane + q * 64] = make_float4( scaled.x + b.x, scaled.y + b.y, scaled.z + b.z, scaled.w + b.w );
+		}
+	}
+}
+
+constexpr int MaxNormalizeWidth = 2048; // eight quads to a lane
+
+// Two parked sums and the chain behind them: true ( launched, the queue empty ) if they are a whole normalisation whose blobs are apart
+static bool launchNormalization( hipStream_t stream, CTinyQueue& queue )
+{
+	CTinyChain& chain = queue.Chain;
+	if( queue.ParkedCount != 2 || chain.Length != 4 ) {
+		return false;
+	}
+	const CPendingColumnSum& first = queue.Parked[0].Sum;
+	const CPendingColumnSum& second = queue.Parked[1].Sum;
+	const CTinyChain& toMean = queue.Parked[0].Tail;
+	const CTinyChain& toDeviation = queue.Parked[1].Tail;
+	const CTinyOp* op = chain.Ops;
+	const int height = first.Height, width = first.Width;
+	const long long count = static_cast<long long>( height ) * width;
+	bool known = toMean.Length == 1 && isKind<CNegMulValueOp>( toMean.Ops[0] ) && toDeviation.Length == 4
+		&& isKind<CMulValueOp<float>>( toDeviation.Ops[0] ) && isKind<CAddValueOp<float>>( toDeviation.Ops[1] )
+		&& isKind<CSqrtOp>( toDeviation.Ops[2] ) && isKind<CInvOp>( toDeviation.Ops[3] );
+	known = known && isKind<CAddOp<float>>( op[0] ) && isKind<CMulOp<float>>( op[1] ) && isKind<CMulOp<float>>( op[2] )
+		&& isKind<CAddOp<float>>( op[3] ) && op[0].Spread == TS_PerRow && op[1].Spread == TS_PerRow && op[2].Spread == TS_PerColumn
+		&& op[3].Spread == TS_PerColumn;
+	float* centred = op[0].Out;
+	float* out = op[2].Out;
+	known = known && op[0].In[0] == first.Matrix && op[0].In[1] == first.Result && op[1].In[0] == centred && op[1].Out == centred
+		&& op[1].In[1] == second.Result && op[2].In[0] == centred && op[3].In[0] == out && op[3].Out == out;
+	for( int k = 0; k < 4; ++k ) {
+		known = known && op[k].Count == count && op[k].Width == width && op[k].Barrier == 0;
+	}
+	if( !known ) {
+		return false;
+	}
+	const bool add = first.AddFirst != nullptr;
+	const float* x = add ? first.AddFirst : first.Matrix;
+	const float* y = add ? first.AddSecond : first.Matrix;
+	const float* scale = op[2].In[1];
+	const float* bias = op[3].In[1];
+	const float* scalars[3] = { toMean.Ops[0].Scalar, toDeviation.Ops[0].Scalar, toDeviation.Ops[1].Scalar };
+	for( const float* p : { x, y, first.Matrix, second.Matrix, static_cast<const float*>( centred ), static_cast<const float*>( out ), scale, bias } ) {
+		if( !isAligned16( p ) ) {
+			return false;
+		}
+	}
+	// what is written and what is read: every blob apart from every other that is written ( a summand may be the sum's own place )
+	struct CBlob { const float* P; long long Count; };
+	CBlob written[6] = { { first.Result, height }, { second.Result, height }, { second.Matrix, count }, { centred, count } };
+	int writtenCount = 4;
+	if( out != centred ) {
+		written[writtenCount++] = { out, count };
+	}
+	if( add ) {
+		written[writtenCount++] = { first.Matrix, count };
+	}
+	const CBlob read[8] = { { x, count }, { y, count }, { first.Matrix, count }, { scale, width }, { bias, width }, { scalars[0], 1 }, { scalars[1], 1 },
+		{ scalars[2], 1 } };
+	for( int i = 0; i < writtenCount; ++i ) {
+		for( int j = i + 1; j < writtenCount; ++j ) {
+			if( rangesMeet( written[i].P, written[i].Count, written[j].P, written[j].Count ) ) {
+				return false;
+			}
+		}
+		for( const CBlob& blob : read ) {
+			if( !( blob.P == first.Matrix && written[i].P == first.Matrix ) && rangesMeet( written[i].P, written[i].Count, blob.P, blob.Count ) ) {
+				return false;
+			}
+		}
+	}
+	auto launch = [&]( auto quadsOf ) {
+		constexpr int Quads = decltype( quadsOf )::value;
+		float* matrix = const_cast<float*>( first.Matrix );
+		float* square = const_cast<float*>( second.Matrix );
+		if( add ) {
+			hipLaunchKernelGGL( ( normalizeRowsKernel<Quads, true> ), dim3( ceilDiv( height, 4 ) ), dim3( 256 ), 0, stream, x, y, matrix, square, centred,
+				out, first.Result, second.Result, scale, bias, scalars[0], scalars[1], scalars[2], height, width );
+		} else {
+			hipLaunchKernelGGL( ( normalizeRowsKernel<Quads, false> ), dim3( ceilDiv( height, 4 ) ), dim3( 256 ), 0, stream, x, y, matrix, square, centred,
+				out, first.Result, second.Result, scale, bias, scalars[0], scalars[1], scalars[2], height, width );
+		}
+	};
+	if( width <= 256 ) {
+		launch( std::integral_constant<int, 1>() );
+	} else if( width <= 512 ) {
+		launch( std::integral_constant<int, 2>() );
+	} else if( width <= 1024 ) {
+		launch( std::integral_constant<int, 4>() );
+	} else {
+		launch( std::integral_constant<int, 8>() );
+	}
+	queue.ParkedCount = 0;
+	chain.Length = 0;
+	__atomic_fetch_sub( &tinyChainsPending, 3, __ATOMIC_RELAXED );
+	return true;
+}
+
+// The sums that wait may wait on while this call ( + a value per row ) is queued: the first call behind the mean, or the first behind
+// the inverse deviation of the same rows
+static bool parkColumnSum( CTinyQueue& queue, const float* matrix, const float* vector, const float* result, int count, int width )
+{
+	const CPendingColumnSum& sum = queue.ColumnSum;
+	if( sum.ColumnsOf > 0 || sum.Width != width || width % 4 != 0 || width > MaxNormalizeWidth
+		|| static_cast<long long>( sum.Height ) * sum.Width != count || result == matrix ) {
+		return false;
+	}
+	if( queue.ParkedCount == 0 ) {
+		if( sum.SquareOf != nullptr || matrix != sum.Matrix || vector != sum.Result ) {
+			return false;
+		}
+	} else {
+		const CPendingColumnSum& first = queue.Parked[0].Sum;
+		if( queue.ParkedCount != 1 || sum.SquareOf != first.Matrix || sum.SquareShift != first.Result || matrix != first.Matrix
+			|| vector != first.Result || sum.Height != first.Height ) {
+			return false;
+		}
+	}
+	CParkedSum& parked = queue.Parked[queue.ParkedCount++]; // ( one thing waits where one waited )
+	parked.Sum = sum;
+	parked.Tail = queue.Chain;
+	queue.ColumnSum.Pending = false;
+	if( queue.Chain.Length > 0 ) {
+		queue.Chain.Length = 0;
+		__atomic_fetch_sub( &tinyChainsPending, 1, __ATOMIC_RELAXED );
+	}
+	return true;
+}
+
+static void launchColumnSum( hipStream_t stream, const CPendingColumnSum& sum, const CTinyChain& tail )
+{
+	const int vec = ( sum.Width % 4 == 0 && isAligned16( sum.Matrix ) && isAligned16( sum.AddFirst ) && isAligned16( sum.AddSecond )
+		&& isAligned16( sum.SquareOf ) ) ? 1 : 0;
+	if( sum.ColumnsOf > 0 ) {
+		launchSumShortRows( stream, sum.ColumnsOf, sum.Result, sum.Matrix, sum.Height, sum.Width, false, tail );
+	} else if( sum.AddFirst != nullptr ) {
+		hipLaunchKernelGGL( sumColumnsTailKernel<1>, dim3( ceilDiv( sum.Height, 4 ) ), dim3( 256 ), 0, stream, sum.Result, sum.Matrix,
+			sum.AddFirst, sum.AddSecond, const_cast<float*>( sum.Matrix ), sum.Height, sum.Width, vec, tail );
+	} else if( sum.SquareOf != nullptr ) {
+		hipLaunchKernelGGL( sumColumnsTailKernel<2>, dim3( ceilDiv( sum.Height, 4 ) ), dim3( 256 ), 0, stream, sum.Result, sum.Matrix,
+			sum.SquareOf, sum.SquareShift, const_cast<float*>( sum.Matrix ), sum.Height, sum.Width, vec, tail );
+	} else {
+		hipLaunchKernelGGL( sumColumnsTailKernel<0>, dim3( ceilDiv( sum.Height, 4 ) ), dim3( 256 ), 0, stream, sum.Result, sum.Matrix,
+			static_cast<const float*>( nullptr ), static_cast<const float*>( nullptr ), static_cast<float*>( nullptr ), sum.Height,
+			sum.Width, vec, tail );
+	}
+}
+
 // what the queue holds: the product that waits for its successor ( then nothing else is queued ), or a chain
 static bool launchPending( hipStream_t stream, CTinyQueue& queue )
 {
+	( void )launchParked( stream, queue ); // ( something else waits behind it )
 	if( queue.ColumnSum.Pending ) {
 		const CPendingColumnSum sum = queue.ColumnSum;
 		queue.ColumnSum.Pending = false;
 		__atomic_fetch_sub( &tinyChainsPending, 1, __ATOMIC_RELAXED );
 		CTinyChain& tail = queue.Chain; // ( calls in place over the sums, nothing else: deferEltwise sees to that )
-		const int vec = ( sum.Width % 4 == 0 && isAligned16( sum.Matrix ) && isAligned16( sum.AddFirst ) && isAligned16( sum.AddSecond )
-			&& isAligned16( sum.SquareOf ) ) ? 1 : 0;
-		if( sum.ColumnsOf > 0 ) {
-			launchSumShortRows( stream, sum.ColumnsOf, sum.Result, sum.Matrix, sum.Height, sum.Width, false, tail );
-		} else if( sum.AddFirst != nullptr ) {
-			hipLaunchKernelGGL( sumColumnsTailKernel<1>, dim3( ceilDiv( sum.Height, 4 ) ), dim3( 256 ), 0, stream, sum.Result, sum.Matrix,
-				sum.AddFirst, sum.AddSecond, const_cast<float*>( sum.Matrix ), sum.Height, sum.Width, vec, tail );
-		} else if( sum.SquareOf != nullptr ) {
-			hipLaunchKernelGGL( sumColumnsTailKernel<2>, dim3( ceilDiv( sum.Height, 4 ) ), dim3( 256 ), 0, stream, sum.Result, sum.Matrix,
-				sum.SquareOf, sum.SquareShift, const_cast<float*>( sum.Matrix ), sum.Height, sum.Width, vec, tail );
-		} else {
-			hipLaunchKernelGGL( sumColumnsTailKernel<0>, dim3( ceilDiv( sum.Height, 4 ) ), dim3( 256 ), 0, stream, sum.Result, sum.Matrix,
-				static_cast<const float*>( nullptr ), static_cast<const float*>( nullptr ), static_cast<float*>( nullptr ), sum.Height,
-				sum.Width, vec, tail );
-		}
+		launchColumnSum( stream, sum, tail );
 		if( tail.Length > 0 ) {
 			tail.Length = 0;
 			__atomic_fetch_sub( &tinyChainsPending, 1, __ATOMIC_RELAXED );
@@ -1462,7 +1699,7 @@ void flushAllTinyOps()
 	{
 		std::lock_guard<std::recursive_mutex> guard( tinyLock );
 		for( auto& entry : tinyQueues() ) {
-			if( entry.second.Chain.Length == 0 && !entry.second.LaunchWaits() ) {
+			if( entry.second.Chain.Length == 0 && entry.second.ParkedCount == 0 && !entry.second.LaunchWaits() ) {
 				continue;
 			}
 			if( entry.first.first != active ) {
@@ -1887,11 +2124,6 @@ static bool fusePendingSum( nhStream s, const float* first, float* result, int c
 	return true;
 }
 
-static bool rangesMeet( const float* a, long long countA, const float* b, long long countB )
-{
-	return a != nullptr && b != nullptr && a < b + countB && b < a + countA;
-}
-
 // whether the convolution reads or writes any of these values
 static bool touches( const CPendingConvolution& c, const float* p, long long count )
 {
@@ -2109,7 +2341,8 @@ static bool deferEltwise( nhStream s, const TIn* a, const TIn* b, const TIn* c, 
 			const float* own = scalarOf( f, 0 );
 			const bool tail = NIN == 1 && spread == TS_None && a == out && out == sum.Result && n == sum.Count()
 				&& found->second.Chain.Length < TinyChainMax && ( own == nullptr || own + 1 <= out || own >= out + n );
-			if( !tail ) {
+			constexpr bool Sum = std::is_same<F, CAddOp<float>>::value;
+			if( !tail && !( Sum && spread == TS_PerRow && parkColumnSum( found->second, a, b, out, n, width ) ) ) {
 				launchPending( stream, found->second );
 			}
 		} else if( found->second.LaunchWaits() ) {
@@ -2212,6 +2445,7 @@ static bool deferEltwise( nhStream s, const TIn* a, const TIn* b, const TIn* c, 
 		}
 		chain.Ops[chain.Length] = op;
 		++chain.Length;
+		( void )launchNormalization( stream, queue );
 		return true;
 	} else {
 		( void )s; ( void )a; ( void )b; ( void )c; ( void )out; ( void )n; ( void )f; ( void )spread; ( void )width; ( void )spreadAlone;
