@@ -649,23 +649,28 @@ static int sumMatrixRowsImpl( nhStream s, int batchSize, float* result, const fl
 }
 
 template<bool LOGSUMEXP>
-static int softmaxImpl( nhStream s, const float* matrix, int height, int width, float* result )
+static int softmaxImpl( hipStream_t stream, const float* matrix, int height, int width, float* result )
 {
 	if( height == 0 || width == 0 ) {
 		return NH_OK;
 	}
 	const dim3 grid( ceilDiv( height, RowsPerBlock ) );
 	if( width <= 64 ) {
-		hipLaunchKernelGGL( ( softmaxRowsKernel<1, LOGSUMEXP> ), grid, dim3( 256 ), 0, toStream( s ), matrix, height, width, result );
+		hipLaunchKernelGGL( ( softmaxRowsKernel<1, LOGSUMEXP> ), grid, dim3( 256 ), 0, stream, matrix, height, width, result );
 	} else if( width <= 256 ) {
-		hipLaunchKernelGGL( ( softmaxRowsKernel<4, LOGSUMEXP> ), grid, dim3( 256 ), 0, toStream( s ), matrix, height, width, result );
+		hipLaunchKernelGGL( ( softmaxRowsKernel<4, LOGSUMEXP> ), grid, dim3( 256 ), 0, stream, matrix, height, width, result );
 	} else if( width <= 1024 ) {
-		hipLaunchKernelGGL( ( softmaxRowsKernel<16, LOGSUMEXP> ), grid, dim3( 256 ), 0, toStream( s ), matrix, height, width, result );
+		hipLaunchKernelGGL( ( softmaxRowsKernel<16, LOGSUMEXP> ), grid, dim3( 256 ), 0, stream, matrix, height, width, result );
 	} else {
-		hipLaunchKernelGGL( ( softmaxRowsKernel<0, LOGSUMEXP> ), grid, dim3( 256 ), 0, toStream( s ), matrix, height, width, result );
+		hipLaunchKernelGGL( ( softmaxRowsKernel<0, LOGSUMEXP> ), grid, dim3( 256 ), 0, stream, matrix, height, width, result );
 	}
 	NH_LAUNCH_CHECK();
 	return NH_OK;
+}
+
+int nh::softmaxRows( hipStream_t stream, const float* matrix, int height, int width, float* result )
+{
+	return softmaxImpl<false>( stream, matrix, height, width, result );
 }
 
 // The launch of a call with a spread vector that a stream had put aside and nothing joined
@@ -824,13 +829,17 @@ int nhSumMatrixColumns( nhStream s, float* result, const float* matrix, int matr
 int nhMatrixSoftmaxByRows( nhStream s, const float* matrix, int height, int width, float* result )
 {
 	NH_REQUIRE( height >= 0 && width >= 0 );
-	return softmaxImpl<false>( s, matrix, height, width, result );
+	if( height > 0 && width > 0 && __atomic_load_n( &tinyChainsPending, __ATOMIC_RELAXED ) != 0
+		&& joinPendingSoftmax( s, matrix, height, width, result ) ) {
+		return NH_OK; // ( the scores of an attention layer were waiting for this call )
+	}
+	return softmaxImpl<false>( toStream( s ), matrix, height, width, result );
 }
 
 int nhMatrixLogSumExpByRows( nhStream s, const float* matrix, int height, int width, float* result, int resultSize )
 {
 	NH_REQUIRE( height >= 0 && width >= 0 && resultSize >= height );
-	return softmaxImpl<true>( s, matrix, height, width, result );
+	return softmaxImpl<true>( toStream( s ), matrix, height, width, result );
 }
 
 int nhFindMaxValueInRows( nhStream s, const float* matrix, int matrixHeight, int matrixWidth,
@@ -863,6 +872,11 @@ int nhFindMaxValueInColumns( nhStream s, int batchSize, const float* matrix, int
 int nhTransposeMatrix( nhStream s, int batchSize, const float* first, int height, int medium, int width,
 	int channels, float* result, int resultBufferSize )
 {
+	int rc = NH_OK;
+	if( __atomic_load_n( &tinyChainsPending, __ATOMIC_RELAXED ) != 0
+		&& fusePendingTransposition( s, batchSize, first, height, medium, width, channels, result, &rc ) ) {
+		return rc; // ( the result of an attention layer's core was waiting for this call )
+	}
 	return transposeImpl<float>( s, batchSize, first, height, medium, width, channels, result, resultBufferSize );
 }
 

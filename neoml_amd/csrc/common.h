@@ -63,10 +63,29 @@ bool fusePendingPadding( nhStream s, const nhPoolingDesc& d, const float* source
 // ( dnn_ops.hip ) the padding by itself; the padding with the pooling over it, false if the pair is not one it takes
 int launchPadding( hipStream_t stream, const CPendingPadding& padding );
 bool launchPaddingWithPooling( hipStream_t stream, const CPendingPadding& padding, const nhPoolingDesc& d, float* result, int* rc );
-// A batch of small dense row-major products that waits for the call behind it ( nhBatchMultiplyMatrixByMatrix followed by
-// nhVectorMultiply over the whole result in place: one launch )
+// A batch of small dense row-major products, Scores[b] = Q[b] * KT[b], that waits for the call behind it ( nhBatchMultiplyMatrixByMatrix ): the
+// factor over the whole result in place ( nhVectorMultiply ), and, where the attention kernel takes them, softmax over its rows
+// ( nhMatrixSoftmaxByRows ), the product of the weights and the values, and the exchange of heads and rows ( nhTransposeMatrix ): one launch.
+struct CPendingAttention {
+	bool Pending = false;
+	int Batch = 0, M = 0, N = 0, K = 0, D = 0, Heads = 1;
+	const float* Q = nullptr;
+	const float* KT = nullptr;
+	const float* V = nullptr;
+	const float* Scale = nullptr;
+	float* Scores = nullptr;
+	float* Weights = nullptr;
+	float* Context = nullptr;
+	float* Transposed = nullptr;
+};
 bool deferBatchedProduct( nhStream s, int batch, const float* first, int height, int width, const float* second, int secondWidth,
 	float* result );
+bool joinPendingSoftmax( nhStream s, const float* matrix, int height, int width, float* result );
+bool fusePendingTransposition( nhStream s, int batch, const float* first, int height, int medium, int width, int channels, float* result, int* rc );
+// ( attention.hip ) whether it takes the core of such a layer, and its launch; ( blas_ops.hip ) softmax over rows by itself
+bool attentionTakes( int batch, int M, int N, int K, int D, const float* q );
+int launchAttention( hipStream_t stream, const CPendingAttention& a );
+int softmaxRows( hipStream_t stream, const float* matrix, int height, int width, float* result );
 // The same for a convolution ( plain or channelwise, its descriptor checked by the caller ) and the VectorReLU over its
 // result in place that follows it in most networks.
 bool deferConvolution( nhStream s, bool channelwise, const nhConvDesc& d, const float* source, const float* filter,

@@ -828,17 +828,6 @@ struct CPendingSum {
 	int Count = 0;
 };
 
-// A batch of small products C[b] = A[b] * B[b] ( dense, row-major ) followed by VectorMultiply over the whole result in place
-// by a device scalar: CMatrixMultiplicationLayer + CLinearLayer, the scores of an attention layer and their 1 / sqrt( d )
-// ( NeoML/src/Dnn/Layers/MultiheadAttentionLayer.cpp:168-183 ). The kernel for such batches multiplies on the way out.
-struct CPendingBatched {
-	bool Pending = false;
-	const float* A = nullptr;
-	const float* B = nullptr;
-	float* C = nullptr;
-	int Batch = 0, M = 0, N = 0, K = 0;
-};
-
 // The sums of the rows of a matrix ( SumMatrixColumns: one value per row ) followed by element-wise calls with one operand
 // in place over those sums: the mean and the inverse deviation of CObjectNormalizationLayer ( sum, x -1/width; sum, x 1/width,
 // + epsilon, sqrt, 1/x ). The sum waits; such calls are queued behind it as its tail ( the queue's chain holds nothing else
@@ -889,7 +878,9 @@ struct CTinyQueue {
 	// with the first ( pending only while that is ).
 	CPendingConvolution Shortcut;
 	CPendingSum Sum;
-	CPendingBatched Batched;
+	// CMatrixMultiplicationLayer + CLinearLayer, the scores of an attention layer and their 1 / sqrt( d ), CSoftmaxLayer, the product with the
+	// values and the exchange of heads and rows ( NeoML/src/Dnn/Layers/MultiheadAttentionLayer.cpp:168-183 )
+	CPendingAttention Batched;
 	CPendingPadding Padding;
 	CPendingColumnSum ColumnSum;
 
@@ -916,10 +907,29 @@ static int launchPendingConvolution( hipStream_t stream, const CPendingConvoluti
 	return launchDeferredConvolution( stream, c.Channelwise, c.Desc, c.Source, c.Filter, c.FreeTerm, c.Result, act, c.Residual );
 }
 
-static int launchBatched( hipStream_t stream, const CPendingBatched& p, const float* scale, bool* scaled )
+static int launchBatched( hipStream_t stream, const CPendingAttention& p, const float* scale, bool* scaled )
 {
-	return matMulNN( stream, p.A, p.K, p.B, p.N, p.C, p.N, p.M, p.N, p.K, p.Batch, static_cast<long long>( p.M ) * p.K,
+	return matMulNN( stream, p.Q, p.K, p.KT, p.N, p.Scores, p.N, p.M, p.N, p.K, p.Batch, static_cast<long long>( p.M ) * p.K,
 		static_cast<long long>( p.K ) * p.N, static_cast<long long>( p.M ) * p.N, false, scale, scaled );
+}
+
+// what of it has been asked for by then
+static int launchPendingAttention( hipStream_t stream, const CPendingAttention& p )
+{
+	if( p.Context != nullptr ) {
+		return launchAttention( stream, p );
+	}
+	bool scaled = false;
+	int rc = launchBatched( stream, p, p.Scale, &scaled );
+	if( rc == NH_OK && p.Scale != nullptr && !scaled ) {
+		CMulValueOp<float> op; op.Ptr = p.Scale; op.Value = 0;
+		rc = launchEltwisePlain<1, float, float>( stream, static_cast<const float*>( p.Scores ), static_cast<const float*>( nullptr ),
+			static_cast<const float*>( nullptr ), p.Scores, p.Batch * p.M * p.N, op );
+	}
+	if( rc == NH_OK && p.Weights != nullptr ) {
+		rc = softmaxRows( stream, p.Scores, p.Batch * p.M, p.N, p.Weights );
+	}
+	return rc;
 }
 
 typedef std::map<std::pair<int, hipStream_t>, CTinyQueue> CTinyQueues;
@@ -1648,10 +1658,10 @@ static bool launchPending( hipStream_t stream, CTinyQueue& queue )
 		return true;
 	}
 	if( queue.Batched.Pending ) {
-		const CPendingBatched p = queue.Batched;
+		const CPendingAttention p = queue.Batched;
 		queue.Batched.Pending = false;
 		__atomic_fetch_sub( &tinyChainsPending, 1, __ATOMIC_RELAXED );
-		( void )launchBatched( stream, p, nullptr, nullptr );
+		( void )launchPendingAttention( stream, p );
 		return true;
 	}
 	if( queue.Padding.Pending ) {
@@ -1984,19 +1994,60 @@ bool fusePendingPadding( nhStream s, const nhPoolingDesc& d, const float* source
 	return false;
 }
 
+// the queue of a stream of the current device that puts calls aside ( with tinyLock held )
+static CTinyQueue* deferringQueue( hipStream_t stream )
+{
+	int device = 0;
+	if( hipGetDevice( &device ) != hipSuccess ) {
+		( void )hipGetLastError();
+		return nullptr;
+	}
+	auto found = tinyQueues().find( std::make_pair( device, stream ) );
+	return found != tinyQueues().end() && found->second.Enabled ? &found->second : nullptr;
+}
+
+// whether a blob that a waiting attention core is to write, or a scalar that it is to read, lies apart from what it has been handed so far
+static bool apartFrom( const CPendingAttention& p, const float* blob, long long count, bool alsoFromInputs )
+{
+	const long long scores = static_cast<long long>( p.Batch ) * p.M * p.N, context = static_cast<long long>( p.Batch ) * p.M * p.D;
+	return !rangesMeet( p.Scores, scores, blob, count ) && !rangesMeet( p.Weights, scores, blob, count ) && !rangesMeet( p.Context, context, blob, count )
+		&& ( !alsoFromInputs || ( !rangesMeet( p.Q, static_cast<long long>( p.Batch ) * p.M * p.K, blob, count )
+			&& !rangesMeet( p.KT, static_cast<long long>( p.Batch ) * p.K * p.N, blob, count )
+			&& !rangesMeet( p.V, static_cast<long long>( p.Batch ) * p.N * p.D, blob, count ) && !rangesMeet( p.Scale, 1, blob, count ) ) );
+}
+
 bool deferBatchedProduct( nhStream s, int batch, const float* first, int height, int width, const float* second, int secondWidth,
 	float* result )
 {
-	// ( only what the kernel for batches of small products may take: the others have nothing to gain from waiting )
-	if( __atomic_load_n( &tinyDeferringStreams, __ATOMIC_RELAXED ) == 0 || batch < 2 || height <= 0 || width <= 0 || width > 256
+	// ( only what the kernel for batches of small products may take, or the attention kernel: the others have nothing to gain from waiting )
+	if( __atomic_load_n( &tinyDeferringStreams, __ATOMIC_RELAXED ) == 0 || batch < 1 || height <= 0 || width <= 0
 		|| secondWidth <= 0 || first == nullptr || second == nullptr || result == nullptr
 		|| static_cast<long long>( batch ) * height * secondWidth > 0x7fffffffLL ) {
 		return false;
 	}
+	if( __atomic_load_n( &tinyChainsPending, __ATOMIC_RELAXED ) != 0 ) {
+		// the product of the weights that wait and their values
+		std::lock_guard<std::recursive_mutex> guard( tinyLock );
+		CTinyQueue* queue = deferringQueue( reinterpret_cast<hipStream_t>( s ) );
+		if( queue != nullptr && queue->Batched.Pending && queue->Batched.Weights != nullptr && queue->Batched.Context == nullptr ) {
+			CPendingAttention& p = queue->Batched;
+			if( first == p.Weights && batch == p.Batch && height == p.M && width == p.N
+				&& attentionTakes( batch, p.M, p.N, p.K, secondWidth, p.Q ) && apartFrom( p, second, static_cast<long long>( batch ) * width * secondWidth, false )
+				&& apartFrom( p, result, static_cast<long long>( batch ) * height * secondWidth, true )
+				&& !rangesMeet( second, static_cast<long long>( batch ) * width * secondWidth, result, static_cast<long long>( batch ) * height * secondWidth ) ) {
+				p.V = second;
+				p.D = secondWidth;
+				p.Context = result;
+				return true;
+			}
+		}
+	}
+	if( width > 256 || ( batch < 2 && !attentionTakes( batch, height, secondWidth, width, 64, first ) ) ) {
+		return false;
+	}
 	const hipStream_t stream = toStream( s ); // ( what the stream holds goes out first )
-	int device = 0;
 	hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-	if( hipGetDevice( &device ) != hipSuccess || hipStreamIsCapturing( stream, &capture ) != hipSuccess ) {
+	if( hipStreamIsCapturing( stream, &capture ) != hipSuccess ) {
 		( void )hipGetLastError();
 		return false;
 	}
@@ -2004,41 +2055,42 @@ bool deferBatchedProduct( nhStream s, int batch, const float* first, int height,
 		return false;
 	}
 	std::lock_guard<std::recursive_mutex> guard( tinyLock );
-	auto found = tinyQueues().find( std::make_pair( device, stream ) );
-	if( found == tinyQueues().end() || !found->second.Enabled || found->second.Chain.Length != 0 || found->second.LaunchWaits() ) {
+	CTinyQueue* queue = deferringQueue( stream );
+	if( queue == nullptr || queue->Chain.Length != 0 || queue->LaunchWaits() ) {
 		return false;
 	}
-	CPendingBatched& p = found->second.Batched;
+	CPendingAttention& p = queue->Batched;
+	p = CPendingAttention();
 	p.Pending = true;
-	p.A = first; p.B = second; p.C = result; p.Batch = batch; p.M = height; p.N = secondWidth; p.K = width;
+	p.Q = first; p.KT = second; p.Scores = result; p.Batch = batch; p.M = height; p.N = secondWidth; p.K = width;
 	__atomic_fetch_add( &tinyChainsPending, 1, __ATOMIC_RELAXED );
 	return true;
 }
 
 // VectorMultiply( first -> result, count, multiplier ) asks whether it is the call a batch of products waits for. true: both
-// have been launched as one ( *rc ). false: the caller goes on as usual ( a waiting batch has then been launched by itself if
-// this call is over its result but its kernel cannot multiply; otherwise the caller's own launch sends it out first ).
+// have been launched as one ( *rc ), or wait on as the scores of an attention layer. false: the caller goes on as usual ( a waiting batch has
+// then been launched by itself if this call is over its result but its kernel cannot multiply; otherwise the caller's own launch sends it out
+// first ).
 static bool fusePendingBatched( nhStream s, const float* first, float* result, int count, const float* multiplier, int* rc )
 {
 	const hipStream_t stream = reinterpret_cast<hipStream_t>( s );
-	int device = 0;
-	if( hipGetDevice( &device ) != hipSuccess ) {
-		( void )hipGetLastError();
-		return false;
-	}
-	CPendingBatched p;
+	CPendingAttention p;
 	{
 		std::lock_guard<std::recursive_mutex> guard( tinyLock );
-		auto found = tinyQueues().find( std::make_pair( device, stream ) );
-		if( found == tinyQueues().end() || !found->second.Batched.Pending ) {
+		CTinyQueue* queue = deferringQueue( stream );
+		if( queue == nullptr || !queue->Batched.Pending || queue->Batched.Weights != nullptr ) {
 			return false;
 		}
-		p = found->second.Batched;
-		if( first != p.C || result != p.C || multiplier == nullptr
+		p = queue->Batched;
+		if( first != p.Scores || result != p.Scores || multiplier == nullptr || p.Scale != nullptr
 			|| static_cast<long long>( count ) != static_cast<long long>( p.Batch ) * p.M * p.N ) {
 			return false;
 		}
-		found->second.Batched.Pending = false;
+		if( attentionTakes( p.Batch, p.M, p.N, p.K, 64, p.Q ) && apartFrom( p, multiplier, 1, false ) ) {
+			queue->Batched.Scale = multiplier;
+			return true;
+		}
+		queue->Batched.Pending = false;
 		__atomic_fetch_sub( &tinyChainsPending, 1, __ATOMIC_RELAXED );
 	}
 	bool scaled = false;
@@ -2047,6 +2099,50 @@ static bool fusePendingBatched( nhStream s, const float* first, float* result, i
 		noteStreamUse( stream );
 	}
 	return scaled || *rc != NH_OK;
+}
+
+bool joinPendingSoftmax( nhStream s, const float* matrix, int height, int width, float* result )
+{
+	std::lock_guard<std::recursive_mutex> guard( tinyLock );
+	CTinyQueue* queue = deferringQueue( reinterpret_cast<hipStream_t>( s ) );
+	if( queue == nullptr || !queue->Batched.Pending || queue->Batched.Weights != nullptr || result == nullptr ) {
+		return false;
+	}
+	CPendingAttention& p = queue->Batched;
+	const long long count = static_cast<long long>( height ) * width;
+	if( matrix != p.Scores || width != p.N || height != static_cast<long long>( p.Batch ) * p.M || !attentionTakes( p.Batch, p.M, p.N, p.K, 64, p.Q )
+		|| !apartFrom( p, result, count, true ) ) {
+		return false;
+	}
+	p.Weights = result;
+	return true;
+}
+
+bool fusePendingTransposition( nhStream s, int batch, const float* first, int height, int medium, int width, int channels, float* result, int* rc )
+{
+	const hipStream_t stream = reinterpret_cast<hipStream_t>( s );
+	CPendingAttention p;
+	{
+		std::lock_guard<std::recursive_mutex> guard( tinyLock );
+		CTinyQueue* queue = deferringQueue( stream );
+		if( queue == nullptr || !queue->Batched.Pending || queue->Batched.Context == nullptr || result == nullptr ) {
+			return false;
+		}
+		p = queue->Batched;
+		if( first != p.Context || medium != 1 || batch <= 0 || height <= 0 || static_cast<long long>( batch ) * height != p.Batch || width != p.M || channels != p.D
+			|| !apartFrom( p, result, static_cast<long long>( p.Batch ) * p.M * p.D, true ) ) {
+			return false;
+		}
+		queue->Batched.Pending = false;
+		__atomic_fetch_sub( &tinyChainsPending, 1, __ATOMIC_RELAXED );
+	}
+	p.Transposed = result;
+	p.Heads = height;
+	*rc = launchAttention( stream, p );
+	if( __atomic_load_n( &lstmPartnersAwaited, __ATOMIC_RELAXED ) != 0 ) {
+		noteStreamUse( stream );
+	}
+	return true;
 }
 
 static int launchPlainSum( hipStream_t stream, const CPendingSum& sum )
@@ -2131,17 +2227,6 @@ static bool touches( const CPendingConvolution& c, const float* p, long long cou
 	return rangesMeet( c.Source, static_cast<long long>( d.batch ) * d.height * d.width * d.channels, p, count )
 		|| rangesMeet( c.Filter, static_cast<long long>( d.filterCount ) * d.filterHeight * d.filterWidth * d.channels, p, count )
 		|| rangesMeet( c.FreeTerm, d.filterCount, p, count ) || rangesMeet( c.Result, c.ResultCount(), p, count );
-}
-
-static CTinyQueue* deferringQueue( hipStream_t stream )
-{
-	int device = 0;
-	if( hipGetDevice( &device ) != hipSuccess ) {
-		( void )hipGetLastError();
-		return nullptr;
-	}
-	auto found = tinyQueues().find( std::make_pair( device, stream ) );
-	return found != tinyQueues().end() && found->second.Enabled ? &found->second : nullptr;
 }
 
 bool deferConvolution( nhStream s, bool channelwise, const nhConvDesc& d, const float* source, const float* filter,
