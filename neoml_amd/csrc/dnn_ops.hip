@@ -389,6 +389,7 @@ struct CPadPoolArgs {
 	float DefaultValue;
 	int StrideHeight, StrideWidth, ResultHeight, ResultWidth, RowChunks, RowsPerItem;
 	long long TotalItems;
+	unsigned GroupsMagic, WidthMagic, ChunksMagic;
 };
 
 __device__ __forceinline__ float4 paddedPixel( const CPadPoolArgs& a, const float* image, int py, int px )
@@ -406,10 +407,12 @@ void padMaxPool3x3Kernel( const CPadPoolArgs a )
 	const int cg = a.Channels / 4;
 	const long long step = static_cast<long long>( gridDim.x ) * 256;
 	for( long long item = xcdSwizzle( blockIdx.x, gridDim.x ) * 256LL + threadIdx.x; item < a.TotalItems; item += step ) {
-		long long t = item;
-		const int c = static_cast<int>( t % cg ) * 4; t /= cg;
-		const int wo = static_cast<int>( t % a.ResultWidth ); t /= a.ResultWidth;
-		const int ho0 = static_cast<int>( t % a.RowChunks ) * a.RowsPerItem; t /= a.RowChunks;
+		int t = static_cast<int>( item ), c, wo, chunk; // ( the items can be counted in 31 bits )
+		fastDivMod( t, cg, a.GroupsMagic, t, c );
+		fastDivMod( t, a.ResultWidth, a.WidthMagic, t, wo );
+		fastDivMod( t, a.RowChunks, a.ChunksMagic, t, chunk );
+		c *= 4;
+		const int ho0 = chunk * a.RowsPerItem;
 		const long long n = t;
 		const int hoEnd = min( ho0 + a.RowsPerItem, a.ResultHeight );
 		const float* image = a.From + n * a.Height * a.Width * a.Channels + c;
@@ -2976,8 +2979,16 @@ bool launchPaddingWithPooling( hipStream_t stream, const CPendingPadding& p, con
 	}
 	const long long perRow = static_cast<long long>( d.batch ) * d.resultWidth * ( d.channels / 4 );
 	int rowChunks = 1, rowsPerItem = 1;
-	chooseRowChunks( perRow, d.resultHeight, 4, 8192, &rowChunks, &rowsPerItem );
+	// A row to a thread while there are few: a thread that walks down four has their loads one behind the other. us, four rows ( and divisions in
+	// 64 bits ) and one: 1 x 112 x 112 x 64 10.2 and 5.0, 9 images 13.9 and 11.4, 32 35.1 and 29.4, 9 x 56 x 56 x 64 11.0 and 6.0; 64 images, where the
+	// row that neighbours share counts, stay with four ( 2^21.6 rows: 95 ).
+	const int minRows = perRow * d.resultHeight <= ( 1 << 21 ) ? 1 : 4;
+	chooseRowChunks( perRow, d.resultHeight, minRows, 8192, &rowChunks, &rowsPerItem );
+	if( perRow * rowChunks > 0x7fffffffLL ) {
+		return false;
+	}
 	CPadPoolArgs a;
+	a.GroupsMagic = divisionMagic( d.channels / 4 ); a.WidthMagic = divisionMagic( d.resultWidth ); a.ChunksMagic = divisionMagic( rowChunks );
 	a.From = p.From; a.Padded = p.To; a.Result = result;
 	a.Height = p.Height; a.Width = p.Width; a.Channels = p.Channels; a.ToHeight = p.ToHeight; a.ToWidth = p.ToWidth;
 	a.DeltaTop = p.DeltaTop; a.DeltaLeft = p.DeltaLeft; a.DefaultValue = p.DefaultValue;
