@@ -3,6 +3,7 @@
 #pragma once
 
 #include <hip/hip_runtime.h>
+#include <float.h>
 #include <stdint.h>
 #include <stdio.h>
 #include "../../include/neoml_hip.h"
@@ -247,6 +248,25 @@ __device__ __forceinline__ float applyActivation( float v, const CFusedActivatio
 		v = v <= -3.f ? 0.f : ( v >= 3.f ? v : v * ( v + 3.f ) * ( 1.f / 6.f ) );
 	}
 	return v;
+}
+
+// exp with the reference's clamps (src/CPU/x86/CpuX86.h:55: below -87.33654474 -> 0, above 88 -> FLT_MAX)
+__device__ __forceinline__ float expClamped( float x )
+{
+	if( x < -87.33654474f ) {
+		return 0.f;
+	}
+	if( x > 88.f ) {
+		return FLT_MAX;
+	}
+	return expf( x );
+}
+
+// e / ( e + 1 ), e = clamped exp( x ) (src/CPU/x86/CpuX86MathEngineVectorMathPrivate.h:1200-1228)
+__device__ __forceinline__ float sigmoidOf( float x )
+{
+	const float e = expClamped( x );
+	return e / ( e + 1.f );
 }
 
 // The same activation with its type fixed at compile time and the upper threshold of ReLU given as a value that is

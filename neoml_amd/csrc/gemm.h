@@ -66,6 +66,9 @@ struct CMatMulArgs {
 	// AM_ConvClasses: the dense result is [images][OutH][OutW][Ldc], DenseM pixels in all
 	int OutH, OutW, OutUpH, OutUpW, DenseM;
 	CConvClass Class[MaxConvClasses];
+	// C = x * gate with gate = sigmoid( x * *GateScale ), x = A * B + bias, the gates stored too ( C's layout; null: none ): a GELU taken along
+	float* Gate;
+	const float* GateScale;
 	int SmallTile; // smallProductKernel: 0: 16 x 16, 1: 16 x 32, 2: 32 x 32
 	// epilogue of the fused blocks: C = act( A * B + bias ) + Residual; Residual has C's layout, may be C itself
 	CFusedActivation Act;

@@ -96,6 +96,7 @@ __device__ __forceinline__ void smallProductTile( const CMatMulArgs& args, float
 	// what the thread adds behind the sums, asked for in front of them: columns of its elements e = tid + i T ( see below )
 	float free[PerThread] = {};
 	const CFusedActivation act = withParam( args.Act );
+	const float gateScale = args.Gate != nullptr ? *args.GateScale : 0.f;
 	if( args.Bias != nullptr ) {
 		const __amdgpu_buffer_rsrc_t bias = __builtin_amdgcn_make_buffer_rsrc( const_cast<float*>( args.Bias ), 0, N * 4u, 0x00020000 );
 #pragma unroll
@@ -337,7 +338,11 @@ __device__ __forceinline__ void smallProductTile( const CMatMulArgs& args, float
 			if( args.Accumulate ) {
 				v += C[at];
 			}
-			if( residual != nullptr ) {
+			if( args.Gate != nullptr ) {
+				const float gate = sigmoidOf( v * gateScale );
+				args.Gate[at] = gate;
+				v *= gate;
+			} else if( residual != nullptr ) {
 				const float r = residual[at];
 				v = act.BehindResidual != 0 ? applyActivation( v + r, act ) : applyActivation( v, act ) + r;
 			} else {

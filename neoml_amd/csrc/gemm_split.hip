@@ -332,6 +332,9 @@ void splitProductKernel( const CMatMulArgs args )
 	const float actParam = withParam( args.Act ).Param; // ( the threshold may live in device memory )
 	const float reluTop = actParam > 0.f ? actParam : __builtin_inff();
 	const bool behind = args.Act.BehindResidual != 0;
+	constexpr int GateType = -1; // ( beside the activations: the gates of a GELU )
+	const float gateScale = args.Gate != nullptr ? *args.GateScale : 0.f;
+	const __amdgpu_buffer_rsrc_t bufGate = __builtin_amdgcn_make_buffer_rsrc( args.Gate != nullptr ? args.Gate : C, 0, args.CBytes, 0x00020000 );
 	const unsigned pitchBytes = static_cast<unsigned>( args.Ldc ) * 4u;
 	auto write = [&]( auto typeOf, auto extraOf, auto insideOf ) {
 		constexpr int Type = decltype( typeOf )::value;
@@ -352,7 +355,15 @@ void splitProductKernel( const CMatMulArgs args )
 					const unsigned groupOffset = laneOffset + static_cast<unsigned>( row & ~3 ) * pitchBytes;
 					const unsigned rowBytes = static_cast<unsigned>( row & 3 ) * pitchBytes;
 					float v = acc[mi][ni][r] + bias;
-					if constexpr( Extra ) {
+					if constexpr( Type == GateType ) {
+						const float gate = sigmoidOf( v * gateScale );
+						v *= gate;
+						if constexpr( Inside ) {
+							__builtin_amdgcn_raw_buffer_store_b32( __float_as_uint( gate ), bufGate, groupOffset, rowBytes, 0 );
+						} else {
+							__builtin_amdgcn_raw_buffer_store_b32( __float_as_uint( gate ), bufGate, groupOffset + rowBytes, 0, 0 );
+						}
+					} else if constexpr( Extra ) {
 						const bool ok = n < N && rowBase + row < M;
 						const long long at = static_cast<long long>( rowBase + row ) * args.Ldc + n;
 						if( args.Accumulate && ok ) {
@@ -381,7 +392,13 @@ void splitProductKernel( const CMatMulArgs args )
 			write( typeOf, std::false_type(), std::false_type() );
 		}
 	};
-	if( args.Act.Type == NH_ACT_RELU ) {
+	if( args.Gate != nullptr ) {
+		if( m0 + BM <= M ) {
+			write( std::integral_constant<int, GateType>(), std::false_type(), std::true_type() );
+		} else {
+			write( std::integral_constant<int, GateType>(), std::false_type(), std::false_type() );
+		}
+	} else if( args.Act.Type == NH_ACT_RELU ) {
 		writeAs( std::integral_constant<int, NH_ACT_RELU>() );
 	} else if( args.Act.Type == NH_ACT_HSWISH ) {
 		writeAs( std::integral_constant<int, NH_ACT_HSWISH>() );

@@ -165,18 +165,6 @@ static int launchEltwisePlain( hipStream_t stream, const TIn* a, const TIn* b, c
 	return NH_OK;
 }
 
-// exp with the reference's clamps (src/CPU/x86/CpuX86.h:55: below -87.33654474 -> 0, above 88 -> FLT_MAX)
-__device__ __forceinline__ float expClamped( float x )
-{
-	if( x < -87.33654474f ) {
-		return 0.f;
-	}
-	if( x > 88.f ) {
-		return FLT_MAX;
-	}
-	return expf( x );
-}
-
 // ---- functors: operator()( a, b, c ) with unused operands ignored ---------------------------------------
 
 struct CNoScalar { __device__ void prepare() {} };
@@ -341,11 +329,9 @@ struct CMinMaxOp {
 	}
 };
 struct CSigmoidOp : CNoScalar {
-	// e / ( e + 1 ), e = clamped exp( x ) (src/CPU/x86/CpuX86MathEngineVectorMathPrivate.h:1200-1228)
 	__device__ float operator()( float a, float, float ) const
 	{
-		const float e = expClamped( a );
-		return e / ( e + 1.f );
+		return sigmoidOf( a );
 	}
 };
 struct CTanhOp : CNoScalar {
@@ -794,6 +780,8 @@ struct CPendingProduct {
 	const float* B = nullptr;
 	float* C = nullptr;
 	int Lda = 0, Ldb = 0, Ldc = 0, M = 0, N = 0, K = 0;
+	// the free term, once it has been asked for: the product waits on, it may be the one in front of a GELU
+	const float* Bias = nullptr;
 };
 
 // A convolution ( plain or channelwise ) that waits for the call behind it in the same way: CConvLayer / CChannelwiseConvLayer
@@ -872,6 +860,8 @@ struct CTinyQueue {
 	void ( *FirstAlone )( hipStream_t, const CTinyOp& ) = nullptr;
 	CSpreadAlone FirstSpreadAlone = nullptr; // ( the same for a call with a spread operand: its own kernel lives with its entry point )
 	CPendingProduct Product;
+	// the product waits behind the calls that the chain holds by then: a GELU over its result, see launchGatedProduct
+	bool ProductParked = false;
 	CPendingConvolution Convolution;
 	// A second convolution with a result of the same size, behind the first: a block's last convolution may be followed by that of
 	// its shortcut, and only then by the sum of the two over the first one's result. The sum launches the second one and waits on
@@ -886,7 +876,7 @@ struct CTinyQueue {
 
 	bool LaunchWaits() const
 	{
-		return Product.Pending || Convolution.Pending || Sum.Pending || Batched.Pending || Padding.Pending || ColumnSum.Pending;
+		return ( Product.Pending && !ProductParked ) || Convolution.Pending || Sum.Pending || Batched.Pending || Padding.Pending || ColumnSum.Pending;
 	}
 };
 
@@ -901,6 +891,10 @@ int matMulNT( hipStream_t stream, const float* a, int lda, const float* b, int l
 int matMulNN( hipStream_t stream, const float* a, int lda, const float* b, int ldb, float* c, int ldc,
 	int M, int N, int K, int batch, long long strideA, long long strideB, long long strideC, bool accumulate,
 	const float* scale, bool* scaled );
+
+// the product of matMulNT with a GELU over its result in place: gate = sigmoid( c * scale ), c *= gate. false: no kernel takes it, nothing done
+bool matMulNTGated( hipStream_t stream, const float* a, int lda, const float* b, int ldb, float* c, int ldc, int M, int N, int K, const float* bias,
+	float* gate, const float* gateScale, int* rc );
 
 static int launchPendingConvolution( hipStream_t stream, const CPendingConvolution& c, const CFusedActivation& act )
 {
@@ -1164,6 +1158,18 @@ static bool launchKnownChain( hipStream_t stream, const CTinyChain& chain )
 
 static void launchColumnSum( hipStream_t stream, const CPendingColumnSum& sum, const CTinyChain& tail );
 
+static bool launchPendingProduct( hipStream_t stream, CTinyQueue& queue )
+{
+	const CPendingProduct p = queue.Product;
+	queue.Product.Pending = false;
+	queue.ProductParked = false;
+	__atomic_fetch_sub( &tinyChainsPending, 1, __ATOMIC_RELAXED );
+	// ( a launch that fails leaves its message with nhGetLastError and its HIP error to the next launch check )
+	( void )matMulNT( stream, p.A, p.Lda, p.B, p.Ldb, p.C, p.Ldc, p.M, p.N, p.K, 1, 0, 0, 0, p.Bias, false );
+	return true;
+}
+
+// ( a product or sums of rows that wait in front of whatever else the queue holds )
 static bool launchParked( hipStream_t stream, CTinyQueue& queue )
 {
 	const int count = queue.ParkedCount;
@@ -1172,7 +1178,7 @@ static bool launchParked( hipStream_t stream, CTinyQueue& queue )
 		launchColumnSum( stream, queue.Parked[i].Sum, queue.Parked[i].Tail );
 		__atomic_fetch_sub( &tinyChainsPending, 1, __ATOMIC_RELAXED );
 	}
-	return count > 0;
+	return ( queue.Product.Pending && launchPendingProduct( stream, queue ) ) || count > 0;
 }
 
 static bool launchTinyChain( hipStream_t stream, CTinyQueue& queue )
@@ -1624,7 +1630,7 @@ static void launchColumnSum( hipStream_t stream, const CPendingColumnSum& sum, c
 // what the queue holds: the product that waits for its successor ( then nothing else is queued ), or a chain
 static bool launchPending( hipStream_t stream, CTinyQueue& queue )
 {
-	( void )launchParked( stream, queue ); // ( something else waits behind it )
+	const bool parked = launchParked( stream, queue );
 	if( queue.ColumnSum.Pending ) {
 		const CPendingColumnSum sum = queue.ColumnSum;
 		queue.ColumnSum.Pending = false;
@@ -1635,14 +1641,6 @@ static bool launchPending( hipStream_t stream, CTinyQueue& queue )
 			tail.Length = 0;
 			__atomic_fetch_sub( &tinyChainsPending, 1, __ATOMIC_RELAXED );
 		}
-		return true;
-	}
-	if( queue.Product.Pending ) {
-		const CPendingProduct p = queue.Product;
-		queue.Product.Pending = false;
-		__atomic_fetch_sub( &tinyChainsPending, 1, __ATOMIC_RELAXED );
-		// ( a launch that fails leaves its message with nhGetLastError and its HIP error to the next launch check )
-		( void )matMulNT( stream, p.A, p.Lda, p.B, p.Ldb, p.C, p.Ldc, p.M, p.N, p.K, 1, 0, 0, 0, nullptr, false );
 		return true;
 	}
 	if( queue.Convolution.Pending ) {
@@ -1678,7 +1676,7 @@ static bool launchPending( hipStream_t stream, CTinyQueue& queue )
 		( void )launchPlainSum( stream, sum );
 		return true;
 	}
-	return launchTinyChain( stream, queue );
+	return launchTinyChain( stream, queue ) || parked;
 }
 
 bool flushTinyOps( hipStream_t stream )
@@ -1709,7 +1707,7 @@ void flushAllTinyOps()
 	{
 		std::lock_guard<std::recursive_mutex> guard( tinyLock );
 		for( auto& entry : tinyQueues() ) {
-			if( entry.second.Chain.Length == 0 && entry.second.ParkedCount == 0 && !entry.second.LaunchWaits() ) {
+			if( entry.second.Chain.Length == 0 && entry.second.ParkedCount == 0 && !entry.second.Product.Pending && !entry.second.LaunchWaits() ) {
 				continue;
 			}
 			if( entry.first.first != active ) {
@@ -1782,39 +1780,87 @@ bool deferProduct( nhStream s, const float* a, int lda, const float* b, int ldb,
 		return false;
 	}
 	CPendingProduct& p = found->second.Product;
+	p = CPendingProduct();
 	p.Pending = true;
 	p.A = a; p.Lda = lda; p.B = b; p.Ldb = ldb; p.C = c; p.Ldc = ldc; p.M = M; p.N = N; p.K = K;
 	__atomic_fetch_add( &tinyChainsPending, 1, __ATOMIC_RELAXED );
 	return true;
 }
 
-bool fusePendingProduct( nhStream s, const float* matrix, float* result, int height, int width, const float* vector, int* rc )
+// the queue of a stream of the current device that puts calls aside ( with tinyLock held )
+static CTinyQueue* deferringQueue( hipStream_t stream )
 {
-	const hipStream_t stream = reinterpret_cast<hipStream_t>( s );
 	int device = 0;
 	if( hipGetDevice( &device ) != hipSuccess ) {
 		( void )hipGetLastError();
+		return nullptr;
+	}
+	auto found = tinyQueues().find( std::make_pair( device, stream ) );
+	return found != tinyQueues().end() && found->second.Enabled ? &found->second : nullptr;
+}
+
+// AddVectorToMatrixRows asks whether it is the free term of a product that waits: true, the product waits on with it
+bool fusePendingProduct( nhStream s, const float* matrix, float* result, int height, int width, const float* vector, int* rc )
+{
+	std::lock_guard<std::recursive_mutex> guard( tinyLock );
+	CTinyQueue* queue = deferringQueue( reinterpret_cast<hipStream_t>( s ) );
+	if( queue == nullptr || !queue->Product.Pending || queue->ProductParked || queue->Product.Bias != nullptr ) {
 		return false;
 	}
-	CPendingProduct p;
-	{
-		std::lock_guard<std::recursive_mutex> guard( tinyLock );
-		auto found = tinyQueues().find( std::make_pair( device, stream ) );
-		if( found == tinyQueues().end() || !found->second.Product.Pending ) {
-			return false;
-		}
-		p = found->second.Product;
-		if( matrix != p.C || result != p.C || height != p.M || width != p.N || vector == nullptr ) {
-			return false; // ( the caller's own launch sends the product out first, as it was asked for )
-		}
-		found->second.Product.Pending = false;
-		__atomic_fetch_sub( &tinyChainsPending, 1, __ATOMIC_RELAXED );
+	CPendingProduct& p = queue->Product;
+	if( matrix != p.C || result != p.C || height != p.M || width != p.N || vector == nullptr
+		|| rangesMeet( vector, width, p.C, static_cast<long long>( height ) * width ) ) {
+		return false; // ( the caller's own launch sends the product out first, as it was asked for )
 	}
-	*rc = matMulNT( stream, p.A, p.Lda, p.B, p.Ldb, p.C, p.Ldc, p.M, p.N, p.K, 1, 0, 0, 0, vector, false );
-	if( __atomic_load_n( &lstmPartnersAwaited, __ATOMIC_RELAXED ) != 0 ) {
-		noteStreamUse( stream );
-	}
+	p.Bias = vector;
+	*rc = NH_OK;
 	return true;
+}
+
+// A product with its free term that waits may wait on while this call ( its result times a device scalar into another matrix ) is queued:
+// the first of the three that CGELULayer::runFastApproximate asks for
+static bool parkProduct( CTinyQueue& queue, const float* x, const float* t, int count, const float* scale )
+{
+	const CPendingProduct& p = queue.Product;
+	const long long size = static_cast<long long>( p.M ) * p.N;
+	if( !p.Pending || p.Bias == nullptr || queue.ProductParked || x != p.C || count != size || rangesMeet( t, count, p.C, size )
+		|| rangesMeet( t, count, p.A, static_cast<long long>( p.M - 1 ) * p.Lda + p.K ) || rangesMeet( t, count, p.B, static_cast<long long>( p.N - 1 ) * p.Ldb + p.K )
+		|| rangesMeet( t, count, p.Bias, p.N ) || rangesMeet( scale, 1, p.C, size ) || rangesMeet( scale, 1, t, count ) ) {
+		return false;
+	}
+	queue.ProductParked = true;
+	return true;
+}
+
+// true ( launched, the queue empty ) if the chain behind a parked product is t = x * scale; t = sigmoid( t ); x = x * t and a kernel takes
+// them along
+static bool launchGatedProduct( hipStream_t stream, CTinyQueue& queue )
+{
+	CTinyChain& chain = queue.Chain;
+	const CTinyOp* op = chain.Ops;
+	const CPendingProduct p = queue.Product;
+	if( !queue.ProductParked || queue.ParkedCount > 0 || chain.Length != 3 || !isKind<CMulValueOp<float>>( op[0] ) || !isKind<CSigmoidOp>( op[1] )
+		|| !isKind<CMulOp<float>>( op[2] ) || op[2].Spread != TS_None || op[0].Barrier != 0 || op[1].Barrier != 0 || op[2].Barrier != 0 ) {
+		return false;
+	}
+	float* t = op[0].Out;
+	const bool product = ( op[2].In[0] == p.C && op[2].In[1] == t ) || ( op[2].In[0] == t && op[2].In[1] == p.C );
+	if( op[1].In[0] != t || op[1].Out != t || op[1].Count != op[0].Count || !product || op[2].Out != p.C || op[2].Count != op[0].Count ) {
+		return false;
+	}
+	const float* scale = op[0].Scalar;
+	queue.Product.Pending = false; // ( as elsewhere: a launch may ask a pool for memory, which sends out what the queues hold )
+	const CTinyChain held = chain;
+	chain.Length = 0;
+	int rc = NH_OK;
+	if( matMulNTGated( stream, p.A, p.Lda, p.B, p.Ldb, p.C, p.Ldc, p.M, p.N, p.K, p.Bias, t, scale, &rc ) ) {
+		queue.ProductParked = false;
+		__atomic_fetch_sub( &tinyChainsPending, 2, __ATOMIC_RELAXED );
+		return true;
+	}
+	chain = held;
+	queue.Product.Pending = true;
+	return false;
 }
 
 bool deferColumnSum( nhStream s, float* result, const float* matrix, int height, int width )
@@ -1992,18 +2038,6 @@ bool fusePendingPadding( nhStream s, const nhPoolingDesc& d, const float* source
 	}
 	( void )launchPadding( stream, p ); // ( not a pair for one launch: the padding as it was asked for, the pooling is the caller's )
 	return false;
-}
-
-// the queue of a stream of the current device that puts calls aside ( with tinyLock held )
-static CTinyQueue* deferringQueue( hipStream_t stream )
-{
-	int device = 0;
-	if( hipGetDevice( &device ) != hipSuccess ) {
-		( void )hipGetLastError();
-		return nullptr;
-	}
-	auto found = tinyQueues().find( std::make_pair( device, stream ) );
-	return found != tinyQueues().end() && found->second.Enabled ? &found->second : nullptr;
 }
 
 // whether a blob that a waiting attention core is to write, or a scalar that it is to read, lies apart from what it has been handed so far
@@ -2430,7 +2464,8 @@ static bool deferEltwise( nhStream s, const TIn* a, const TIn* b, const TIn* c, 
 			if( !tail && !( Sum && spread == TS_PerRow && parkColumnSum( found->second, a, b, out, n, width ) ) ) {
 				launchPending( stream, found->second );
 			}
-		} else if( found->second.LaunchWaits() ) {
+		} else if( found->second.LaunchWaits() && !( std::is_same<F, CMulValueOp<float>>::value && spread == TS_None
+			&& parkProduct( found->second, a, out, n, scalarOf( f, 0 ) ) ) ) {
 			launchPending( stream, found->second ); // ( a launch that waited for its successor: this call is not the one )
 		}
 		CTinyQueue& queue = found->second;
@@ -2530,7 +2565,9 @@ static bool deferEltwise( nhStream s, const TIn* a, const TIn* b, const TIn* c, 
 		}
 		chain.Ops[chain.Length] = op;
 		++chain.Length;
-		( void )launchNormalization( stream, queue );
+		if( !launchNormalization( stream, queue ) ) {
+			( void )launchGatedProduct( stream, queue );
+		}
 		return true;
 	} else {
 		( void )s; ( void )a; ( void )b; ( void )c; ( void )out; ( void )n; ( void )f; ( void )spread; ( void )width; ( void )spreadAlone;
