@@ -33,6 +33,7 @@ struct CConvClass {
 };
 
 constexpr int MaxConvClasses = 4;
+constexpr int MaxProductGroup = 3;
 
 struct CMatMulArgs {
 	const float* A;
@@ -66,6 +67,11 @@ struct CMatMulArgs {
 	// AM_ConvClasses: the dense result is [images][OutH][OutW][Ldc], DenseM pixels in all
 	int OutH, OutW, OutUpH, OutUpW, DenseM;
 	CConvClass Class[MaxConvClasses];
+	// products of one A ( grid y ): each with its own B, free term and result
+	int Group;
+	const float* GroupB[MaxProductGroup];
+	const float* GroupBias[MaxProductGroup];
+	float* GroupC[MaxProductGroup];
 	// C = x * gate with gate = sigmoid( x * *GateScale ), x = A * B + bias, the gates stored too ( C's layout; null: none ): a GELU taken along
 	float* Gate;
 	const float* GateScale;

@@ -2436,6 +2436,26 @@ static int matMulNTMeeting( hipStream_t stream, const float* a, int lda, const f
 	return launchMatMul<AM_RowsK, BM_RowsK>( stream, args, batch, vec, fixedMeeting );
 }
 
+// Two or three products of one A as one launch, if the kernel for few tiles takes them ( the queries, keys and values of a short sequence:
+// three of 37 x 512 x 512 13.5 us and 6.2, and two launches less for the host )
+bool matMulNTGroup( hipStream_t stream, const float* a, int lda, int ldb, int M, int N, int K, int count, const float* const* b,
+	const float* const* bias, float* const* c, int* rc )
+{
+	CMatMulArgs args = {};
+	args.A = a; args.B = b[0]; args.C = c[0]; args.Bias = bias[0];
+	args.M = M; args.N = N; args.K = K;
+	args.Lda = lda; args.Ldb = ldb; args.Ldc = N;
+	args.Group = 1;
+	bool vec = isAligned16( a ) && K % 4 == 0 && lda % 4 == 0 && ldb % 4 == 0 && fitsBuffer( M, lda, K ) && fitsBuffer( N, ldb, K );
+	for( int i = 0; i < count; ++i ) {
+		args.GroupB[i] = b[i];
+		args.GroupBias[i] = bias[i];
+		args.GroupC[i] = c[i];
+		vec = vec && isAligned16( b[i] );
+	}
+	return trySmallProduct( stream, args, false, count, vec, rc, nullptr );
+}
+
 // The product with the GELU over its result, where the kernel that takes the product does that on the way out: for few tiles it saves a
 // launch, for many the pass over the result: 8192 x 2048 x 512 90 us and 31 for the pass, 107 together.
 bool matMulNTGated( hipStream_t stream, const float* a, int lda, const float* b, int ldb, float* c, int ldc, int M, int N, int K, const float* bias,

@@ -42,7 +42,9 @@ __device__ __forceinline__ void smallProductTile( const CMatMulArgs& args, float
 	const int batch = blockIdx.y, slice = blockIdx.z;
 	const int M = args.M, N = args.N, K = args.K;
 	const float* baseA = args.A + batch * args.BatchStrideA;
-	const float* baseB = args.B + batch * args.BatchStrideB;
+	const bool group = !IsTaps && args.Group != 0;
+	const float* baseB = group ? args.GroupB[batch] : args.B + batch * args.BatchStrideB;
+	const float* freeTerm = group ? args.GroupBias[batch] : args.Bias;
 
 	// this wavefront's groups
 	const int groups = ( K + 15 ) / 16;
@@ -97,8 +99,8 @@ __device__ __forceinline__ void smallProductTile( const CMatMulArgs& args, float
 	float free[PerThread] = {};
 	const CFusedActivation act = withParam( args.Act );
 	const float gateScale = args.Gate != nullptr ? *args.GateScale : 0.f;
-	if( args.Bias != nullptr ) {
-		const __amdgpu_buffer_rsrc_t bias = __builtin_amdgcn_make_buffer_rsrc( const_cast<float*>( args.Bias ), 0, N * 4u, 0x00020000 );
+	if( freeTerm != nullptr ) {
+		const __amdgpu_buffer_rsrc_t bias = __builtin_amdgcn_make_buffer_rsrc( const_cast<float*>( freeTerm ), 0, N * 4u, 0x00020000 );
 #pragma unroll
 		for( int i = 0; i < PerThread; ++i ) {
 			free[i] = bufferLoad1( bias, ( n0 + ( ( wave + i * WAVES ) / 4 % NB ) * 16 + l16 ) * 4u );
@@ -326,7 +328,7 @@ __device__ __forceinline__ void smallProductTile( const CMatMulArgs& args, float
 		return;
 	}
 	// element ( r, lane ): block ( r / ( 4 NB ), r / 4 % NB ), of it column lane % 16 of row 4 ( lane / 16 ) + r % 4
-	float* C = args.C + batch * args.BatchStrideC;
+	float* C = group ? args.GroupC[batch] : args.C + batch * args.BatchStrideC;
 	const float* residual = args.Residual != nullptr ? args.Residual + batch * args.BatchStrideC : nullptr;
 #pragma unroll
 	for( int i = 0; i < PerThread; ++i ) {

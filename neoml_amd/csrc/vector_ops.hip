@@ -860,6 +860,10 @@ struct CTinyQueue {
 	void ( *FirstAlone )( hipStream_t, const CTinyOp& ) = nullptr;
 	CSpreadAlone FirstSpreadAlone = nullptr; // ( the same for a call with a spread operand: its own kernel lives with its entry point )
 	CPendingProduct Product;
+	// Products of the same A, with their free terms, that were asked for in front of it: the queries and keys of an attention layer in front
+	// of its values
+	CPendingProduct Siblings[2] = {};
+	int SiblingCount = 0;
 	// the product waits behind the calls that the chain holds by then: a GELU over its result, see launchGatedProduct
 	bool ProductParked = false;
 	CPendingConvolution Convolution;
@@ -1158,14 +1162,41 @@ static bool launchKnownChain( hipStream_t stream, const CTinyChain& chain )
 
 static void launchColumnSum( hipStream_t stream, const CPendingColumnSum& sum, const CTinyChain& tail );
 
+bool matMulNTGroup( hipStream_t stream, const float* a, int lda, int ldb, int M, int N, int K, int count, const float* const* b,
+	const float* const* bias, float* const* c, int* rc );
+
 static bool launchPendingProduct( hipStream_t stream, CTinyQueue& queue )
 {
-	const CPendingProduct p = queue.Product;
+	CPendingProduct products[3];
+	int count = 0;
+	for( ; count < queue.SiblingCount; ++count ) {
+		products[count] = queue.Siblings[count];
+	}
+	products[count++] = queue.Product;
 	queue.Product.Pending = false;
 	queue.ProductParked = false;
+	queue.SiblingCount = 0;
 	__atomic_fetch_sub( &tinyChainsPending, 1, __ATOMIC_RELAXED );
+	if( count > 1 ) {
+		const float* b[3];
+		const float* bias[3];
+		float* c[3];
+		for( int i = 0; i < count; ++i ) {
+			b[i] = products[i].B;
+			bias[i] = products[i].Bias;
+			c[i] = products[i].C;
+		}
+		const CPendingProduct& p = products[0];
+		int rc = NH_OK;
+		if( matMulNTGroup( stream, p.A, p.Lda, p.Ldb, p.M, p.N, p.K, count, b, bias, c, &rc ) ) {
+			return true;
+		}
+	}
 	// ( a launch that fails leaves its message with nhGetLastError and its HIP error to the next launch check )
-	( void )matMulNT( stream, p.A, p.Lda, p.B, p.Ldb, p.C, p.Ldc, p.M, p.N, p.K, 1, 0, 0, 0, p.Bias, false );
+	for( int i = 0; i < count; ++i ) {
+		const CPendingProduct& p = products[i];
+		( void )matMulNT( stream, p.A, p.Lda, p.B, p.Ldb, p.C, p.Ldc, p.M, p.N, p.K, 1, 0, 0, 0, p.Bias, false );
+	}
 	return true;
 }
 
@@ -1758,10 +1789,47 @@ void releaseTinyQueue( hipStream_t stream )
 	}
 }
 
+// the queue of a stream of the current device that puts calls aside ( with tinyLock held )
+static CTinyQueue* deferringQueue( hipStream_t stream )
+{
+	int device = 0;
+	if( hipGetDevice( &device ) != hipSuccess ) {
+		( void )hipGetLastError();
+		return nullptr;
+	}
+	auto found = tinyQueues().find( std::make_pair( device, stream ) );
+	return found != tinyQueues().end() && found->second.Enabled ? &found->second : nullptr;
+}
+
+constexpr long long MaxGroupedProduct = 1 << 18; // ( values of a result: what the kernel for few tiles may take three of )
+
 bool deferProduct( nhStream s, const float* a, int lda, const float* b, int ldb, float* c, int ldc, int M, int N, int K )
 {
 	if( __atomic_load_n( &tinyDeferringStreams, __ATOMIC_RELAXED ) == 0 || M <= 0 || N <= 0 || K <= 0 || ldc != N ) {
 		return false;
+	}
+	if( static_cast<long long>( M ) * N <= MaxGroupedProduct && __atomic_load_n( &tinyChainsPending, __ATOMIC_RELAXED ) != 0 ) {
+		// a product of the same A that waits with its free term: the two wait on, apart from each other as they must be
+		std::lock_guard<std::recursive_mutex> guard( tinyLock );
+		CTinyQueue* queue = deferringQueue( reinterpret_cast<hipStream_t>( s ) );
+		if( queue != nullptr && queue->Product.Pending && !queue->ProductParked && queue->Product.Bias != nullptr && queue->SiblingCount < 2
+			&& queue->Chain.Length == 0 && queue->ParkedCount == 0 ) {
+			const CPendingProduct& last = queue->Product;
+			const long long sizeA = static_cast<long long>( M - 1 ) * lda + K, sizeB = static_cast<long long>( N - 1 ) * ldb + K, sizeC = static_cast<long long>( M ) * N;
+			bool joins = last.A == a && last.Lda == lda && last.Ldb == ldb && last.M == M && last.N == N && last.K == K && !rangesMeet( c, sizeC, a, sizeA )
+				&& !rangesMeet( c, sizeC, b, sizeB );
+			for( int i = 0; joins && i <= queue->SiblingCount; ++i ) {
+				const CPendingProduct& other = i < queue->SiblingCount ? queue->Siblings[i] : last;
+				joins = !rangesMeet( c, sizeC, other.C, sizeC ) && !rangesMeet( c, sizeC, other.B, sizeB ) && !rangesMeet( c, sizeC, other.Bias, N )
+					&& !rangesMeet( b, sizeB, other.C, sizeC ) && !rangesMeet( a, sizeA, other.C, sizeC );
+			}
+			if( joins ) {
+				queue->Siblings[queue->SiblingCount++] = last;
+				CPendingProduct& p = queue->Product;
+				p.B = b; p.C = c; p.Bias = nullptr; // ( one thing waits where one waited )
+				return true;
+			}
+		}
 	}
 	const hipStream_t stream = toStream( s ); // ( what the stream holds goes out first )
 	int device = 0;
@@ -1781,22 +1849,11 @@ bool deferProduct( nhStream s, const float* a, int lda, const float* b, int ldb,
 	}
 	CPendingProduct& p = found->second.Product;
 	p = CPendingProduct();
+	found->second.SiblingCount = 0;
 	p.Pending = true;
 	p.A = a; p.Lda = lda; p.B = b; p.Ldb = ldb; p.C = c; p.Ldc = ldc; p.M = M; p.N = N; p.K = K;
 	__atomic_fetch_add( &tinyChainsPending, 1, __ATOMIC_RELAXED );
 	return true;
-}
-
-// the queue of a stream of the current device that puts calls aside ( with tinyLock held )
-static CTinyQueue* deferringQueue( hipStream_t stream )
-{
-	int device = 0;
-	if( hipGetDevice( &device ) != hipSuccess ) {
-		( void )hipGetLastError();
-		return nullptr;
-	}
-	auto found = tinyQueues().find( std::make_pair( device, stream ) );
-	return found != tinyQueues().end() && found->second.Enabled ? &found->second : nullptr;
 }
 
 // AddVectorToMatrixRows asks whether it is the free term of a product that waits: true, the product waits on with it
@@ -1812,6 +1869,11 @@ bool fusePendingProduct( nhStream s, const float* matrix, float* result, int hei
 		|| rangesMeet( vector, width, p.C, static_cast<long long>( height ) * width ) ) {
 		return false; // ( the caller's own launch sends the product out first, as it was asked for )
 	}
+	for( int i = 0; i < queue->SiblingCount; ++i ) {
+		if( rangesMeet( vector, width, queue->Siblings[i].C, static_cast<long long>( height ) * width ) ) {
+			return false;
+		}
+	}
 	p.Bias = vector;
 	*rc = NH_OK;
 	return true;
@@ -1823,7 +1885,7 @@ static bool parkProduct( CTinyQueue& queue, const float* x, const float* t, int 
 {
 	const CPendingProduct& p = queue.Product;
 	const long long size = static_cast<long long>( p.M ) * p.N;
-	if( !p.Pending || p.Bias == nullptr || queue.ProductParked || x != p.C || count != size || rangesMeet( t, count, p.C, size )
+	if( !p.Pending || p.Bias == nullptr || queue.ProductParked || queue.SiblingCount > 0 || x != p.C || count != size || rangesMeet( t, count, p.C, size )
 		|| rangesMeet( t, count, p.A, static_cast<long long>( p.M - 1 ) * p.Lda + p.K ) || rangesMeet( t, count, p.B, static_cast<long long>( p.N - 1 ) * p.Ldb + p.K )
 		|| rangesMeet( t, count, p.Bias, p.N ) || rangesMeet( scale, 1, p.C, size ) || rangesMeet( scale, 1, t, count ) ) {
 		return false;
