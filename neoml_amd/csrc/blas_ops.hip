@@ -1,7 +1,7 @@
 // Bandwidth-bound matrix helpers of IBlasEngine: row/column broadcasts, row/column sums, softmax, arg-max,
 // diagonal products and the blob transpose. Row reductions give one 64-lane wavefront to each row and reduce
 // with cross-lane shuffles; element-wise broadcasts use 128-bit accesses when shapes and pointers allow it.
-#include "common.h"
+#include "gemm.h"
 #include <float.h>
 
 namespace nh {
@@ -527,6 +527,67 @@ void transposePlainQuadKernel( const T* in, T* out, int height, int width )
 	}
 }
 
+// Up to four transpositions of a few thousand values each that do not depend on one another ( the queries, keys and values of a short
+// sequence ), by one launch: a thread owns four channels or, where there are no four, one value of the result. What bounds it is the launch, so
+// that the reads of a plain transposition, a row apart from each other, do not count: 37 x 512 4.7 us by tiles through LDS ( one value
+// to a thread and pass ), 1.9 here; 37 x 8 x 64, 37 x 512 and 37 x 8 x 64 one by one 12.2 us, as one launch 2.6. Up to 65536 values ( 256 x 256 2.04 us
+// by the tiles that read four values, 2.09 here; 256 x 512 2.07 and 2.71 ).
+__global__ __launch_bounds__( 256 )
+void transposeSmallKernel( const CTranspositions args )
+{
+	const CTransposition& t = args.Items[blockIdx.y];
+	const int g = blockIdx.x * 256 + threadIdx.x;
+	if( g >= t.Threads ) {
+		return;
+	}
+	int rest, channel, row, middle, column, image;
+	fastDivMod( g, t.ChannelGroups, t.ChannelsMagic, rest, channel );
+	fastDivMod( rest, t.Height, t.HeightMagic, rest, row );
+	fastDivMod( rest, t.Medium, t.MediumMagic, rest, middle );
+	fastDivMod( rest, t.Width, t.WidthMagic, image, column );
+	const int from = ( ( ( image * t.Height + row ) * t.Medium + middle ) * t.Width + column ) * t.ChannelGroups + channel;
+	if( t.Quads != 0 ) {
+		reinterpret_cast<float4*>( t.To )[g] = reinterpret_cast<const float4*>( t.From )[from];
+	} else {
+		t.To[g] = t.From[from];
+	}
+}
+
+// true: t describes a transposition that transposeSmallKernel is for
+static bool smallTransposition( int batch, const float* first, int height, int medium, int width, int channels, float* result, CTransposition& t )
+{
+	if( batch <= 0 || height <= 0 || medium <= 0 || width <= 0 || channels <= 0 || first == nullptr || result == nullptr || first == result
+		|| ( medium == 1 && ( height == 1 || width == 1 ) ) ) {
+		return false;
+	}
+	long long total = batch;
+	for( int dim : { height, medium, width, channels } ) {
+		total *= dim;
+		if( total > MaxSmallTransposition ) {
+			return false;
+		}
+	}
+	t.From = first; t.To = result;
+	t.Quads = channels % 4 == 0 && isAligned16( first ) && isAligned16( result ) ? 1 : 0;
+	t.Count = static_cast<int>( total );
+	t.Threads = t.Quads != 0 ? t.Count / 4 : t.Count;
+	t.Height = height; t.Medium = medium; t.Width = width; t.ChannelGroups = t.Quads != 0 ? channels / 4 : channels;
+	t.HeightMagic = divisionMagic( height ); t.MediumMagic = divisionMagic( medium ); t.WidthMagic = divisionMagic( width );
+	t.ChannelsMagic = divisionMagic( t.ChannelGroups );
+	return true;
+}
+
+int launchTranspositions( hipStream_t stream, const CTranspositions& t )
+{
+	int threads = 0;
+	for( int i = 0; i < t.Length; ++i ) {
+		threads = t.Items[i].Threads > threads ? t.Items[i].Threads : threads;
+	}
+	hipLaunchKernelGGL( transposeSmallKernel, dim3( ceilDiv( threads, 256 ), t.Length ), dim3( 256 ), 0, stream, t );
+	NH_LAUNCH_CHECK();
+	return NH_OK;
+}
+
 template<typename T>
 static int transposeImpl( nhStream s, int batchSize, const T* first, int height, int medium, int width, int channels,
 	T* result, int resultBufferSize )
@@ -876,6 +937,14 @@ int nhTransposeMatrix( nhStream s, int batchSize, const float* first, int height
 	if( __atomic_load_n( &tinyChainsPending, __ATOMIC_RELAXED ) != 0
 		&& fusePendingTransposition( s, batchSize, first, height, medium, width, channels, result, &rc ) ) {
 		return rc; // ( the result of an attention layer's core was waiting for this call )
+	}
+	CTranspositions one = {};
+	if( smallTransposition( batchSize, first, height, medium, width, channels, result, one.Items[0] ) ) {
+		if( deferTransposition( s, one.Items[0] ) ) {
+			return NH_OK;
+		}
+		one.Length = 1;
+		return launchTranspositions( toStream( s ), one );
 	}
 	return transposeImpl<float>( s, batchSize, first, height, medium, width, channels, result, resultBufferSize );
 }

@@ -64,6 +64,21 @@ bool fusePendingPadding( nhStream s, const nhPoolingDesc& d, const float* source
 // ( dnn_ops.hip ) the padding by itself; the padding with the pooling over it, false if the pair is not one it takes
 int launchPadding( hipStream_t stream, const CPendingPadding& padding );
 bool launchPaddingWithPooling( hipStream_t stream, const CPendingPadding& padding, const nhPoolingDesc& d, float* result, int* rc );
+// Small transpositions ( nhTransposeMatrix ) that do not depend on one another wait for one another: one launch ( launchTranspositions, blas_ops.hip )
+constexpr int MaxTranspositions = 4;
+constexpr long long MaxSmallTransposition = 1 << 16; // values: a thread to each, and they come from the caches
+struct CTransposition {
+	const float* From;
+	float* To;
+	int Count, Threads, Quads, Height, Medium, Width, ChannelGroups; // Quads: four channels to a thread
+	unsigned HeightMagic, MediumMagic, WidthMagic, ChannelsMagic;
+};
+struct CTranspositions {
+	int Length;
+	CTransposition Items[MaxTranspositions];
+};
+bool deferTransposition( nhStream s, const CTransposition& t );
+int launchTranspositions( hipStream_t stream, const CTranspositions& t );
 // A batch of small dense row-major products, Scores[b] = Q[b] * KT[b], that waits for the call behind it ( nhBatchMultiplyMatrixByMatrix ): the
 // factor over the whole result in place ( nhVectorMultiply ), and, where the attention kernel takes them, softmax over its rows
 // ( nhMatrixSoftmaxByRows ), the product of the weights and the values, and the exchange of heads and rows ( nhTransposeMatrix ): one launch.

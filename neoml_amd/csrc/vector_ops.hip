@@ -877,10 +877,12 @@ struct CTinyQueue {
 	CPendingAttention Batched;
 	CPendingPadding Padding;
 	CPendingColumnSum ColumnSum;
+	CTranspositions Transpositions = {};
 
 	bool LaunchWaits() const
 	{
-		return ( Product.Pending && !ProductParked ) || Convolution.Pending || Sum.Pending || Batched.Pending || Padding.Pending || ColumnSum.Pending;
+		return ( Product.Pending && !ProductParked ) || Convolution.Pending || Sum.Pending || Batched.Pending || Padding.Pending || ColumnSum.Pending
+			|| Transpositions.Length > 0;
 	}
 };
 
@@ -1693,6 +1695,13 @@ static bool launchPending( hipStream_t stream, CTinyQueue& queue )
 		( void )launchPendingAttention( stream, p );
 		return true;
 	}
+	if( queue.Transpositions.Length > 0 ) {
+		const CTranspositions t = queue.Transpositions;
+		queue.Transpositions.Length = 0;
+		__atomic_fetch_sub( &tinyChainsPending, 1, __ATOMIC_RELAXED );
+		( void )launchTranspositions( stream, t );
+		return true;
+	}
 	if( queue.Padding.Pending ) {
 		const CPendingPadding p = queue.Padding;
 		queue.Padding.Pending = false;
@@ -2238,6 +2247,48 @@ bool fusePendingTransposition( nhStream s, int batch, const float* first, int he
 	if( __atomic_load_n( &lstmPartnersAwaited, __ATOMIC_RELAXED ) != 0 ) {
 		noteStreamUse( stream );
 	}
+	return true;
+}
+
+bool deferTransposition( nhStream s, const CTransposition& t )
+{
+	if( __atomic_load_n( &tinyDeferringStreams, __ATOMIC_RELAXED ) == 0 ) {
+		return false;
+	}
+	if( __atomic_load_n( &tinyChainsPending, __ATOMIC_RELAXED ) != 0 ) {
+		std::lock_guard<std::recursive_mutex> guard( tinyLock );
+		CTinyQueue* queue = deferringQueue( reinterpret_cast<hipStream_t>( s ) );
+		if( queue != nullptr && queue->Transpositions.Length > 0 && queue->Transpositions.Length < MaxTranspositions ) {
+			CTranspositions& waiting = queue->Transpositions;
+			bool joins = !rangesMeet( t.From, t.Count, t.To, t.Count );
+			for( int i = 0; joins && i < waiting.Length; ++i ) {
+				const CTransposition& other = waiting.Items[i];
+				joins = !rangesMeet( t.To, t.Count, other.To, other.Count ) && !rangesMeet( t.To, t.Count, other.From, other.Count )
+					&& !rangesMeet( t.From, t.Count, other.To, other.Count );
+			}
+			if( joins ) {
+				waiting.Items[waiting.Length++] = t; // ( one thing waits where one waited )
+				return true;
+			}
+		}
+	}
+	const hipStream_t stream = toStream( s ); // ( what the stream holds goes out first )
+	hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+	if( hipStreamIsCapturing( stream, &capture ) != hipSuccess ) {
+		( void )hipGetLastError();
+		return false;
+	}
+	if( capture != hipStreamCaptureStatusNone ) {
+		return false;
+	}
+	std::lock_guard<std::recursive_mutex> guard( tinyLock );
+	CTinyQueue* queue = deferringQueue( stream );
+	if( queue == nullptr || queue->Chain.Length != 0 || queue->LaunchWaits() ) {
+		return false;
+	}
+	queue->Transpositions.Items[0] = t;
+	queue->Transpositions.Length = 1;
+	__atomic_fetch_add( &tinyChainsPending, 1, __ATOMIC_RELAXED );
 	return true;
 }
 
