@@ -26,6 +26,17 @@ void noteStreamUse( hipStream_t stream );
 // that is asked of the stream, so they too are caught here: tinyChainsPending counts the streams that hold some.
 // flushTinyOps launches what the stream of the current device holds; flushAllTinyOps does so for every stream of every
 // device ( before device memory is given back ). releaseTinyQueue: the stream is being destroyed.
+// Inside a launch of calls that were put aside ( CHeldLaunch; launchingHeldCalls: of this thread ) both do nothing, so that the calls
+// behind the one that is being launched stay behind it, and a pool neither gives nor releases cached blocks: the calls' operands
+// may be among them, given back behind the calls.
+class CHeldLaunch {
+public:
+	CHeldLaunch();
+	~CHeldLaunch();
+	CHeldLaunch( const CHeldLaunch& ) = delete;
+	CHeldLaunch& operator=( const CHeldLaunch& ) = delete;
+};
+bool launchingHeldCalls();
 extern int tinyChainsPending;
 bool flushTinyOps( hipStream_t stream ); // true: something was launched
 void flushAllTinyOps();
@@ -126,6 +137,11 @@ inline hipStream_t toStream( nhStream s )
 // Frees the scratch blocks that sliced reductions keep for a stream of the current device ( gemm_mfma.hip ); the stream
 // must have been drained. unbind: the stream is going away, its binding to a pool goes with the blocks.
 void releaseSliceScratch( hipStream_t stream, bool unbind );
+
+// Scratch that such launches were refused by a pool at its limit, asked for once more: by a call that is about to be put aside,
+// with nothing in front of it.
+extern int sliceScratchWanted;
+void growWantedScratch( hipStream_t stream );
 
 // Scratch of the stream for reductions that meet inside a launch ( gemm_mfma.hip ): `partialFloats` floats and one arrival
 // counter that is zero between launches and must be left at zero. false: none to be had, take another way.

@@ -1032,12 +1032,16 @@ void matMulKernel( const CMatMulArgs launchArgs )
 // (nhStreamReleaseScratch); those of other streams live until the process ends.
 // A stream that has been bound to a caching pool (nhStreamBindPool) takes its blocks from that pool and gives them back
 // to it, so the pool's memory limit, statistics and clean-up cover them; other streams use the raw allocator.
+// A launch of calls that were put aside gets none of the pool's cached blocks, which may hold its operands, and has none
+// released (mem_pool.cpp): what a pool at its limit refuses it is asked for again when the next call is put aside (Wanted).
 // The counters start at zero and every launch leaves them at zero.
 struct CSliceScratch {
 	float* Partials = nullptr;
 	size_t PartialFloats = 0;
 	unsigned* Counters = nullptr;
 	size_t CounterCount = 0;
+	size_t WantedFloats = 0;
+	size_t WantedCounters = 0;
 	std::vector<void*> Blocks; // every allocation made for the stream
 	nhPool Pool = nullptr;     // where the blocks came from; null = the raw allocator
 };
@@ -1054,8 +1058,13 @@ static std::map<std::pair<int, hipStream_t>, nhPool>& poolByStream()
 	return byStream;
 }
 
+int sliceScratchWanted = 0; // streams with a wish
+
 static void freeSliceBlocks( CSliceScratch& scratch )
 {
+	if( scratch.WantedFloats > 0 ) {
+		__atomic_fetch_sub( &sliceScratchWanted, 1, __ATOMIC_RELAXED );
+	}
 	for( void* block : scratch.Blocks ) {
 		if( scratch.Pool != nullptr ) {
 			( void )nhPoolHeapFree( scratch.Pool, block );
@@ -1144,6 +1153,13 @@ static bool sliceScratch( hipStream_t stream, size_t partialFloats, size_t count
 		void* block = nullptr;
 		if( scratch.Pool != nullptr ) {
 			if( nhPoolHeapAlloc( scratch.Pool, bytes, &block ) != NH_OK ) {
+				if( launchingHeldCalls() ) {
+					if( scratch.WantedFloats == 0 ) {
+						__atomic_fetch_add( &sliceScratchWanted, 1, __ATOMIC_RELAXED );
+					}
+					scratch.WantedFloats = partialFloats > scratch.WantedFloats ? partialFloats : scratch.WantedFloats;
+					scratch.WantedCounters = counters > scratch.WantedCounters ? counters : scratch.WantedCounters;
+				}
 				return nullptr;
 			}
 		} else if( hipMalloc( &block, bytes ) != hipSuccess ) {
@@ -1180,6 +1196,32 @@ static bool sliceScratch( hipStream_t stream, size_t partialFloats, size_t count
 	out.Partials = scratch.Partials;
 	out.Counters = scratch.Counters;
 	return true;
+}
+
+// What launches of calls that had been put aside could not get is asked for again, from a call with nothing in front of it on
+// the stream ( deferProduct, deferConvolution )
+void growWantedScratch( hipStream_t stream )
+{
+	int device = 0;
+	if( hipGetDevice( &device ) != hipSuccess ) {
+		( void )hipGetLastError();
+		return;
+	}
+	size_t floats = 0, counters = 0;
+	{
+		std::lock_guard<std::mutex> guard( sliceScratchLock );
+		auto found = sliceScratchByStream().find( std::make_pair( device, stream ) );
+		if( found == sliceScratchByStream().end() || found->second.WantedFloats == 0 ) {
+			return;
+		}
+		floats = found->second.WantedFloats;
+		counters = found->second.WantedCounters;
+		found->second.WantedFloats = 0;
+		found->second.WantedCounters = 0;
+		__atomic_fetch_sub( &sliceScratchWanted, 1, __ATOMIC_RELAXED );
+	}
+	CSliceScratch scratch;
+	( void )sliceScratch( stream, floats, counters, scratch );
 }
 
 // The same block for other reductions that meet inside a launch ( vector sums ): partial results and one arrival counter,

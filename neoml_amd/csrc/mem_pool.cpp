@@ -9,6 +9,8 @@
 //     raw allocator and straight back on free;
 //   - the raw allocator may hold at most `memoryLimit` bytes (0 = unlimited); when a request fails the calling
 //     thread's cached blocks are released and the request is tried once more, then NH_ERR_MEMORY;
+//   - a launch of calls that were put aside (nh::launchingHeldCalls) may find their operands in these caches, freed behind
+//     the calls: its requests take no cached block and release none, they get new memory within the limit or none;
 //   - CleanUp releases the cached blocks and the empty stack of the calling thread only;
 //   - the stack grows in 64 KiB quanta; while it is empty its single block is re-allocated to the high-water
 //     mark, so a steady-state workload ends up with one block and no raw allocations.
@@ -25,6 +27,7 @@
 
 namespace nh {
 void setLastError( const char* fmt, ... );
+bool launchingHeldCalls();
 }
 
 namespace {
@@ -169,7 +172,7 @@ void* CPool::tryAlloc( size_t size, CThreadState& st )
 	const std::vector<size_t>& classes = sizeClasses();
 	const int cls = static_cast<int>( std::lower_bound( classes.begin(), classes.end(), size ) - classes.begin() );
 	void* ptr = nullptr;
-	if( !st.FreeLists[cls].empty() ) {
+	if( !st.FreeLists[cls].empty() && !nh::launchingHeldCalls() ) {
 		ptr = st.FreeLists[cls].back();
 		st.FreeLists[cls].pop_back();
 	} else {
@@ -198,7 +201,7 @@ void* CPool::heapAllocLocked( size_t size )
 {
 	CThreadState& st = state();
 	void* ptr = tryAlloc( size, st );
-	if( ptr == nullptr ) {
+	if( ptr == nullptr && !nh::launchingHeldCalls() ) {
 		releaseCached( st );
 		ptr = tryAlloc( size, st );
 	}

@@ -933,9 +933,12 @@ static int launchPendingAttention( hipStream_t stream, const CPendingAttention& 
 }
 
 typedef std::map<std::pair<int, hipStream_t>, CTinyQueue> CTinyQueues;
-// ( recursive: a product launched from under the lock may ask its stream's pool for scratch memory, a pool at its limit
-// gives memory back first, and giving memory back launches what every stream holds )
+// ( recursive: what is launched from under the lock may turn a stream handle into a stream, which looks for calls to launch )
 static std::recursive_mutex tinyLock;
+static thread_local int heldLaunches = 0;
+CHeldLaunch::CHeldLaunch() { ++heldLaunches; }
+CHeldLaunch::~CHeldLaunch() { --heldLaunches; }
+bool launchingHeldCalls() { return heldLaunches != 0; }
 static CTinyQueues& tinyQueues()
 {
 	static CTinyQueues* queues = new CTinyQueues; // never destroyed: calls may still arrive while the process unloads
@@ -1216,6 +1219,7 @@ static bool launchParked( hipStream_t stream, CTinyQueue& queue )
 
 static bool launchTinyChain( hipStream_t stream, CTinyQueue& queue )
 {
+	const CHeldLaunch held;
 	CTinyChain& chain = queue.Chain;
 	const bool parked = launchParked( stream, queue );
 	if( chain.Length == 0 ) {
@@ -1663,6 +1667,7 @@ static void launchColumnSum( hipStream_t stream, const CPendingColumnSum& sum, c
 // what the queue holds: the product that waits for its successor ( then nothing else is queued ), or a chain
 static bool launchPending( hipStream_t stream, CTinyQueue& queue )
 {
+	const CHeldLaunch held;
 	const bool parked = launchParked( stream, queue );
 	if( queue.ColumnSum.Pending ) {
 		const CPendingColumnSum sum = queue.ColumnSum;
@@ -1721,6 +1726,9 @@ static bool launchPending( hipStream_t stream, CTinyQueue& queue )
 
 bool flushTinyOps( hipStream_t stream )
 {
+	if( launchingHeldCalls() ) {
+		return false;
+	}
 	int device = 0;
 	if( hipGetDevice( &device ) != hipSuccess ) {
 		( void )hipGetLastError();
@@ -1733,7 +1741,7 @@ bool flushTinyOps( hipStream_t stream )
 
 void flushAllTinyOps()
 {
-	if( __atomic_load_n( &tinyChainsPending, __ATOMIC_RELAXED ) == 0 ) {
+	if( __atomic_load_n( &tinyChainsPending, __ATOMIC_RELAXED ) == 0 || launchingHeldCalls() ) {
 		return;
 	}
 	int current = 0;
@@ -1850,6 +1858,9 @@ bool deferProduct( nhStream s, const float* a, int lda, const float* b, int ldb,
 	if( capture != hipStreamCaptureStatusNone ) {
 		return false;
 	}
+	if( __atomic_load_n( &sliceScratchWanted, __ATOMIC_RELAXED ) != 0 ) {
+		growWantedScratch( stream );
+	}
 	std::lock_guard<std::recursive_mutex> guard( tinyLock );
 	auto found = tinyQueues().find( std::make_pair( device, stream ) );
 	if( found == tinyQueues().end() || !found->second.Enabled || found->second.Chain.Length != 0 || found->second.LaunchWaits() )
@@ -1919,19 +1930,16 @@ static bool launchGatedProduct( hipStream_t stream, CTinyQueue& queue )
 	if( op[1].In[0] != t || op[1].Out != t || op[1].Count != op[0].Count || !product || op[2].Out != p.C || op[2].Count != op[0].Count ) {
 		return false;
 	}
-	const float* scale = op[0].Scalar;
-	queue.Product.Pending = false; // ( as elsewhere: a launch may ask a pool for memory, which sends out what the queues hold )
-	const CTinyChain held = chain;
-	chain.Length = 0;
+	const CHeldLaunch held;
 	int rc = NH_OK;
-	if( matMulNTGated( stream, p.A, p.Lda, p.B, p.Ldb, p.C, p.Ldc, p.M, p.N, p.K, p.Bias, t, scale, &rc ) ) {
-		queue.ProductParked = false;
-		__atomic_fetch_sub( &tinyChainsPending, 2, __ATOMIC_RELAXED );
-		return true;
+	if( !matMulNTGated( stream, p.A, p.Lda, p.B, p.Ldb, p.C, p.Ldc, p.M, p.N, p.K, p.Bias, t, op[0].Scalar, &rc ) ) {
+		return false;
 	}
-	chain = held;
-	queue.Product.Pending = true;
-	return false;
+	queue.Product.Pending = false;
+	queue.ProductParked = false;
+	chain.Length = 0;
+	__atomic_fetch_sub( &tinyChainsPending, 2, __ATOMIC_RELAXED );
+	return true;
 }
 
 bool deferColumnSum( nhStream s, float* result, const float* matrix, int height, int width )
@@ -2198,6 +2206,7 @@ static bool fusePendingBatched( nhStream s, const float* first, float* result, i
 		queue->Batched.Pending = false;
 		__atomic_fetch_sub( &tinyChainsPending, 1, __ATOMIC_RELAXED );
 	}
+	const CHeldLaunch held;
 	bool scaled = false;
 	*rc = launchBatched( stream, p, multiplier, &scaled );
 	if( __atomic_load_n( &lstmPartnersAwaited, __ATOMIC_RELAXED ) != 0 ) {
@@ -2243,6 +2252,7 @@ bool fusePendingTransposition( nhStream s, int batch, const float* first, int he
 	}
 	p.Transposed = result;
 	p.Heads = height;
+	const CHeldLaunch held;
 	*rc = launchAttention( stream, p );
 	if( __atomic_load_n( &lstmPartnersAwaited, __ATOMIC_RELAXED ) != 0 ) {
 		noteStreamUse( stream );
@@ -2405,6 +2415,9 @@ bool deferConvolution( nhStream s, bool channelwise, const nhConvDesc& d, const 
 	if( capture != hipStreamCaptureStatusNone ) {
 		return false;
 	}
+	if( __atomic_load_n( &sliceScratchWanted, __ATOMIC_RELAXED ) != 0 ) {
+		growWantedScratch( stream );
+	}
 	std::lock_guard<std::recursive_mutex> guard( tinyLock );
 	CTinyQueue* queue = deferringQueue( stream );
 	if( queue == nullptr || queue->Chain.Length != 0 || queue->LaunchWaits() ) {
@@ -2447,11 +2460,11 @@ bool joinPendingConvolution( nhStream s, const float* first, const float* second
 		if( other != shortcut.Result || touches( c, shortcut.Result, count ) || touches( shortcut, c.Result, count ) ) {
 			return false;
 		}
-		// ( both leave the queue: the launch may ask a pool for memory, which sends out what the queues hold )
 		queue->Convolution.Pending = false;
 		queue->Shortcut.Pending = false;
 		__atomic_fetch_sub( &tinyChainsPending, 1, __ATOMIC_RELAXED );
 	}
+	const CHeldLaunch held;
 	const CFusedActivation none = { NH_ACT_NONE, 0.f };
 	( void )launchPendingConvolution( stream, shortcut, none );
 	if( __atomic_load_n( &lstmPartnersAwaited, __ATOMIC_RELAXED ) != 0 ) {
@@ -2494,6 +2507,7 @@ bool fusePendingConvolution( nhStream s, const float* first, float* result, long
 		queue->Shortcut.Pending = false;
 		__atomic_fetch_sub( &tinyChainsPending, 1, __ATOMIC_RELAXED );
 	}
+	const CHeldLaunch held;
 	if( front.Pending ) {
 		const CFusedActivation none = { NH_ACT_NONE, 0.f };
 		( void )launchPendingConvolution( stream, front, none );
