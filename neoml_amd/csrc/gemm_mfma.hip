@@ -43,9 +43,20 @@ namespace nh {
 // over one half of the K steps of the tile, then the second group hands its accumulators to the first through LDS.
 // For problems of a few hundred tiles with a reduction long enough to cut in two: the same number of waves per compute
 // unit as two K slices in separate workgroups, without the preset of C, the atomics and the separate activation pass.
-template<int BM, int BN, int WAVES_M, int WAVES_N, int AMODE, int BMODE, bool VEC, int KGROUPS = 1>
-__global__ __launch_bounds__( Threads * KGROUPS, KGROUPS == 1 ? 2 : 1 )
-void matMulKernel( const CMatMulArgs launchArgs )
+// Wavefronts to a SIMD that the kernels of matMulTile are compiled for, at least and at most. How many workgroups a compute unit takes at once
+// decides how whole the last round of a launch is, and launchTile cuts K by it. The two modes that run the large products and 3x3
+// convolutions have room for eight ( 64 registers ). With 90, five, launches of five to eight workgroups a compute unit are uneven: us with five
+// and eight, 2880 x 256 x 1152 in 4 slices 47.6 and 43.5, 5672 x 256 x 2304 in 5 58.8 and 53, 1421 x 512 x 4608 in 8 63.6 and 57; with seven
+// 2048 workgroups of a 2304-long reduction take 298 instead of 270. The operands from columns ( the gradient by a filter above all, whose slices
+// were fitted to five ) stay at five: with seven the gradients of 57 x 13 x 14 x 256 take 3 % longer.
+template<int BM, int AMODE, int BMODE>
+constexpr int leastWaves() { return BM == 64 && BMODE == BM_RowsK && ( AMODE == AM_RowsK || AMODE == AM_ConvTaps ) ? 8 : 2; }
+template<int BMODE>
+constexpr int mostWaves() { return BMODE == BM_RowsK ? 8 : 5; }
+
+// RESIDUAL: the launch adds one ( a kernel of its own, below: its epilogue would cost the others registers )
+template<int BM, int BN, int WAVES_M, int WAVES_N, int AMODE, int BMODE, bool VEC, int KGROUPS, bool RESIDUAL>
+__device__ __forceinline__ void matMulTile( const CMatMulArgs& launchArgs )
 {
 	constexpr bool IsClasses = ( AMODE == AM_ConvClasses );
 	CMatMulArgs args = launchArgs;
@@ -761,9 +772,21 @@ void matMulKernel( const CMatMulArgs launchArgs )
 		}
 	}
 
+	// The thread's place again, for what follows: its parts, kept across the loop, would take the registers that the eighth
+	// workgroup of a compute unit needs.
+	int endTid = threadIdx.x;
+	asm volatile( "" : "+v"( endTid ) );
+	endTid = KGROUPS == 1 ? endTid : endTid % Threads;
+	const int endLane = endTid & 63;
+	const int endWave = endTid >> 6;
+	const int endWaveM = endWave / WAVES_N;
+	const int endWaveN = endWave % WAVES_N;
+	const int endL32 = endLane & 31;
+	const int endHalf = endLane >> 5;
+
 	if constexpr( KGROUPS == 2 ) {
 		// every wave has passed the last barrier of its loop behind its last LDS read: the buffers are free
-		float* hand = &lds[1][0][0] + wave * ( MI * NI * 16 * 64 ) + lane;
+		float* hand = &lds[1][0][0] + endWave * ( MI * NI * 16 * 64 ) + endLane;
 		if( kGroup == 1 ) {
 #pragma unroll
 			for( int mi = 0; mi < MI; ++mi ) {
@@ -813,7 +836,7 @@ void matMulKernel( const CMatMulArgs launchArgs )
 			// 123 us to 145 / 166 / 159 us ( 64 x 28 x 28 x 128, 64 x 14 x 14 x 256, 64 x 7 x 7 x 512 ).
 			const int slicedTile = args.FullTiles > 0 ? tile - args.FullTiles : tile;
 			unsigned* mine = reinterpret_cast<unsigned*>( args.Partials )
-				+ ( static_cast<long long>( slicedTile ) * splitK + split ) * ( BM * BN ) + wave * 64 + lane;
+				+ ( static_cast<long long>( slicedTile ) * splitK + split ) * ( BM * BN ) + endWave * 64 + endLane;
 #pragma unroll
 			for( int r = 0; r < 16; ++r ) {
 				__hip_atomic_store( mine + r * Threads, __float_as_uint( acc[0][0][r] ), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT );
@@ -821,7 +844,7 @@ void matMulKernel( const CMatMulArgs launchArgs )
 			__builtin_amdgcn_s_waitcnt( 0x0F70 ); // vmcnt( 0 ): this wave's stores have been acknowledged
 			__syncthreads();
 			unsigned* arrived = reinterpret_cast<unsigned*>( &lds[0][0][0] );
-			if( tid == 0 ) {
+			if( endTid == 0 ) {
 				*arrived = __hip_atomic_fetch_add( args.Counters + slicedTile, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT );
 			}
 			__syncthreads();
@@ -849,7 +872,7 @@ void matMulKernel( const CMatMulArgs launchArgs )
 				}
 			}
 			acc[0][0] = total;
-			if( tid == 0 ) {
+			if( endTid == 0 ) {
 				__hip_atomic_store( args.Counters + slicedTile, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT );
 			}
 			splitK = 1; // from here on: the one workgroup that writes the tile
@@ -866,8 +889,8 @@ void matMulKernel( const CMatMulArgs launchArgs )
 	if constexpr( !IsClasses && BMODE != BM_ConvN ) {
 		if( args.CBytes != 0 && splitK == 1 && !args.Accumulate ) {
 			const __amdgpu_buffer_rsrc_t bufC = __builtin_amdgcn_make_buffer_rsrc( C, 0, args.CBytes, 0x00020000 );
-			const __amdgpu_buffer_rsrc_t bufR = __builtin_amdgcn_make_buffer_rsrc(
-				const_cast<float*>( args.Residual != nullptr ? args.Residual + batch * args.BatchStrideC : C ), 0, args.CBytes, 0x00020000 );
+			const __amdgpu_buffer_rsrc_t bufR = RESIDUAL ? __builtin_amdgcn_make_buffer_rsrc(
+				const_cast<float*>( args.Residual + batch * args.BatchStrideC ), 0, args.CBytes, 0x00020000 ) : bufC;
 			const float actParam = withParam( args.Act ).Param; // ( the threshold may live in device memory )
 			const float reluTop = actParam > 0.f ? actParam : __builtin_inff();
 			const unsigned pitchBytes = static_cast<unsigned>( args.Ldc ) * 4u;
@@ -879,10 +902,10 @@ void matMulKernel( const CMatMulArgs launchArgs )
 				constexpr int Residual = decltype( residualOf )::value;
 #pragma unroll
 				for( int ni = 0; ni < NI; ++ni ) {
-					const int n = n0 + waveN * WN + ni * 32 + l32;
+					const int n = n0 + endWaveN * WN + ni * 32 + endL32;
 					const float bias = ( args.Bias != nullptr && n < N ) ? args.Bias[n] : 0.f;
 					const unsigned laneOffset = n < N
-						? static_cast<unsigned>( ( m0 + waveM * WM + half * 4 ) * args.Ldc + n ) * 4u : OutOfRange;
+						? static_cast<unsigned>( ( m0 + endWaveM * WM + endHalf * 4 ) * args.Ldc + n ) * 4u : OutOfRange;
 #pragma unroll
 					for( int mi = 0; mi < MI; ++mi ) {
 						auto rowBytesOf = [&]( int r ) {
@@ -925,7 +948,7 @@ void matMulKernel( const CMatMulArgs launchArgs )
 				}
 			};
 			auto storeAs = [&]( auto typeOf ) {
-				if( args.Residual == nullptr ) {
+				if constexpr( !RESIDUAL ) {
 					storeBy( typeOf, std::integral_constant<int, 0>() );
 				} else if( args.Act.BehindResidual == 0 || decltype( typeOf )::value == NH_ACT_NONE ) {
 					storeBy( typeOf, std::integral_constant<int, 1>() );
@@ -944,9 +967,41 @@ void matMulKernel( const CMatMulArgs launchArgs )
 		}
 	}
 
+	if constexpr( RESIDUAL ) {
+		// A residual with a result beyond 32-bit offsets ( one slice or the last to arrive, see launchTile ): element after element, the others
+		// moving up, so that it takes none of the registers that the common case has no use for ( unrolled it takes 90 of
+		// them, five workgroups to a compute unit instead of eight ).
+		const CFusedActivation act = withParam( args.Act );
+#pragma unroll
+		for( int ni = 0; ni < NI; ++ni ) {
+			const int n = n0 + endWaveN * WN + ni * 32 + endL32;
+#pragma unroll
+			for( int mi = 0; mi < MI; ++mi ) {
+#pragma unroll 1
+				for( int r = 0; r < 16; ++r ) {
+					const int m = m0 + endWaveM * WM + mi * 32 + ( r >> 2 ) * 8 + endHalf * 4 + ( r & 3 );
+					if( m < M && n < N ) {
+						const long long at = static_cast<long long>( m ) * args.Ldc + n;
+						const float other = args.Residual[batch * args.BatchStrideC + at];
+						float v = acc[mi][ni][0] + ( args.Bias != nullptr ? args.Bias[n] : 0.f );
+						if( args.Accumulate ) {
+							v += C[at];
+						}
+						C[at] = args.Act.BehindResidual != 0 ? applyActivation( v + other, act ) : applyActivation( v, act ) + other;
+					}
+#pragma unroll
+					for( int e = 0; e + 1 < 16; ++e ) {
+						acc[mi][ni][e] = acc[mi][ni][e + 1];
+					}
+				}
+			}
+		}
+		return;
+	}
+
 #pragma unroll
 	for( int ni = 0; ni < NI; ++ni ) {
-		int n = n0 + waveN * WN + ni * 32 + l32;
+		int n = n0 + endWaveN * WN + ni * 32 + endL32;
 		if( n >= N ) {
 			continue;
 		}
@@ -961,9 +1016,9 @@ void matMulKernel( const CMatMulArgs launchArgs )
 		}
 		const float bias = ( args.Bias != nullptr ) ? args.Bias[n] : 0.f;
 		const float actParam = withParam( args.Act ).Param; // ( the threshold may live in device memory )
-	const float reluTop = actParam > 0.f ? actParam : __builtin_inff();
+		const float reluTop = actParam > 0.f ? actParam : __builtin_inff();
 		// Mode: 0 adds onto C with atomics ( K slices that meet in C: it was set to the free term, or left as it was when
-		// accumulating, before the launch ), 1 stores act( acc + bias ), 2 also accumulates and / or adds the residual.
+		// accumulating, before the launch ), 1 stores act( acc + bias ), 2 also accumulates.
 		// What is the same for the whole tile is decided once per tile, not per element: with up to eight wavefronts per SIMD
 		// a handful of branches in front of every one of a lane's 16 or 32 stores costs microseconds per launch.
 		auto write = [&]( auto modeOf, auto typeOf ) {
@@ -973,7 +1028,7 @@ void matMulKernel( const CMatMulArgs launchArgs )
 			for( int mi = 0; mi < MI; ++mi ) {
 #pragma unroll
 				for( int r = 0; r < 16; ++r ) {
-					const int m = m0 + waveM * WM + mi * 32 + ( r >> 2 ) * 8 + half * 4 + ( r & 3 );
+					const int m = m0 + endWaveM * WM + mi * 32 + ( r >> 2 ) * 8 + endHalf * 4 + ( r & 3 );
 					if( m < M ) {
 						long long row = m;
 						if constexpr( IsClasses ) {
@@ -989,24 +1044,16 @@ void matMulKernel( const CMatMulArgs launchArgs )
 						} else {
 							float v = acc[mi][ni][r] + bias;
 							if constexpr( Mode == 2 ) {
-								if( args.Accumulate ) {
-									v += *p;
-								}
+								v += *p;
 							}
-							if constexpr( Mode == 2 ) {
-								const float r = args.Residual != nullptr ? args.Residual[batch * args.BatchStrideC + row * args.Ldc + n] : 0.f;
-								v = args.Act.BehindResidual != 0 ? applyActivationOf<Type>( v + r, reluTop ) : applyActivationOf<Type>( v, reluTop ) + r;
-							} else {
-								v = applyActivationOf<Type>( v, reluTop );
-							}
-							*p = v;
+							*p = applyActivationOf<Type>( v, reluTop );
 						}
 					}
 				}
 			}
 		};
 		auto writeAs = [&]( auto typeOf ) {
-			if( args.Accumulate || args.Residual != nullptr ) {
+			if( args.Accumulate ) {
 				write( std::integral_constant<int, 2>(), typeOf );
 			} else {
 				write( std::integral_constant<int, 1>(), typeOf );
@@ -1022,6 +1069,20 @@ void matMulKernel( const CMatMulArgs launchArgs )
 			writeAs( std::integral_constant<int, NH_ACT_NONE>() );
 		}
 	}
+}
+
+template<int BM, int BN, int WAVES_M, int WAVES_N, int AMODE, int BMODE, bool VEC, int KGROUPS = 1>
+__global__ __launch_bounds__( Threads * KGROUPS ) __attribute__(( amdgpu_waves_per_eu( ( leastWaves<BM, AMODE, BMODE>() ), ( mostWaves<BMODE>() ) ) ))
+void matMulKernel( const CMatMulArgs args )
+{
+	matMulTile<BM, BN, WAVES_M, WAVES_N, AMODE, BMODE, VEC, KGROUPS, false>( args );
+}
+
+template<int BM, int BN, int WAVES_M, int WAVES_N, int AMODE, int BMODE, bool VEC, int KGROUPS = 1>
+__global__ __launch_bounds__( Threads * KGROUPS ) __attribute__(( amdgpu_waves_per_eu( ( leastWaves<BM, AMODE, BMODE>() ), ( mostWaves<BMODE>() ) ) ))
+void matMulResidualKernel( const CMatMulArgs args )
+{
+	matMulTile<BM, BN, WAVES_M, WAVES_N, AMODE, BMODE, VEC, KGROUPS, true>( args );
 }
 
 // Scratch of the K slices that meet without atomics: partial tiles and arrival counters, one pair per stream (launches
@@ -1357,6 +1418,8 @@ static int presetResult( hipStream_t stream, const CMatMulArgs& args, int batch 
 template<int BM, int BN, int WAVES_M, int WAVES_N, int AMODE, int BMODE>
 static int launchTile( hipStream_t stream, CMatMulArgs& args, int batch, bool vec, const CSliceMeeting* fixedMeeting )
 {
+	constexpr bool TakesResidual = BMODE == BM_RowsK && AMODE != AM_ConvClasses;
+	NH_REQUIRE( TakesResidual || args.Residual == nullptr );
 	args.TilesM = ceilDiv( args.M, BM );
 	args.TilesN = ceilDiv( args.N, BN );
 	args.TilesNMagic = divisionMagic( args.TilesN );
@@ -1535,14 +1598,25 @@ static int launchTile( hipStream_t stream, CMatMulArgs& args, int batch, bool ve
 		a.B += b0 * args.BatchStrideB;
 		a.C += b0 * args.BatchStrideC;
 		const dim3 grid( static_cast<unsigned>( gridX ), nb, args.SplitK );
+		auto launch = [&]( auto vecOf, auto groupsOf ) {
+			constexpr bool Vec = decltype( vecOf )::value;
+			constexpr int Groups = decltype( groupsOf )::value;
+			if constexpr( TakesResidual ) {
+				if( args.Residual != nullptr ) {
+					hipLaunchKernelGGL( ( matMulResidualKernel<BM, BN, WAVES_M, WAVES_N, AMODE, BMODE, Vec, Groups> ), grid, dim3( Threads * Groups ), 0, stream, a );
+					return;
+				}
+			}
+			hipLaunchKernelGGL( ( matMulKernel<BM, BN, WAVES_M, WAVES_N, AMODE, BMODE, Vec, Groups> ), grid, dim3( Threads * Groups ), 0, stream, a );
+		};
 		if( twoGroups ) {
 			if constexpr( BM == 64 && BN == 64 && BMODE == BM_RowsK && ( AMODE == AM_Conv || AMODE == AM_ConvTaps || AMODE == AM_RowsK ) ) {
-				hipLaunchKernelGGL( ( matMulKernel<BM, BN, WAVES_M, WAVES_N, AMODE, BMODE, true, 2> ), grid, dim3( Threads * 2 ), 0, stream, a );
+				launch( std::true_type(), std::integral_constant<int, 2>() );
 			}
 		} else if( vec ) {
-			hipLaunchKernelGGL( ( matMulKernel<BM, BN, WAVES_M, WAVES_N, AMODE, BMODE, true> ), grid, dim3( Threads ), 0, stream, a );
+			launch( std::true_type(), std::integral_constant<int, 1>() );
 		} else if constexpr( AMODE != AM_ConvTaps ) {
-			hipLaunchKernelGGL( ( matMulKernel<BM, BN, WAVES_M, WAVES_N, AMODE, BMODE, false> ), grid, dim3( Threads ), 0, stream, a );
+			launch( std::false_type(), std::integral_constant<int, 1>() );
 		}
 		if( args.FullTiles > 0 && actAfter.Type != NH_ACT_NONE && !meetInScratch ) {
 			const long long total = static_cast<long long>( tail.M ) * args.N;

@@ -90,3 +90,33 @@ def test_sum_and_relu(streams, n, h, w, cin, cout, f, stride):
             results.append((y.view(torch.int32), s.view(torch.int32)))
         assert torch.equal(results[0][0], results[1][0]), what
         assert torch.equal(results[0][1], results[1][1]), what
+
+
+def test_a_result_beyond_32_bit_offsets(streams):
+    import nhtest
+    torch, lib, na = streams.torch, streams.lib, streams.na
+    hip = nhtest.Hip()
+    size, cin, cout = 2899, 16, 64  # 2.15 GB
+    g = torch.Generator(device=streams.dev).manual_seed(5)
+    d = hip.conv_desc(1, size, size, cin, cout, 3, 3, 1, 1, 1, 1)
+    count = size * size * cout
+    assert count * 4 > 2 ** 31
+    x, filt, bias, other = (torch.randn(shape, generator=g, device=streams.dev) for shape in ((1, size, size, cin), (cout, 3, 3, cin), (cout,), (count,)))
+    top = torch.full((1,), 6.0, device=streams.dev)
+
+    def p(t):
+        return ctypes.c_void_p(t.data_ptr())
+
+    for activation in ([], [("nhVectorReLU", count, p(top))], [("nhVectorHSwish", count)]):
+        results = []
+        for stream in (streams.plain, streams.deferring):
+            y = torch.empty(count, device=streams.dev)
+            torch.cuda.synchronize()
+            na.check(lib.nhBlobConvolution(stream, ctypes.byref(d), p(x), p(filt), p(bias), p(y)))
+            na.check(lib.nhVectorAdd(stream, p(y), p(other), p(y), count))
+            for name, *args in activation:
+                na.check(getattr(lib, name)(stream, p(y), p(y), *args))
+            na.check(lib.nhStreamSynchronize(stream))
+            results.append(y)
+        assert torch.equal(results[0].view(torch.int32), results[1].view(torch.int32))
+        del results, y
