@@ -1095,6 +1095,8 @@ void matMulResidualKernel( const CMatMulArgs args )
 // to it, so the pool's memory limit, statistics and clean-up cover them; other streams use the raw allocator.
 // A launch of calls that were put aside gets none of the pool's cached blocks, which may hold its operands, and has none
 // released (mem_pool.cpp): what a pool at its limit refuses it is asked for again when the next call is put aside (Wanted).
+// Blocks are taken and given back with the lock open: a pool that releases memory launches what streams hold, and those
+// launches come here.
 // The counters start at zero and every launch leaves them at zero.
 struct CSliceScratch {
 	float* Partials = nullptr;
@@ -1103,8 +1105,8 @@ struct CSliceScratch {
 	size_t CounterCount = 0;
 	size_t WantedFloats = 0;
 	size_t WantedCounters = 0;
-	std::vector<void*> Blocks; // every allocation made for the stream
-	nhPool Pool = nullptr;     // where the blocks came from; null = the raw allocator
+	std::vector<std::pair<void*, nhPool>> Blocks; // every allocation made for the stream and where it came from; null = the raw allocator
+	nhPool Pool = nullptr;                        // where the next one comes from
 };
 
 static std::mutex sliceScratchLock;
@@ -1121,19 +1123,31 @@ static std::map<std::pair<int, hipStream_t>, nhPool>& poolByStream()
 
 int sliceScratchWanted = 0; // streams with a wish
 
-static void freeSliceBlocks( CSliceScratch& scratch )
+// ( with the lock held: what the stream keeps leaves the table )
+static CSliceScratch takeSliceScratch( const std::pair<int, hipStream_t>& key )
 {
-	if( scratch.WantedFloats > 0 ) {
-		__atomic_fetch_sub( &sliceScratchWanted, 1, __ATOMIC_RELAXED );
+	CSliceScratch taken;
+	auto& byStream = sliceScratchByStream();
+	auto found = byStream.find( key );
+	if( found != byStream.end() ) {
+		taken = found->second;
+		if( taken.WantedFloats > 0 ) {
+			__atomic_fetch_sub( &sliceScratchWanted, 1, __ATOMIC_RELAXED );
+		}
+		byStream.erase( found );
 	}
-	for( void* block : scratch.Blocks ) {
-		if( scratch.Pool != nullptr ) {
-			( void )nhPoolHeapFree( scratch.Pool, block );
+	return taken;
+}
+
+static void freeSliceBlocks( const CSliceScratch& scratch )
+{
+	for( const auto& block : scratch.Blocks ) {
+		if( block.second != nullptr ) {
+			( void )nhPoolHeapFree( block.second, block.first );
 		} else {
-			( void )hipFree( block );
+			( void )hipFree( block.first );
 		}
 	}
-	scratch = CSliceScratch();
 }
 
 void releaseSliceScratch( hipStream_t stream, bool unbind )
@@ -1143,37 +1157,38 @@ void releaseSliceScratch( hipStream_t stream, bool unbind )
 		( void )hipGetLastError();
 		return;
 	}
-	std::lock_guard<std::mutex> guard( sliceScratchLock );
 	const std::pair<int, hipStream_t> key = std::make_pair( device, stream );
-	auto& byStream = sliceScratchByStream();
-	auto found = byStream.find( key );
-	if( found != byStream.end() ) {
-		freeSliceBlocks( found->second );
-		byStream.erase( found );
+	CSliceScratch taken;
+	{
+		std::lock_guard<std::mutex> guard( sliceScratchLock );
+		taken = takeSliceScratch( key );
+		if( unbind ) {
+			poolByStream().erase( key );
+		}
 	}
-	if( unbind ) {
-		poolByStream().erase( key );
-	}
+	freeSliceBlocks( taken );
 }
 
 int bindSliceScratchPool( hipStream_t stream, nhPool pool )
 {
 	int device = 0;
 	NH_HIP( hipGetDevice( &device ) );
-	std::lock_guard<std::mutex> guard( sliceScratchLock );
 	const std::pair<int, hipStream_t> key = std::make_pair( device, stream );
-	auto& byStream = sliceScratchByStream();
-	auto found = byStream.find( key );
-	if( found != byStream.end() && found->second.Pool != pool ) {
-		// blocks from the previous source go back there ( the caller has drained the stream )
-		freeSliceBlocks( found->second );
-		byStream.erase( found );
+	CSliceScratch taken;
+	{
+		std::lock_guard<std::mutex> guard( sliceScratchLock );
+		auto& byStream = sliceScratchByStream();
+		auto found = byStream.find( key );
+		if( found != byStream.end() && found->second.Pool != pool ) {
+			taken = takeSliceScratch( key );
+		}
+		if( pool != nullptr ) {
+			poolByStream()[key] = pool;
+		} else {
+			poolByStream().erase( key );
+		}
 	}
-	if( pool != nullptr ) {
-		poolByStream()[key] = pool;
-	} else {
-		poolByStream().erase( key );
-	}
+	freeSliceBlocks( taken ); // ( back to the previous source; the caller has drained the stream )
 	return NH_OK;
 }
 
@@ -1194,8 +1209,6 @@ static bool sliceScratch( hipStream_t stream, size_t partialFloats, size_t count
 	if( hipGetDevice( &device ) != hipSuccess ) {
 		return false;
 	}
-	std::lock_guard<std::mutex> guard( sliceScratchLock );
-	auto& byStream = sliceScratchByStream();
 	// A recorded graph may replay on another stream, beside launches that use this stream's block: launches under
 	// capture take the atomic path.
 	hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
@@ -1204,43 +1217,55 @@ static bool sliceScratch( hipStream_t stream, size_t partialFloats, size_t count
 		return false;
 	}
 	const std::pair<int, hipStream_t> key = std::make_pair( device, stream );
-	CSliceScratch& scratch = byStream[key];
-	if( scratch.Blocks.empty() ) {
-		auto bound = poolByStream().find( key );
-		scratch.Pool = bound != poolByStream().end() ? bound->second : nullptr;
-	}
+	std::unique_lock<std::mutex> guard( sliceScratchLock );
+	CSliceScratch* scratch = nullptr;
+	auto find = [&]() {
+		scratch = &sliceScratchByStream()[key];
+		if( scratch->Blocks.empty() ) {
+			auto bound = poolByStream().find( key );
+			scratch->Pool = bound != poolByStream().end() ? bound->second : nullptr;
+		}
+	};
+	find();
 	// a pool that cannot give the block ( its memory limit ) is not an error here: the slices then meet through atomics
 	auto allocate = [&]( size_t bytes ) -> void* {
+		const nhPool pool = scratch->Pool;
 		void* block = nullptr;
-		if( scratch.Pool != nullptr ) {
-			if( nhPoolHeapAlloc( scratch.Pool, bytes, &block ) != NH_OK ) {
-				if( launchingHeldCalls() ) {
-					if( scratch.WantedFloats == 0 ) {
-						__atomic_fetch_add( &sliceScratchWanted, 1, __ATOMIC_RELAXED );
-					}
-					scratch.WantedFloats = partialFloats > scratch.WantedFloats ? partialFloats : scratch.WantedFloats;
-					scratch.WantedCounters = counters > scratch.WantedCounters ? counters : scratch.WantedCounters;
-				}
-				return nullptr;
+		guard.unlock();
+		if( pool != nullptr ) {
+			if( nhPoolHeapAlloc( pool, bytes, &block ) != NH_OK ) {
+				block = nullptr;
 			}
 		} else if( hipMalloc( &block, bytes ) != hipSuccess ) {
 			( void )hipGetLastError();
-			return nullptr;
+			block = nullptr;
 		}
-		scratch.Blocks.push_back( block );
+		guard.lock();
+		find();
+		if( block != nullptr ) {
+			scratch->Blocks.emplace_back( block, pool );
+		} else if( pool != nullptr && launchingHeldCalls() ) {
+			if( scratch->WantedFloats == 0 ) {
+				__atomic_fetch_add( &sliceScratchWanted, 1, __ATOMIC_RELAXED );
+			}
+			scratch->WantedFloats = partialFloats > scratch->WantedFloats ? partialFloats : scratch->WantedFloats;
+			scratch->WantedCounters = counters > scratch->WantedCounters ? counters : scratch->WantedCounters;
+		}
 		return block;
 	};
-	if( scratch.PartialFloats < partialFloats ) {
-		const size_t grown = partialFloats > 2 * scratch.PartialFloats ? partialFloats : 2 * scratch.PartialFloats;
+	if( scratch->PartialFloats < partialFloats ) {
+		const size_t grown = partialFloats > 2 * scratch->PartialFloats ? partialFloats : 2 * scratch->PartialFloats;
 		float* block = static_cast<float*>( allocate( grown * sizeof( float ) ) );
 		if( block == nullptr ) {
 			return false;
 		}
-		scratch.Partials = block;
-		scratch.PartialFloats = grown;
+		if( scratch->PartialFloats < grown ) { // ( another thread may have been here meanwhile )
+			scratch->Partials = block;
+			scratch->PartialFloats = grown;
+		}
 	}
-	if( scratch.CounterCount < counters ) {
-		size_t grown = counters > 2 * scratch.CounterCount ? counters : 2 * scratch.CounterCount;
+	if( scratch->CounterCount < counters ) {
+		size_t grown = counters > 2 * scratch->CounterCount ? counters : 2 * scratch->CounterCount;
 		grown = grown > 4096 ? grown : 4096;
 		unsigned* block = static_cast<unsigned*>( allocate( grown * sizeof( unsigned ) ) );
 		if( block == nullptr ) {
@@ -1251,11 +1276,13 @@ static bool sliceScratch( hipStream_t stream, size_t partialFloats, size_t count
 			( void )hipGetLastError();
 			return false;
 		}
-		scratch.Counters = block;
-		scratch.CounterCount = grown;
+		if( scratch->CounterCount < grown ) {
+			scratch->Counters = block;
+			scratch->CounterCount = grown;
+		}
 	}
-	out.Partials = scratch.Partials;
-	out.Counters = scratch.Counters;
+	out.Partials = scratch->Partials;
+	out.Counters = scratch->Counters;
 	return true;
 }
 

@@ -9,6 +9,9 @@
 //     raw allocator and straight back on free;
 //   - the raw allocator may hold at most `memoryLimit` bytes (0 = unlimited); when a request fails the calling
 //     thread's cached blocks are released and the request is tried once more, then NH_ERR_MEMORY;
+//   - a block is given back to the raw allocator with the pool's lock open: giving device memory back launches what streams
+//     have put aside (nhRawFree), and such a launch may ask this pool for scratch memory. Requests that fail meanwhile wait
+//     and are tried again;
 //   - a launch of calls that were put aside (nh::launchingHeldCalls) may find their operands in these caches, freed behind
 //     the calls: its requests take no cached block and release none, they get new memory within the limit or none;
 //   - CleanUp releases the cached blocks and the empty stack of the calling thread only;
@@ -18,6 +21,7 @@
 #include "../../include/neoml_hip.h"
 
 #include <algorithm>
+#include <condition_variable>
 #include <map>
 #include <mutex>
 #include <stdlib.h>
@@ -103,16 +107,21 @@ private:
 	size_t peak;
 	size_t freeSize;
 	std::mutex mutex;
+	int givingBack = 0; // threads that are giving blocks back with the lock open
+	std::condition_variable gaveBack;
 	std::map<std::thread::id, CThreadState> threads;
 	std::unordered_map<void*, CUsedBlock> used;
 
+	typedef std::vector<std::pair<void*, size_t>> CRawBlocks;
+
 	CThreadState& state();
 	void* rawAlloc( size_t size );
-	void rawFree( void* ptr, size_t size );
+	void rawFree( void* ptr );
 	void* tryAlloc( size_t size, CThreadState& st );
-	void* heapAllocLocked( size_t size );
-	void heapFreeLocked( void* ptr );
-	void releaseCached( CThreadState& st );
+	void* heapAlloc( std::unique_lock<std::mutex>& lock, size_t size );
+	void heapFree( void* ptr, CRawBlocks& toGiveBack );
+	void takeCached( CThreadState& st, CRawBlocks& toGiveBack );
+	void giveBack( std::unique_lock<std::mutex>& lock, const CRawBlocks& blocks );
 };
 
 CThreadState& CPool::state()
@@ -149,14 +158,32 @@ void* CPool::rawAlloc( size_t size )
 	return ptr;
 }
 
-void CPool::rawFree( void* ptr, size_t size )
+void CPool::rawFree( void* ptr )
 {
-	allocated -= size;
 	if( kind == 0 ) {
 		nhRawFree( ptr );
 	} else {
 		free( ptr );
 	}
+}
+
+// opens the lock meanwhile; the blocks count as held until they are gone
+void CPool::giveBack( std::unique_lock<std::mutex>& lock, const CRawBlocks& blocks )
+{
+	if( blocks.empty() ) {
+		return;
+	}
+	++givingBack;
+	lock.unlock();
+	size_t size = 0;
+	for( const auto& block : blocks ) {
+		rawFree( block.first );
+		size += block.second;
+	}
+	lock.lock();
+	allocated -= size;
+	--givingBack;
+	gaveBack.notify_all();
 }
 
 void* CPool::tryAlloc( size_t size, CThreadState& st )
@@ -186,41 +213,46 @@ void* CPool::tryAlloc( size_t size, CThreadState& st )
 	return ptr;
 }
 
-void CPool::releaseCached( CThreadState& st )
+void CPool::takeCached( CThreadState& st, CRawBlocks& toGiveBack )
 {
 	const std::vector<size_t>& classes = sizeClasses();
 	for( size_t cls = 0; cls < st.FreeLists.size(); ++cls ) {
 		for( void* ptr : st.FreeLists[cls] ) {
-			rawFree( ptr, classes[cls] );
+			toGiveBack.emplace_back( ptr, classes[cls] );
 		}
 		st.FreeLists[cls].clear();
 	}
 }
 
-void* CPool::heapAllocLocked( size_t size )
+void* CPool::heapAlloc( std::unique_lock<std::mutex>& lock, size_t size )
 {
 	CThreadState& st = state();
 	void* ptr = tryAlloc( size, st );
-	if( ptr == nullptr && !nh::launchingHeldCalls() ) {
-		releaseCached( st );
+	if( ptr != nullptr || nh::launchingHeldCalls() ) {
+		return ptr;
+	}
+	while( ptr == nullptr && givingBack > 0 ) {
+		gaveBack.wait( lock );
+		ptr = tryAlloc( size, st );
+	}
+	if( ptr == nullptr ) {
+		CRawBlocks blocks;
+		takeCached( st, blocks );
+		giveBack( lock, blocks );
 		ptr = tryAlloc( size, st );
 	}
 	return ptr;
 }
 
-void CPool::heapFreeLocked( void* ptr )
+void CPool::heapFree( void* ptr, CRawBlocks& toGiveBack )
 {
 	auto it = used.find( ptr );
 	const CUsedBlock block = it->second;
 	used.erase( it );
 	freeSize += block.Size;
-	if( block.Class < 0 ) {
-		rawFree( ptr, block.Size );
-		return;
-	}
 	auto owner = threads.find( block.Owner );
-	if( owner == threads.end() ) {
-		rawFree( ptr, block.Size );
+	if( block.Class < 0 || owner == threads.end() ) {
+		toGiveBack.emplace_back( ptr, block.Size );
 		return;
 	}
 	owner->second.FreeLists[block.Class].push_back( ptr );
@@ -228,8 +260,8 @@ void CPool::heapFreeLocked( void* ptr )
 
 int CPool::HeapAlloc( size_t size, void** ptr )
 {
-	std::lock_guard<std::mutex> lock( mutex );
-	*ptr = heapAllocLocked( size == 0 ? 1 : size );
+	std::unique_lock<std::mutex> lock( mutex );
+	*ptr = heapAlloc( lock, size == 0 ? 1 : size );
 	if( *ptr == nullptr ) {
 		nh::setLastError( "HeapAlloc: cannot allocate %zu bytes (in use %zu, limit %zu)", size, allocated, limit );
 		return NH_ERR_MEMORY;
@@ -239,12 +271,14 @@ int CPool::HeapAlloc( size_t size, void** ptr )
 
 int CPool::HeapFree( void* ptr )
 {
-	std::lock_guard<std::mutex> lock( mutex );
+	std::unique_lock<std::mutex> lock( mutex );
 	if( used.find( ptr ) == used.end() ) {
 		nh::setLastError( "HeapFree: the pointer was not allocated by this pool" );
 		return NH_ERR_ARGUMENT;
 	}
-	heapFreeLocked( ptr );
+	CRawBlocks blocks;
+	heapFree( ptr, blocks );
+	giveBack( lock, blocks );
 	return NH_OK;
 }
 
@@ -274,7 +308,7 @@ int CPool::Transfer( void* ptr, size_t size )
 
 int CPool::StackAlloc( size_t size, void** ptr )
 {
-	std::lock_guard<std::mutex> lock( mutex );
+	std::unique_lock<std::mutex> lock( mutex );
 	size = ( std::max<size_t>( size, 1 ) + StackAlignment - 1 ) / StackAlignment * StackAlignment;
 	CThreadState& st = state();
 	st.StackCurrent += size;
@@ -283,11 +317,13 @@ int CPool::StackAlloc( size_t size, void** ptr )
 	const bool regrow = st.Stack.size() == 1 && st.Stack[0].Used == 0 && st.Stack[0].BlockSize < st.StackHighWater;
 	if( st.Stack.empty() || regrow ) {
 		if( regrow ) {
-			heapFreeLocked( st.Stack[0].Base );
+			CRawBlocks blocks;
+			heapFree( st.Stack[0].Base, blocks );
 			st.Stack.clear();
+			giveBack( lock, blocks );
 		}
 		const size_t blockSize = ( st.StackHighWater + StackQuantum - 1 ) / StackQuantum * StackQuantum;
-		void* base = heapAllocLocked( blockSize );
+		void* base = heapAlloc( lock, blockSize );
 		if( base == nullptr ) {
 			st.StackCurrent -= size;
 			nh::setLastError( "StackAlloc: cannot allocate a %zu byte stack block", blockSize );
@@ -304,7 +340,7 @@ int CPool::StackAlloc( size_t size, void** ptr )
 		return NH_OK;
 	}
 	const size_t blockSize = ( size + StackQuantum - 1 ) / StackQuantum * StackQuantum;
-	void* base = heapAllocLocked( blockSize );
+	void* base = heapAlloc( lock, blockSize );
 	if( base == nullptr ) {
 		st.StackCurrent -= size;
 		nh::setLastError( "StackAlloc: cannot allocate a %zu byte stack block", blockSize );
@@ -320,7 +356,7 @@ int CPool::StackFree( void* ptr )
 	if( ptr == nullptr ) {
 		return NH_OK;
 	}
-	std::lock_guard<std::mutex> lock( mutex );
+	std::unique_lock<std::mutex> lock( mutex );
 	CThreadState& st = state();
 	if( st.Stack.empty() ) {
 		nh::setLastError( "StackFree: the stack of this thread is empty" );
@@ -336,27 +372,31 @@ int CPool::StackFree( void* ptr )
 	st.StackCurrent -= top.Used - offset;
 	top.Used = offset;
 	if( top.Used == 0 && st.Stack.size() > 1 ) {
-		heapFreeLocked( top.Base );
+		CRawBlocks blocks;
+		heapFree( top.Base, blocks );
 		st.Stack.pop_back();
+		giveBack( lock, blocks );
 	}
 	return NH_OK;
 }
 
 void CPool::CleanUp()
 {
-	std::lock_guard<std::mutex> lock( mutex );
+	std::unique_lock<std::mutex> lock( mutex );
 	auto it = threads.find( std::this_thread::get_id() );
 	if( it == threads.end() ) {
 		return;
 	}
 	CThreadState& st = it->second;
+	CRawBlocks blocks;
 	if( st.Stack.size() == 1 && st.Stack[0].Used == 0 ) {
-		heapFreeLocked( st.Stack[0].Base );
+		heapFree( st.Stack[0].Base, blocks );
 		st.Stack.clear();
 		st.StackCurrent = 0;
 		st.StackHighWater = 0;
 	}
-	releaseCached( st );
+	takeCached( st, blocks );
+	giveBack( lock, blocks );
 }
 
 size_t CPool::InPools()
@@ -375,19 +415,16 @@ size_t CPool::InPools()
 
 CPool::~CPool()
 {
+	CRawBlocks blocks;
 	for( auto& t : threads ) {
-		for( CStackBlock& b : t.second.Stack ) {
-			auto it = used.find( b.Base );
-			if( it != used.end() ) {
-				rawFree( b.Base, it->second.Size );
-				used.erase( it );
-			}
-		}
-		releaseCached( t.second );
+		takeCached( t.second, blocks );
 	}
-	// blocks the caller never freed
+	// the threads' stacks, and blocks the caller never freed
 	for( auto& u : used ) {
-		rawFree( u.first, u.second.Size );
+		blocks.emplace_back( u.first, u.second.Size );
+	}
+	for( const auto& block : blocks ) {
+		rawFree( block.first );
 	}
 }
 

@@ -118,3 +118,117 @@ def test_an_operand_is_not_released_under_a_waiting_call():
         want = a.double() @ b.double().T + bias.double()
         bound = (k + 40) * 2.0 ** -24 * (a.double().abs() @ b.double().abs().T + bias.double().abs())
         assert ((x.double() - want).abs() <= bound).all()
+
+
+# what gives memory back to the device while a product waits that will ask the same pool for scratch: a request at the limit, the release of a
+# block that was not from the caches, a clean-up, a stack, the scratch of another stream, a product on another stream
+@pytest.mark.parametrize("what", ["request", "direct block", "clean-up", "stack", "stack of blocks", "scratch", "product"])
+def test_memory_given_back_while_a_product_waits(what):
+    m, n, k = 8, 64, 8192
+    with Pooled(8 * MB) as s:
+        torch, lib, na = s.torch, s.lib, s.na
+        a, b, bias = s.draw(1, m, k), s.draw(2, n, k) * k ** -0.5, s.draw(3, n)
+        x, y = torch.zeros((m, n), device="cuda:0"), torch.zeros((m, n), device="cuda:0")
+        other = ctypes.c_void_p()
+        na.check(lib.nhStreamCreate(ctypes.byref(other)))
+        na.check(lib.nhStreamBindPool(other, s.pool))
+        try:
+            direct, top = ctypes.c_void_p(), []
+            if what == "direct block":
+                na.check(lib.nhPoolSetReuseMemoryMode(s.pool, 0))
+                direct = s.alloc(1 * MB)
+                na.check(lib.nhPoolSetReuseMemoryMode(s.pool, 1))
+            if what == "stack of blocks":
+                na.check(lib.nhPoolSetReuseMemoryMode(s.pool, 0))
+            if what in ("stack", "stack of blocks"):
+                for size in (100000, 200000):
+                    top.append(ctypes.c_void_p())
+                    na.check(lib.nhPoolStackAlloc(s.pool, size, ctypes.byref(top[-1])))
+            if what == "scratch":
+                na.check(lib.nhPoolSetReuseMemoryMode(s.pool, 0))
+                s.call(other, "nhMultiplyMatrixByTransposedMatrix", a, m, k, k, b, n, k, y, n, m * n)
+                na.check(lib.nhStreamSynchronize(other))
+            if what in ("request", "clean-up", "product"):
+                for p in [s.alloc(1 * MB) for _ in range(8)]:
+                    s.free(p)
+            torch.cuda.synchronize()
+            s.call(s.stream, "nhMultiplyMatrixByTransposedMatrix", a, m, k, k, b, n, k, x, n, m * n)
+            s.call(s.stream, "nhAddVectorToMatrixRows", 1, x, x, m, n, bias)
+            if what == "request":
+                s.free(s.alloc(3 * MB))
+            elif what == "direct block":
+                s.free(direct)
+            elif what == "clean-up":
+                na.check(lib.nhPoolCleanUp(s.pool))
+            elif what in ("stack", "stack of blocks"):
+                while top:
+                    na.check(lib.nhPoolStackFree(s.pool, top.pop()))
+                na.check(lib.nhPoolStackAlloc(s.pool, 400000, ctypes.byref(direct)))
+                na.check(lib.nhPoolStackFree(s.pool, direct))
+                na.check(lib.nhPoolCleanUp(s.pool))
+            elif what == "scratch":
+                na.check(lib.nhStreamReleaseScratch(other))
+            else:
+                s.call(other, "nhMultiplyMatrixByTransposedMatrix", a, m, k, k, b, n, k, y, n, m * n)
+                na.check(lib.nhStreamSynchronize(other))
+            na.check(lib.nhStreamSynchronize(s.stream))
+            used, cached = ctypes.c_size_t(), ctypes.c_size_t()
+            na.check(lib.nhPoolGetCurrentMemoryUsage(s.pool, ctypes.byref(used)))
+            na.check(lib.nhPoolGetMemoryInPools(s.pool, ctypes.byref(cached)))
+            assert cached.value <= used.value <= 8 * MB
+        finally:
+            na.check(lib.nhStreamDestroy(other))
+        want = a.double() @ b.double().T
+        bound = (k + 40) * 2.0 ** -24 * (a.double().abs() @ b.double().abs().T + bias.double().abs())
+        assert ((x.double() - (want + bias.double())).abs() <= bound).all()
+        if what in ("scratch", "product"):
+            assert ((y.double() - want).abs() <= bound).all()
+
+
+def test_threads_at_the_limit_of_one_pool():
+    """Threads that ask a pool at its limit, each with what the others need in its caches at times, and with calls that wait on streams of
+    their own: every request that fits is met."""
+    import threading
+    m, n, k, threads = 8, 64, 8192, 4
+    # one thread's caches come to 3.75 MB at most, so 14 hold what three keep and the largest request of the fourth, and a little scratch; not
+    # what all four would keep
+    sizes = [MB // 2, MB * 3 // 4, MB, MB * 3 // 2]
+    with Pooled(14 * MB) as s:
+        torch, lib, na = s.torch, s.lib, s.na
+        a, b, bias = s.draw(1, m, k), s.draw(2, n, k) * k ** -0.5, s.draw(3, n)
+        results = [torch.zeros((m, n), device="cuda:0") for _ in range(threads)]
+        torch.cuda.synchronize()
+        errors = []
+
+        def work(i):
+            stream = ctypes.c_void_p()
+            try:
+                na.check(lib.nhStreamCreate(ctypes.byref(stream)))
+                na.check(lib.nhStreamBindPool(stream, s.pool))
+                na.check(lib.nhStreamDeferSmallOps(stream, 1))
+                for r in range(40):
+                    s.call(stream, "nhMultiplyMatrixByTransposedMatrix", a, m, k, k, b, n, k, results[i], n, m * n)
+                    s.call(stream, "nhAddVectorToMatrixRows", 1, results[i], results[i], m, n, bias)
+                    p = s.alloc(sizes[(r + i) % 4])
+                    s.call(stream, "nhVectorFill", p, ctypes.c_float(1.0), 1024)
+                    s.free(p)
+                    if r % 16 == 15:
+                        na.check(lib.nhPoolCleanUp(s.pool))
+                na.check(lib.nhStreamSynchronize(stream))
+            except Exception as e:  # noqa: BLE001
+                errors.append(repr(e))
+            finally:
+                lib.nhStreamDestroy(stream)
+                lib.nhPoolCleanUp(s.pool)
+
+        running = [threading.Thread(target=work, args=(i,)) for i in range(threads)]
+        for t in running:
+            t.start()
+        for t in running:
+            t.join(60)
+        assert not any(t.is_alive() for t in running)
+        assert not errors, errors
+        want = a.double() @ b.double().T + bias.double()
+        bound = (k + 40) * 2.0 ** -24 * (a.double().abs() @ b.double().abs().T + bias.double().abs())
+        for x in results:
+            assert ((x.double() - want).abs() <= bound).all()
