@@ -25,8 +25,9 @@ void noteStreamUse( hipStream_t stream );
 // Small element-wise calls that a stream has put aside ( nhStreamDeferSmallOps, vector_ops.hip ) run before anything else
 // that is asked of the stream, so they too are caught here: tinyChainsPending counts the streams that hold some.
 // flushTinyOps launches what the stream of the current device holds; flushAllTinyOps does so for every stream of every
-// device ( before device memory is given back ). releaseTinyQueue: the stream is being destroyed.
-// Inside a launch of calls that were put aside ( CHeldLaunch; launchingHeldCalls: of this thread ) both do nothing, so that the calls
+// device, and finishHeldCalls also waits for other threads that are launching such calls ( before device memory is given back ).
+// releaseTinyQueue: the stream is being destroyed.
+// Inside a launch of calls that were put aside ( CHeldLaunch, from before they leave the queue; launchingHeldCalls: of this thread ) they do nothing, so that the calls
 // behind the one that is being launched stay behind it, and a pool neither gives nor releases cached blocks: the calls' operands
 // may be among them, given back behind the calls.
 class CHeldLaunch {
@@ -40,6 +41,7 @@ bool launchingHeldCalls();
 extern int tinyChainsPending;
 bool flushTinyOps( hipStream_t stream ); // true: something was launched
 void flushAllTinyOps();
+void finishHeldCalls();
 void releaseTinyQueue( hipStream_t stream );
 // On such a stream a product A * B^T with a dense result may wait for the call behind it ( deferProduct: true, nothing
 // launched ); an AddVectorToMatrixRows over that result in place then launches both as one ( fusePendingProduct: true,

@@ -122,7 +122,7 @@ int nhRawAlloc( void** ptr, size_t size )
 int nhRawFree( void* ptr )
 {
 	if( ptr != nullptr ) {
-		flushAllTinyOps(); // a call that has been put aside may still name this block
+		finishHeldCalls(); // a call that has been put aside may still name this block
 		NH_HIP( hipFree( ptr ) );
 	}
 	return NH_OK;

@@ -10,6 +10,8 @@
 #include <float.h>
 #include <map>
 #include <mutex>
+#include <optional>
+#include <shared_mutex>
 #include <stddef.h>
 #include <type_traits>
 #include <utility>
@@ -936,8 +938,20 @@ typedef std::map<std::pair<int, hipStream_t>, CTinyQueue> CTinyQueues;
 // ( recursive: what is launched from under the lock may turn a stream handle into a stream, which looks for calls to launch )
 static std::recursive_mutex tinyLock;
 static thread_local int heldLaunches = 0;
-CHeldLaunch::CHeldLaunch() { ++heldLaunches; }
-CHeldLaunch::~CHeldLaunch() { --heldLaunches; }
+// held by the threads that have taken calls out of a queue and not launched them all yet
+static std::shared_mutex heldLaunchLock;
+CHeldLaunch::CHeldLaunch()
+{
+	if( heldLaunches++ == 0 ) {
+		heldLaunchLock.lock_shared();
+	}
+}
+CHeldLaunch::~CHeldLaunch()
+{
+	if( --heldLaunches == 0 ) {
+		heldLaunchLock.unlock_shared();
+	}
+}
 bool launchingHeldCalls() { return heldLaunches != 0; }
 static CTinyQueues& tinyQueues()
 {
@@ -1787,6 +1801,16 @@ void flushAllTinyOps()
 	}
 }
 
+// what device memory is about to be given back after: every call that any thread has been asked for so far is on its stream
+void finishHeldCalls()
+{
+	flushAllTinyOps();
+	if( !launchingHeldCalls() ) {
+		heldLaunchLock.lock();
+		heldLaunchLock.unlock();
+	}
+}
+
 // the stream is going away ( drained by the caller ): a later stream may be handed the same handle
 void releaseTinyQueue( hipStream_t stream )
 {
@@ -2109,6 +2133,7 @@ bool fusePendingPadding( nhStream s, const nhPoolingDesc& d, const float* source
 	if( found == tinyQueues().end() || !found->second.Padding.Pending || found->second.Padding.To != source ) {
 		return false; // ( the caller's own launch sends the padding out first )
 	}
+	const CHeldLaunch held;
 	const CPendingPadding p = found->second.Padding;
 	found->second.Padding.Pending = false;
 	__atomic_fetch_sub( &tinyChainsPending, 1, __ATOMIC_RELAXED );
@@ -2187,6 +2212,7 @@ bool deferBatchedProduct( nhStream s, int batch, const float* first, int height,
 static bool fusePendingBatched( nhStream s, const float* first, float* result, int count, const float* multiplier, int* rc )
 {
 	const hipStream_t stream = reinterpret_cast<hipStream_t>( s );
+	std::optional<CHeldLaunch> held;
 	CPendingAttention p;
 	{
 		std::lock_guard<std::recursive_mutex> guard( tinyLock );
@@ -2203,10 +2229,10 @@ static bool fusePendingBatched( nhStream s, const float* first, float* result, i
 			queue->Batched.Scale = multiplier;
 			return true;
 		}
+		held.emplace();
 		queue->Batched.Pending = false;
 		__atomic_fetch_sub( &tinyChainsPending, 1, __ATOMIC_RELAXED );
 	}
-	const CHeldLaunch held;
 	bool scaled = false;
 	*rc = launchBatched( stream, p, multiplier, &scaled );
 	if( __atomic_load_n( &lstmPartnersAwaited, __ATOMIC_RELAXED ) != 0 ) {
@@ -2235,6 +2261,7 @@ bool joinPendingSoftmax( nhStream s, const float* matrix, int height, int width,
 bool fusePendingTransposition( nhStream s, int batch, const float* first, int height, int medium, int width, int channels, float* result, int* rc )
 {
 	const hipStream_t stream = reinterpret_cast<hipStream_t>( s );
+	std::optional<CHeldLaunch> held;
 	CPendingAttention p;
 	{
 		std::lock_guard<std::recursive_mutex> guard( tinyLock );
@@ -2247,12 +2274,12 @@ bool fusePendingTransposition( nhStream s, int batch, const float* first, int he
 			|| !apartFrom( p, result, static_cast<long long>( p.Batch ) * p.M * p.D, true ) ) {
 			return false;
 		}
+		held.emplace();
 		queue->Batched.Pending = false;
 		__atomic_fetch_sub( &tinyChainsPending, 1, __ATOMIC_RELAXED );
 	}
 	p.Transposed = result;
 	p.Heads = height;
-	const CHeldLaunch held;
 	*rc = launchAttention( stream, p );
 	if( __atomic_load_n( &lstmPartnersAwaited, __ATOMIC_RELAXED ) != 0 ) {
 		noteStreamUse( stream );
@@ -2358,6 +2385,7 @@ static bool fusePendingSum( nhStream s, const float* first, float* result, int c
 		( void )hipGetLastError();
 		return false;
 	}
+	std::optional<CHeldLaunch> held;
 	CPendingSum sum;
 	{
 		std::lock_guard<std::recursive_mutex> guard( tinyLock );
@@ -2369,6 +2397,7 @@ static bool fusePendingSum( nhStream s, const float* first, float* result, int c
 		if( first != sum.Result || result != sum.Result || count != sum.Count ) {
 			return false; // ( the caller's own launch sends the sum out first, as it was asked for )
 		}
+		held.emplace();
 		found->second.Sum.Pending = false;
 		__atomic_fetch_sub( &tinyChainsPending, 1, __ATOMIC_RELAXED );
 	}
@@ -2435,6 +2464,7 @@ bool joinPendingConvolution( nhStream s, const float* first, const float* second
 		return false;
 	}
 	const hipStream_t stream = reinterpret_cast<hipStream_t>( s );
+	std::optional<CHeldLaunch> held;
 	CPendingConvolution shortcut, c;
 	{
 		std::lock_guard<std::recursive_mutex> guard( tinyLock );
@@ -2460,11 +2490,11 @@ bool joinPendingConvolution( nhStream s, const float* first, const float* second
 		if( other != shortcut.Result || touches( c, shortcut.Result, count ) || touches( shortcut, c.Result, count ) ) {
 			return false;
 		}
+		held.emplace();
 		queue->Convolution.Pending = false;
 		queue->Shortcut.Pending = false;
 		__atomic_fetch_sub( &tinyChainsPending, 1, __ATOMIC_RELAXED );
 	}
-	const CHeldLaunch held;
 	const CFusedActivation none = { NH_ACT_NONE, 0.f };
 	( void )launchPendingConvolution( stream, shortcut, none );
 	if( __atomic_load_n( &lstmPartnersAwaited, __ATOMIC_RELAXED ) != 0 ) {
@@ -2488,6 +2518,7 @@ bool fusePendingConvolution( nhStream s, const float* first, float* result, long
 	const float* upperThreshold, int* rc )
 {
 	const hipStream_t stream = reinterpret_cast<hipStream_t>( s );
+	std::optional<CHeldLaunch> held;
 	CPendingConvolution c, front;
 	{
 		std::lock_guard<std::recursive_mutex> guard( tinyLock );
@@ -2503,11 +2534,11 @@ bool fusePendingConvolution( nhStream s, const float* first, float* result, long
 		if( first != c.Result || result != c.Result || count != c.ResultCount() || ( activation == NH_ACT_RELU && ( upperThreshold == nullptr || rangesMeet( upperThreshold, 1, c.Result, count ) ) ) ) {
 			return false; // ( the caller's own launch sends the convolution out first, as it was asked for )
 		}
+		held.emplace();
 		queue->Convolution.Pending = false;
 		queue->Shortcut.Pending = false;
 		__atomic_fetch_sub( &tinyChainsPending, 1, __ATOMIC_RELAXED );
 	}
-	const CHeldLaunch held;
 	if( front.Pending ) {
 		const CFusedActivation none = { NH_ACT_NONE, 0.f };
 		( void )launchPendingConvolution( stream, front, none );

@@ -232,3 +232,41 @@ def test_threads_at_the_limit_of_one_pool():
         bound = (k + 40) * 2.0 ** -24 * (a.double().abs() @ b.double().abs().T + bias.double().abs())
         for x in results:
             assert ((x.double() - want).abs() <= bound).all()
+
+
+def test_another_thread_frees_what_a_waiting_call_reads():
+    """A thread may free the source of a convolution as soon as the call has returned, also while the thread that asked for it is in the call
+    behind it."""
+    import threading
+    import nhtest
+    hip = nhtest.Hip()
+    d = hip.conv_desc(2, 32, 32, 32, 64, 3, 3, 1, 1, 1, 1)
+    with Pooled(0) as s:
+        torch, lib, na = s.torch, s.lib, s.na
+        x, filt, zero = s.draw(1, 2, 32, 32, 32), s.draw(2, 64, 3, 3, 32) / 17, torch.zeros(1, device="cuda:0")
+        want, y = torch.empty(2, 32, 32, 64, device="cuda:0"), torch.empty(2, 32, 32, 64, device="cuda:0")
+        s.call(s.plain, "nhBlobConvolution", ctypes.byref(d), x, filt, None, want)
+        s.call(s.plain, "nhVectorReLU", want, want, want.numel(), zero)
+        na.check(lib.nhStreamSynchronize(s.plain))
+        errors = []
+        for _ in range(20):
+            source, asked = ctypes.c_void_p(), threading.Event()
+            na.check(lib.nhRawAlloc(ctypes.byref(source), x.numel() * 4))
+            s.call(s.plain, "nhCopyDeviceToDevice", source, x, x.numel() * 4)
+            na.check(lib.nhStreamSynchronize(s.plain))
+
+            def free():
+                asked.wait()
+                if lib.nhRawFree(source) != 0:
+                    errors.append(na.last_error())
+
+            thread = threading.Thread(target=free)
+            thread.start()
+            s.call(s.stream, "nhBlobConvolution", ctypes.byref(d), source, filt, None, y)
+            asked.set()
+            s.call(s.stream, "nhVectorReLU", y, y, y.numel(), zero)
+            na.check(lib.nhStreamSynchronize(s.stream))
+            thread.join(60)
+            assert not thread.is_alive() and not errors
+            # ( sent out with its ReLU or in front of it: the same convolution, the same bits )
+            assert torch.equal(y.view(torch.int32), want.view(torch.int32))
