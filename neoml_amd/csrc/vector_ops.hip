@@ -886,6 +886,7 @@ struct CTinyQueue {
 		return ( Product.Pending && !ProductParked ) || Convolution.Pending || Sum.Pending || Batched.Pending || Padding.Pending || ColumnSum.Pending
 			|| Transpositions.Length > 0;
 	}
+	bool Holds() const { return Chain.Length != 0 || ParkedCount != 0 || Product.Pending || LaunchWaits(); }
 };
 
 static int launchPlainSum( hipStream_t stream, const CPendingSum& sum );
@@ -960,6 +961,17 @@ static CTinyQueues& tinyQueues()
 }
 int tinyChainsPending = 0;
 static int tinyDeferringStreams = 0;
+// streams on which a product, a convolution, a batch of products waits: calls that such a one may take along ask here before they ask for
+// the device and the lock ( 75 ns )
+static int productsWaiting = 0, convolutionsWaiting = 0, batchesWaiting = 0;
+static void setWaiting( bool& pending, int& count, bool value )
+{
+	if( pending != value ) {
+		pending = value;
+		__atomic_fetch_add( &count, value ? 1 : -1, __ATOMIC_RELAXED );
+	}
+}
+static bool someWait( const int& count ) { return __atomic_load_n( &count, __ATOMIC_RELAXED ) != 0; }
 
 // With tinyLock held and the queue's device current. true: something was launched ( telling a stream's one-launch LSTMs
 // about it, noteStreamUse, is left to the callers: that takes a lock that a caller of toStream may hold ).
@@ -1192,7 +1204,7 @@ static bool launchPendingProduct( hipStream_t stream, CTinyQueue& queue )
 		products[count] = queue.Siblings[count];
 	}
 	products[count++] = queue.Product;
-	queue.Product.Pending = false;
+	setWaiting( queue.Product.Pending, productsWaiting, false );
 	queue.ProductParked = false;
 	queue.SiblingCount = 0;
 	__atomic_fetch_sub( &tinyChainsPending, 1, __ATOMIC_RELAXED );
@@ -1697,7 +1709,7 @@ static bool launchPending( hipStream_t stream, CTinyQueue& queue )
 	}
 	if( queue.Convolution.Pending ) {
 		const CPendingConvolution c = queue.Convolution, shortcut = queue.Shortcut;
-		queue.Convolution.Pending = false;
+		setWaiting( queue.Convolution.Pending, convolutionsWaiting, false );
 		queue.Shortcut.Pending = false;
 		__atomic_fetch_sub( &tinyChainsPending, 1, __ATOMIC_RELAXED );
 		const CFusedActivation none = { NH_ACT_NONE, 0.f };
@@ -1709,7 +1721,7 @@ static bool launchPending( hipStream_t stream, CTinyQueue& queue )
 	}
 	if( queue.Batched.Pending ) {
 		const CPendingAttention p = queue.Batched;
-		queue.Batched.Pending = false;
+		setWaiting( queue.Batched.Pending, batchesWaiting, false );
 		__atomic_fetch_sub( &tinyChainsPending, 1, __ATOMIC_RELAXED );
 		( void )launchPendingAttention( stream, p );
 		return true;
@@ -1750,7 +1762,7 @@ bool flushTinyOps( hipStream_t stream )
 	}
 	std::lock_guard<std::recursive_mutex> guard( tinyLock );
 	auto found = tinyQueues().find( std::make_pair( device, stream ) );
-	return found != tinyQueues().end() && launchPending( stream, found->second );
+	return found != tinyQueues().end() && found->second.Holds() && launchPending( stream, found->second );
 }
 
 void flushAllTinyOps()
@@ -1769,7 +1781,7 @@ void flushAllTinyOps()
 	{
 		std::lock_guard<std::recursive_mutex> guard( tinyLock );
 		for( auto& entry : tinyQueues() ) {
-			if( entry.second.Chain.Length == 0 && entry.second.ParkedCount == 0 && !entry.second.Product.Pending && !entry.second.LaunchWaits() ) {
+			if( !entry.second.Holds() ) {
 				continue;
 			}
 			if( entry.first.first != active ) {
@@ -1842,6 +1854,46 @@ static CTinyQueue* deferringQueue( hipStream_t stream )
 	return found != tinyQueues().end() && found->second.Enabled ? &found->second : nullptr;
 }
 
+// A call joins what waits on its stream only where the stream is not being recorded into a graph: what joined would be missing from the graph and
+// would run once, behind it. ( What waits goes out as the graph's first launch then, through toStream. Asked for where the call is found to be the
+// one that is waited for, not in every call. )
+static bool recorded( hipStream_t stream )
+{
+	hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+	if( hipStreamIsCapturing( stream, &capture ) != hipSuccess ) {
+		( void )hipGetLastError();
+		return true;
+	}
+	return capture != hipStreamCaptureStatusNone;
+}
+
+// The queue of the stream with nothing in it, what it held sent out, for a call that may begin to wait there; null: none ( a stream that puts
+// no calls aside, or that is being recorded ). Locked by guard. One question for the device and one for the recording, 50 ns each, in place
+// of one for every step.
+static CTinyQueue* emptiedQueue( nhStream s, std::unique_lock<std::recursive_mutex>& guard )
+{
+	const hipStream_t stream = reinterpret_cast<hipStream_t>( s );
+	guard = std::unique_lock<std::recursive_mutex>( tinyLock );
+	CTinyQueue* queue = deferringQueue( stream );
+	if( queue == nullptr || launchingHeldCalls() ) {
+		return nullptr;
+	}
+	if( queue->Holds() ) {
+		launchPending( stream, *queue );
+	}
+	if( __atomic_load_n( &lstmPartnersAwaited, __ATOMIC_RELAXED ) != 0 || __atomic_load_n( &sliceScratchWanted, __ATOMIC_RELAXED ) != 0 ) {
+		guard.unlock(); // ( neither is asked for with the lock held )
+		if( __atomic_load_n( &lstmPartnersAwaited, __ATOMIC_RELAXED ) != 0 ) {
+			noteStreamUse( stream );
+		}
+		if( __atomic_load_n( &sliceScratchWanted, __ATOMIC_RELAXED ) != 0 ) {
+			growWantedScratch( stream );
+		}
+		guard.lock();
+	}
+	return recorded( stream ) || queue->Holds() ? nullptr : queue;
+}
+
 constexpr long long MaxGroupedProduct = 1 << 18; // ( values of a result: what the kernel for few tiles may take three of )
 
 bool deferProduct( nhStream s, const float* a, int lda, const float* b, int ldb, float* c, int ldc, int M, int N, int K )
@@ -1849,7 +1901,7 @@ bool deferProduct( nhStream s, const float* a, int lda, const float* b, int ldb,
 	if( __atomic_load_n( &tinyDeferringStreams, __ATOMIC_RELAXED ) == 0 || M <= 0 || N <= 0 || K <= 0 || ldc != N ) {
 		return false;
 	}
-	if( static_cast<long long>( M ) * N <= MaxGroupedProduct && __atomic_load_n( &tinyChainsPending, __ATOMIC_RELAXED ) != 0 ) {
+	if( static_cast<long long>( M ) * N <= MaxGroupedProduct && someWait( productsWaiting ) ) {
 		// a product of the same A that waits with its free term: the two wait on, apart from each other as they must be
 		std::lock_guard<std::recursive_mutex> guard( tinyLock );
 		CTinyQueue* queue = deferringQueue( reinterpret_cast<hipStream_t>( s ) );
@@ -1864,7 +1916,7 @@ bool deferProduct( nhStream s, const float* a, int lda, const float* b, int ldb,
 				joins = !rangesMeet( c, sizeC, other.C, sizeC ) && !rangesMeet( c, sizeC, other.B, sizeB ) && !rangesMeet( c, sizeC, other.Bias, N )
 					&& !rangesMeet( b, sizeB, other.C, sizeC ) && !rangesMeet( a, sizeA, other.C, sizeC );
 			}
-			if( joins ) {
+			if( joins && !recorded( reinterpret_cast<hipStream_t>( s ) ) ) {
 				queue->Siblings[queue->SiblingCount++] = last;
 				CPendingProduct& p = queue->Product;
 				p.B = b; p.C = c; p.Bias = nullptr; // ( one thing waits where one waited )
@@ -1872,29 +1924,15 @@ bool deferProduct( nhStream s, const float* a, int lda, const float* b, int ldb,
 			}
 		}
 	}
-	const hipStream_t stream = toStream( s ); // ( what the stream holds goes out first )
-	int device = 0;
-	hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-	if( hipGetDevice( &device ) != hipSuccess || hipStreamIsCapturing( stream, &capture ) != hipSuccess ) {
-		( void )hipGetLastError();
+	std::unique_lock<std::recursive_mutex> guard;
+	CTinyQueue* queue = emptiedQueue( s, guard );
+	if( queue == nullptr ) {
 		return false;
 	}
-	if( capture != hipStreamCaptureStatusNone ) {
-		return false;
-	}
-	if( __atomic_load_n( &sliceScratchWanted, __ATOMIC_RELAXED ) != 0 ) {
-		growWantedScratch( stream );
-	}
-	std::lock_guard<std::recursive_mutex> guard( tinyLock );
-	auto found = tinyQueues().find( std::make_pair( device, stream ) );
-	if( found == tinyQueues().end() || !found->second.Enabled || found->second.Chain.Length != 0 || found->second.LaunchWaits() )
-	{
-		return false;
-	}
-	CPendingProduct& p = found->second.Product;
+	CPendingProduct& p = queue->Product;
 	p = CPendingProduct();
-	found->second.SiblingCount = 0;
-	p.Pending = true;
+	queue->SiblingCount = 0;
+	setWaiting( p.Pending, productsWaiting, true );
 	p.A = a; p.Lda = lda; p.B = b; p.Ldb = ldb; p.C = c; p.Ldc = ldc; p.M = M; p.N = N; p.K = K;
 	__atomic_fetch_add( &tinyChainsPending, 1, __ATOMIC_RELAXED );
 	return true;
@@ -1903,6 +1941,9 @@ bool deferProduct( nhStream s, const float* a, int lda, const float* b, int ldb,
 // AddVectorToMatrixRows asks whether it is the free term of a product that waits: true, the product waits on with it
 bool fusePendingProduct( nhStream s, const float* matrix, float* result, int height, int width, const float* vector, int* rc )
 {
+	if( !someWait( productsWaiting ) ) {
+		return false;
+	}
 	std::lock_guard<std::recursive_mutex> guard( tinyLock );
 	CTinyQueue* queue = deferringQueue( reinterpret_cast<hipStream_t>( s ) );
 	if( queue == nullptr || !queue->Product.Pending || queue->ProductParked || queue->Product.Bias != nullptr ) {
@@ -1917,6 +1958,9 @@ bool fusePendingProduct( nhStream s, const float* matrix, float* result, int hei
 		if( rangesMeet( vector, width, queue->Siblings[i].C, static_cast<long long>( height ) * width ) ) {
 			return false;
 		}
+	}
+	if( recorded( reinterpret_cast<hipStream_t>( s ) ) ) {
+		return false;
 	}
 	p.Bias = vector;
 	*rc = NH_OK;
@@ -1959,7 +2003,7 @@ static bool launchGatedProduct( hipStream_t stream, CTinyQueue& queue )
 	if( !matMulNTGated( stream, p.A, p.Lda, p.B, p.Ldb, p.C, p.Ldc, p.M, p.N, p.K, p.Bias, t, op[0].Scalar, &rc ) ) {
 		return false;
 	}
-	queue.Product.Pending = false;
+	setWaiting( queue.Product.Pending, productsWaiting, false );
 	queue.ProductParked = false;
 	chain.Length = 0;
 	__atomic_fetch_sub( &tinyChainsPending, 2, __ATOMIC_RELAXED );
@@ -1985,7 +2029,8 @@ bool deferColumnSum( nhStream s, float* result, const float* matrix, int height,
 			const CPendingSum added = waiting->second.Sum;
 			const float* resultEnd = result + height;
 			const bool apart = resultEnd <= added.Result || added.Result + added.Count <= result;
-			if( added.Result == matrix && static_cast<long long>( added.Count ) == static_cast<long long>( height ) * width && apart ) {
+			if( added.Result == matrix && static_cast<long long>( added.Count ) == static_cast<long long>( height ) * width && apart
+				&& !recorded( reinterpret_cast<hipStream_t>( s ) ) ) {
 				waiting->second.Sum.Pending = false; // ( one thing waits where one waited: the count of waiting queues stays )
 				CPendingColumnSum& sum = waiting->second.ColumnSum;
 				sum.Pending = true;
@@ -2005,7 +2050,8 @@ bool deferColumnSum( nhStream s, float* result, const float* matrix, int height,
 			const float* resultEnd = result + height;
 			auto apart = [&]( const float* p ) { return resultEnd <= p || p + count <= result; };
 			if( added.Kind == CKindOf<CAddOp<float>, CTinyKinds>::Value && added.Spread == TS_None && added.Out == matrix
-				&& added.Count == count && apart( added.Out ) && apart( added.In[0] ) && apart( added.In[1] ) ) {
+				&& added.Count == count && apart( added.Out ) && apart( added.In[0] ) && apart( added.In[1] )
+				&& !recorded( reinterpret_cast<hipStream_t>( s ) ) ) {
 				CPendingColumnSum& sum = waiting->second.ColumnSum;
 				sum.Pending = true;
 				sum.Result = result; sum.Matrix = matrix; sum.Height = height; sum.Width = width; sum.ColumnsOf = 0;
@@ -2028,7 +2074,7 @@ bool deferColumnSum( nhStream s, float* result, const float* matrix, int height,
 			if( centre.Kind == CKindOf<CAddOp<float>, CTinyKinds>::Value && square.Kind == CKindOf<CMulOp<float>, CTinyKinds>::Value
 				&& centre.Spread == TS_PerRow && square.Spread == TS_None && centre.Width == width && centre.Count == count
 				&& square.Count == count && centre.Out == matrix && square.In[0] == matrix && square.In[1] == matrix && square.Out == matrix
-				&& centre.Barrier == 0 && square.Barrier == 0 && apart ) {
+				&& centre.Barrier == 0 && square.Barrier == 0 && apart && !recorded( reinterpret_cast<hipStream_t>( s ) ) ) {
 				CPendingColumnSum& sum = waiting->second.ColumnSum;
 				sum.Pending = true;
 				sum.Result = result; sum.Matrix = matrix; sum.Height = height; sum.Width = width; sum.ColumnsOf = 0;
@@ -2039,22 +2085,12 @@ bool deferColumnSum( nhStream s, float* result, const float* matrix, int height,
 			}
 		}
 	}
-	const hipStream_t stream = toStream( s ); // ( what the stream holds goes out first )
-	int device = 0;
-	hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-	if( hipGetDevice( &device ) != hipSuccess || hipStreamIsCapturing( stream, &capture ) != hipSuccess ) {
-		( void )hipGetLastError();
+	std::unique_lock<std::recursive_mutex> guard;
+	CTinyQueue* queue = emptiedQueue( s, guard );
+	if( queue == nullptr ) {
 		return false;
 	}
-	if( capture != hipStreamCaptureStatusNone ) {
-		return false;
-	}
-	std::lock_guard<std::recursive_mutex> guard( tinyLock );
-	auto found = tinyQueues().find( std::make_pair( device, stream ) );
-	if( found == tinyQueues().end() || !found->second.Enabled || found->second.Chain.Length != 0 || found->second.LaunchWaits() ) {
-		return false;
-	}
-	CPendingColumnSum& sum = found->second.ColumnSum;
+	CPendingColumnSum& sum = queue->ColumnSum;
 	sum.Pending = true;
 	sum.Result = result; sum.Matrix = matrix; sum.Height = height; sum.Width = width; sum.ColumnsOf = 0;
 	sum.AddFirst = nullptr; sum.AddSecond = nullptr;
@@ -2070,22 +2106,12 @@ bool deferRowSums( nhStream s, int batch, float* result, const float* matrix, in
 		|| static_cast<long long>( batch ) * width > 0x7fffffffLL ) {
 		return false;
 	}
-	const hipStream_t stream = toStream( s ); // ( what the stream holds goes out first )
-	int device = 0;
-	hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-	if( hipGetDevice( &device ) != hipSuccess || hipStreamIsCapturing( stream, &capture ) != hipSuccess ) {
-		( void )hipGetLastError();
+	std::unique_lock<std::recursive_mutex> guard;
+	CTinyQueue* queue = emptiedQueue( s, guard );
+	if( queue == nullptr ) {
 		return false;
 	}
-	if( capture != hipStreamCaptureStatusNone ) {
-		return false;
-	}
-	std::lock_guard<std::recursive_mutex> guard( tinyLock );
-	auto found = tinyQueues().find( std::make_pair( device, stream ) );
-	if( found == tinyQueues().end() || !found->second.Enabled || found->second.Chain.Length != 0 || found->second.LaunchWaits() ) {
-		return false;
-	}
-	CPendingColumnSum& sum = found->second.ColumnSum;
+	CPendingColumnSum& sum = queue->ColumnSum;
 	sum = CPendingColumnSum();
 	sum.Pending = true;
 	sum.Result = result; sum.Matrix = matrix; sum.Height = height; sum.Width = width; sum.ColumnsOf = batch;
@@ -2098,23 +2124,13 @@ bool deferPadding( nhStream s, const CPendingPadding& padding )
 	if( __atomic_load_n( &tinyDeferringStreams, __ATOMIC_RELAXED ) == 0 ) {
 		return false;
 	}
-	const hipStream_t stream = toStream( s ); // ( what the stream holds goes out first )
-	int device = 0;
-	hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-	if( hipGetDevice( &device ) != hipSuccess || hipStreamIsCapturing( stream, &capture ) != hipSuccess ) {
-		( void )hipGetLastError();
+	std::unique_lock<std::recursive_mutex> guard;
+	CTinyQueue* queue = emptiedQueue( s, guard );
+	if( queue == nullptr ) {
 		return false;
 	}
-	if( capture != hipStreamCaptureStatusNone ) {
-		return false;
-	}
-	std::lock_guard<std::recursive_mutex> guard( tinyLock );
-	auto found = tinyQueues().find( std::make_pair( device, stream ) );
-	if( found == tinyQueues().end() || !found->second.Enabled || found->second.Chain.Length != 0 || found->second.LaunchWaits() ) {
-		return false;
-	}
-	found->second.Padding = padding;
-	found->second.Padding.Pending = true;
+	queue->Padding = padding;
+	queue->Padding.Pending = true;
 	__atomic_fetch_add( &tinyChainsPending, 1, __ATOMIC_RELAXED );
 	return true;
 }
@@ -2163,7 +2179,7 @@ bool deferBatchedProduct( nhStream s, int batch, const float* first, int height,
 		|| static_cast<long long>( batch ) * height * secondWidth > 0x7fffffffLL ) {
 		return false;
 	}
-	if( __atomic_load_n( &tinyChainsPending, __ATOMIC_RELAXED ) != 0 ) {
+	if( someWait( batchesWaiting ) ) {
 		// the product of the weights that wait and their values
 		std::lock_guard<std::recursive_mutex> guard( tinyLock );
 		CTinyQueue* queue = deferringQueue( reinterpret_cast<hipStream_t>( s ) );
@@ -2172,7 +2188,8 @@ bool deferBatchedProduct( nhStream s, int batch, const float* first, int height,
 			if( first == p.Weights && batch == p.Batch && height == p.M && width == p.N
 				&& attentionTakes( batch, p.M, p.N, p.K, secondWidth, p.Q ) && apartFrom( p, second, static_cast<long long>( batch ) * width * secondWidth, false )
 				&& apartFrom( p, result, static_cast<long long>( batch ) * height * secondWidth, true )
-				&& !rangesMeet( second, static_cast<long long>( batch ) * width * secondWidth, result, static_cast<long long>( batch ) * height * secondWidth ) ) {
+				&& !rangesMeet( second, static_cast<long long>( batch ) * width * secondWidth, result, static_cast<long long>( batch ) * height * secondWidth )
+				&& !recorded( reinterpret_cast<hipStream_t>( s ) ) ) {
 				p.V = second;
 				p.D = secondWidth;
 				p.Context = result;
@@ -2183,23 +2200,14 @@ bool deferBatchedProduct( nhStream s, int batch, const float* first, int height,
 	if( width > 256 || ( batch < 2 && !attentionTakes( batch, height, secondWidth, width, 64, first ) ) ) {
 		return false;
 	}
-	const hipStream_t stream = toStream( s ); // ( what the stream holds goes out first )
-	hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-	if( hipStreamIsCapturing( stream, &capture ) != hipSuccess ) {
-		( void )hipGetLastError();
-		return false;
-	}
-	if( capture != hipStreamCaptureStatusNone ) {
-		return false;
-	}
-	std::lock_guard<std::recursive_mutex> guard( tinyLock );
-	CTinyQueue* queue = deferringQueue( stream );
-	if( queue == nullptr || queue->Chain.Length != 0 || queue->LaunchWaits() ) {
+	std::unique_lock<std::recursive_mutex> guard;
+	CTinyQueue* queue = emptiedQueue( s, guard );
+	if( queue == nullptr ) {
 		return false;
 	}
 	CPendingAttention& p = queue->Batched;
 	p = CPendingAttention();
-	p.Pending = true;
+	setWaiting( p.Pending, batchesWaiting, true );
 	p.Q = first; p.KT = second; p.Scores = result; p.Batch = batch; p.M = height; p.N = secondWidth; p.K = width;
 	__atomic_fetch_add( &tinyChainsPending, 1, __ATOMIC_RELAXED );
 	return true;
@@ -2211,6 +2219,9 @@ bool deferBatchedProduct( nhStream s, int batch, const float* first, int height,
 // first ).
 static bool fusePendingBatched( nhStream s, const float* first, float* result, int count, const float* multiplier, int* rc )
 {
+	if( !someWait( batchesWaiting ) ) {
+		return false;
+	}
 	const hipStream_t stream = reinterpret_cast<hipStream_t>( s );
 	std::optional<CHeldLaunch> held;
 	CPendingAttention p;
@@ -2225,12 +2236,12 @@ static bool fusePendingBatched( nhStream s, const float* first, float* result, i
 			|| static_cast<long long>( count ) != static_cast<long long>( p.Batch ) * p.M * p.N ) {
 			return false;
 		}
-		if( attentionTakes( p.Batch, p.M, p.N, p.K, 64, p.Q ) && apartFrom( p, multiplier, 1, false ) ) {
+		if( attentionTakes( p.Batch, p.M, p.N, p.K, 64, p.Q ) && apartFrom( p, multiplier, 1, false ) && !recorded( stream ) ) {
 			queue->Batched.Scale = multiplier;
 			return true;
 		}
 		held.emplace();
-		queue->Batched.Pending = false;
+		setWaiting( queue->Batched.Pending, batchesWaiting, false );
 		__atomic_fetch_sub( &tinyChainsPending, 1, __ATOMIC_RELAXED );
 	}
 	bool scaled = false;
@@ -2243,6 +2254,9 @@ static bool fusePendingBatched( nhStream s, const float* first, float* result, i
 
 bool joinPendingSoftmax( nhStream s, const float* matrix, int height, int width, float* result )
 {
+	if( !someWait( batchesWaiting ) ) {
+		return false;
+	}
 	std::lock_guard<std::recursive_mutex> guard( tinyLock );
 	CTinyQueue* queue = deferringQueue( reinterpret_cast<hipStream_t>( s ) );
 	if( queue == nullptr || !queue->Batched.Pending || queue->Batched.Weights != nullptr || result == nullptr ) {
@@ -2251,7 +2265,7 @@ bool joinPendingSoftmax( nhStream s, const float* matrix, int height, int width,
 	CPendingAttention& p = queue->Batched;
 	const long long count = static_cast<long long>( height ) * width;
 	if( matrix != p.Scores || width != p.N || height != static_cast<long long>( p.Batch ) * p.M || !attentionTakes( p.Batch, p.M, p.N, p.K, 64, p.Q )
-		|| !apartFrom( p, result, count, true ) ) {
+		|| !apartFrom( p, result, count, true ) || recorded( reinterpret_cast<hipStream_t>( s ) ) ) {
 		return false;
 	}
 	p.Weights = result;
@@ -2260,6 +2274,9 @@ bool joinPendingSoftmax( nhStream s, const float* matrix, int height, int width,
 
 bool fusePendingTransposition( nhStream s, int batch, const float* first, int height, int medium, int width, int channels, float* result, int* rc )
 {
+	if( !someWait( batchesWaiting ) ) {
+		return false;
+	}
 	const hipStream_t stream = reinterpret_cast<hipStream_t>( s );
 	std::optional<CHeldLaunch> held;
 	CPendingAttention p;
@@ -2275,7 +2292,7 @@ bool fusePendingTransposition( nhStream s, int batch, const float* first, int he
 			return false;
 		}
 		held.emplace();
-		queue->Batched.Pending = false;
+		setWaiting( queue->Batched.Pending, batchesWaiting, false );
 		__atomic_fetch_sub( &tinyChainsPending, 1, __ATOMIC_RELAXED );
 	}
 	p.Transposed = result;
@@ -2303,24 +2320,15 @@ bool deferTransposition( nhStream s, const CTransposition& t )
 				joins = !rangesMeet( t.To, t.Count, other.To, other.Count ) && !rangesMeet( t.To, t.Count, other.From, other.Count )
 					&& !rangesMeet( t.From, t.Count, other.To, other.Count );
 			}
-			if( joins ) {
+			if( joins && !recorded( reinterpret_cast<hipStream_t>( s ) ) ) {
 				waiting.Items[waiting.Length++] = t; // ( one thing waits where one waited )
 				return true;
 			}
 		}
 	}
-	const hipStream_t stream = toStream( s ); // ( what the stream holds goes out first )
-	hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-	if( hipStreamIsCapturing( stream, &capture ) != hipSuccess ) {
-		( void )hipGetLastError();
-		return false;
-	}
-	if( capture != hipStreamCaptureStatusNone ) {
-		return false;
-	}
-	std::lock_guard<std::recursive_mutex> guard( tinyLock );
-	CTinyQueue* queue = deferringQueue( stream );
-	if( queue == nullptr || queue->Chain.Length != 0 || queue->LaunchWaits() ) {
+	std::unique_lock<std::recursive_mutex> guard;
+	CTinyQueue* queue = emptiedQueue( s, guard );
+	if( queue == nullptr ) {
 		return false;
 	}
 	queue->Transpositions.Items[0] = t;
@@ -2355,22 +2363,12 @@ static bool deferSum( nhStream s, const float* first, const float* second, float
 			return false;
 		}
 	}
-	const hipStream_t stream = toStream( s ); // ( what the stream holds goes out first )
-	int device = 0;
-	hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-	if( hipGetDevice( &device ) != hipSuccess || hipStreamIsCapturing( stream, &capture ) != hipSuccess ) {
-		( void )hipGetLastError();
+	std::unique_lock<std::recursive_mutex> guard;
+	CTinyQueue* queue = emptiedQueue( s, guard );
+	if( queue == nullptr ) {
 		return false;
 	}
-	if( capture != hipStreamCaptureStatusNone ) {
-		return false;
-	}
-	std::lock_guard<std::recursive_mutex> guard( tinyLock );
-	auto found = tinyQueues().find( std::make_pair( device, stream ) );
-	if( found == tinyQueues().end() || !found->second.Enabled || found->second.Chain.Length != 0 || found->second.LaunchWaits() ) {
-		return false;
-	}
-	CPendingSum& sum = found->second.Sum;
+	CPendingSum& sum = queue->Sum;
 	sum.Pending = true;
 	sum.First = first; sum.Second = second; sum.Result = result; sum.Count = count;
 	__atomic_fetch_add( &tinyChainsPending, 1, __ATOMIC_RELAXED );
@@ -2406,6 +2404,14 @@ static bool fusePendingSum( nhStream s, const float* first, float* result, int c
 	return true;
 }
 
+// ( where none waits )
+static void setConvolution( CTinyQueue& queue, const CPendingConvolution& c )
+{
+	queue.Convolution = c;
+	queue.Convolution.Pending = false;
+	setWaiting( queue.Convolution.Pending, convolutionsWaiting, true );
+}
+
 // whether the convolution reads or writes any of these values
 static bool touches( const CPendingConvolution& c, const float* p, long long count )
 {
@@ -2426,33 +2432,21 @@ bool deferConvolution( nhStream s, bool channelwise, const nhConvDesc& d, const 
 	c.Channelwise = channelwise;
 	c.Desc = d;
 	c.Source = source; c.Filter = filter; c.FreeTerm = freeTerm; c.Result = result;
-	if( !channelwise && __atomic_load_n( &tinyChainsPending, __ATOMIC_RELAXED ) != 0 ) {
+	if( !channelwise && someWait( convolutionsWaiting ) ) {
 		std::lock_guard<std::recursive_mutex> guard( tinyLock );
 		CTinyQueue* queue = deferringQueue( reinterpret_cast<hipStream_t>( s ) );
 		if( queue != nullptr && queue->Convolution.Pending && !queue->Convolution.Channelwise && queue->Convolution.Residual == nullptr
-			&& !queue->Shortcut.Pending && queue->Convolution.ResultCount() == c.ResultCount() ) {
+			&& !queue->Shortcut.Pending && queue->Convolution.ResultCount() == c.ResultCount() && !recorded( reinterpret_cast<hipStream_t>( s ) ) ) {
 			queue->Shortcut = c;
 			return true;
 		}
 	}
-	const hipStream_t stream = toStream( s ); // ( what the stream holds goes out first )
-	hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-	if( hipStreamIsCapturing( stream, &capture ) != hipSuccess ) {
-		( void )hipGetLastError();
+	std::unique_lock<std::recursive_mutex> guard;
+	CTinyQueue* queue = emptiedQueue( s, guard );
+	if( queue == nullptr ) {
 		return false;
 	}
-	if( capture != hipStreamCaptureStatusNone ) {
-		return false;
-	}
-	if( __atomic_load_n( &sliceScratchWanted, __ATOMIC_RELAXED ) != 0 ) {
-		growWantedScratch( stream );
-	}
-	std::lock_guard<std::recursive_mutex> guard( tinyLock );
-	CTinyQueue* queue = deferringQueue( stream );
-	if( queue == nullptr || queue->Chain.Length != 0 || queue->LaunchWaits() ) {
-		return false;
-	}
-	queue->Convolution = c;
+	setConvolution( *queue, c );
 	queue->Shortcut.Pending = false;
 	__atomic_fetch_add( &tinyChainsPending, 1, __ATOMIC_RELAXED );
 	return true;
@@ -2460,7 +2454,7 @@ bool deferConvolution( nhStream s, bool channelwise, const nhConvDesc& d, const 
 
 bool joinPendingConvolution( nhStream s, const float* first, const float* second, float* result, long long count )
 {
-	if( first == nullptr || second == nullptr || result == nullptr || first == second ) {
+	if( !someWait( convolutionsWaiting ) || first == nullptr || second == nullptr || result == nullptr || first == second ) {
 		return false;
 	}
 	const hipStream_t stream = reinterpret_cast<hipStream_t>( s );
@@ -2479,7 +2473,7 @@ bool joinPendingConvolution( nhStream s, const float* first, const float* second
 		}
 		const float* other = first == c.Result ? second : first;
 		if( ( first != c.Result && second != c.Result ) || result != c.Result || count != c.ResultCount()
-			|| rangesMeet( other, count, c.Result, count ) ) {
+			|| rangesMeet( other, count, c.Result, count ) || recorded( stream ) ) {
 			return false; // ( the caller's own launch sends the convolutions out first, as they were asked for )
 		}
 		if( !shortcut.Pending ) {
@@ -2491,7 +2485,7 @@ bool joinPendingConvolution( nhStream s, const float* first, const float* second
 			return false;
 		}
 		held.emplace();
-		queue->Convolution.Pending = false;
+		setWaiting( queue->Convolution.Pending, convolutionsWaiting, false );
 		queue->Shortcut.Pending = false;
 		__atomic_fetch_sub( &tinyChainsPending, 1, __ATOMIC_RELAXED );
 	}
@@ -2505,7 +2499,7 @@ bool joinPendingConvolution( nhStream s, const float* first, const float* second
 		std::lock_guard<std::recursive_mutex> guard( tinyLock );
 		CTinyQueue* queue = deferringQueue( stream );
 		if( queue != nullptr && queue->Chain.Length == 0 && !queue->LaunchWaits() ) {
-			queue->Convolution = c;
+			setConvolution( *queue, c );
 			__atomic_fetch_add( &tinyChainsPending, 1, __ATOMIC_RELAXED );
 			return true;
 		}
@@ -2517,6 +2511,9 @@ bool joinPendingConvolution( nhStream s, const float* first, const float* second
 bool fusePendingConvolution( nhStream s, const float* first, float* result, long long count, int activation,
 	const float* upperThreshold, int* rc )
 {
+	if( !someWait( convolutionsWaiting ) ) {
+		return false;
+	}
 	const hipStream_t stream = reinterpret_cast<hipStream_t>( s );
 	std::optional<CHeldLaunch> held;
 	CPendingConvolution c, front;
@@ -2535,7 +2532,7 @@ bool fusePendingConvolution( nhStream s, const float* first, float* result, long
 			return false; // ( the caller's own launch sends the convolution out first, as it was asked for )
 		}
 		held.emplace();
-		queue->Convolution.Pending = false;
+		setWaiting( queue->Convolution.Pending, convolutionsWaiting, false );
 		queue->Shortcut.Pending = false;
 		__atomic_fetch_sub( &tinyChainsPending, 1, __ATOMIC_RELAXED );
 	}
