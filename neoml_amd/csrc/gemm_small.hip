@@ -408,14 +408,15 @@ static double tilesCost( int M, int N, int K, int batch, bool convolution )
 // of the other kernels win: 9 x 12 x 14 x 256 3 x 3 22 and 26 us, 410 x 1121 x 832 14.7 and 16.9.
 static void chooseSmall( const CMatMulArgs& args, bool convolution, int batch, int waves, int maxSlices, int& tile, int& slices )
 {
-	const int groups = ceilDiv( args.K, 16 );
+	const int perWave = ceilDiv( ceilDiv( args.K, 16 ), waves );
 	tile = -1;
 	double cost = tilesCost( args.M, args.N, args.K, batch, convolution );
 	for( int t = 0; t < SmallTiles; ++t ) {
 		const long long tiles = static_cast<long long>( ceilDiv( args.M, SmallTileM[t] ) ) * ceilDiv( args.N, SmallTileN[t] ) * batch;
-		for( int s = 1; s <= maxSlices && tiles * s <= MaxSmallWorkgroups; ++s ) {
-			const int share = ceilDiv( groups, static_cast<long long>( s ) * waves );
-			if( ceilDiv( groups, static_cast<long long>( share ) * waves ) != s ) {
+		// ( a slice's share in groups to each of its wavefronts; beyond perWave slices some would have none )
+		for( int s = 1; s <= maxSlices && s <= perWave && tiles * s <= MaxSmallWorkgroups; ++s ) {
+			const int share = ( perWave + s - 1 ) / s;
+			if( ( perWave + share - 1 ) / share != s ) {
 				continue; // ( fewer slices have the same share )
 			}
 			const double c = smallCost( t, waves, share, s, tiles, convolution );
