@@ -316,10 +316,11 @@ NH_API int nhBlobConvolution(nhStream s, const nhConvDesc* desc_host, const floa
 
 /* nhBlobConvolution for callers that cannot allocate device memory: code recording a HIP graph, serving loops and
  * harnesses that forbid hipMalloc. No counterpart in the reference. Same arguments and results as nhBlobConvolution
- * (bit for bit: the same kernels and the same summation order). Where nhBlobConvolution lets the K slices of a launch
+ * (bit for bit: the same kernels and the same summation order; not for large pointwise convolutions, whose split in three
+ * needs scratch of the stream's own). Where nhBlobConvolution lets the K slices of a launch
  * meet in a block it allocates per stream, this one uses a fixed array inside the library's device image: it never
  * calls hipMalloc / hipFree, also not while the stream is being captured (its counters are cleared by a fill kernel).
- * Limits: the partial tiles of one launch (sliced tiles x slices x 16 KiB) must fit NH_NOALLOC_SCRATCH_BYTES and the
+ * Limits: the partial tiles of one launch (sliced tiles x slices x at most 16 KiB) must fit NH_NOALLOC_SCRATCH_BYTES and the
  * sliced tiles NH_NOALLOC_MAX_SLICED_TILES, otherwise NH_ERR_ARGUMENT and nothing is launched (the ResNet-18 stages at
  * batch 64 need up to 38.5 MB). Every GPU the library runs on holds its own copy of the array until the process ends.
  * All calls on one GPU share that copy: calls that may overlap there (different streams, replays of graphs recorded

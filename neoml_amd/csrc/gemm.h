@@ -122,6 +122,9 @@ struct CSliceMeeting {
 	size_t CounterCount;
 };
 
+// The counters of such a place are whatever the last call left there: cleared on the stream in front of each launch.
+void clearCounters( hipStream_t stream, unsigned* counters, size_t count );
+
 // ( gemm_small.hip ) the same for results of a few tiles; A also as the im2col view of an image whose channel count is a multiple
 // of 16. fixedMeeting: where its slices meet ( none if they would not fit ) instead of the stream's block.
 constexpr int MaxSmallSlices = 16;

@@ -1380,6 +1380,12 @@ __global__ __launch_bounds__( 256 ) void clearCountersKernel( unsigned* counters
 	}
 }
 
+void clearCounters( hipStream_t stream, unsigned* counters, size_t count )
+{
+	hipLaunchKernelGGL( clearCountersKernel, dim3( ceilDiv( static_cast<long long>( count ), 1024 ) ), dim3( 256 ), 0, stream, counters,
+		static_cast<int>( count ) );
+}
+
 // C[b][m][n] = bias[n] (or 0): the starting value that the K slices add their partial products to
 __global__ __launch_bounds__( 256 ) void presetResultKernel( float* c, const float* bias, int M, int N, int ldc, long long batchStride )
 {
@@ -1575,8 +1581,7 @@ static int launchTile( hipStream_t stream, CMatMulArgs& args, int batch, bool ve
 					fixedMeeting->PartialFloats * sizeof( float ), fixedMeeting->CounterCount );
 				return NH_ERR_ARGUMENT;
 			}
-			hipLaunchKernelGGL( clearCountersKernel, dim3( ceilDiv( static_cast<long long>( slicedTiles ), 1024 ) ), dim3( 256 ), 0, stream,
-				fixedMeeting->Counters, static_cast<int>( slicedTiles ) );
+			clearCounters( stream, fixedMeeting->Counters, slicedTiles );
 			args.Partials = fixedMeeting->Partials;
 			args.Counters = fixedMeeting->Counters;
 		} else if( sliceScratch( stream, slicedTiles * slices * 4096, slicedTiles, scratch ) ) {

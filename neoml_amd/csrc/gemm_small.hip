@@ -448,6 +448,9 @@ bool trySmallProduct( hipStream_t stream, const CMatMulArgs& given, bool convolu
 			place = floats <= fixedMeeting->PartialFloats && tiles <= fixedMeeting->CounterCount;
 			args.Partials = fixedMeeting->Partials;
 			args.Counters = fixedMeeting->Counters;
+			if( place ) {
+				clearCounters( stream, args.Counters, tiles );
+			}
 		} else {
 			place = sliceMeetingPlace( stream, floats, tiles, &args.Partials, &args.Counters );
 		}

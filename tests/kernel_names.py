@@ -1,7 +1,7 @@
 """Which kernels the engine's calls launch: a program of its own, so that the profiler it asks stays out of the tests' process.
 
 Standard input: a JSON list of calls, ["nt", batch, m, n, k, pitch of C], ["conv", n, h, w, cin, cout, filter size, padding, stride],
-["conv_backward", ...the same] or ["lstm", steps, batch, width, hidden]. Standard output: a JSON list of lists of the kernels' names."""
+["conv_no_alloc", ...the same], ["conv_backward", ...the same] or ["lstm", steps, batch, width, hidden]. Standard output: a JSON list of lists of the kernels' names."""
 import ctypes
 import json
 import sys
@@ -37,8 +37,8 @@ def main():
         batch, h, w, cin, cout, f, pad, stride = sizes
         d = hip.conv_desc(batch, h, w, cin, cout, f, f, pad, pad, stride, stride)
         x, filt, y = blob(batch, h, w, cin), blob(cout, f, f, cin), blob(batch, d.resultHeight, d.resultWidth, cout)
-        if kind == "conv":
-            return (x, filt, y), lambda: hip.call("nhBlobConvolution", ctypes.byref(d), hip.p(x), hip.p(filt), None, hip.p(y))
+        if kind in ("conv", "conv_no_alloc"):
+            return (x, filt, y), lambda: hip.call("nhBlobConvolution" if kind == "conv" else "nhBlobConvolutionNoAlloc", ctypes.byref(d), hip.p(x), hip.p(filt), None, hip.p(y))
         size = ctypes.c_size_t(0)
         hip.na.check(hip.lib.nhBlobConvolutionBackwardWorkspaceSize(ctypes.byref(d), ctypes.byref(size)))
         work = blob(size.value // 4 + 1)

@@ -109,3 +109,13 @@ def test_no_alloc_convolution_refuses_what_does_not_fit_its_array():
             assert (hip.down(out) == 7.0).all()
     if refused == 0:
         pytest.skip("none of the shapes tried was cut into more slices than the fixed array holds")
+
+
+def test_no_alloc_convolution_clears_its_counters_itself():
+    """The arrival counters of the fixed array are whatever the last call there left, which may have been cut short: every launch whose slices meet
+    there clears them first, that of the kernel for few tiles as that of the larger ones; one without slices has nothing to clear."""
+    few, many, whole = (1, 7, 7, 512, 512, 3, 1, 1), (64, 7, 7, 512, 512, 3, 1, 1), (64, 56, 56, 16, 64, 3, 1, 1)
+    names = nhtest.kernel_names([("conv_no_alloc",) + c for c in (few, many, whole)])
+    assert sorted(n.split("<")[0] for n in names[0]) == ["clearCountersKernel", "smallProductKernel"]
+    assert sorted(n.split("<")[0] for n in names[1]) == ["clearCountersKernel", "matMulKernel"]
+    assert [n.split("<")[0] for n in names[2]] == ["matMulKernel"]
