@@ -691,7 +691,12 @@ static int sumMatrixRowsImpl( nhStream s, int batchSize, float* result, const fl
 			return rc;
 		}
 	}
-	if( slices == 1 && matrixHeight < 256 && batchSize <= 65535 ) {
+	// The rows shared by the lanes of a workgroup, 32 columns ( 8 where they are not read four at a time ) to each: where the columns alone are few,
+	// or where all lanes have a row and four columns to read. us, a thread to a column and shared: 2 x 10^7 24.6 and 116, 16 x 2^20 13.4 and 15.3,
+	// 49 x 65536 6.3 and 3.9, one column at a time 6.4 and 12.7, 16 of 16 x 4096 3.5 and 4.9; 49 x 512 5.9 and 2.0.
+	const bool quads = matrixWidth % 4 == 0 && isAligned16( matrix );
+	const bool shared = base * ( quads ? 1 : 4 ) < 512 || ( quads && matrixHeight >= 32 && matrixWidth <= ( 1 << 28 ) );
+	if( slices == 1 && matrixHeight < 256 && batchSize <= 65535 && shared ) {
 		if( !accumulate && deferRowSums( s, batchSize, result, matrix, matrixHeight, matrixWidth ) ) {
 			return NH_OK;
 		}

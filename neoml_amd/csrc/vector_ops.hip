@@ -1394,9 +1394,12 @@ void sumColumnsTailKernel( float* result, const float* matrix, const float* firs
 // column has its loads one behind the other. So 8 lanes cover a run of 8 V columns and the other 32 share the rows, at most
 // eight loads of a lane in flight, and the lanes' sums meet in LDS. 49 rows of 512 / 1280 / 64 x 512 columns: 5.9 / 5.9 / 6.1 us with a
 // thread to a column, 2.0 / 2.0 / 2.3 us like this; the factor that follows, a launch of 2.0 us, goes along on a deferring stream.
-template<int V>
+// Without a tail the chain is no argument either: its 900 bytes take the host 0.8 us a launch.
+struct CNoTail {};
+template<int V, bool TAIL>
 __global__ __launch_bounds__( 256 )
-void sumShortRowsKernel( float* result, const float* matrix, int height, int width, int accumulate, const CTinyChain tail )
+void sumShortRowsKernel( float* result, const float* matrix, int height, int width, int accumulate,
+	const std::conditional_t<TAIL, CTinyChain, CNoTail> tail )
 {
 	constexpr int Lanes = 32, Columns = 8 * V;
 	__shared__ float meet[Lanes][Columns];
@@ -1433,33 +1436,41 @@ void sumShortRowsKernel( float* result, const float* matrix, int height, int wid
 	if( accumulate ) {
 		s += *out;
 	}
-	const float none = 0.f;
-	for( int k = 0; k < tail.Length; ++k ) {
-		const CTinyOp& op = tail.Ops[k];
-		const float scalar = op.Scalar != nullptr ? *op.Scalar : 0.f;
-		float next = 0.f;
-		CTinyApply<CTinyKinds>::template Run<1>( op.Kind, op, scalar, &s, &none, &none, &next );
-		s = next;
+	if constexpr( TAIL ) {
+		const float none = 0.f;
+		for( int k = 0; k < tail.Length; ++k ) {
+			const CTinyOp& op = tail.Ops[k];
+			const float scalar = op.Scalar != nullptr ? *op.Scalar : 0.f;
+			float next = 0.f;
+			CTinyApply<CTinyKinds>::template Run<1>( op.Kind, op, scalar, &s, &none, &none, &next );
+			s = next;
+		}
 	}
 	*out = s;
 }
 
 static void launchSumShortRows( hipStream_t stream, int batch, float* result, const float* matrix, int height, int width, bool accumulate,
-	const CTinyChain& tail )
+	const CTinyChain* tail )
 {
+	auto launch = [&]( auto valuesOf ) {
+		constexpr int V = decltype( valuesOf )::value;
+		const dim3 grid( ceilDiv( width, 8 * V ), batch );
+		if( tail != nullptr && tail->Length > 0 ) {
+			hipLaunchKernelGGL( ( sumShortRowsKernel<V, true> ), grid, dim3( 256 ), 0, stream, result, matrix, height, width, accumulate ? 1 : 0, *tail );
+		} else {
+			hipLaunchKernelGGL( ( sumShortRowsKernel<V, false> ), grid, dim3( 256 ), 0, stream, result, matrix, height, width, accumulate ? 1 : 0, CNoTail() );
+		}
+	};
 	if( width % 4 == 0 && isAligned16( matrix ) ) {
-		hipLaunchKernelGGL( sumShortRowsKernel<4>, dim3( ceilDiv( width, 32 ), batch ), dim3( 256 ), 0, stream, result, matrix, height, width,
-			accumulate ? 1 : 0, tail );
+		launch( std::integral_constant<int, 4>() );
 	} else {
-		hipLaunchKernelGGL( sumShortRowsKernel<1>, dim3( ceilDiv( width, 8 ), batch ), dim3( 256 ), 0, stream, result, matrix, height, width,
-			accumulate ? 1 : 0, tail );
+		launch( std::integral_constant<int, 1>() );
 	}
 }
 
 int sumShortRows( hipStream_t stream, int batch, float* result, const float* matrix, int height, int width, bool accumulate )
 {
-	const CTinyChain none = {};
-	launchSumShortRows( stream, batch, result, matrix, height, width, accumulate, none );
+	launchSumShortRows( stream, batch, result, matrix, height, width, accumulate, nullptr );
 	NH_LAUNCH_CHECK();
 	return NH_OK;
 }
@@ -1676,7 +1687,7 @@ static void launchColumnSum( hipStream_t stream, const CPendingColumnSum& sum, c
 	const int vec = ( sum.Width % 4 == 0 && isAligned16( sum.Matrix ) && isAligned16( sum.AddFirst ) && isAligned16( sum.AddSecond )
 		&& isAligned16( sum.SquareOf ) ) ? 1 : 0;
 	if( sum.ColumnsOf > 0 ) {
-		launchSumShortRows( stream, sum.ColumnsOf, sum.Result, sum.Matrix, sum.Height, sum.Width, false, tail );
+		launchSumShortRows( stream, sum.ColumnsOf, sum.Result, sum.Matrix, sum.Height, sum.Width, false, &tail );
 	} else if( sum.AddFirst != nullptr ) {
 		hipLaunchKernelGGL( sumColumnsTailKernel<1>, dim3( ceilDiv( sum.Height, 4 ) ), dim3( 256 ), 0, stream, sum.Result, sum.Matrix,
 			sum.AddFirst, sum.AddSecond, const_cast<float*>( sum.Matrix ), sum.Height, sum.Width, vec, tail );

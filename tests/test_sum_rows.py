@@ -35,3 +35,27 @@ def test_sums(streams, batch, height, width, shift):  # noqa: F811
     for tail in tails:
         program = [("nhSumMatrixRows", [batch, at(RESULT), at(m), height, width])] + tail
         assert same_bits(streams.run(streams.plain, program, start), streams.run(streams.deferring, program, start))
+
+
+# on either side of the line between a thread to a column and rows shared by lanes: 511 and 512 runs of 256 columns ( 127 and 128 where they are read one by
+# one ), 31 and 32 rows beyond it; more columns than a launch of 8 or of 32 to a workgroup could have
+@pytest.mark.parametrize("batch,height,width,shift", [
+    (1, 31, 511 * 256, 0), (1, 31, 512 * 256, 0), (1, 32, 512 * 256, 0), (7, 3, 73 * 256, 0), (8, 3, 64 * 256, 0), (1, 40, 127 * 256 - 1, 0), (1, 40, 127 * 256 + 1, 0), (1, 40, 128 * 256, 1),
+    (1, 2, (1 << 27) + 5, 0), (1, 1, (1 << 29) + 4, 0)])
+def test_wide_matrices(streams, batch, height, width, shift):  # noqa: F811
+    torch, lib, na = streams.torch, streams.lib, streams.na
+    g = torch.Generator(device=streams.dev).manual_seed(width)
+    values = torch.rand(batch * height * width + shift, generator=g, device=streams.dev)[shift:].view(batch, height, width)
+    factor = torch.full((1,), 0.5, device=streams.dev)
+    want = sum(values[:, i].double() for i in range(height)) if height < 8 else values.double().sum(dim=1)
+    results = []
+    for stream in (streams.plain, streams.deferring):
+        out = torch.full((batch, width), 7.0, device=streams.dev)
+        torch.cuda.synchronize()
+        na.check(lib.nhSumMatrixRows(stream, batch, ctypes.c_void_p(out.data_ptr()), ctypes.c_void_p(values.data_ptr()), height, width))
+        na.check(lib.nhVectorMultiply(stream, ctypes.c_void_p(out.data_ptr()), ctypes.c_void_p(out.data_ptr()), batch * width, ctypes.c_void_p(factor.data_ptr())))
+        na.check(lib.nhStreamSynchronize(stream))
+        # ( sums of values between 0 and 1, halved )
+        assert ((out.double() - want * 0.5).abs() <= (height + 2) * 2.0 ** -24 * want + 1e-30).all()
+        results.append(out)
+    assert torch.equal(results[0].view(torch.int32), results[1].view(torch.int32))
