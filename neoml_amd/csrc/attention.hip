@@ -209,13 +209,14 @@ void attentionKernel( const CAttentionArgs args )
 }
 
 constexpr int MaxAttentionColumns = 512;
+constexpr long long MaxWorkgroups = ( 1 << 24 ) - 1; // a launch has fewer than 2^32 threads
 
 // Whether it takes the core of this layer. Scores of more than 256 columns only where the kernel for batches of products does not
 // have enough strips of 64 rows to take the two products by itself.
 bool attentionTakes( int batch, int M, int N, int K, int D, const float* q )
 {
 	return batch > 0 && M > 0 && N > 0 && N <= MaxAttentionColumns && K > 0 && K <= 64 && K % 16 == 0 && D > 0 && D <= 64 && isAligned16( q )
-		&& ( N <= 256 || static_cast<long long>( ceilDiv( M, 64 ) ) * batch < 512 ) && static_cast<long long>( ceilDiv( M, 16 ) ) * batch <= 0x7ffffff0LL;
+		&& ( N <= 256 || static_cast<long long>( ceilDiv( M, 64 ) ) * batch < 512 ) && static_cast<long long>( ceilDiv( M, 16 ) ) * batch <= MaxWorkgroups;
 }
 
 int launchAttention( hipStream_t stream, const CPendingAttention& a )

@@ -2778,7 +2778,7 @@ static bool tryBatchedStrips( hipStream_t stream, const CMatMulArgs& args, int b
 	constexpr int KS = 32;
 	const int tilesM = ceilDiv( args.M, 64 );
 	const long long groups = static_cast<long long>( tilesM ) * batch;
-	if( groups < 512 || groups > 0x7fffffffLL ) {
+	if( groups < 512 || groups >= ( 1 << 24 ) ) { // ( a launch has fewer than 2^32 threads )
 		return false;
 	}
 	hipLaunchKernelGGL( ( batchedStripKernel<1, KS> ), dim3( static_cast<unsigned>( groups ) ), dim3( Threads ), 0, stream,

@@ -113,3 +113,20 @@ def test_other_sequences(streams):
         plain, deferred = (layer.run(s, program) for s in (streams.plain, streams.deferring))
         for blob in plain:
             assert streams.torch.allclose(plain[blob], deferred[blob], rtol=1e-4, atol=1e-5, equal_nan=True), (what, blob)
+
+
+# as many strips as a launch has workgroups for, and one more, which goes out as separate launches: fewer than 2^32 threads to a launch
+@pytest.mark.parametrize("batch", [(1 << 24) - 1, 1 << 24])
+def test_the_most_workgroups(streams, batch):
+    torch = streams.torch
+    layer = Layer(streams, batch, 1, 1, 4, 16, 1)
+    got = layer.run(streams.deferring, layer.calls()[1])
+    at = torch.cat([torch.arange(1000, device=streams.dev), torch.arange(batch - 1000, batch, device=streams.dev)])
+    scores = layer.q[at].double() @ layer.kt[at].double().contiguous() * 0.125
+    weights = torch.softmax(scores, -1)
+    context = weights @ layer.v[at].double()
+    # ( 16 products of normal values, their sum of sizes below 100, times 0.125: 20 * 2^-24 * 12.5; weights below one, twice that relatively )
+    for name, want in (("scores", scores), ("weights", weights), ("context", context), ("out", context)):
+        found = got[name][:batch * want[0].numel()].view(batch, -1)[at].double()
+        assert torch.allclose(found, want.reshape(found.shape), rtol=0, atol=1e-4), name
+        assert not (got[name][:batch * want[0].numel()] == 7.0).any() and (got[name][batch * want[0].numel():] == 7.0).all()
