@@ -43,16 +43,13 @@ namespace nh {
 // over one half of the K steps of the tile, then the second group hands its accumulators to the first through LDS.
 // For problems of a few hundred tiles with a reduction long enough to cut in two: the same number of waves per compute
 // unit as two K slices in separate workgroups, without the preset of C, the atomics and the separate activation pass.
-// Wavefronts to a SIMD that the kernels of matMulTile are compiled for, at least and at most. How many workgroups a compute unit takes at once
-// decides how whole the last round of a launch is, and launchTile cuts K by it. The two modes that run the large products and 3x3
-// convolutions have room for eight ( 64 registers ). With 90, five, launches of five to eight workgroups a compute unit are uneven: us with five
-// and eight, 2880 x 256 x 1152 in 4 slices 47.6 and 43.5, 5672 x 256 x 2304 in 5 58.8 and 53, 1421 x 512 x 4608 in 8 63.6 and 57; with seven
-// 2048 workgroups of a 2304-long reduction take 298 instead of 270. The operands from columns ( the gradient by a filter above all, whose slices
-// were fitted to five ) stay at five: with seven the gradients of 57 x 13 x 14 x 256 take 3 % longer.
+// Wavefronts to a SIMD that the kernels of matMulTile are compiled for, at least. How many workgroups a compute unit takes at once decides how
+// whole the last round of a launch is, and launchTile cuts K by it. The two modes that run the large products and 3x3 convolutions have room for
+// eight ( 64 registers ). With 90, five, launches of five to eight workgroups a compute unit are uneven: us with five and eight, 2880 x 256 x 1152
+// in 4 slices 47.6 and 43.5, 5672 x 256 x 2304 in 5 58.8 and 53, 1421 x 512 x 4608 in 8 63.6 and 57; with seven 2048 workgroups of a 2304-long
+// reduction take 298 instead of 270.
 template<int BM, int AMODE, int BMODE>
 constexpr int leastWaves() { return BM == 64 && BMODE == BM_RowsK && ( AMODE == AM_RowsK || AMODE == AM_ConvTaps ) ? 8 : 2; }
-template<int BMODE>
-constexpr int mostWaves() { return BMODE == BM_RowsK ? 8 : 5; }
 
 // RESIDUAL: the launch adds one ( a kernel of its own, below: its epilogue would cost the others registers )
 template<int BM, int BN, int WAVES_M, int WAVES_N, int AMODE, int BMODE, bool VEC, int KGROUPS, bool RESIDUAL>
@@ -1072,14 +1069,14 @@ __device__ __forceinline__ void matMulTile( const CMatMulArgs& launchArgs )
 }
 
 template<int BM, int BN, int WAVES_M, int WAVES_N, int AMODE, int BMODE, bool VEC, int KGROUPS = 1>
-__global__ __launch_bounds__( Threads * KGROUPS ) __attribute__(( amdgpu_waves_per_eu( ( leastWaves<BM, AMODE, BMODE>() ), ( mostWaves<BMODE>() ) ) ))
+__global__ __launch_bounds__( Threads * KGROUPS, ( leastWaves<BM, AMODE, BMODE>() ) )
 void matMulKernel( const CMatMulArgs args )
 {
 	matMulTile<BM, BN, WAVES_M, WAVES_N, AMODE, BMODE, VEC, KGROUPS, false>( args );
 }
 
 template<int BM, int BN, int WAVES_M, int WAVES_N, int AMODE, int BMODE, bool VEC, int KGROUPS = 1>
-__global__ __launch_bounds__( Threads * KGROUPS ) __attribute__(( amdgpu_waves_per_eu( ( leastWaves<BM, AMODE, BMODE>() ), ( mostWaves<BMODE>() ) ) ))
+__global__ __launch_bounds__( Threads * KGROUPS, ( leastWaves<BM, AMODE, BMODE>() ) )
 void matMulResidualKernel( const CMatMulArgs args )
 {
 	matMulTile<BM, BN, WAVES_M, WAVES_N, AMODE, BMODE, VEC, KGROUPS, true>( args );
