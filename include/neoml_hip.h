@@ -449,27 +449,41 @@ NH_API int nhStreamOverlapLstm(nhStream s, int enable);
  * nhStreamDestroy, enable = 0, or a release of device memory (nhRawFree, a pool's clean-up). Until then their results are
  * not in memory and their operands must stay valid, so this is only for streams whose work, synchronisation included,
  * all goes through this library (an engine's own stream): synchronise with nhStreamSynchronize, not with HIP calls of
- * your own. Nothing is put aside while the stream is being captured into a graph (synchronise through the library
- * before a capture begins: what was put aside before it would otherwise become the graph's first launch). What it
+ * your own. Nothing is put aside, and no call joins what waits, while the stream is being captured into a graph (synchronise through
+ * the library before a capture begins: what was put aside before it would otherwise become the graph's first launch). What it
  * saves: a row-normalising
  * layer (CObjectNormalizationLayer) asks for five such calls per run, each a launch of about 4 us.
- * On such a stream nhMultiplyMatrixByTransposedMatrix with a dense result (resultRowSize == secondHeight) waits for the
- * call behind it as well: nhAddVectorToMatrixRows over that result in place (batchSize 1, the same height and width) is
- * then part of the product's launch, the vector added to the accumulators on their way out, as the fully connected
- * layer's two calls ask (NeoML/src/Dnn/Layers/FullyConnectedLayer.cpp:91-99); any other call launches the product first,
- * as it was asked for. The sum is the same; where the product is cut into slices of its reduction the vector is added
- * in front of the slices instead of behind them, i.e. the last bits may differ from the two launches'.
- * In the same way nhBlobConvolution and nhBlobChannelwiseConvolution wait for an nhVectorReLU or nhVectorHSwish over
- * their result in place
- * (CConvLayer / CChannelwiseConvLayer followed by CReLULayer: the activation runs on the accumulators' way out, its
- * threshold read from the device scalar), and an nhVectorAdd over more than 262144 elements waits for an nhVectorReLU
- * over the sum in place (CEltwiseSumLayer + CReLULayer at the end of a residual block: one pass), and
- * nhBatchMultiplyMatrixByMatrix with a reduction of at most 256 waits for an nhVectorMultiply over its whole result in
- * place (CMatrixMultiplicationLayer + CLinearLayer: an attention layer's scores and their factor), and nhBlobResizeImage
- * with constant padding waits for an nhBlobMaxPooling (3x3, no indices) over the padded blob (CImageResizeLayer +
- * CMaxPoolingLayer: one launch writes both blobs), and nhSumMatrixColumns waits for the element-wise calls with one
- * operand in place over its sums (the mean and the inverse deviation of CObjectNormalizationLayer: the reduction's launch
- * applies them to each row's value). Same bits as the separate launches. */
+ * On such a stream larger calls wait too, each for the calls that NeoML's layers ask for behind it; what was asked for by then goes
+ * out as one launch, any other call sends it out first, as it was asked for, and blobs that overlap in a way that one launch
+ * would not keep are launched one by one:
+ * - nhMultiplyMatrixByTransposedMatrix with a dense result (resultRowSize == secondHeight): nhAddVectorToMatrixRows over that
+ *   result in place (batchSize 1, the same height and width; CFullyConnectedLayer,
+ *   NeoML/src/Dnn/Layers/FullyConnectedLayer.cpp:91-99), then either the three calls of CGELULayer's sigmoid form over it
+ *   (nhVectorMultiply into another blob, nhVectorSigmoid there, nhVectorEltwiseMultiply back; the gates are stored too) or, for
+ *   small results, up to two further products of the same first matrix with their free terms (queries, keys, values). The free
+ *   term is added to the accumulators on their way out: where the product is cut into slices of its reduction that is
+ *   in front of the slices instead of behind them, i.e. the last bits may differ from the separate launches'.
+ * - nhBlobConvolution and nhBlobChannelwiseConvolution: nhVectorReLU or nhVectorHSwish over their result in place (CConvLayer /
+ *   CChannelwiseConvLayer followed by CReLULayer; the threshold is read from the device scalar). nhBlobConvolution with a
+ *   channel count that is a multiple of 4 also: nhVectorAdd of another blob over its result in place (CEltwiseSumLayer at the end of a
+ *   residual block), directly or behind a second nhBlobConvolution that writes the other summand (the shortcut), then the activation.
+ * - nhVectorAdd over more than 262144 elements: nhVectorReLU over the sum in place.
+ * - nhBatchMultiplyMatrixByMatrix with a reduction of at most 256: nhVectorMultiply over its whole result in place by a
+ *   device scalar (an attention layer's scores and their factor), and, with reductions that are a multiple of 16 up to 64 and
+ *   up to 512 columns, nhMatrixSoftmaxByRows into another blob, nhBatchMultiplyMatrixByMatrix of that and the values (at most 64
+ *   columns) and nhTransposeMatrix of its result (heads and rows exchanged): the core of CMultiheadAttentionLayer. Scores, weights and
+ *   context are stored as by the separate launches.
+ * - nhTransposeMatrix of at most 65536 values: up to three more of them.
+ * - nhBlobResizeImage with constant padding: nhBlobMaxPooling (3x3, no indices) over the padded blob (CImageResizeLayer +
+ *   CMaxPoolingLayer: one launch writes both blobs).
+ * - nhSumMatrixColumns, and nhSumMatrixRows over fewer than 256 rows: the element-wise calls with one operand in place over the sums.
+ *   Two such sums of columns with their calls and the four calls over the matrix behind them, CObjectNormalizationLayer with rows of
+ *   at most 2048 elements, are one pass, with the sum of two blobs in front of them if there is one.
+ * Same bits as the separate launches but for the free term as said, and for the attention core, whose products are summed up in
+ * another order. A launch that needs scratch memory takes it from the stream's pool (nhStreamBindPool). Operands may have been
+ * given back to a pool by then (nhPoolHeapFree behind the call that names them): inside such a launch a pool gives only new memory
+ * within its limit, never a cached block, and releases none; what it refuses is asked for again with the next product or convolution, and
+ * the launch does without. */
 NH_API int nhStreamDeferSmallOps(nhStream s, int enable);
 /* LSTM (NME.h:1005-1011). Weights: inputWeights [4H x objectSize], recurrentWeights [4H x H]; gate order in
  * the 4H vector: main(tanh) | forget | input | output (src/CPU/CpuMathEngineDnnLstm.h:49-90).

@@ -44,8 +44,8 @@ void flushAllTinyOps();
 void finishHeldCalls();
 void releaseTinyQueue( hipStream_t stream );
 // On such a stream a product A * B^T with a dense result may wait for the call behind it ( deferProduct: true, nothing
-// launched ); an AddVectorToMatrixRows over that result in place then launches both as one ( fusePendingProduct: true,
-// *rc is the launch's code ), any other call sends the product out first, through toStream.
+// launched ); an AddVectorToMatrixRows over that result in place waits on with it ( fusePendingProduct: true ), for the calls of a GELU or
+// for a further product of the same A; any other call sends the product out first, through toStream.
 bool deferProduct( nhStream s, const float* a, int lda, const float* b, int ldb, float* c, int ldc, int M, int N, int K );
 bool fusePendingProduct( nhStream s, const float* matrix, float* result, int height, int width, const float* vector, int* rc );
 // An element-wise call over a height x width matrix whose second operand is a vector spread over the rows or the columns

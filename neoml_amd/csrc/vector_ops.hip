@@ -775,7 +775,8 @@ __global__ __launch_bounds__( QuadThreads ) void quadChainKernel( const CTinyCha
 // product's rows in place, a pass over the whole result for one add per element. On a stream that puts small calls aside
 // the product is put aside too ( nothing else is pending then ), and if the next call is that AddVectorToMatrixRows, both
 // go out as the one launch the product's kernels have for it ( the free term added to the accumulators on their way
-// out ); any other call launches the product as it was asked for, first.
+// out ), once the call behind them is neither the first of a GELU over the result ( parkProduct ) nor a product of the same A; any other
+// call launches the product as it was asked for, first.
 struct CPendingProduct {
 	bool Pending = false;
 	const float* A = nullptr;
@@ -1701,7 +1702,7 @@ static void launchColumnSum( hipStream_t stream, const CPendingColumnSum& sum, c
 	}
 }
 
-// what the queue holds: the product that waits for its successor ( then nothing else is queued ), or a chain
+// what the queue holds: what is parked, then the launch that waits for its successor, or a chain
 static bool launchPending( hipStream_t stream, CTinyQueue& queue )
 {
 	const CHeldLaunch held;
