@@ -7,11 +7,11 @@
 // Results may alias an input exactly (in-place layers): every element is read before it is written by the
 // same thread, so no __restrict__ is put on the pointers.
 #include "common.h"
+#include "launch_gate.h"
 #include <float.h>
 #include <map>
 #include <mutex>
 #include <optional>
-#include <shared_mutex>
 #include <stddef.h>
 #include <type_traits>
 #include <utility>
@@ -940,18 +940,27 @@ typedef std::map<std::pair<int, hipStream_t>, CTinyQueue> CTinyQueues;
 // ( recursive: what is launched from under the lock may turn a stream handle into a stream, which looks for calls to launch )
 static std::recursive_mutex tinyLock;
 static thread_local int heldLaunches = 0;
-// held by the threads that have taken calls out of a queue and not launched them all yet
-static std::shared_mutex heldLaunchLock;
+// inside: the threads that have taken calls out of a queue and not launched them all yet
+static CLaunchGate& heldLaunchGate()
+{
+	static CLaunchGate* gate = new CLaunchGate; // ( never destroyed, as the queues )
+	return *gate;
+}
+static CLaunchGate::CThread& heldLaunchThread()
+{
+	static thread_local CLaunchGate::CThread thread( heldLaunchGate() );
+	return thread;
+}
 CHeldLaunch::CHeldLaunch()
 {
 	if( heldLaunches++ == 0 ) {
-		heldLaunchLock.lock_shared();
+		heldLaunchThread().Enter();
 	}
 }
 CHeldLaunch::~CHeldLaunch()
 {
 	if( --heldLaunches == 0 ) {
-		heldLaunchLock.unlock_shared();
+		heldLaunchThread().Leave();
 	}
 }
 bool launchingHeldCalls() { return heldLaunches != 0; }
@@ -1830,8 +1839,7 @@ void finishHeldCalls()
 {
 	flushAllTinyOps();
 	if( !launchingHeldCalls() ) {
-		heldLaunchLock.lock();
-		heldLaunchLock.unlock();
+		heldLaunchGate().WaitForThoseInside();
 	}
 }
 
