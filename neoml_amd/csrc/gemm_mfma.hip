@@ -1622,6 +1622,16 @@ static int launchTile( hipStream_t stream, CMatMulArgs& args, int batch, bool ve
 	// blockIdx.y is limited to 65535: walk larger batches in slices
 	for( int b0 = 0; b0 < batch; b0 += 65535 ) {
 		const int nb = batch - b0 < 65535 ? batch - b0 : 65535;
+		// A little more than the eight workgroups of every compute unit would be one round, in which all end at about the same time, and a
+		// second one with most of the unit idle. With six at once two rounds are even: us with eight and six, 2136 workgroups of 48 steps
+		// 118 and 109, 2176 of 72 177 and 158, 2292 of 144 346 and 314, 2352 of 48 126 and 120, 2560 of 36 102 and 95, 2496 of 72 199 and 176;
+		// of 12 such launches between 2048 and 3072 none lost more than 1 %. From there on six would be three rounds ( 3136 of 36 steps 119.5 and
+		// 121.3 ); up to 2048 eight are one ( 2048 of 36 77 and 84 ); the uneven ones with tail tiles gain 10 % here and lose 6 there. Launches of less than
+		// four steps are bound by memory and want all eight ( 11464 x 1024 x 16 11.1 and 12.2, x 24 some 3 %; x 48 and x 64 even, x 96 28.3 and 26.7 ).
+		const long long workgroups = gridX * nb * args.SplitK;
+		const bool sixAtOnce = leastWaves<BM, AMODE, BMODE>() == 8 && !twoGroups && args.FullTiles == 0 && args.StepsPerSplit >= 4 && workgroups > 8 * 256
+			&& workgroups <= 12 * 256;
+		const unsigned moreLds = sixAtOnce ? 4096 : 0; // with the 20 KB of a workgroup, of the 160 KB of a compute unit
 		CMatMulArgs a = args;
 		a.A += b0 * args.BatchStrideA;
 		a.B += b0 * args.BatchStrideB;
@@ -1632,11 +1642,11 @@ static int launchTile( hipStream_t stream, CMatMulArgs& args, int batch, bool ve
 			constexpr int Groups = decltype( groupsOf )::value;
 			if constexpr( TakesResidual ) {
 				if( args.Residual != nullptr ) {
-					hipLaunchKernelGGL( ( matMulResidualKernel<BM, BN, WAVES_M, WAVES_N, AMODE, BMODE, Vec, Groups> ), grid, dim3( Threads * Groups ), 0, stream, a );
+					hipLaunchKernelGGL( ( matMulResidualKernel<BM, BN, WAVES_M, WAVES_N, AMODE, BMODE, Vec, Groups> ), grid, dim3( Threads * Groups ), moreLds, stream, a );
 					return;
 				}
 			}
-			hipLaunchKernelGGL( ( matMulKernel<BM, BN, WAVES_M, WAVES_N, AMODE, BMODE, Vec, Groups> ), grid, dim3( Threads * Groups ), 0, stream, a );
+			hipLaunchKernelGGL( ( matMulKernel<BM, BN, WAVES_M, WAVES_N, AMODE, BMODE, Vec, Groups> ), grid, dim3( Threads * Groups ), moreLds, stream, a );
 		};
 		if( twoGroups ) {
 			if constexpr( BM == 64 && BN == 64 && BMODE == BM_RowsK && ( AMODE == AM_Conv || AMODE == AM_ConvTaps || AMODE == AM_RowsK ) ) {
